@@ -298,29 +298,59 @@ __global__ __launch_bounds__(256) void k_dense_scatter(const K *__restrict__ key
     }
 }
 
-// 65536-bin histogram of 16-bit symbols.  Lanes holding the same symbol are
-// grouped with a ballot peer mask, so each distinct symbol of a wave costs one global
-// atomic.  In GSA mode it also counts the invalid positions (a 0 first, or two
-// adjacent 0s).
-__global__ __launch_bounds__(256) void k_hist16(const uint16_t *__restrict__ T, u64 n, int gsa, u64 *__restrict__ hist,
-                                                u32 *__restrict__ bad)
+// Dense ranks of an integer alphabet through a table of its values: table[v] = 1 where
+// value v occurs, an exclusive scan turns that into v's rank, and a gather replaces
+// the symbols.  The flag is read before it is written: in Zipf-like texts most symbols
+// find it set, and the few hot words would otherwise take every write.
+template <typename ST>
+__global__ __launch_bounds__(256) void k_mark_values(const ST *__restrict__ T, u64 n, u32 *__restrict__ table)
 {
     const u64 stride = (u64)gridDim.x * blockDim.x;
-    const u64 lane = lane_id();
+    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        u32 *f = table + (u32)T[i];
+        if (!*f) *f = 1u;
+    }
+}
+
+template <typename ST>
+__global__ __launch_bounds__(256) void k_value_ranks(const ST *__restrict__ T, u64 n, const u32 *__restrict__ table,
+                                                     u32 *__restrict__ S)
+{
+    const u64 stride = (u64)gridDim.x * blockDim.x;
+    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) S[i] = table[(u32)T[i]];
+}
+
+// 65536-bin histogram of 16-bit symbols.  Each workgroup counts stretches of at most
+// H16_TILE symbols in LDS, two 16-bit counters per word (H16_TILE < 65536, so a half
+// never carries), and adds the bins it met to the global table: a symbol of a
+// Zipf-like text costs one LDS atomic instead of a global one on a few hot addresses
+// (4 M token ids: 790 us with one global atomic per distinct symbol of a wave step).
+// 128 KB of counters are one workgroup per CU, so it has 1024 threads.  In GSA mode it
+// also counts the invalid positions (a 0 first, or two adjacent 0s).
+constexpr u32 H16_TILE = 16384, H16_THREADS = 1024;
+
+__global__ __launch_bounds__(H16_THREADS) void k_hist16(const uint16_t *__restrict__ T, u64 n, u64 span, int gsa,
+                                                        u64 *__restrict__ hist, u32 *__restrict__ bad)
+{
+    __shared__ u32 s_h[32768];
     u32 nbad = 0;
-    for (u64 base = (u64)blockIdx.x * blockDim.x + threadIdx.x - lane; base < n; base += stride) {
-        const u64 i = base + lane;
-        const bool ok = i < n;
-        const u32 v = ok ? T[i] : 0u;
-        if (gsa && ok && v == 0 && (i == 0 || T[i - 1] == 0)) nbad++;
-        u64 m = __ballot(ok);
-#pragma unroll
-        for (int b = 0; b < 16; b++) {
-            const bool bit = (v >> b) & 1u;
-            const u64 bb = __ballot(bit);
-            m &= bit ? bb : ~bb;
+    const u64 lo = (u64)blockIdx.x * span, hi = lo + span < n ? lo + span : n;
+    for (u64 base = lo; base < hi; base += H16_TILE) {
+        for (u32 b = threadIdx.x; b < 32768; b += H16_THREADS) s_h[b] = 0;
+        __syncthreads();
+        const u64 end = base + H16_TILE < hi ? base + H16_TILE : hi;
+        for (u64 i = base + threadIdx.x; i < end; i += H16_THREADS) {
+            const u32 v = T[i];
+            if (gsa && v == 0 && (i == 0 || T[i - 1] == 0)) nbad++;
+            atomicAdd(&s_h[v >> 1], 1u << (16 * (v & 1)));
         }
-        if (ok && __popcll(m & lanemask_lt()) == 0) atomicAdd((unsigned long long *)&hist[v], (unsigned long long)__popcll(m));
+        __syncthreads();
+        for (u32 b = threadIdx.x; b < 32768; b += H16_THREADS) {
+            const u32 x = s_h[b];
+            if (x & 0xFFFFu) atomicAdd((unsigned long long *)&hist[2 * b], (unsigned long long)(x & 0xFFFFu));
+            if (x >> 16) atomicAdd((unsigned long long *)&hist[2 * b + 1], (unsigned long long)(x >> 16));
+        }
+        __syncthreads();
     }
     if (gsa && nbad) atomicAdd(bad, nbad);
 }
@@ -367,8 +397,11 @@ int launch_pack_keys32(const uint8_t *T, u64 n, const uint8_t *lut, int bits, in
 
 int launch_hist16(const uint16_t *T, u64 n, int gsa, u64 *hist65536, u32 *bad, hipStream_t s)
 {
-    // the loop steps a whole wave at a time, so the grid is a multiple of 64 threads
-    hipLaunchKernelGGL(k_hist16, dim3(grid_for(n, 256 * 16, 4096)), dim3(256), 0, s, T, n, gsa, hist65536, bad);
+    // whole tiles per workgroup, at most 1024 workgroups (four rounds over the 256 CUs)
+    const u64 tiles = (n + H16_TILE - 1) / H16_TILE;
+    const u64 per = (tiles + 1023) / 1024;
+    hipLaunchKernelGGL(k_hist16, dim3(ceil_div_u(tiles, per)), dim3(H16_THREADS), 0, s, T, n, per * H16_TILE, gsa,
+                       hist65536, bad);
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
