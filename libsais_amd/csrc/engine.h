@@ -395,6 +395,10 @@ int launch_hist16(const uint16_t *T, u64 n, int gsa, u64 *hist65536, u32 *bad, h
 int launch_map16(const uint16_t *T, u64 n, const u32 *lut, u32 *S, hipStream_t s);
 int launch_max_sym(const void *T, int width, u64 n, u64 *out, hipStream_t s);
 int launch_sym_narrow(const void *T, int width, u64 n, u32 *S, hipStream_t s);
+// table[v] = 1 for every value v of T (the table is zeroed by the caller); S[i] =
+// table[T[i]] (the values' ranks once the table is scanned).
+int launch_mark_values(const void *T, int width, u64 n, u32 *table, hipStream_t s);
+int launch_value_ranks(const void *T, int width, u64 n, const u32 *table, u32 *S, hipStream_t s);
 int launch_sym_keys64(const void *T, int width, u64 n, u64 *keys, u32 *vals, hipStream_t s);
 int launch_run_flags64(const u64 *keys, u64 n, u32 *flags, hipStream_t s);
 int launch_dense_scatter64(const u64 *keys, const u32 *vals, const u32 *excl, u64 n, u32 *S, hipStream_t s);

@@ -1732,6 +1732,22 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_sa_int(const void *T, void *SA, int64
         if (maxv < (1ull << 16)) {
             SAGPU_TRY(launch_sym_narrow(dTin, width, N, dSym, s));
             bits = maxv ? bits_for(maxv) : 1;
+        } else if (maxv < 4 * N && maxv < (1ull << 31)) {
+            // Values below 4 N: ranks from a table of the values.  Its 4 passes (zeroed,
+            // marked, scanned, gathered) move at most as many bytes as one pass of the
+            // sort below, which takes 3 passes or more for values of 17 bits and up (6 M
+            // token ids below 100,000: 0.06 ms against 0.36 ms)
+            const u64 slots = maxv + 1, pcap = slots / 4096 + 2;
+            u32 *table = in.get<u32>(slots + 1), *part = in.get<u32>(pcap);
+            if (!table || !part) return SAGPU_ENOMEM;
+            SAGPU_TRY(launch_fill_u32(table, slots + 1, 0, s));
+            SAGPU_TRY(launch_mark_values(dTin, width, N, table, s));
+            ScanScratch ssc{part, pcap};
+            SAGPU_TRY(scan_exclusive_u32(ssc, table, slots + 1, s));
+            SAGPU_TRY(launch_value_ranks(dTin, width, N, table, dSym, s));
+            u32 distinct = 0;
+            SAGPU_TRY(read_u32(*c, table + slots, &distinct));
+            bits = distinct > 1 ? bits_for((u64)distinct - 1) : 1;
         } else {
             u64 *k0 = in.get<u64>(N), *k1 = in.get<u64>(N);
             u32 *v0 = in.get<u32>(N), *v1 = in.get<u32>(N), *flags = in.get<u32>(N);

@@ -37,3 +37,20 @@ def test_hist16(n):
         T[:] = 40001
         SA, f = _freq16(T)
         assert f[40001] == n and f.sum() == n and np.array_equal(SA, np.arange(n)[::-1])
+
+
+@pytest.mark.parametrize("n", [2, 5, 20001])
+@pytest.mark.parametrize("wide", [False, True])
+def test_int_value_table(n, wide):
+    """Alphabets ranked through a table of the values (largest value below 4 n) and, one
+    above, through the sort; both from the first value past 16 bits on."""
+    for largest in (65536, 4 * n - 1, 4 * n):
+        print(f"[int table] n={n} largest={largest} wide={wide}", flush=True)
+        rng = np.random.default_rng(largest)
+        T = rng.integers(0, max(2, largest // 3), n).astype(np.int64 if wide else np.int32)
+        T[0], T[n // 2] = largest, largest
+        ref = ol.sa_int(T)
+        SA = np.zeros(n, T.dtype)
+        f = la.libsais64_long if wide else la.libsais_int
+        assert f(T, SA, n, largest + 1, 0) == 0, la.last_error()
+        assert np.array_equal(SA, ref)
