@@ -371,16 +371,30 @@ int launch_lcp_fix(const u32 *PLCP, const u32 *SA, u64 n, u32 *LCP, hipStream_t 
 int launch_aux_samples(const u32 *ISA, u64 n, u64 r, u64 count, u32 *out, hipStream_t s);
 u64 unbwt_count_slots(u64 n);
 int launch_unbwt_succ(const uint8_t *U, u64 n, u64 p, u32 *counts, ScanScratch &sc, u32 *S, hipStream_t s);
+// scanned: the scanned counts launch_unbwt_succ leaves (byte symbols; unused for 16 bits).
 int launch_unbwt_aux_walk(const void *U, int sym_bytes, const u32 *S, u64 n, u64 p, u64 r, const u64 *rows,
-                          u64 chunks, void *out, u32 *err, hipStream_t s);
+                          u64 chunks, const u32 *scanned, void *out, u32 *err, hipStream_t s);
+// Samples of the list-ranking inverse BWT: m of them, one in `gap` of 2^k numbers (2^k
+// is the power of two at or above n).  More samples shorten the walks (the longest
+// of m geometric gaps is about gap ln m dependent reads of 0.4-0.7 us) and lengthen the
+// pointer jumping (log2 m rounds over m words, launch-bound below about 2^18).  32 MiB of
+// text, gap 64: walk 0.91 ms, 21 jumps of 7 us, copy 0.12 ms; before (gap 256, the text
+// walked twice) 1.27, 18 jumps of 5 us and 2.40 ms.
+struct UbPlan {
+    int k;
+    u32 m, gap;
+    u32 pages, segs;   // pages for long gaps, and the counters they are taken from
+};
+UbPlan unbwt_plan(u64 n);
 // 16-bit symbols: sort keys for the stable rank, then the successor array from the
 // sorted positions.
 int launch_unbwt_succ16(const uint16_t *U, u64 n, u64 p, u32 *keys, u32 *vals, u32 *S, hipStream_t s);
 int launch_unbwt_succ_sorted(const u32 *V, u64 n, u64 p, u32 *S, hipStream_t s);
-int launch_unbwt_flags(u64 n, u32 *flags, hipStream_t s);
-int launch_unbwt_sample_total(const u32 *sid, u64 n, u32 *out, hipStream_t s);
-int launch_unbwt_rank(const void *U, int sym_bytes, const u32 *S, const u32 *sid, u64 n, u32 m, u32 *samp_q,
-                      u32 *nxt[2], u64 *dist[2], u64 *gap, void *out, u32 *err, hipStream_t s);
+// nd: 3 arrays of m words; buf: (m + pages) * cap symbols (cap a multiple of 8); link:
+// m + pages words; more: m words; used: segs words.
+int launch_unbwt_rank(const void *U, int sym_bytes, const u32 *S, u64 n, u64 p, const UbPlan &pl, u32 cap,
+                      const u32 *scanned, u64 *const nd[3], void *buf, u32 *link, u32 *more, u32 *used, void *out,
+                      u32 *err, hipStream_t s);
 int launch_lcp(const u32 *PLCP, const u32 *SA, u64 n, u32 *LCP, hipStream_t s);
 
 // Tiny fill kernel (graph-capture safe replacement for hipMemsetAsync).

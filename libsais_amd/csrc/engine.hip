@@ -1862,10 +1862,11 @@ int unbwt_host(Ctx &c, const void *T, void *U, u64 N, u64 r, const void *I, int 
     SAGPU_TRY(h2d(c, dB, T, bytes));
     SAGPU_CHECK(hipMemsetAsync(dOut, 0, bytes, s));
     SAGPU_TRY(launch_fill_u32(d_err, 2, 0, s));
-    const u64 pcap = N / 4096 + 2;
+    u32 *counts = nullptr;   // scanned byte counts: the walks decode symbols from them
     if (sym_bytes == 1) {
         const u64 slots = unbwt_count_slots(N);
-        GET(counts, u32, slots);
+        counts = sc.get<u32>(slots);
+        if (!counts) return SAGPU_ENOMEM;
         const u64 scap = slots / 4096 + 2;
         GET(part, u32, scap);
         ScanScratch ssc{part, scap};
@@ -1885,29 +1886,29 @@ int unbwt_host(Ctx &c, const void *T, void *U, u64 N, u64 r, const void *I, int 
     if (r < N && chunks >= 32768) {
         GET(d_rows, u64, chunks);
         SAGPU_CHECK(hipMemcpyAsync(d_rows, rows.data(), chunks * 8, hipMemcpyHostToDevice, s));
-        SAGPU_TRY(launch_unbwt_aux_walk(dB, sym_bytes, S, N, rows[0], r, d_rows, chunks, dOut, d_err, s));
+        SAGPU_TRY(launch_unbwt_aux_walk(dB, sym_bytes, S, N, rows[0], r, d_rows, chunks, counts, dOut, d_err, s));
     } else {
-        GET(part, u32, pcap);
-        ScanScratch ssc{part, pcap};
-        GET(sid, u32, N);
-        SAGPU_TRY(launch_unbwt_flags(N, sid, s));
-        SAGPU_TRY(scan_exclusive_u32(ssc, sid, N, s));
-        SAGPU_TRY(launch_unbwt_sample_total(sid, N, d_err + 1, s));
-        u32 m = 0;
-        SAGPU_TRY(read_u32(c, d_err + 1, &m));
-        if (m == 0 || m > N) {
-            sagpu_set_error("inverse BWT: sample count inconsistent", __FILE__, __LINE__);
-            return SAGPU_EDEVICE;
+        const UbPlan pl = unbwt_plan(N);
+        u64 *nd[3];
+        for (auto &q : nd) {
+            q = sc.get<u64>(pl.m);
+            if (!q) return SAGPU_ENOMEM;
         }
-        GET(samp_q, u32, m);
-        GET(nxt0, u32, m);
-        GET(nxt1, u32, m);
-        GET(dist0, u64, m);
-        GET(dist1, u64, m);
-        GET(gap, u64, m);
-        u32 *nxt[2] = {nxt0, nxt1};
-        u64 *dist[2] = {dist0, dist1};
-        SAGPU_TRY(launch_unbwt_rank(dB, sym_bytes, S, sid, N, m, samp_q, nxt, dist, gap, dOut, d_err, s));
+        GET(more, u32, pl.m);
+        GET(link, u32, pl.m + pl.pages);
+        GET(used, u32, pl.segs);
+        // room for gaps of three times the mean (one in twenty goes on in pages); less
+        // where memory is short
+        void *buf = nullptr;
+        u32 cap = 0;
+        for (u32 want : {3 * pl.gap, pl.gap, 8u}) {
+            cap = want;
+            buf = sc.get<uint8_t>((u64)(pl.m + pl.pages) * cap * (u64)sym_bytes);
+            if (buf) break;
+        }
+        if (!buf) return SAGPU_ENOMEM;
+        SAGPU_TRY(launch_unbwt_rank(dB, sym_bytes, S, N, rows[0], pl, cap, counts, nd, buf, link, more, used, dOut,
+                                    d_err, s));
     }
     u32 err = 0;
     SAGPU_TRY(read_u32(c, d_err, &err));

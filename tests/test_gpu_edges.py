@@ -54,3 +54,80 @@ def test_int_value_table(n, wide):
         f = la.libsais64_long if wide else la.libsais_int
         assert f(T, SA, n, largest + 1, 0) == 0, la.last_error()
         assert np.array_equal(SA, ref)
+
+
+@pytest.mark.parametrize("n", [2, 3, 15, 16, 17, 31, 32, 33, 47, 49, 255, 256, 257, 4095, 4096, 4097, 65537])
+def test_unbwt_edges(n):
+    """Inverse BWT around the sample spacing, the words a walk keeps, powers of two (the
+    width of the position hash) and the decode table; every text form whose walks
+    run differently (one symbol, two, all 256, 16-bit symbols), plain and with samples
+    closer than an output word."""
+    rng = np.random.default_rng(n)
+    for name, T in (("one", np.full(n, 7, np.uint8)), ("two", rng.integers(0, 2, n).astype(np.uint8) * 255),
+                    ("bytes", rng.integers(0, 256, n).astype(np.uint8)), ("period", np.arange(n, dtype=np.uint8) % 5)):
+        print(f"[unbwt] n={n} {name}", flush=True)
+        rc, SA = ol.sa(T)
+        U, p = ol.bwt(T, SA)
+        out, A = np.zeros(n, np.uint8), np.zeros(n + 1, np.int32)
+        assert la.libsais_unbwt(U, out, A, n, None, p) == 0, la.last_error()
+        assert np.array_equal(out, T), name
+        for r in (2, 4, 16):
+            U, I = ol.bwt_aux(T, SA, r)
+            out[:] = 9
+            assert la.libsais_unbwt_aux(U, out, A, n, None, r, I.astype(np.int32)) == 0, la.last_error()
+            assert np.array_equal(out, T), (name, r)
+    T = rng.integers(0, 65536, n).astype(np.uint16)
+    rc, SA = ol.sa16(T)
+    U, p = ol.bwt16(T, SA)
+    out, A = np.zeros(n, np.uint16), np.zeros(n + 1, np.int32)
+    assert la.libsais16_unbwt(U, out, A, n, None, p) == 0, la.last_error()
+    assert np.array_equal(out, T)
+
+
+@pytest.mark.parametrize("n,r", [(1 << 22, 0), ((1 << 22) + 1, 0), ((1 << 24) - 1, 0), ((1 << 24) + 3, 0),
+                                 (100003, 2), ((1 << 22) + 5, 64), ((1 << 22) + 5, 2048)])
+def test_unbwt_spacing(n, r):
+    """The sizes where the sample spacing changes, and both decoders of auxiliary samples
+    (many chunks of odd total length; few)."""
+    print(f"[unbwt] n={n} r={r}", flush=True)
+    T = workloads.dna_like(n, seed=n)
+    U, out, A = np.zeros(n, np.uint8), np.zeros(n, np.uint8), np.zeros(n + 1, np.int32)
+    if r:
+        I = np.zeros((n - 1) // r + 1, np.int32)
+        assert la.libsais_bwt_aux(T, U, A, n, 0, None, r, I) == 0, la.last_error()
+        assert la.libsais_unbwt_aux(U, out, A, n, None, r, I) == 0, la.last_error()
+    else:
+        p = la.libsais_bwt(T, U, A, n, 0, None)
+        assert p > 0
+        assert la.libsais_unbwt(U, out, A, n, None, p) == 0, la.last_error()
+    assert np.array_equal(out, T)
+
+
+def test_unbwt_short_of_memory():
+    """Under a falling memory cap the walks get less room (shorter chunks, pages that run
+    out, gaps walked twice): the call returns the text or -2, nothing else."""
+    n = 65537
+    T = workloads.dna_like(n, seed=5)
+    rc, SA = ol.sa(T)
+    U, p = ol.bwt(T, SA)
+    lib = la.load()
+    out, A = np.zeros(n, np.uint8), np.zeros(n + 1, np.int32)
+
+    def capped(limit):
+        lib.sagpu_set_memory_limit(limit)
+        out[:] = 0
+        rc = la.libsais_unbwt(U, out, A, n, None, p)
+        assert rc in (0, -2), rc
+        assert rc == -2 or np.array_equal(out, T), limit
+        return rc == 0
+
+    try:
+        low, high = 1, 1 << 36   # the context keeps scratch of earlier calls: look for the least cap
+        while high - low > (16 << 10):
+            mid = (low + high) // 2
+            low, high = (low, mid) if capped(mid) else (mid, high)
+        for step in range(64):
+            capped(low + (step << 14))
+    finally:
+        lib.sagpu_set_memory_limit(0)
+    assert la.libsais_unbwt(U, out, A, n, None, p) == 0 and np.array_equal(out, T)
