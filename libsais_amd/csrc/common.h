@@ -34,6 +34,35 @@ __device__ __forceinline__ u32 lane_id() { return __lane_id(); }
 
 __device__ __forceinline__ u64 lanemask_lt() { return (1ull << lane_id()) - 1ull; }
 
+// Lanes of `active` that hold the same low BITS bits of d as this lane.  Four vector
+// instructions per bit: the bit spread over a word (x), its ballot, and for each half
+// of the mask m & ~(ballot ^ x), one three-input operation (the empty asm keeps the
+// compiler from testing the bit a second way).  Written as m &= bit ? ballot : ~ballot
+// it compiled to nine; a radix pass ranks every key with eight of these, and a pass over
+// 2^28 u32 pairs went from 1.21 to 1.12 ms with the four (116 to 75 vector instructions
+// per key).
+template <int BITS> __device__ __forceinline__ u64 wave_peers(u32 d, u64 active)
+{
+    u32 lo = (u32)active, hi = (u32)(active >> 32);
+#pragma unroll
+    for (int b = 0; b < BITS; b++) {
+        u32 x = (u32)__builtin_amdgcn_sbfe((int)d, b, 1);
+        asm("" : "+v"(x));
+        const u64 bb = __ballot(x != 0);
+        lo &= ~((u32)bb ^ x);
+        asm("" : "+v"(lo));
+        hi &= ~((u32)(bb >> 32) ^ x);
+        asm("" : "+v"(hi));
+    }
+    return (u64)hi << 32 | lo;
+}
+
+// Set bits of m below this lane.
+__device__ __forceinline__ u32 mask_below(u64 m)
+{
+    return __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
+}
+
 // Inclusive wave-level scan (sum) over 64 lanes.
 __device__ __forceinline__ u32 wave_incl_sum(u32 v)
 {

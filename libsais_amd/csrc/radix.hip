@@ -202,6 +202,11 @@ __global__ __launch_bounds__(256) void k_radix_offsets(u64 *hist, int npass, int
 // ticket, aggregate publish, decoupled look-back).  LOOKBACK = false: the tile's
 // global digit offsets were produced by an upsweep + scan (reduce-then-scan).
 // GEN: the input keys and values are generated (KeyGen) instead of read.
+// Bound by memory: 2^28 u32 pairs take 1.11 ms, 3.87 TB/s of the 16 bytes per pair that a
+// pass cannot do without (a 4 GiB copy on the same card: 4.76 TB/s); 1.21 ms before the
+// ranking took fewer vector instructions (wave_peers), digit starts were folded into
+// one LDS read per element and values were loaded under the key writes.  u64 keys:
+// 3.37 ms for 2^29 pairs (3.72 before).
 template <typename K, bool HAS_VALS, bool LOOKBACK, int ITEMS, bool GEN = false, int NT = RS_THREADS, int DB = 8>
 __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, const u32 *__restrict__ vin,
                                                            K *__restrict__ kout, u32 *__restrict__ vout, u64 n,
@@ -221,8 +226,7 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     constexpr int DPB = DB > 8 ? 16 : 8, DPW = 32 / DPB;
     __shared__ u32 s_tile;
     __shared__ u32 s_wcnt[NW][BINS];
-    __shared__ u32 s_dstart[BINS];
-    __shared__ u64 s_gbase[BINS];
+    __shared__ u32 s_gofs[BINS];   // output index of a staged element - its staged index (mod 2^32)
     __shared__ u32 s_wsum[NW];
     __shared__ K s_keys[TILE_];
 
@@ -236,8 +240,8 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     const u64 tile = LOOKBACK ? (u64)s_tile : (u64)blockIdx.x;
     const u64 wbase = tile * TILE_ + (u64)w * WAVE_ITEMS_;
 
-    // Values are loaded only for the value phase, after the keys have left the
-    // registers: fewer live registers per wave, more waves per SIMD.
+    // Values are loaded after the keys have left the registers: fewer live registers
+    // per wave, more waves per SIMD.
     //
     // Positions past n (only in the last tile) take the largest key.  They rank
     // after every real key of the largest digit (position order is the tie-break),
@@ -295,16 +299,10 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
         u32 d = (u32)(key[j] >> shift) & dmask;
-        u64 m = ~0ull;
-#pragma unroll
-        for (int b = 0; b < DB; b++) {
-            bool bit = (d >> b) & 1u;
-            u64 bb = __ballot(bit);
-            m &= bit ? bb : ~bb;
-        }
-        u32 below = __popcll(m & lanemask_lt());
-        u32 old = s_wcnt[w][d];
-        if (below == 0) s_wcnt[w][d] = old + (u32)__popcll(m);
+        const u64 m = wave_peers<DB>(d, ~0ull);
+        const u32 below = mask_below(m);
+        const u32 old = s_wcnt[w][d];
+        s_wcnt[w][d] = old + (u32)__popcll(m);   // the same value from every peer
         // rank inside the wave (< 2^16) with the digit above it: one live register
         // per item until the reorder instead of three (rank, digit, LDS address)
         rank[j] = (old + below) | (d << 16);
@@ -316,7 +314,7 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     __syncthreads();
 
     // Per digit: wave offsets, tile count, global offset.
-    u32 run[DPT];
+    u32 run[DPT], gbase[DPT];   // (output indexes fit 32 bits: n <= 2^32)
     u32 tsum = 0;
     const bool dthread = tid * DPT < (u32)BINS;
 #pragma unroll
@@ -349,7 +347,6 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
 #pragma unroll
         for (int qd = 0; qd < DPT; qd++) {
             const u32 d = tid * DPT + qd;
-            u64 gbase;
             if (LOOKBACK) {
                 u64 *my = lookback + tile * BINS + d;
                 u64 excl = 0;
@@ -379,11 +376,10 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
                     }
                     st_release_u64(my, lb_pack(epoch, LB_PRE, excl + run[qd]));
                 }
-                gbase = offsets[d] + excl;
+                gbase[qd] = (u32)(offsets[d] + excl);
             } else {
-                gbase = scanned[(u64)d * tiles + tile];
+                gbase[qd] = scanned[(u64)d * tiles + tile];
             }
-            s_gbase[d] = gbase;
         }
     }
     __syncthreads();
@@ -393,7 +389,12 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
         u32 st = carry + inc - tsum;
 #pragma unroll
         for (int qd = 0; qd < DPT; qd++) {
-            s_dstart[tid * DPT + qd] = st;
+            const u32 d = tid * DPT + qd;
+            // the digit's start in the tile goes into its waves' offsets and, negated,
+            // into its output offset: one LDS read per element in each place
+#pragma unroll
+            for (int q = 0; q < NW; q++) s_wcnt[q][d] += st;
+            s_gofs[d] = gbase[qd] - st;
             st += run[qd];
         }
     }
@@ -403,9 +404,25 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
         const u32 d = rank[j] >> 16;
-        const u32 lp = s_dstart[d] + s_wcnt[w][d] + (rank[j] & 0xFFFFu);
+        const u32 lp = s_wcnt[w][d] + (rank[j] & 0xFFFFu);
         s_keys[lp] = key[j];
         rank[j] = lp;
+    }
+    // The values take the registers the keys have left: loaded here, they arrive while
+    // the keys are written out.
+    constexpr bool LOAD_VALS = HAS_VALS && !GEN;
+    u32 val[LOAD_VALS ? ITEMS : 1];
+    if constexpr (LOAD_VALS) {
+        if (full) {
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) val[j] = vin[wbase + (u64)j * SAGPU_WAVE + lane];
+        } else {
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) {
+                const u64 pos = wbase + (u64)j * SAGPU_WAVE + lane;
+                val[j] = pos < n ? vin[pos] : 0u;
+            }
+        }
     }
     __syncthreads();
     const u64 tbase = tile * TILE_;
@@ -415,17 +432,26 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     u32 dpack[(ITEMS + DPW - 1) / DPW];
 #pragma unroll
     for (int q = 0; q < (ITEMS + DPW - 1) / DPW; q++) dpack[q] = 0;
+    auto put_key = [&](int j, u32 idx) {
+        const K kk = s_keys[idx];
+        const u32 d = (u32)(kk >> shift) & dmask;
+        dpack[j / DPW] |= d << (DPB * (j % DPW));
+        kout[s_gofs[d] + idx] = kk;
+    };
+    if (full) {
 #pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        const u32 idx = tid + (u32)j * NT;
-        if (idx < tile_n) {
-            const K kk = s_keys[idx];
-            const u32 d = (u32)(kk >> shift) & dmask;
-            dpack[j / DPW] |= d << (DPB * (j % DPW));
-            kout[s_gbase[d] + (idx - s_dstart[d])] = kk;
+        for (int j = 0; j < ITEMS; j++) {
+            put_key(j, tid + (u32)j * NT);
+            // bound the LDS loads the scheduler hoists (each item holds four registers)
+            if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
         }
-        // bound the LDS loads the scheduler hoists (each item holds four registers)
-        if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const u32 idx = tid + (u32)j * NT;
+            if (idx < tile_n) put_key(j, idx);
+            if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+        }
     }
     if (HAS_VALS) {
         __syncthreads();
@@ -439,25 +465,29 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
                 const u32 pc = (prevc[j / 4] >> (8 * (j % 4))) & 255u;
                 if (pos <= nn) s_vals[rank[j]] = (pos << gen.cb) | pc;
             }
-        } else if (full) {
+        } else {
+            // (past-the-end values land in the slots of past-the-end keys)
 #pragma unroll
-            for (int j = 0; j < ITEMS; j++) s_vals[rank[j]] = vin[wbase + (u64)j * SAGPU_WAVE + lane];
+            for (int j = 0; j < ITEMS; j++) s_vals[rank[j]] = val[j];
+        }
+        __syncthreads();
+        auto put_val = [&](int j, u32 idx) {
+            const u32 d = (dpack[j / DPW] >> (DPB * (j % DPW))) & ((1u << DPB) - 1u);
+            vout[s_gofs[d] + idx] = s_vals[idx];
+        };
+        if (full) {
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) {
+                put_val(j, tid + (u32)j * NT);
+                if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+            }
         } else {
 #pragma unroll
             for (int j = 0; j < ITEMS; j++) {
-                u64 pos = wbase + (u64)j * SAGPU_WAVE + lane;
-                if (pos < n) s_vals[rank[j]] = vin[pos];
+                const u32 idx = tid + (u32)j * NT;
+                if (idx < tile_n) put_val(j, idx);
+                if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
             }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < ITEMS; j++) {
-            const u32 idx = tid + (u32)j * NT;
-            if (idx < tile_n) {
-                const u32 d = (dpack[j / DPW] >> (DPB * (j % DPW))) & ((1u << DPB) - 1u);
-                vout[s_gbase[d] + (idx - s_dstart[d])] = s_vals[idx];
-            }
-            if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
         }
     }
 }

@@ -114,17 +114,13 @@ __global__ __launch_bounds__(UB_THREADS) void k_ub_succ(const uint8_t *__restric
         u64 pos = wbase + (u64)j * SAGPU_WAVE + lane;
         bool ok = pos < n;
         u32 d = ok ? (u32)U[pos] : 0u;
-        u64 m = __ballot(ok);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            bool bit = (d >> b) & 1u;
-            u64 bb = __ballot(bit);
-            m &= bit ? bb : ~bb;
-        }
-        u32 below = __popcll(m & lanemask_lt());
+        const u64 m = wave_peers<8>(d, __ballot(ok));
+        const u32 below = mask_below(m);
         u32 old = 0;
-        if (ok) old = s_wcnt[w][d];
-        if (ok && below == 0) s_wcnt[w][d] = old + (u32)__popcll(m);
+        if (ok) {
+            old = s_wcnt[w][d];
+            s_wcnt[w][d] = old + (u32)__popcll(m);   // the same value from every peer
+        }
         dig[j] = d;
         rank[j] = old + below;
     }
