@@ -273,6 +273,9 @@ SAGPU_API int32_t sagpu_sort_pairs_u64(uint64_t *d_keys, uint32_t *d_vals, int64
  *   "hist_windows"   1 = the initial sort's histograms, when its keys come from the code stream
  *                    with whole symbols per 8-bit digit, are derived from one histogram of the
  *                    stream's 8-bit windows (default); 0 = counted per pass
+ *   "small_build"    1 = texts of at most 24 KiB are built by one workgroup in one kernel, while the
+ *                    other engine knobs above hold their defaults and timing is off (default);
+ *                    0 = by the general engine
  *   "api_slots"      contexts that calls made without a libsais context share, 1-16
  *                    (default 8): that many such calls run at once, each on its own stream
  * Returns 0, or -1 for an unknown name or value.

@@ -300,6 +300,32 @@ int big_piv_emit(const u32 *pq, const PivRegions &reg, const u32 *rk, const u32 
                  u64 base, u64 h, u32 *ISA, const u32 *out_i, u32 *out_g, u32 *LCP, int cb, const u32 *cscan, u32 nb,
                  u64 total, hipStream_t s);
 
+// ------------------------------------------------- short texts (small.hip)
+// A build of at most SMALL_MAX bytes in one workgroup, all of it in LDS.  T and the
+// outputs may be device memory or pinned host memory; out is pinned host memory.
+constexpr u32 SMALL_MAX = 24 * 1024;
+enum { SMALL_NOT_TAKEN = 1 };   // status: a GSA text that does not end in a separator
+struct SmallOut {
+    int32_t status;          // SAGPU_OK, SAGPU_EINVAL (GSA validity) or SMALL_NOT_TAKEN
+    u32 primary, rounds, ksym, sigma;
+    u32 active[64];          // members of groups entering each round
+    u64 freq[256];           // when want_freq
+};
+struct SmallJob {
+    const uint8_t *T;
+    u32 n;
+    int gsa, want_freq;
+    int wide;                // 1: SA, PLCP, LCP and I (and in_SA) are int64
+    const void *in_SA;       // null, or the caller's suffix array: PLCP / LCP from it
+    void *SA;                // outputs, each may be null
+    uint8_t *U;
+    void *PLCP, *LCP;
+    void *I;                 // auxiliary samples: I[k] = 1 + slot of suffix k * r
+    u32 r;
+    SmallOut *out;
+};
+int launch_small_build(const SmallJob &j, hipStream_t s);
+
 // ------------------------------------------------------------ SA kernels
 int launch_histogram(const uint8_t *T, u64 n, int gsa, u64 *hist256, u32 *gsa_bad, hipStream_t s);
 // vals[p] = p, or (p << cb) | code of T[p-1] with cb > 0 (n - 1 < 2^(32 - cb)).

@@ -303,6 +303,7 @@ struct Ctx {
     Timer timer;
     sagpu_stats stats{};
     bool sort_u32 = false;  // the radix passes being timed are u32-key passes
+    uint8_t *small_io = nullptr;   // pinned: result block and host arrays of small builds
     // Executable graphs of a doubling round, one per buffer parity (rounds 2, 4, ...
     // and 3, 5, ...), kept across builds: reused as they are while every argument and
     // launch size of the round is the same (round_sig), else captured again and
@@ -365,6 +366,11 @@ int g_perm_hist = 1;
 // radix sorts of fewer keys use the smallest tiles (2048 keys), whatever radix_items
 // and radix_threads say
 int g_radix_small_n = 1 << 20;
+
+// 1: texts of at most SMALL_MAX bytes are built by one workgroup in one kernel
+// (small.hip); 0: by the general engine
+int g_small_build = 1;
+u32 g_knobs_off = 0;   // bit k: general-engine knob g_knobs[k] is off its default
 
 // A context is one stream with its own pooled buffers and scratch; calls on one
 // context are serialised, different contexts run concurrently on the device.
@@ -438,6 +444,7 @@ void ctx_destroy(Ctx *c)
     if (c->xs) (void)hipHostFree(c->xs);
     for (auto &e : c->xs_ev)
         if (e) (void)hipEventDestroy(e);
+    if (c->small_io) (void)hipHostFree(c->small_io);
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1498,6 +1505,97 @@ void stats_reset(Ctx &c)
     c.stats_fresh = true;
 }
 
+// Whether a text of n bytes is built by one workgroup (small.hip).  The line is what
+// its LDS holds; at the largest size it still beats the general engine by far (see
+// small.hip).  Timing mode wants the general engine's kernels, a knob off its default
+// its effect, and the allocation-free build its static scratch only.
+bool small_text(const Ctx &c, u64 n)
+{
+    return n >= 2 && n <= SMALL_MAX && g_small_build && !g_knobs_off && !g_timing && !c.pool.arena;
+}
+
+// Pinned block of small builds: the kernel's result, then the host arrays it reads and
+// writes over the bus (text, in_SA, and up to three outputs), each 8-byte aligned.
+constexpr size_t SMALL_IO = 4096 + SMALL_MAX + 4 * 8 * (size_t)SMALL_MAX;
+
+int small_block(Ctx &c, SmallOut **out, uint8_t **arrays)
+{
+    static_assert(sizeof(SmallOut) <= 4096, "result block");
+    if (!c.small_io) {
+        g_device_allocs++;
+        if (hipHostMalloc((void **)&c.small_io, SMALL_IO, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c.small_io = nullptr;
+            sagpu_set_error("pinned host allocation failed", __FILE__, __LINE__);
+            return SAGPU_ENOMEM;
+        }
+    }
+    *out = (SmallOut *)c.small_io;
+    *arrays = c.small_io + 4096;
+    return SAGPU_OK;
+}
+
+// Runs a small build and waits for it.  SMALL_NOT_TAKEN: the general engine's case.
+int small_run(Ctx &c, const SmallJob &j)
+{
+    j.out->status = SAGPU_EDEVICE;
+    SAGPU_TRY(launch_small_build(j, c.stream));
+    SAGPU_CHECK(hipStreamSynchronize(c.stream));
+    const SmallOut &o = *j.out;
+    if (o.status != SAGPU_OK) return o.status;
+    c.stats.rounds = (int32_t)o.rounds;
+    c.stats.initial_symbols = (int32_t)o.ksym;
+    c.stats.bits_per_symbol = o.sigma <= 2 ? 1 : bits_for((u64)o.sigma - 1);
+    for (u32 r = 0; r < o.rounds && r < 64; r++) c.stats.active[r] = (int64_t)o.active[r];
+    return SAGPU_OK;
+}
+
+// The same from and to host arrays, which pass through the pinned block: the kernel
+// reads and writes it over the bus, so the call is one launch and one wait.
+// SA, PLCP, LCP and I (auxiliary samples, one in r) have `width` bytes per entry.
+int small_host(Ctx &c, const uint8_t *T, u64 n, int gsa, int width, const void *in_SA, void *SA, uint8_t *U,
+               void *PLCP, void *LCP, void *I, u64 r, u64 *freq, u64 *primary)
+{
+    SmallOut *out;
+    uint8_t *at;
+    SAGPU_TRY(small_block(c, &out, &at));
+    const size_t text = (n + 7) & ~(size_t)7, index = n * (size_t)width;
+    auto take = [&](bool wanted, size_t bytes) {
+        uint8_t *p = wanted ? at : nullptr;
+        if (wanted) at += (bytes + 7) & ~(size_t)7;
+        return p;
+    };
+    SmallJob j{};
+    uint8_t *hT = take(true, text), *hS = take(in_SA != nullptr, index), *hSA = take(SA != nullptr, index);
+    uint8_t *hU = take(U != nullptr, text), *hP = take(PLCP != nullptr, index), *hL = take(LCP != nullptr, index);
+    const u64 samples = I ? (n - 1) / r + 1 : 0;
+    uint8_t *hI = take(I != nullptr, samples * width);
+    memcpy(hT, T, n);
+    if (hS) memcpy(hS, in_SA, index);
+    j.T = hT;
+    j.n = (u32)n;
+    j.gsa = gsa;
+    j.want_freq = freq != nullptr;
+    j.wide = width == 8;
+    j.in_SA = hS;
+    j.SA = hSA;
+    j.U = hU;
+    j.PLCP = hP;
+    j.LCP = hL;
+    j.I = hI;
+    j.r = (u32)(r < n ? r : n);
+    j.out = out;
+    SAGPU_TRY(small_run(c, j));
+    if (SA) memcpy(SA, hSA, index);
+    if (U) memcpy(U, hU, n);
+    if (PLCP) memcpy(PLCP, hP, index);
+    if (LCP) memcpy(LCP, hL, index);
+    if (I) memcpy(I, hI, samples * width);
+    if (freq) memcpy(freq, out->freq, sizeof out->freq);
+    if (primary) *primary = out->primary;
+    return SAGPU_OK;
+}
+
 // Fused device pipeline.  Returns 0 or the primary index when U is requested.
 int64_t build_dev(Ctx &c, Scope &sc, const uint8_t *dTpad, u64 n, int gsa, u32 *dSA, uint8_t *dU, u32 *dPLCP,
                   u32 *dLCP, u64 *freq, u32 *dISA = nullptr)
@@ -1663,6 +1761,13 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_sa(const uint8_t *T, void *SA, int64_
     }
     stats_reset(*c);
     int64_t rc;
+    if (small_text(*c, (u64)n)) {
+        u64 f[256];
+        rc = small_host(*c, T, (u64)n, gsa, width, nullptr, SA, nullptr, nullptr, nullptr, nullptr, 0,
+                        freq ? f : nullptr, nullptr);
+        if (rc == SAGPU_OK) store_freq(f, freq, width);
+        if (rc != SMALL_NOT_TAKEN) return rc;
+    }
     {
         Scope sc(*c);
         uint8_t *dT;
@@ -1687,6 +1792,13 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_bwt(const uint8_t *T, uint8_t *U, int
         return SAGPU_ENOMEM;
     }
     stats_reset(*c);
+    if (small_text(*c, (u64)n)) {
+        u64 fr[256], primary = 0;
+        SAGPU_TRY(small_host(*c, T, (u64)n, 0, width, nullptr, nullptr, U, nullptr, nullptr, nullptr, 0,
+                             freq ? fr : nullptr, &primary));
+        store_freq(fr, freq, width);
+        return (int64_t)primary;
+    }
     Scope sc(*c);
     uint8_t *dT;
     SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT));
@@ -1819,6 +1931,13 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_bwt_aux(const uint8_t *T, uint8_t *U,
         return SAGPU_ENOMEM;
     }
     stats_reset(*c);
+    if (small_text(*c, (u64)n)) {
+        u64 fr[256];
+        SAGPU_TRY(small_host(*c, T, (u64)n, 0, width, nullptr, nullptr, U, nullptr, nullptr, I, (u64)r,
+                             freq ? fr : nullptr, nullptr));
+        store_freq(fr, freq, width);
+        return 0;
+    }
     Scope sc(*c);
     uint8_t *dT;
     SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT));
@@ -2085,6 +2204,11 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_plcp(const uint8_t *T, const void *SA
         return SAGPU_ENOMEM;
     }
     stats_reset(*c);
+    if (small_text(*c, (u64)n)) {
+        const int rc = small_host(*c, T, (u64)n, gsa, width, SA, nullptr, nullptr, PLCP, nullptr, nullptr, 0, nullptr,
+                                  nullptr);
+        if (rc != SMALL_NOT_TAKEN) return rc;
+    }
     Scope sc(*c);
     uint8_t *dT;
     SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT));
@@ -2215,7 +2339,33 @@ extern "C" void sagpu_trim(void) { trim_idle_slots(); }
 
 extern "C" void sagpu_set_timing(int32_t enabled) { g_timing = enabled != 0; }
 
+namespace {
+// The knobs of the general engine and their defaults.  While one of them is off its
+// default, short texts take the general engine too, so that the knob has its effect.
+const struct { const char *name; int64_t value; } g_knobs[] = {
+    {"radix_items", 32}, {"radix_threads", 512}, {"radix_variant", RADIX_ONESWEEP}, {"radix_bits", 8},
+    {"radix_small_n", 1 << 20}, {"bucketed_phi", 1}, {"plcp_hint", 1}, {"exact_round1", 1}, {"stream_compare", 1},
+    {"raw_round1", 1}, {"key_stream", 1}, {"round_graphs", 1}, {"big_pivot_min", 1 << 20}, {"perm_hist", 1},
+    {"group_flags", 1}, {"windowed_scatter", 1}, {"plcp_pairs", 1}, {"bwt_variant", 0}, {"hist_windows", 1},
+    {"init_rows", 8}, {"tile_range", 512}, {"isa_window_log2", 25}, {"wide_from", 0x7FFFFFFF}};
+
+int set_option(const char *name, int64_t value);
+} // namespace
+
 extern "C" int32_t sagpu_set_option(const char *name, int64_t value)
+{
+    const int rc = set_option(name, value);
+    if (rc == 0) {
+        std::lock_guard<std::mutex> lk(g_opt_mu);
+        for (size_t k = 0; k < sizeof g_knobs / sizeof g_knobs[0]; k++)
+            if (!strcmp(name, g_knobs[k].name))
+                g_knobs_off = value == g_knobs[k].value ? g_knobs_off & ~(1u << k) : g_knobs_off | 1u << k;
+    }
+    return rc;
+}
+
+namespace {
+int set_option(const char *name, int64_t value)
 {
     if (!name) return SAGPU_EINVAL;
     std::lock_guard<std::mutex> lk(g_opt_mu);
@@ -2349,10 +2499,13 @@ extern "C" int32_t sagpu_set_option(const char *name, int64_t value)
         g_wide_from = (u64)value;
         return 0;
     }
+    if (!strcmp(name, "small_build")) {
+        if (value != 0 && value != 1) return SAGPU_EINVAL;
+        g_small_build = (int)value;
+        return 0;
+    }
     return SAGPU_EINVAL;
 }
-
-namespace {
 
 template <typename K>
 int sort_pairs_dev(K *d_keys, u32 *d_vals, int64_t n, int begin_bit, int end_bit)
@@ -2477,6 +2630,24 @@ int64_t build32_on(Ctx &c, const uint8_t *d_T, u64 n, int32_t flags, int32_t *d_
                    int32_t *d_LCP, int64_t *h_freq)
 {
     stats_reset(c);
+    if (small_text(c, n)) {
+        SmallJob j{};
+        uint8_t *arrays;
+        SAGPU_TRY(small_block(c, &j.out, &arrays));
+        j.T = d_T;
+        j.n = (u32)n;
+        j.gsa = (flags & SAGPU_FLAG_GSA) ? 1 : 0;
+        j.want_freq = h_freq != nullptr;
+        j.SA = d_SA;
+        j.U = d_U;
+        j.PLCP = d_PLCP;
+        j.LCP = d_LCP;
+        const int rc = small_run(c, j);
+        if (rc == SAGPU_OK && h_freq)
+            for (int ch = 0; ch < 256; ch++) h_freq[ch] = (int64_t)j.out->freq[ch];
+        if (rc == SAGPU_OK) return d_U ? (int64_t)j.out->primary : 0;
+        if (rc != SMALL_NOT_TAKEN) return rc;
+    }
     Scope sc(c);
     uint8_t *dT;
     SAGPU_TRY(padded_text(c, sc, d_T, n, SRC_DEVICE, &dT));
@@ -2717,6 +2888,13 @@ int run_single(Ctx &c, sagpu_job *j)
     const u64 n = (u64)j->n;
     if (n > (u64)INT32_MAX) return SAGPU_ENOMEM;
     stats_reset(c);
+    if (small_text(c, n)) {
+        u64 primary = 0;
+        SAGPU_TRY(small_host(c, j->T, n, 0, 4, nullptr, j->SA, j->kind == SAGPU_JOB_BWT ? j->U : nullptr, nullptr,
+                             j->kind == SAGPU_JOB_LCP ? j->LCP : nullptr, nullptr, 0, nullptr, &primary));
+        if (j->kind == SAGPU_JOB_BWT) j->primary = (int64_t)primary;
+        return 0;
+    }
     Scope sc(c);
     uint8_t *dT;
     SAGPU_TRY(padded_text(c, sc, j->T, n, SRC_HOST, &dT));

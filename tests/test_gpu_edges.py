@@ -131,3 +131,91 @@ def test_unbwt_short_of_memory():
     finally:
         lib.sagpu_set_memory_limit(0)
     assert la.libsais_unbwt(U, out, A, n, None, p) == 0 and np.array_equal(out, T)
+
+
+SMALL_MAX = 24 * 1024   # the longest text one workgroup builds
+
+
+def _small_texts(n, rng):
+    yield "one", np.full(n, 65, np.uint8)
+    yield "two", rng.integers(0, 2, n).astype(np.uint8)
+    yield "bytes", rng.integers(0, 256, n).astype(np.uint8)
+    yield "acgt", workloads.iid(n, seed=n, alphabet=b"ACGT")
+    yield "period", workloads.periodic(n, 17, 3)
+    yield "fibonacci", workloads.fibonacci(n)
+    copies = np.tile(workloads.iid(max(2, n // 3), seed=n, alphabet=b"abcdefghijklmnopqrstuvwxyz"), 4)[:n].copy()
+    yield "copies", copies
+    runs = copies.copy()
+    runs[n // 4: n // 4 + 300] = 97   # one group on either side of what is ranked by counting
+    runs[n // 2: n // 2 + 90] = 97
+    yield "runs", runs
+
+
+@pytest.mark.parametrize("n", [2, 3, 17, 63, 64, 65, 1023, 1024, 1025, 2049, 4096, 4097, 8192, 8193, 16384, 16385,
+                               SMALL_MAX - 1, SMALL_MAX, SMALL_MAX + 1])
+def test_small_build(n):
+    """Texts built by one workgroup, at the edges of its rows and of its range, and the
+    first size past it: every output of the device and the host entry points (both
+    index widths) against the oracle, and the general engine on the same text."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    rng = np.random.default_rng(n)
+    for name, T in _small_texts(n, rng):
+        print(f"[small] n={n} {name}", flush=True)
+        rc, SA = ol.sa(T)
+        U, p = ol.bwt(T, SA)
+        P = ol.plcp(T, SA)
+        L, f = ol.lcp(P, SA), ol.freq(T)
+        for small in (1, 0):
+            assert lib.sagpu_set_option(b"small_build", small) == 0
+            try:
+                gSA, gU, gp, gP, gL, gf = fused(T)
+            finally:
+                assert lib.sagpu_set_option(b"small_build", 1) == 0
+            assert np.array_equal(gSA, SA), (name, small)
+            assert gp == p and np.array_equal(gU, U), (name, small)
+            assert np.array_equal(gP, P) and np.array_equal(gL, L) and np.array_equal(gf, f), (name, small)
+        for dt, sa, bwt, plcp, aux in ((np.int32, la.libsais, la.libsais_bwt, la.libsais_plcp, la.libsais_bwt_aux),
+                                       (np.int64, la.libsais64, la.libsais64_bwt, la.libsais64_plcp,
+                                        la.libsais64_bwt_aux)):
+            out, fr, hU, A = np.zeros(n, dt), np.zeros(256, dt), T.copy(), np.zeros(n, dt)
+            assert sa(T, out, n, 0, fr) == 0 and np.array_equal(out, SA) and np.array_equal(fr, f), name
+            assert bwt(hU, hU, A, n, 0, fr) == p and np.array_equal(hU, U) and np.array_equal(fr, f), name
+            out[:] = 0
+            assert plcp(T, np.ascontiguousarray(SA, dt), out, n) == 0 and np.array_equal(out, P), name
+            for r in (2, 64, 1 << 30):
+                I = np.zeros((n - 1) // r + 1, dt)
+                rU, rI = ol.bwt_aux(T, SA, r)
+                assert aux(T, hU, A, n, 0, None, r, I) == 0 and np.array_equal(hU, rU), (name, r)
+                assert np.array_equal(I, rI), (name, r)
+
+
+@pytest.mark.parametrize("n", [2, 65, 1025, 4097, 16385, SMALL_MAX, SMALL_MAX + 1])
+def test_small_gsa(n):
+    """String sets built by one workgroup: SA, PLCP and LCP against the oracle; invalid
+    sets refused."""
+    from tests.test_gpu_parity import fused
+    rng = np.random.default_rng(n)
+    unit = rng.integers(1, 4, 200).astype(np.uint8)
+    for name, every in (("single", 0), ("many", 23), ("alike", 201)):
+        T = np.tile(unit, n // 200 + 1)[:n].copy() if every == 201 else rng.integers(1, 5, n).astype(np.uint8)
+        if every:
+            T[every - 1::every] = 0
+        if n > 1:
+            T[-2:] = (1, 0)
+        print(f"[small gsa] n={n} {name}", flush=True)
+        rc, SA = ol.sa(T, gsa=True)
+        assert rc == 0
+        P = ol.plcp(T, SA, gsa=True)
+        gSA, _, _, gP, gL, _ = fused(T, gsa=True)
+        assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA)), name
+        out = np.zeros(n, np.int32)
+        assert la.libsais_gsa(T, out, n, 0, None) == 0 and np.array_equal(out, SA)
+        assert la.libsais_plcp_gsa(T, out, out, n) == 0 and np.array_equal(out, P)
+        bad = T.copy()
+        bad[0] = 0
+        assert la.libsais_gsa(bad, out, n, 0, None) == -1
+        if n > 64:
+            bad = T.copy()
+            bad[30:32] = 0
+            assert la.libsais_gsa(bad, out, n, 0, None) == -1
