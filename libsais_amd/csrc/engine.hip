@@ -12,7 +12,9 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <deque>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <pthread.h>
@@ -169,16 +171,17 @@ struct Timer {
 };
 
 // ------------------------------------------------------ host copies
-// Bulk copies between caller host memory (pageable) and the device run through
-// pinned slots: the host side of each chunk is copied by a pool of threads while
-// the DMA of the neighbouring chunk runs.  On the MI355X host, pageable hipMemcpy
-// moves 22-29 GB/s to the device and 4 GB/s into pages the caller has not touched
-// yet (first-touch faults taken by one thread); the staged form 54 GB/s and
-// 27-29 GB/s with 16 copy threads.
-constexpr int XS_SLOTS = 4;
-// 1: copies of at least 4 MiB staged in 32 MiB chunks (default); 0: every copy
-// direct; 2: every copy staged in 64 KiB chunks (exercises the chunk logic on
-// small inputs)
+// Bulk copies between caller host memory (pageable) and the device run through a ring of
+// pinned memory in chunks: a pool of threads fills (or drains) several chunks at once
+// while the DMA of others runs.  On the MI355X host, pageable hipMemcpy moves 22-29 GB/s
+// to the device and 4 GB/s into pages the caller has not touched yet (first-touch faults
+// taken by one thread); pinned DMA 57 GB/s.  64-bit index arrays are narrowed and widened
+// by the copy threads, so only 4 bytes per index cross the bus.
+constexpr u64 XS_RING = 32ull << 20;
+constexpr int XS_EVENTS = 8, XS_AHEAD = 24;   // upload chunks whose host copies may run ahead of the DMA
+enum { XS_TODO = -1, XS_QUEUED = -2 };        // a region's DMA is not queued / queued, no event after it yet
+// 1: copies of at least XS_MIN bytes staged (default); 0: every copy direct; 2: every
+// copy staged in 64 KiB chunks (exercises the chunk logic on small inputs)
 int g_host_staging = 1;
 int g_copy_threads = 0;   // 0: min(16, hardware threads)
 
@@ -189,50 +192,153 @@ int copy_threads()
     return hw == 0 ? 4 : (int)(hw < 16 ? hw : 16);
 }
 
-// memcpy split over worker threads; the calling thread takes parts too.  Workers
-// are detached and live until the process ends; a forked child starts a new pool.
+// Copies split over worker threads.  Workers are detached and live until the process
+// ends; a forked child starts a new pool.  Parts are small (128 KiB take a thread about
+// 40 us while 16 of them share the memory), so that the first ones are soon ready for
+// the DMA; they are taken and reported without a lock, and a thread looks for the next
+// one for some time before it sleeps (waking one takes longer than a part).
 class CopyPool {
-    struct Job {
+  public:
+    struct Part {
         uint8_t *d;
         const uint8_t *s;
-        u64 len, per;
-        int parts, next, left;
+        u64 len;     // bytes written
+        int conv;    // 0: bytes; 1: int64 narrowed to u32; 2: u32 widened to int64
     };
-    std::mutex m;
-    std::condition_variable work_cv, done_cv;
-    std::vector<Job *> open;   // jobs with parts not taken yet
+    // At most `most` parts, granted by the owner in order as they become ready, taken in
+    // that order, and done in any.
+    struct Job {
+        explicit Job(u64 most) : part(most), done(new std::atomic<char>[most])
+        {
+            for (u64 k = 0; k < most; k++) done[k].store(0, std::memory_order_relaxed);
+        }
+        std::vector<Part> part;
+        std::unique_ptr<std::atomic<char>[]> done;
+        std::atomic<int> granted{0}, next{0}, users{0};
+        std::atomic<bool> closing{false};
+        int prefix = 0;   // the owner's: parts [0, prefix) are done
+    };
+
+  private:
+    std::mutex m;   // open, workers, sleeping
+    std::condition_variable work_cv;
+    std::vector<Job *> open;
+    std::atomic<int> sleeping{0};
+    std::atomic<u32> epoch{0};   // grants so far, of all jobs
     int workers = 0;
 
-    static void run(Job *j, int p)
+    static void run(const Part &p)
     {
-        const u64 a = (u64)p * j->per;
-        if (a >= j->len) return;
-        const u64 b = a + j->per < j->len ? a + j->per : j->len;
-        memcpy(j->d + a, j->s + a, b - a);
+        if (p.conv == 1) {
+            const int64_t *s = (const int64_t *)p.s;
+            u32 *d = (u32 *)p.d;
+            for (u64 i = 0; i < p.len / 4; i++) d[i] = (u32)s[i];
+        } else if (p.conv == 2) {
+            const u32 *s = (const u32 *)p.s;
+            int64_t *d = (int64_t *)p.d;
+            for (u64 i = 0; i < p.len / 8; i++) d[i] = (int64_t)s[i];
+        } else {
+            memcpy(p.d, p.s, p.len);
+        }
     }
-    // Takes the next part of the first open job; m is held.
-    Job *take(int *p)
+    // Takes and runs one part, if there is one.
+    static bool take(Job &j)
     {
-        Job *j = open.front();
-        *p = j->next++;
-        if (j->next == j->parts) open.erase(open.begin());
-        return j;
+        int k = j.next.load();
+        while (k < j.granted.load())
+            if (j.next.compare_exchange_weak(k, k + 1)) {
+                run(j.part[k]);
+                j.done[k].store(1, std::memory_order_release);
+                return true;
+            }
+        return false;
+    }
+    Job *find()   // m is held
+    {
+        for (Job *j : open)
+            if (j->next.load() < j->granted.load()) return j;
+        return nullptr;
     }
     void loop()
     {
         std::unique_lock<std::mutex> lk(m);
         for (;;) {
-            work_cv.wait(lk, [&] { return !open.empty(); });
-            int p;
-            Job *j = take(&p);
+            Job *j = find();
+            if (!j) {   // look out for a grant for some 50 us, then sleep
+                const u32 seen = epoch.load();
+                lk.unlock();
+                for (int k = 0; k < 2000 && epoch.load() == seen; k++) __builtin_ia32_pause();
+                lk.lock();
+                if (epoch.load() != seen) continue;
+                sleeping++;
+                work_cv.wait(lk, [&] { return (j = find()) != nullptr; });
+                sleeping--;
+            }
+            j->users++;
             lk.unlock();
-            run(j, p);
+            for (int idle = 0; idle < 2000 && !j->closing.load(); idle++) {
+                if (take(*j)) idle = 0;
+                else __builtin_ia32_pause();
+            }
+            j->users--;
             lk.lock();
-            if (--j->left == 0) done_cv.notify_all();
         }
     }
 
   public:
+    // Opens a job (no parts yet) for up to `threads` threads.
+    void begin(Job &j, int threads)
+    {
+        std::lock_guard<std::mutex> lk(m);
+        while (workers < threads - 1) {
+            std::thread([this] { loop(); }).detach();
+            workers++;
+        }
+        open.push_back(&j);
+    }
+    void end(Job &j)   // waits for every part granted, and for the workers to leave the job
+    {
+        wait(j, j.granted.load());
+        j.closing.store(true);
+        {
+            std::lock_guard<std::mutex> lk(m);
+            open.erase(std::find(open.begin(), open.end(), &j));
+        }
+        while (j.users.load() > 0) __builtin_ia32_pause();
+    }
+    // Grants a stretch in parts of `per` written bytes.
+    void grant(Job &j, Part all, u64 per)
+    {
+        const u64 sper = all.conv == 1 ? 2 * per : all.conv == 2 ? per / 2 : per;
+        int g = j.granted.load();
+        for (; all.len; all.d += per, all.s += sper) {
+            Part p = all;
+            p.len = all.len < per ? all.len : per;
+            all.len -= p.len;
+            j.part[g++] = p;
+        }
+        j.granted.store(g);
+        epoch++;
+        if (sleeping.load() > 0) {
+            { std::lock_guard<std::mutex> lk(m); }
+            work_cv.notify_all();
+        }
+    }
+    // Waits until parts [0, upto) are done; takes parts itself when that is not soon.
+    void wait(Job &j, int upto)
+    {
+        for (int idle = 0; j.prefix < upto; idle++) {
+            if (j.done[j.prefix].load(std::memory_order_acquire)) {
+                j.prefix++;
+                idle = 0;
+            } else if (idle < 2000 && workers > 0) {
+                __builtin_ia32_pause();
+            } else if (!take(j)) {
+                std::this_thread::yield();
+            }
+        }
+    }
+    static u64 parts_of(u64 len, u64 per) { return (len + per - 1) / per; }
     void copy(void *d, const void *s, u64 len, int threads)
     {
         if (threads <= 1 || len < (1u << 20)) {
@@ -242,24 +348,10 @@ class CopyPool {
         // parts of whole pages, at least 1 MiB
         u64 per = (len + threads - 1) / threads;
         per = per < (1u << 20) ? (1u << 20) : (per + 4095) & ~(u64)4095;
-        Job j{(uint8_t *)d, (const uint8_t *)s, len, per, (int)((len + per - 1) / per), 0, 0};
-        j.left = j.parts;
-        std::unique_lock<std::mutex> lk(m);
-        while (workers < threads - 1) {
-            std::thread([this] { loop(); }).detach();
-            workers++;
-        }
-        open.push_back(&j);
-        work_cv.notify_all();
-        while (j.next < j.parts) {
-            int p = j.next++;
-            if (j.next == j.parts) open.erase(std::find(open.begin(), open.end(), &j));
-            lk.unlock();
-            run(&j, p);
-            lk.lock();
-            j.left--;
-        }
-        done_cv.wait(lk, [&] { return j.left == 0; });
+        Job j(parts_of(len, per));
+        begin(j, threads);
+        grant(j, Part{(uint8_t *)d, (const uint8_t *)s, len, 0}, per);
+        end(j);
     }
     void lock() { m.lock(); }
     void unlock() { m.unlock(); }
@@ -294,12 +386,17 @@ struct Ctx {
     u64 *pinned = nullptr;      // small pinned host staging (counts, histograms)
     uint8_t *stage = nullptr;   // large pinned staging for batched jobs
     size_t stage_cap = 0;
-    // pinned slots for copies from and to caller host memory (h2d / d2h)
+    // pinned ring for copies from and to caller host memory (h2d / d2h).  Uploads take
+    // regions of it in order, each free again once its DMA is over; a download has the
+    // ring to itself (its kernel follows the uploads on the stream)
+    struct XsRegion { u64 at, len; int ev; };   // ev: the event after its DMA, or XS_TODO / XS_QUEUED
     uint8_t *xs = nullptr;
-    u64 xs_chunk = 0;
-    hipEvent_t xs_ev[XS_SLOTS] = {};
-    bool xs_busy[XS_SLOTS] = {};
-    int xs_next = 0;
+    u64 xs_head = 0;
+    std::deque<XsRegion> xs_used;
+    hipEvent_t xs_ev[XS_EVENTS] = {};
+    int xs_next_ev = 0;
+    u32 *xs_ctr = nullptr;    // device: workgroups done with each chunk of a download
+    u32 xs_tick = 0;          // value that marks the current download's chunks in the pinned flags
     Timer timer;
     sagpu_stats stats{};
     bool sort_u32 = false;  // the radix passes being timed are u32-key passes
@@ -442,6 +539,7 @@ void ctx_destroy(Ctx *c)
         if (e) (void)hipGraphExecDestroy(e);
     if (c->stage) (void)hipHostFree(c->stage);
     if (c->xs) (void)hipHostFree(c->xs);
+    if (c->xs_ctr) c->pool.put(c->xs_ctr);
     for (auto &e : c->xs_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->small_io) (void)hipHostFree(c->small_io);
@@ -1385,97 +1483,253 @@ int plcp_run(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, const u32 *PH
                        cs && g_stream_compare ? cs->pw : nullptr, cs ? cs->bits : 0, hint_off);
 }
 
-// Pinned slots of `chunk` bytes for the staged copies; false if the mode asks for
-// direct copies of this size (or pinned memory is not available).
-bool xs_ready(Ctx &c, u64 bytes)
+// Least size of a staged copy, in device bytes.  libsais_lcp of 600,000 entries (three
+// copies of 2.4 MB): 312 us direct, 345 us staged; 1,200,000: 560 and 500 us.  64-bit
+// arrays save half the bus time: 150,000 entries (0.6 MB on the device) 204 us direct, 275 us
+// staged; 300,000: 328 and 255 us.
+constexpr u64 XS_MIN = 4u << 20, XS_MIN_INDEX64 = 1u << 20;
+
+// Chunks of a download in the ring, and the workgroups that copy them: every workgroup
+// fences each chunk (about 0.1 us in all), so 256 of them reach 35 GB/s with 1 MiB chunks,
+// 128 49 GB/s; a plain copy 56.
+constexpr u32 XP_CHUNKS = 64, XP_WGS = 64;
+
+// Whether a copy of this size is staged (and pinned memory is available).
+bool xs_ready(Ctx &c, u64 bytes, u64 least = XS_MIN)
 {
-    if (g_host_staging == 0 || (g_host_staging == 1 && bytes < (4u << 20))) return false;
-    const u64 chunk = g_host_staging == 2 ? (64u << 10) : (32u << 20);
-    if (c.xs && c.xs_chunk == chunk) return true;
-    if (c.xs) {
-        for (int q = 0; q < XS_SLOTS; q++)
-            if (c.xs_busy[q]) (void)hipEventSynchronize(c.xs_ev[q]);
-        (void)hipHostFree(c.xs);
-        c.xs = nullptr;
-    }
-    for (int q = 0; q < XS_SLOTS; q++) {
-        c.xs_busy[q] = false;
-        if (!c.xs_ev[q] && hipEventCreateWithFlags(&c.xs_ev[q], hipEventDisableTiming) != hipSuccess) {
+    if (g_host_staging == 0 || (g_host_staging == 1 && bytes < least)) return false;
+    if (c.xs) return true;
+    for (auto &e : c.xs_ev)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
             return false;
         }
+    if (!c.xs_ctr) {
+        c.xs_ctr = (u32 *)c.pool.get(XP_CHUNKS * sizeof(u32));
+        if (!c.xs_ctr) return false;
+        if (launch_fill_u32(c.xs_ctr, XP_CHUNKS, 0, c.stream) != SAGPU_OK) return false;
     }
-    if (hipHostMalloc((void **)&c.xs, XS_SLOTS * chunk, hipHostMallocDefault) != hipSuccess) {
+    // the ring, then the flags of a download's chunks
+    g_device_allocs++;
+    if (hipHostMalloc((void **)&c.xs, XS_RING + XP_CHUNKS * sizeof(u32), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         c.xs = nullptr;
         return false;
     }
-    c.xs_chunk = chunk;
+    memset(c.xs + XS_RING, 0, XP_CHUNKS * sizeof(u32));
     return true;
 }
 
-// Host to device on the context's stream.  Returns once every byte of src has
-// been read, so the caller may then overwrite it (outputs that alias inputs);
-// the DMA of the last chunks may still be running.
-int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
+// Bytes of upload chunk k, and of the parts its host copy is split into.  The first
+// chunks are small, so that DMA and host copies overlap from early on; later ones keep
+// the DMA's start-up small beside it (a 4 MiB chunk takes 73 us).
+u64 xs_chunk(int k) { return g_host_staging == 2 ? 64u << 10 : k < 4 ? (512ull << 10) << k : k < 8 ? 4ull << 20 : 8ull << 20; }
+u64 xs_part() { return g_host_staging == 2 ? 16u << 10 : 128u << 10; }
+
+// An event after everything queued so far: it frees every region queued before it.
+int xs_mark(Ctx &c)
 {
-    if (!bytes) return SAGPU_OK;
-    if (!xs_ready(c, bytes)) {
-        SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
-        return SAGPU_OK;
-    }
-    const int th = copy_threads();
-    for (u64 off = 0; off < bytes; off += c.xs_chunk) {
-        const int q = c.xs_next;
-        c.xs_next = (q + 1) % XS_SLOTS;
-        if (c.xs_busy[q]) {
-            SAGPU_CHECK(hipEventSynchronize(c.xs_ev[q]));
-            c.xs_busy[q] = false;
+    const int ev = c.xs_next_ev;
+    c.xs_next_ev = (ev + 1) % XS_EVENTS;
+    for (auto &r : c.xs_used)   // an event still in use covers what comes before it, too
+        if (r.ev == ev) {
+            SAGPU_CHECK(hipEventSynchronize(c.xs_ev[ev]));
+            break;
         }
-        const u64 len = bytes - off < c.xs_chunk ? bytes - off : c.xs_chunk;
-        uint8_t *slot = c.xs + (u64)q * c.xs_chunk;
-        copies().copy(slot, (const uint8_t *)src + off, len, th);
-        SAGPU_CHECK(hipMemcpyAsync((uint8_t *)dst + off, slot, len, hipMemcpyHostToDevice, c.stream));
-        SAGPU_CHECK(hipEventRecord(c.xs_ev[q], c.stream));
-        c.xs_busy[q] = true;
-    }
+    while (!c.xs_used.empty() && c.xs_used.front().ev == ev) c.xs_used.pop_front();
+    SAGPU_CHECK(hipEventRecord(c.xs_ev[ev], c.stream));
+    for (auto &r : c.xs_used)
+        if (r.ev == XS_QUEUED) r.ev = ev;
     return SAGPU_OK;
 }
 
-// Device to host after the work already queued on the context's stream.  With
-// staging it returns with every byte in dst; the direct form leaves the copy to
-// the caller's stream synchronisation.
+// Takes the ring's next `len` bytes for an upload.  Regions of finished DMAs in the way
+// are given back, after waiting for them when `block`.  *ok = false when the space is
+// not free yet.
+int xs_take(Ctx &c, u64 len, bool block, u64 *at, bool *ok)
+{
+    *ok = false;
+    const u64 head = c.xs_head + len > XS_RING ? 0 : c.xs_head;
+    for (;;) {
+        bool clash = false;
+        for (const auto &r : c.xs_used)
+            if (head < r.at + r.len && r.at < head + len) clash = true;
+        if (!clash) break;
+        if (c.xs_used.front().ev == XS_QUEUED) SAGPU_TRY(xs_mark(c));
+        const int ev = c.xs_used.front().ev;   // regions are freed in order
+        if (ev < 0) return SAGPU_OK;
+        if (!block && hipEventQuery(c.xs_ev[ev]) == hipErrorNotReady) return SAGPU_OK;
+        SAGPU_CHECK(hipEventSynchronize(c.xs_ev[ev]));
+        while (!c.xs_used.empty() && c.xs_used.front().ev == ev) c.xs_used.pop_front();
+    }
+    c.xs_used.push_back({head, len, XS_TODO});
+    c.xs_head = head + len;
+    *at = head;
+    *ok = true;
+    return SAGPU_OK;
+}
+
+// Ends a transfer's host copies; a failed one also gives the whole ring back.
+struct XsGuard {
+    Ctx &c;
+    CopyPool::Job &j;
+    bool fine = false;
+    ~XsGuard()
+    {
+        if (!fine) {
+            (void)hipStreamSynchronize(c.stream);
+            (void)hipGetLastError();
+        }
+        copies().end(j);
+        if (!fine) {
+            c.xs_used.clear();
+            c.xs_head = 0;
+        }
+    }
+};
+
+// Host to device on the context's stream: `bytes` device bytes; narrow: src holds int64
+// entries that become u32.  Returns once every byte of src has been read, so the
+// caller may then overwrite it (outputs that alias inputs); the DMA of the last
+// chunks may still be running.
+int h2d_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool narrow)
+{
+    CopyPool::Job j(bytes / xs_part() + bytes / xs_chunk(0) + 2);   // (every chunk may end in a short part)
+    copies().begin(j, copy_threads());
+    XsGuard guard{c, j};
+    // an idle ring starts over: its first pages are the ones the CPU has mapped and cached
+    if (!c.xs_used.empty() && c.xs_used.back().ev >= 0 && hipEventQuery(c.xs_ev[c.xs_used.back().ev]) == hipSuccess)
+        c.xs_used.clear();
+    if (c.xs_used.empty()) c.xs_head = 0;
+    struct Sent { u64 off; int upto; };   // a chunk's place in dst, and the parts through its end
+    std::deque<Sent> ahead;               // chunks whose DMA is not queued yet
+    u64 given = 0;
+    for (int k = 0; given < bytes || !ahead.empty();) {
+        // regions and host copies of the chunks ahead of the DMA
+        while (given < bytes && (int)ahead.size() < XS_AHEAD) {
+            const u64 len = bytes - given < xs_chunk(k) ? bytes - given : xs_chunk(k);
+            u64 at = 0;
+            bool ok;
+            SAGPU_TRY(xs_take(c, len, ahead.empty(), &at, &ok));
+            if (!ok) break;
+            copies().grant(j, {c.xs + at, (const uint8_t *)src + (narrow ? 2 : 1) * given, len, narrow ? 1 : 0},
+                           xs_part());
+            ahead.push_back({given, j.granted.load()});
+            given += len;
+            k++;
+        }
+        copies().wait(j, ahead.front().upto);
+        Ctx::XsRegion &r = c.xs_used[c.xs_used.size() - ahead.size()];
+        SAGPU_CHECK(hipMemcpyAsync((uint8_t *)dst + ahead.front().off, c.xs + r.at, r.len, hipMemcpyHostToDevice,
+                                   c.stream));
+        r.ev = XS_QUEUED;
+        ahead.pop_front();
+    }
+    SAGPU_TRY(xs_mark(c));
+    guard.fine = true;
+    return SAGPU_OK;
+}
+
+// Copies device memory into the pinned ring, chunk after chunk, each divided over all
+// workgroups; the workgroup that finishes a chunk last sets its flag, so the host can
+// drain it while the kernel goes on.  (Single hipMemcpyAsync calls with an event each
+// leave the bus idle for about 18 us per chunk.)  ctr: a counter per chunk, zero before
+// and after.
+__global__ __launch_bounds__(256) void k_push(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, u64 bytes,
+                                              u64 chunk, u32 *__restrict__ ctr, u32 *__restrict__ flags, u32 tick)
+{
+    u32 k = 0;
+    for (u64 off = 0; off < bytes; off += chunk, k++) {
+        const u64 len = bytes - off < chunk ? bytes - off : chunk;
+        const uint4 *s = reinterpret_cast<const uint4 *>(src + off);
+        uint4 *d = reinterpret_cast<uint4 *>(dst + off);
+        for (u64 i = (u64)blockIdx.x * 256 + threadIdx.x; i < len / 16; i += (u64)gridDim.x * 256) d[i] = s[i];
+        if (blockIdx.x == 0 && threadIdx.x < len % 16)
+            dst[off + len / 16 * 16 + threadIdx.x] = src[off + len / 16 * 16 + threadIdx.x];
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0 && atomicAdd(&ctr[k], 1u) == gridDim.x - 1) {
+            ctr[k] = 0;
+            __threadfence_system();
+            __hip_atomic_store(&flags[k], tick, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
+// Device to host after the work already queued on the context's stream: `bytes` device
+// bytes (src aligned to 16); widen: u32 entries become int64.  Returns with every byte
+// in dst.
+int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool widen)
+{
+    CopyPool::Job j(bytes / xs_part() + bytes / xs_chunk(0) + 2);
+    copies().begin(j, copy_threads());
+    XsGuard guard{c, j};
+    volatile u32 *flags = (volatile u32 *)(c.xs + XS_RING);
+    // two halves of the ring, a kernel each; a half is filled again once it is drained
+    const u64 half = XS_RING / 2, chunk = g_host_staging == 2 ? 64u << 10 : bytes < (32u << 20) ? 1u << 20 : 4u << 20;
+    const u64 batch = chunk * (XP_CHUNKS / 2) < half ? chunk * (XP_CHUNKS / 2) : half;
+    const u64 nb = (bytes + batch - 1) / batch;
+    const u64 per = widen ? 2 * xs_part() : xs_part();
+    std::vector<int> upto(nb + 1, 0);   // parts through the end of every batch
+    u32 ticks[2] = {0, 0};
+    auto launch = [&](u64 b) -> int {
+        const u64 off = b * batch, len = bytes - off < batch ? bytes - off : batch;
+        const u32 side = (u32)(b & 1);
+        ticks[side] = ++c.xs_tick;
+        const u64 wgs = (len + 8191) / 8192;
+        hipLaunchKernelGGL(k_push, dim3((unsigned)(wgs < XP_WGS ? wgs : XP_WGS)), dim3(256), 0, c.stream,
+                           (const uint8_t *)src + off, c.xs + side * half, len, chunk, c.xs_ctr + side * (XP_CHUNKS / 2),
+                           (u32 *)flags + side * (XP_CHUNKS / 2), ticks[side]);
+        SAGPU_CHECK(hipGetLastError());
+        return SAGPU_OK;
+    };
+    for (u64 b = 0; b < nb && b < 2; b++) SAGPU_TRY(launch(b));
+    for (u64 b = 0; b < nb; b++) {
+        const u64 off = b * batch, len = bytes - off < batch ? bytes - off : batch;
+        const u32 side = (u32)(b & 1);
+        u32 k = side * (XP_CHUNKS / 2);
+        for (u64 o = 0; o < len; o += chunk, k++) {
+            for (u32 spins = 1; flags[k] != ticks[side]; spins++) {
+                __builtin_ia32_pause();
+                // a stream that has stopped (or failed) sets no more flags
+                if (spins % 65536 == 0 && hipStreamQuery(c.stream) != hipErrorNotReady && flags[k] != ticks[side]) {
+                    SAGPU_CHECK(hipStreamSynchronize(c.stream));
+                    if (flags[k] == ticks[side]) break;
+                    sagpu_set_error("download stopped early", __FILE__, __LINE__);
+                    return SAGPU_EDEVICE;
+                }
+            }
+            std::atomic_thread_fence(std::memory_order_acquire);
+            const u64 l = len - o < chunk ? len - o : chunk;
+            copies().grant(j, {(uint8_t *)dst + (widen ? 2 : 1) * (off + o), c.xs + side * half + o, widen ? 2 * l : l,
+                               widen ? 2 : 0}, per);
+        }
+        upto[b + 1] = j.granted.load();
+        // the half of batch b + 1 is being filled or drained; batch b + 2 needs this one
+        if (b + 2 < nb) {
+            copies().wait(j, upto[b + 1]);
+            SAGPU_TRY(launch(b + 2));
+        }
+    }
+    copies().wait(j, j.granted.load());
+    guard.fine = true;
+    return SAGPU_OK;
+}
+
+int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
+{
+    if (!bytes) return SAGPU_OK;
+    if (xs_ready(c, bytes)) return h2d_staged(c, dst, src, bytes, false);
+    SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+    return SAGPU_OK;
+}
+
+// The direct form leaves the copy to the caller's stream synchronisation.
 int d2h(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    if (!xs_ready(c, bytes)) {
-        SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
-        return SAGPU_OK;
-    }
-    const int th = copy_threads();
-    const u64 ch = c.xs_chunk, nch = (bytes + ch - 1) / ch;
-    auto issue = [&](u64 k) -> int {
-        const int q = (int)(k % XS_SLOTS);
-        if (c.xs_busy[q]) {
-            SAGPU_CHECK(hipEventSynchronize(c.xs_ev[q]));
-            c.xs_busy[q] = false;
-        }
-        const u64 len = bytes - k * ch < ch ? bytes - k * ch : ch;
-        SAGPU_CHECK(hipMemcpyAsync(c.xs + (u64)q * ch, (const uint8_t *)src + k * ch, len, hipMemcpyDeviceToHost,
-                                   c.stream));
-        SAGPU_CHECK(hipEventRecord(c.xs_ev[q], c.stream));
-        c.xs_busy[q] = true;
-        return SAGPU_OK;
-    };
-    for (u64 k = 0; k < nch && k < (u64)XS_SLOTS; k++) SAGPU_TRY(issue(k));
-    for (u64 k = 0; k < nch; k++) {
-        const int q = (int)(k % XS_SLOTS);
-        SAGPU_CHECK(hipEventSynchronize(c.xs_ev[q]));
-        c.xs_busy[q] = false;
-        const u64 len = bytes - k * ch < ch ? bytes - k * ch : ch;
-        copies().copy((uint8_t *)dst + k * ch, c.xs + (u64)q * ch, len, th);
-        if (k + XS_SLOTS < nch) SAGPU_TRY(issue(k + XS_SLOTS));
-    }
+    if ((uintptr_t)src % 16 == 0 && xs_ready(c, bytes)) return d2h_staged(c, dst, src, bytes, false);
+    SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
     return SAGPU_OK;
 }
 
@@ -1690,6 +1944,8 @@ int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 {
     if (width == 4) {
         SAGPU_TRY(d2h(c, h, d, n * 4));
+    } else if (n && xs_ready(c, n * 4, XS_MIN_INDEX64)) {
+        SAGPU_TRY(d2h_staged(c, h, d, n * 4, true));
     } else {
         GET(w, int64_t, n);
         hipLaunchKernelGGL(k_widen, dim3(grid_n(n)), dim3(256), 0, c.stream, d, w, n);
@@ -1703,6 +1959,8 @@ int upload_idx(Ctx &c, Scope &sc, const void *h, u64 n, int width, u32 **out)
     GET(d, u32, n);
     if (width == 4) {
         SAGPU_TRY(h2d(c, d, h, n * 4));
+    } else if (n && xs_ready(c, n * 4, XS_MIN_INDEX64)) {
+        SAGPU_TRY(h2d_staged(c, d, h, n * 4, true));
     } else {
         GET(w, int64_t, n);
         SAGPU_TRY(h2d(c, w, h, n * 8));
@@ -2852,6 +3110,7 @@ extern "C" int32_t sagpu_gsa_batch32(const uint8_t *d_T, int64_t n, const int64_
 
 #include <chrono>
 #include <condition_variable>
+#include <deque>
 #include <deque>
 #include <thread>
 
