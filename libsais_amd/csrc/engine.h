@@ -215,29 +215,39 @@ struct ExactLcp {
     }
 };
 // Rounds.  wide = 0: key2 is u32 (n < 2^31); wide = 1: key2 is u64 (n up to 2^32).
-// The round's list length a and offset h are read from rp[0], rp[1] in device memory
-// (the launch geometry is sized on the host for a list of a_grid entries, which
-// must be at least rp[0]), so one captured launch serves every later round.
+// The round's list length a and offset h live in device memory, rp[0] and rp[1]: put
+// there by its gather kernel (RoundStart with h > 0) or by the end of the round
+// before (h = 0).  The launch geometry is sized on the host for a list of a_grid
+// entries, which must be at least the length.
+struct RoundStart {
+    u64 h;              // 0: take rp as it stands
+    u64 a;              // the length, or where to read it
+    const u64 *a_src;
+};
 extern int g_tile_range;
 // rows of 64 positions per wave span in the initial grouping of texts of at least
 // INIT_SMALL_N suffixes (8 or 16: tiles of 2048 or 4096 positions; the "init_rows" option)
 extern int g_init_rows;   // list entries per workgroup of the tile kernel (the "tile_range" option)
-int round_gather(const u32 *act_i, const u32 *act_g, u64 a_grid, const u64 *rp, const u32 *ISA, u64 n, void *key2,
-                 int wide, hipStream_t s, const RawKey1 *rk = nullptr, int cb = 0);
+// Sets rp for a round whose gather takes it as it stands (a captured one).
+int launch_round_start(u64 *rp, u64 a, u64 h, hipStream_t s);
+// cnt: 8 u64 (0 list length out, 4 big groups | err << 32, 5 big-group members); the
+// gather clears them and seg_ctr (128 u64).
+int round_gather(const u32 *act_i, const u32 *act_g, u64 a_grid, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
+                 const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk = nullptr, int cb = 0);
 // The tile kernel's survivors go to 8 per-XCD segments of seg_i / seg_g (capacity
 // 8 * round_seg_cap(a_grid) each) and are concatenated into out_i / out_g, whose
-// length goes to *out_counter; seg_ctr: 128 u64.  Big-group heads go the same way
-// to 8 segments of bseg_h / bseg_g (round_bigseg_cap(n) entries each, n >= every
-// list length) and are concatenated into big_head / big_g / big_size, their count
-// to *big_counter; boff (big_cap + 1 entries) gets their offsets in the
-// concatenation of their members, *big_total the member count.
+// length goes to cnt[0].  Big-group heads go the same way to 8 segments of bseg_h /
+// bseg_g (round_bigseg_cap(n) entries each, n >= every list length) and are
+// concatenated into big_head / big_g / big_size; boff (big_cap + 1 entries) gets their
+// offsets in the concatenation of their members.  rec (pinned, 7 u64) receives cnt's
+// words at their indexes and in rec[6], last, the length the round started with;
+// rp_next the next round's length (0 when there are big groups) and offset.
 u64 round_seg_cap(u64 a);
 u64 round_bigseg_cap(u64 n);
-int round_tile(const u32 *act_i, const u32 *act_g, const void *key2, int wide, u64 a_grid, const u64 *rp, u32 *SA,
-               u32 *ISA, u32 *out_i, u32 *out_g, u64 *out_counter, u32 *err, u32 *big_head, u32 *big_g, u32 *big_size,
-               u32 *big_counter, u64 big_cap, u32 *LCP, hipStream_t s, const ActCode &ac, const ExactLcp *ex,
-               u32 *seg_i, u32 *seg_g, u64 *seg_ctr, u32 *bseg_h, u32 *bseg_g, u64 bseg_cap, u64 *boff,
-               u64 *big_total);
+int round_tile(const u32 *act_i, const u32 *act_g, const void *key2, int wide, u64 a_grid, const u64 *rp, u64 *rp_next,
+               u64 *rec, u32 *SA, u32 *ISA, u32 *out_i, u32 *out_g, u64 *cnt, u32 *big_head, u32 *big_g, u32 *big_size,
+               u64 big_cap, u32 *LCP, hipStream_t s, const ActCode &ac, const ExactLcp *ex, u32 *seg_i, u32 *seg_g,
+               u64 *seg_ctr, u32 *bseg_h, u32 *bseg_g, u64 bseg_cap, u64 *boff);
 // ISA[PV[e]] = PG[e] for e < m, in the pairs' order.
 int launch_isa_scatter(const u32 *PV, const u32 *PG, u64 m, u32 *ISA, hipStream_t s);
 // The same for pairs grouped into windows of the target by a radix pass on bits

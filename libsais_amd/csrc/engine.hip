@@ -375,7 +375,9 @@ CopyPool &copies()
 enum Family { F_ONESWEEP = 0, F_ONESWEEP32, F_INITIAL, F_ROUNDS, F_BWT, F_PLCP, F_LCP, F_TOTAL, F_PLCP_PAIRS, F_COUNT };
 constexpr int F_KERNEL0 = 64;   // + KernelId: one kernel's launches
 
-constexpr int ROUND_SIG = 31;   // words of a round's launch signature (Ctx::round_sig)
+// Rounds with shorter lists are queued two at a time (sa_build).
+constexpr u64 ROUND_AHEAD = 1ull << 20;
+constexpr int ROUND_SIG = 32;   // words of a round's launch signature (Ctx::round_sig)
 
 struct Ctx {
     int device = 0;
@@ -1056,7 +1058,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     GET(bseg_h, u32, 8 * bseg_cap);
     GET(bseg_g, u32, 8 * bseg_cap);
     u64 *out_counter = d_cnt;
-    u32 *big_counter = (u32 *)(d_cnt + 4), *err = (u32 *)(d_cnt + 4) + 1;
+    u32 *err = (u32 *)(d_cnt + 4) + 1;
     u32 *act_i[2] = {aA, kA}, *act_g[2] = {aA + n, kA + n};
     void *key2 = vA;
 
@@ -1168,7 +1170,6 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     // the device (its kernels stop at the list's end); the host learns it with the
     // round's counters.
     const bool lazy_a = !a_known && n < INIT_SMALL_N && !rk1.pw;
-    u64 *h_a1 = c.pinned + 7204;   // past the round parameters and the pivot regions
     if (lazy_a) {
         a = n;
     } else {
@@ -1185,129 +1186,154 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     u64 h = (u64)ksym;
     int cur = 0;
     st.rounds = 0;
-    // The round's list length and offset reach the kernels through device memory
-    // (d_rp), copied from pinned memory as the round's first operation, so rounds
-    // from the second on replay one captured graph per buffer parity: parameter copy,
-    // gather, counter reset, tile kernel, big-group sizes, counter copy back.  The
-    // graph's launch geometry is sized for the round it was captured in; later
-    // rounds of the same parity have shorter lists.
-    GET(d_rp, u64, 2);
-    u64 *h_rp = c.pinned + 7168;   // past the histogram, LUT and tail-rank staging
+    // A round is three kernels: gather, tile, end (five for long lists).  Its length and
+    // offset live in device memory, where the round's start puts them or the round
+    // before leaves them, so a round can be queued before the host knows the outcome
+    // of the one before: with big groups left, it finds a length of 0 and does nothing.
+    // Rounds from the second on replay one captured graph per buffer parity, whose
+    // launch geometry is sized for a list at least as long as the round's.
+    GET(d_rp, u64, 4);   // by parity
+    u64 *const rec[2] = {c.pinned, c.pinned + 32};   // a round's report, by parity
     // per-XCD survivor segments of the tile kernel, sized for the first (longest) list
-    const u64 seg_words = 8 * round_seg_cap(a);
+    const u64 a_first = a, seg_words = 8 * round_seg_cap(a_first);
     GET(seg_i, u32, seg_words);
     GET(seg_g, u32, seg_words);
     GET(seg_ctr, u64, 128);
     // (not in the allocation-free build: instantiating a graph allocates)
     const bool graphs = g_round_graphs && !c.timer.on && !c.pool.arena;
     bool captured[2] = {false, false};
-    while (a > 0) {
-        if (st.rounds < 64) st.active[st.rounds] = (int64_t)a;
-        st.rounds++;
-        const int nxt = cur ^ 1;
-        h_rp[0] = a;
-        h_rp[1] = h;
-        const bool raw = st.rounds == 1 && rk1.pw;
-        const bool lazy_first = lazy_a && st.rounds == 1;
-        // one round's work on the stream (launch geometry for a_grid entries)
-        auto enqueue = [&](u64 a_grid, bool timed) -> int {
-            SAGPU_CHECK(hipMemcpyAsync(d_rp, h_rp, 2 * sizeof(u64), hipMemcpyHostToDevice, s));
-            if (lazy_first) SAGPU_CHECK(hipMemcpyAsync(d_rp, ws.total, sizeof(u64), hipMemcpyDeviceToDevice, s));
+    constexpr u64 NOT_RUN = ~0ull;
+
+    // Queues the round of parity p: a list of at most a_most entries, of exactly that many
+    // and offset h when `given`, else as the round before leaves it.
+    auto launch = [&](int p, u64 a_most, u64 h, bool given, bool raw, const u64 *a_src) -> int {
+        Span sp(c, F_ROUNDS);
+        // the geometry of lists below 2^20 entries is sized by powers of two, so that the
+        // graphs of one build serve the next one of the same size
+        u64 a_grid = a_most;
+        if (a_most < (1ull << 20)) {
+            a_grid = 4096;
+            while (a_grid < a_most) a_grid *= 2;
+            if (a_grid > a_first) a_grid = a_first;
+        }
+        rec[p][6] = NOT_RUN;
+        auto enqueue = [&](const RoundStart &st, bool timed) -> int {
             if (timed) ktime_begin(KI_ROUND_GATHER);
-            SAGPU_TRY(round_gather(act_i[cur], act_g[cur], a_grid, d_rp, dISA, n, key2, wide, s, raw ? &rk1 : nullptr,
-                                   ac.cb));
+            SAGPU_TRY(round_gather(act_i[p], act_g[p], a_grid, d_rp + 2 * p, st, d_cnt, seg_ctr, dISA, n, key2, wide,
+                                   s, raw ? &rk1 : nullptr, ac.cb));
             // suffix read, one random 4-byte read (rank, or code-stream window), key
             // written (+ the group read for the first round's form)
-            if (timed) ktime_end(KI_ROUND_GATHER, a * ((wide ? 16 : 12) + (raw ? 4 : 0)));
-            SAGPU_TRY(launch_fill_u64(d_cnt, 8, 0, s));
+            if (timed) ktime_end(KI_ROUND_GATHER, a_most * ((wide ? 16 : 12) + (raw ? 4 : 0)));
             // (the tile kernel is timed inside round_tile; the timer is off while a
             // round is captured)
-            SAGPU_TRY(round_tile(act_i[cur], act_g[cur], key2, wide, a_grid, d_rp, dSA, dISA, act_i[nxt], act_g[nxt],
-                                 out_counter, err, big_head, big_g, big_size, big_counter, big_cap, dLCP, s, ac,
-                                 raw ? &ex1 : nullptr, seg_i, seg_g, seg_ctr, bseg_h, bseg_g, bseg_cap, d_boff,
-                                 d_cnt + 5));
-            SAGPU_CHECK(hipMemcpyAsync(c.pinned, d_cnt, 6 * sizeof(u64), hipMemcpyDeviceToHost, s));
-            if (lazy_first) SAGPU_CHECK(hipMemcpyAsync(h_a1, d_rp, sizeof(u64), hipMemcpyDeviceToHost, s));
-            return SAGPU_OK;
+            return round_tile(act_i[p], act_g[p], key2, wide, a_grid, d_rp + 2 * p, d_rp + 2 * (p ^ 1), rec[p], dSA,
+                              dISA, act_i[p ^ 1], act_g[p ^ 1], d_cnt, big_head, big_g, big_size, big_cap, dLCP, s, ac,
+                              raw ? &ex1 : nullptr, seg_i, seg_g, seg_ctr, bseg_h, bseg_g, bseg_cap, d_boff);
         };
-        {
-            Span sp(c, F_ROUNDS);
-            if (graphs && !raw && st.rounds >= 2) {
-                hipGraphExec_t &exec = c.round_exec[cur];
-                // every argument and launch size the round's operations take
-                const u64 sig[ROUND_SIG] = {(u64)act_i[cur], (u64)act_g[cur], (u64)act_i[nxt], (u64)act_g[nxt],
-                                            (u64)key2, (u64)dISA, (u64)dSA, (u64)dLCP, (u64)d_cnt, (u64)big_head,
-                                            (u64)big_g, (u64)big_size, (u64)ac.codes, (u64)d_rp, (u64)c.pinned,
-                                            (u64)seg_i, (u64)seg_g, (u64)seg_ctr, (u64)ac.cb, a, n, (u64)wide,
-                                            (u64)g_tile_range, big_cap, (u64)(dLCP != nullptr), (u64)bseg_h,
-                                            (u64)bseg_g, bseg_cap, (u64)ac.gf, (u64)d_boff, (u64)exec};
-                if (!captured[cur] && exec && !memcmp(sig, c.round_sig[cur], sizeof sig)) captured[cur] = true;
-                if (!captured[cur]) {
-                    // capture this parity's round once per build; the executable graph of
-                    // the previous build is updated when its topology still matches
-                    SAGPU_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                    const int rc = enqueue(a, false);
-                    hipGraph_t graph = nullptr;
-                    const hipError_t ec = hipStreamEndCapture(s, &graph);
-                    if (rc != SAGPU_OK || ec != hipSuccess) {
-                        if (graph) (void)hipGraphDestroy(graph);
-                        (void)hipGetLastError();
-                        if (rc != SAGPU_OK) return rc;
-                        sagpu_set_error("round graph capture failed", __FILE__, __LINE__);
-                        return SAGPU_EDEVICE;
-                    }
-                    bool ok = false;
-                    if (exec) {
-                        hipGraphNode_t bad = nullptr;
-                        hipGraphExecUpdateResult ur;
-                        ok = hipGraphExecUpdate(exec, graph, &bad, &ur) == hipSuccess &&
-                             ur == hipGraphExecUpdateSuccess;
-                        if (!ok) {
-                            (void)hipGetLastError();
-                            (void)hipGraphExecDestroy(exec);
-                            exec = nullptr;
-                        }
-                    }
-                    if (!ok && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
-                        (void)hipGetLastError();
-                        exec = nullptr;
-                        (void)hipGraphDestroy(graph);
-                        sagpu_set_error("round graph instantiation failed", __FILE__, __LINE__);
-                        return SAGPU_EDEVICE;
-                    }
-                    (void)hipGraphDestroy(graph);
-                    captured[cur] = true;
-                    st.round_graphs++;
-                    memcpy(c.round_sig[cur], sig, sizeof sig);
-                    c.round_sig[cur][ROUND_SIG - 1] = (u64)exec;   // the executable graph now serving them
+        if (!graphs || st.rounds < 1) return enqueue(given ? RoundStart{h, a_most, a_src} : RoundStart{}, true);
+        if (given) SAGPU_TRY(launch_round_start(d_rp + 2 * p, a_most, h, s));
+        hipGraphExec_t &exec = c.round_exec[p];
+        // every argument and launch size the round's operations take
+        const u64 sig[ROUND_SIG] = {(u64)act_i[p], (u64)act_g[p], (u64)act_i[p ^ 1], (u64)act_g[p ^ 1],
+                                    (u64)key2, (u64)dISA, (u64)dSA, (u64)dLCP, (u64)d_cnt, (u64)big_head,
+                                    (u64)big_g, (u64)big_size, (u64)ac.codes, (u64)d_rp, (u64)c.pinned,
+                                    (u64)seg_i, (u64)seg_g, (u64)seg_ctr, (u64)ac.cb, a_grid, n, (u64)wide,
+                                    (u64)g_tile_range, big_cap, (u64)(dLCP != nullptr), (u64)bseg_h,
+                                    (u64)bseg_g, bseg_cap, (u64)ac.gf, (u64)d_boff, (u64)p, (u64)exec};
+        if (!captured[p] && exec && !memcmp(sig, c.round_sig[p], sizeof sig)) captured[p] = true;
+        if (!captured[p]) {
+            // capture this parity's round once per build; the executable graph of
+            // the previous build is updated when its topology still matches
+            SAGPU_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+            const int rc = enqueue(RoundStart{}, false);
+            hipGraph_t graph = nullptr;
+            const hipError_t ec = hipStreamEndCapture(s, &graph);
+            if (rc != SAGPU_OK || ec != hipSuccess) {
+                if (graph) (void)hipGraphDestroy(graph);
+                (void)hipGetLastError();
+                if (rc != SAGPU_OK) return rc;
+                sagpu_set_error("round graph capture failed", __FILE__, __LINE__);
+                return SAGPU_EDEVICE;
+            }
+            bool ok = false;
+            if (exec) {
+                hipGraphNode_t bad = nullptr;
+                hipGraphExecUpdateResult ur;
+                ok = hipGraphExecUpdate(exec, graph, &bad, &ur) == hipSuccess && ur == hipGraphExecUpdateSuccess;
+                if (!ok) {
+                    (void)hipGetLastError();
+                    (void)hipGraphExecDestroy(exec);
+                    exec = nullptr;
                 }
-                SAGPU_CHECK(hipGraphLaunch(exec, s));
-                st.round_graph_launches++;
-            } else {
-                SAGPU_TRY(enqueue(a, true));
             }
-        }
-        SAGPU_CHECK(hipStreamSynchronize(s));
-        if (lazy_first) {
-            a = *h_a1;
-            st.active[0] = (int64_t)a;
-            if (a == 0) {   // nothing was grouped: no round ran
-                st.rounds = 0;
-                break;
+            if (!ok && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                exec = nullptr;
+                (void)hipGraphDestroy(graph);
+                sagpu_set_error("round graph instantiation failed", __FILE__, __LINE__);
+                return SAGPU_EDEVICE;
             }
+            (void)hipGraphDestroy(graph);
+            captured[p] = true;
+            c.stats.round_graphs++;
+            memcpy(c.round_sig[p], sig, sizeof sig);
+            c.round_sig[p][ROUND_SIG - 1] = (u64)exec;   // the executable graph now serving them
         }
-        u64 out_n = c.pinned[0];
-        const u32 nb = ((u32 *)(c.pinned + 4))[0];
-        if (nb > big_cap || ((u32 *)(c.pinned + 4))[1] != 0 || out_n > a) {
+        SAGPU_CHECK(hipGraphLaunch(exec, s));
+        return SAGPU_OK;
+    };
+
+    bool queued = false, left = false;   // this round is on the stream already; its length is in rp
+    while (a > 0) {
+        const bool raw = st.rounds == 0 && rk1.pw;
+        const bool lazy_first = lazy_a && st.rounds == 0;
+        bool ahead = false;   // the next round was queued behind this one
+        if (!queued) {
+            SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr));
+            // Short rounds cost their launches and the host's wait: queue the next one
+            // behind (its three kernels cost about 12 us when they find nothing to do,
+            // a wait and a late launch about 20)
+            ahead = a < ROUND_AHEAD && !c.timer.on;
+            if (ahead) {
+                st.rounds++;   // (a queued second round is one that replays a graph)
+                const int rc = launch(cur ^ 1, a, 0, false, false, nullptr);
+                st.rounds--;
+                SAGPU_TRY(rc);
+            }
+            SAGPU_CHECK(hipStreamSynchronize(s));
+        }
+        queued = false;
+        if (rec[cur][6] == NOT_RUN) {   // an empty list (the first round's, read on the device)
+            if (!lazy_first) {
+                sagpu_set_error("a queued round did not run", __FILE__, __LINE__);
+                return SAGPU_EDEVICE;
+            }
+            a = 0;
+            break;
+        }
+        if (lazy_first) a = rec[cur][6];
+        if (rec[cur][6] != a) {
+            sagpu_set_error("round length inconsistent", __FILE__, __LINE__);
+            return SAGPU_EDEVICE;
+        }
+        if (st.rounds < 64) st.active[st.rounds] = (int64_t)a;
+        st.rounds++;
+        if (graphs && st.rounds >= 2) st.round_graph_launches++;
+        const int nxt = cur ^ 1;
+        u64 out_n = rec[cur][0];
+        const u32 nb = (u32)rec[cur][4];
+        if (nb > big_cap || rec[cur][4] >> 32 != 0 || out_n > a) {
             sagpu_set_error("round bookkeeping inconsistent", __FILE__, __LINE__);
             return SAGPU_EDEVICE;
         }
+        left = nb == 0;                  // the next round's length is in rp
+        queued = ahead && left && out_n > 0;
         if (nb > 0) {
             // Big groups in the order k_big_sizes listed them (the outputs do not
             // depend on the order of the groups), with their offsets in the
             // concatenation of their members from the round's scan (d_boff) and the
             // member count among the round's counters
-            const u64 total = c.pinned[5];
+            const u64 total = rec[cur][5];
             if (total > a) {
                 sagpu_set_error("big-group list inconsistent", __FILE__, __LINE__);
                 return SAGPU_EDEVICE;

@@ -682,12 +682,23 @@ int ws_run(WsScratch &ws, const F &f, u64 n, u64 *out_counter, hipStream_t s)
 constexpr int IG = 4;
 template <typename KT>
 __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g,
-                                                      const u64 *__restrict__ rp, const u32 *__restrict__ ISA, u64 n,
+                                                      u64 *rp, RoundStart st, u64 *__restrict__ cnt, u64 *__restrict__ seg_ctr, const u32 *__restrict__ ISA, u64 n,
                                                       KT *__restrict__ key2, RawKey1 rk, int cb)
 {
-    // the round's list length and offset come from device memory (RoundParams), so
-    // a captured launch serves every round
-    const u64 a = rp[0], h = rp[1];
+    // The round's list length and offset: from the host (its block 0 puts them where the
+    // round's other kernels read them), or left there by the round before (a length of
+    // 0: nothing to do, and nothing of the round before is touched).  Block 0 also
+    // clears the round's counters.
+    const u64 a = st.h ? (st.a_src ? *st.a_src : st.a) : rp[0], h = st.h ? st.h : rp[1];
+    if (!st.h && a == 0) return;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 128) seg_ctr[threadIdx.x] = 0;
+        if (threadIdx.x == 128) cnt[0] = cnt[4] = cnt[5] = 0;
+        if (threadIdx.x == 129 && st.h) {
+            rp[0] = a;
+            rp[1] = h;
+        }
+    }
     const u64 chunk = 256ull * IG;
     for (u64 base = (u64)blockIdx.x * chunk; base < a; base += (u64)gridDim.x * chunk) {
         u32 i[IG], r[IG];
@@ -728,6 +739,12 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
             key2[k] = raw[q] ? (KT)r[q] : ih < n ? (KT)(h + r[q]) : (KT)(n - 1 - i[q]);
         }
     }
+}
+
+__global__ void k_round_start(u64 *rp, u64 a, u64 h)
+{
+    rp[0] = a;
+    rp[1] = h;
 }
 
 constexpr int RT_THREADS = 256;
@@ -1152,31 +1169,6 @@ __global__ __launch_bounds__(RT_THREADS) void k_round_tile(const u32 *__restrict
     }
 }
 
-// The next active list from the 8 XCD segments of the tile kernel's output
-// (segment x: [x * seg_cap, x * seg_cap + seg_ctr[16 x])), concatenated in segment
-// order; *out_counter = its length (the big-group emission appends behind it).
-__global__ __launch_bounds__(256) void k_seg_gather(const u32 *__restrict__ seg_i, const u32 *__restrict__ seg_g,
-                                                    const u64 *__restrict__ seg_ctr, u64 seg_cap,
-                                                    u32 *__restrict__ out_i, u32 *__restrict__ out_g,
-                                                    u64 *__restrict__ out_counter)
-{
-    u64 pre[9];
-    pre[0] = 0;
-#pragma unroll
-    for (int x = 0; x < 8; x++) pre[x + 1] = pre[x] + seg_ctr[x * 16];
-    const u64 total = pre[8];
-    if (blockIdx.x == 0 && threadIdx.x == 0) *out_counter = total;
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    for (u64 k = (u64)blockIdx.x * blockDim.x + threadIdx.x; k < total; k += stride) {
-        int x = 0;
-#pragma unroll
-        for (int q = 1; q < 8; q++) x += k >= pre[q];
-        const u64 src = (u64)x * seg_cap + (k - pre[x]);
-        out_i[k] = seg_i[src];
-        out_g[k] = seg_g[src];
-    }
-}
-
 // The big groups the tile kernel listed, its 8 XCD segments (segment x: [x *
 // bseg_cap, x * bseg_cap + seg_ctr[16 x + 8])) concatenated in segment order, with
 // their sizes: the entry holding a big group's last list index wrote it to SA[g].
@@ -1265,6 +1257,111 @@ __global__ __launch_bounds__(1024) void k_big_offsets(const u32 *__restrict__ bi
         *total = s_carry;
     }
     if (bad) atomicOr(err, 2u);
+}
+
+// Ends a round: the next active list from the 8 XCD segments of the tile kernel's output
+// (segment x: [x * seg_cap, x * seg_cap + seg_ctr[16 x])), concatenated in segment
+// order; *out_counter = its length (the big-group emission appends behind it).  Block 0
+// then reports to the host (rec, pinned: list length, big groups | err << 32, their
+// members, the length the round started with) and leaves the next round's length and
+// offset in rp_next; with big groups, whose members the host adds first, a length of
+// 0.  MERGED (lists below END_MERGED): it also does the work of k_big_sizes and
+// k_big_offsets, two launches of about 4.5 us less per round.
+constexpr u64 END_MERGED = 1ull << 22;   // at most 2^22 / 257 big groups: 16 K random reads for one workgroup
+template <bool MERGED>
+__global__ __launch_bounds__(256) void k_round_end(const u32 *__restrict__ seg_i, const u32 *__restrict__ seg_g,
+                                                   const u64 *__restrict__ seg_ctr, u64 seg_cap,
+                                                   u32 *__restrict__ out_i, u32 *__restrict__ out_g,
+                                                   u64 *__restrict__ cnt, const u64 *__restrict__ rp,
+                                                   u64 *__restrict__ rp_next, u64 *__restrict__ rec,
+                                                   const u32 *__restrict__ bseg_h, const u32 *__restrict__ bseg_g,
+                                                   u64 bseg_cap, u32 *__restrict__ big_head, u32 *__restrict__ big_g,
+                                                   u32 *__restrict__ big_size, u64 big_cap, u64 *__restrict__ boff,
+                                                   const u32 *__restrict__ SA, u32 gf)
+{
+    const u64 a = rp[0];
+    if (a == 0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) rp_next[0] = 0;
+        return;
+    }
+    u64 pre[9];
+    pre[0] = 0;
+#pragma unroll
+    for (int x = 0; x < 8; x++) pre[x + 1] = pre[x] + seg_ctr[x * 16];
+    const u64 total = pre[8];
+    const u64 stride = (u64)gridDim.x * blockDim.x;
+    for (u64 k = (u64)blockIdx.x * blockDim.x + threadIdx.x; k < total; k += stride) {
+        int x = 0;
+#pragma unroll
+        for (int q = 1; q < 8; q++) x += k >= pre[q];
+        const u64 src = (u64)x * seg_cap + (k - pre[x]);
+        out_i[k] = seg_i[src];
+        out_g[k] = seg_g[src];
+    }
+    if (blockIdx.x != 0) return;
+    u64 nb, members = 0;
+    u32 err = (u32)(cnt[4] >> 32);
+    if (MERGED) {
+        __shared__ u64 s_sum[256 / SAGPU_WAVE];
+        __shared__ u32 s_bad;
+        if (threadIdx.x == 0) s_bad = 0;
+        __syncthreads();
+        u64 bp[9];
+        bp[0] = 0;
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+            const u64 c = seg_ctr[x * 16 + 8];
+            bp[x + 1] = bp[x] + (c < bseg_cap ? c : bseg_cap);
+        }
+        nb = bp[8];
+        const u64 lim = nb < big_cap ? nb : big_cap;
+        for (u64 b0 = 0; b0 < lim; b0 += 256) {
+            const u64 q = b0 + threadIdx.x;
+            u64 v = 0;
+            if (q < lim) {
+                int x = 0;
+#pragma unroll
+                for (int t = 1; t < 8; t++) x += q >= bp[t];
+                const u64 src = (u64)x * bseg_cap + (q - bp[x]);
+                const u32 hd = bseg_h[src], g = bseg_g[src];
+                const u32 size = SA[g & ~gf] - hd;   // minus one
+                big_head[q] = hd;
+                big_g[q] = g;
+                big_size[q] = size;
+                v = (u64)size + 1;
+                if (v <= (u64)RT_SMALL) s_bad = 1;
+            }
+            const u64 is = wave_incl_sum64(v);
+            if (lane_id() == SAGPU_WAVE - 1) s_sum[threadIdx.x / SAGPU_WAVE] = is;
+            __syncthreads();
+            u64 c = members + is - v;
+            for (u32 w = 0; w < 256 / SAGPU_WAVE; w++) {
+                if (w < threadIdx.x / SAGPU_WAVE) c += s_sum[w];
+                members += s_sum[w];
+            }
+            if (q < lim) boff[q] = c;
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            boff[lim] = members;
+            if (s_bad) err |= 2u;
+            cnt[4] = (nb & 0xFFFFFFFFull) | (u64)err << 32;
+            cnt[5] = members;
+        }
+    } else {
+        nb = (u32)cnt[4];
+        members = cnt[5];
+    }
+    if (threadIdx.x == 0) {
+        cnt[0] = total;
+        rp_next[0] = nb ? 0 : total;
+        rp_next[1] = 2 * rp[1];
+        rec[0] = total;
+        rec[4] = (nb & 0xFFFFFFFFull) | (u64)err << 32;
+        rec[5] = members;
+        __threadfence_system();
+        rec[6] = a;
+    }
 }
 
 // Copies the members of the big groups into the sort buffers: comp = (dense group
@@ -1403,11 +1500,11 @@ int group_init64(WsScratch &ws, const u64 *keys, const u32 *vals, u64 n, int bit
 }
 
 template <typename KT>
-int round_gather_t(const u32 *act_i, const u32 *act_g, u64 a, const u64 *rp, const u32 *ISA, u64 n, KT *key2,
-                   hipStream_t s, const RawKey1 &rk, int cb)
+int round_gather_t(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
+                   const u32 *ISA, u64 n, KT *key2, hipStream_t s, const RawKey1 &rk, int cb)
 {
-    hipLaunchKernelGGL(k_round_gather<KT>, dim3(grid_for(a, 256 * IG, 65535)), dim3(256), 0, s, act_i, act_g, rp, ISA,
-                       n, key2, rk, cb);
+    hipLaunchKernelGGL(k_round_gather<KT>, dim3(grid_for(a, 256 * IG, 65535)), dim3(256), 0, s, act_i, act_g, rp, st,
+                       cnt, seg_ctr, ISA, n, key2, rk, cb);
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
@@ -1423,14 +1520,13 @@ u64 round_seg_cap(u64 a) { return (ceil_div_u(a, (u64)g_tile_range) / 8 + 1) * (
 u64 round_bigseg_cap(u64 n) { return n / 2048 + 16; }
 
 template <typename KT>
-int round_tile_t(const u32 *act_i, const u32 *act_g, const KT *key2, u64 a, const u64 *rp, u32 *SA, u32 *ISA,
-                 u32 *out_i, u32 *out_g, u64 *out_counter, u32 *err, u32 *big_head, u32 *big_g, u32 *big_size,
-                 u32 *big_counter, u64 big_cap, u32 *LCP, hipStream_t s, const ActCode &ac, const ExactLcp &ex,
-                 u32 *seg_i, u32 *seg_g, u64 *seg_ctr, u32 *bseg_h, u32 *bseg_g, u64 bseg_cap, u64 *boff,
-                 u64 *big_total)
+int round_tile_t(const u32 *act_i, const u32 *act_g, const KT *key2, u64 a, const u64 *rp, u64 *rp_next, u64 *rec,
+                 u32 *SA, u32 *ISA, u32 *out_i, u32 *out_g, u64 *cnt, u32 *big_head, u32 *big_g, u32 *big_size,
+                 u64 big_cap, u32 *LCP, hipStream_t s, const ActCode &ac, const ExactLcp &ex, u32 *seg_i, u32 *seg_g,
+                 u64 *seg_ctr, u32 *bseg_h, u32 *bseg_g, u64 bseg_cap, u64 *boff)
 {
     const u64 seg_cap = round_seg_cap(a);
-    SAGPU_TRY(launch_fill_u64(seg_ctr, 8 * 16, 0, s));
+    u32 *big_counter = (u32 *)(cnt + 4), *err = big_counter + 1;
 #define RT_LAUNCH(R)                                                                                              \
     hipLaunchKernelGGL((k_round_tile<KT, R>), dim3(ceil_div_u(a, R)), dim3(RT_THREADS), 0, s, act_i, act_g, key2, rp, \
                        SA, ISA, seg_i, seg_g, seg_ctr, seg_cap, err, bseg_h, bseg_g, bseg_cap, LCP, ac, ex)
@@ -1442,11 +1538,20 @@ int round_tile_t(const u32 *act_i, const u32 *act_g, const KT *key2, u64 a, cons
     else RT_LAUNCH(512);
 #undef RT_LAUNCH
     ktime_end(KI_ROUND_TILE, a * (24 + sizeof(KT)));
-    hipLaunchKernelGGL(k_big_sizes, dim3(grid_for(big_cap, 256, 1024)), dim3(256), 0, s, bseg_h, bseg_g,
-                       (const u64 *)seg_ctr, bseg_cap, big_head, big_g, big_counter, big_cap, SA, big_size, ac.gf);
-    hipLaunchKernelGGL(k_big_offsets, dim3(1), dim3(1024), 0, s, big_size, big_counter, big_cap, boff, big_total, err);
-    hipLaunchKernelGGL(k_seg_gather, dim3(grid_for(a, 256 * 4, 65535)), dim3(256), 0, s, seg_i, seg_g,
-                       (const u64 *)seg_ctr, seg_cap, out_i, out_g, out_counter);
+    const dim3 ge(grid_for(a, 256 * 4, 65535));
+#define END_LAUNCH(M)                                                                                             \
+    hipLaunchKernelGGL(k_round_end<M>, ge, dim3(256), 0, s, seg_i, seg_g, (const u64 *)seg_ctr, seg_cap, out_i, out_g, \
+                       cnt, rp, rp_next, rec, bseg_h, bseg_g, bseg_cap, big_head, big_g, big_size, big_cap, boff, SA, \
+                       ac.gf)
+    if (a < END_MERGED) {
+        END_LAUNCH(true);
+    } else {
+        hipLaunchKernelGGL(k_big_sizes, dim3(grid_for(big_cap, 256, 1024)), dim3(256), 0, s, bseg_h, bseg_g,
+                           (const u64 *)seg_ctr, bseg_cap, big_head, big_g, big_counter, big_cap, SA, big_size, ac.gf);
+        hipLaunchKernelGGL(k_big_offsets, dim3(1), dim3(1024), 0, s, big_size, big_counter, big_cap, boff, cnt + 5, err);
+        END_LAUNCH(false);
+    }
+#undef END_LAUNCH
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
@@ -1461,27 +1566,33 @@ int big_extract_t(const u32 *act_i, const KT *key2, const u32 *bhead, const u64 
     return SAGPU_OK;
 }
 
-int round_gather(const u32 *act_i, const u32 *act_g, u64 a, const u64 *rp, const u32 *ISA, u64 n, void *key2,
-                 int wide, hipStream_t s, const RawKey1 *rk, int cb)
+int round_gather(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
+                 const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk, int cb)
 {
     const RawKey1 r = rk ? *rk : RawKey1{};
-    return wide ? round_gather_t<u64>(act_i, act_g, a, rp, ISA, n, (u64 *)key2, s, r, cb)
-                : round_gather_t<u32>(act_i, act_g, a, rp, ISA, n, (u32 *)key2, s, r, cb);
+    return wide ? round_gather_t<u64>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u64 *)key2, s, r, cb)
+                : round_gather_t<u32>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u32 *)key2, s, r, cb);
 }
 
-int round_tile(const u32 *act_i, const u32 *act_g, const void *key2, int wide, u64 a, const u64 *rp, u32 *SA,
-               u32 *ISA, u32 *out_i, u32 *out_g, u64 *out_counter, u32 *err, u32 *big_head, u32 *big_g, u32 *big_size,
-               u32 *big_counter, u64 big_cap, u32 *LCP, hipStream_t s, const ActCode &ac, const ExactLcp *ex,
-               u32 *seg_i, u32 *seg_g, u64 *seg_ctr, u32 *bseg_h, u32 *bseg_g, u64 bseg_cap, u64 *boff,
-               u64 *big_total)
+int launch_round_start(u64 *rp, u64 a, u64 h, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_round_start, dim3(1), dim3(1), 0, s, rp, a, h);
+    SAGPU_CHECK(hipGetLastError());
+    return SAGPU_OK;
+}
+
+int round_tile(const u32 *act_i, const u32 *act_g, const void *key2, int wide, u64 a, const u64 *rp, u64 *rp_next,
+               u64 *rec, u32 *SA, u32 *ISA, u32 *out_i, u32 *out_g, u64 *cnt, u32 *big_head, u32 *big_g, u32 *big_size,
+               u64 big_cap, u32 *LCP, hipStream_t s, const ActCode &ac, const ExactLcp *ex, u32 *seg_i, u32 *seg_g,
+               u64 *seg_ctr, u32 *bseg_h, u32 *bseg_g, u64 bseg_cap, u64 *boff)
 {
     const ExactLcp e = ex ? *ex : ExactLcp{};
-    return wide ? round_tile_t<u64>(act_i, act_g, (const u64 *)key2, a, rp, SA, ISA, out_i, out_g, out_counter, err,
-                                    big_head, big_g, big_size, big_counter, big_cap, LCP, s, ac, e, seg_i, seg_g,
-                                    seg_ctr, bseg_h, bseg_g, bseg_cap, boff, big_total)
-                : round_tile_t<u32>(act_i, act_g, (const u32 *)key2, a, rp, SA, ISA, out_i, out_g, out_counter, err,
-                                    big_head, big_g, big_size, big_counter, big_cap, LCP, s, ac, e, seg_i, seg_g,
-                                    seg_ctr, bseg_h, bseg_g, bseg_cap, boff, big_total);
+    return wide ? round_tile_t<u64>(act_i, act_g, (const u64 *)key2, a, rp, rp_next, rec, SA, ISA, out_i, out_g, cnt,
+                                    big_head, big_g, big_size, big_cap, LCP, s, ac, e, seg_i, seg_g, seg_ctr, bseg_h,
+                                    bseg_g, bseg_cap, boff)
+                : round_tile_t<u32>(act_i, act_g, (const u32 *)key2, a, rp, rp_next, rec, SA, ISA, out_i, out_g, cnt,
+                                    big_head, big_g, big_size, big_cap, LCP, s, ac, e, seg_i, seg_g, seg_ctr, bseg_h,
+                                    bseg_g, bseg_cap, boff);
 }
 
 int big_extract(const u32 *act_i, const void *key2, int wide, const u32 *bhead, const u64 *boff, u32 nb, u64 total,
