@@ -462,8 +462,8 @@ int g_group_flags = 1;
 // 1: the radix pass that groups the ISA pairs into windows takes its digit histogram
 // from the closed form of a permutation's (the "perm_hist" option)
 int g_perm_hist = 1;
-// radix sorts of fewer keys use the smallest tiles (2048 keys), whatever radix_items
-// and radix_threads say
+// radix sorts of fewer keys choose their tiles by size, whatever radix_items and
+// radix_threads say
 int g_radix_small_n = 1 << 20;
 
 // 1: texts of at most SMALL_MAX bytes are built by one workgroup in one kernel
@@ -823,6 +823,8 @@ int ensure_radix_scratch(Ctx &c, Scope &sc, u64 n)
         c.rs.hist = (u64 *)c.pool.get(2 * RADIX_HIST_WORDS * sizeof(u64));
         c.rs.tile_ctr = (u32 *)c.pool.get(64 * sizeof(u32));
         if (!c.rs.hist || !c.rs.tile_ctr) return SAGPU_ENOMEM;
+        // (every sort leaves its counts cleared)
+        SAGPU_TRY(launch_fill_u64(c.rs.hist, RADIX_HIST_WORDS, 0, c.stream));
     }
     if (c.rs.counts_cap < tiles * 256) {
         if (c.rs.counts) c.pool.put(c.rs.counts);

@@ -21,10 +21,13 @@ int g_hist_windows = 1;
 namespace {
 
 constexpr int RS_WAVES = RS_THREADS / SAGPU_WAVE;
+constexpr u64 RS_TINY_N = 1ull << 18;   // fewer keys take 2048-key tiles
+// fewer take 8192-key tiles (256 threads) where 16384-key tiles are asked for
+constexpr u64 RS_WIDE_N = 3ull << 19;
 constexpr int LB_VAL_BITS = 40;
 constexpr u64 LB_VAL_MASK = (1ull << LB_VAL_BITS) - 1ull;
 constexpr u64 LB_AGG = 1ull, LB_PRE = 2ull;
-constexpr int LB_WIN = 2;
+constexpr int LB_WIN = 2;   // predecessors a look-back reads at once (8: no faster at any tile size)
 
 __device__ __forceinline__ u64 lb_pack(u32 epoch, u64 flag, u64 v)
 {
@@ -169,8 +172,11 @@ __global__ __launch_bounds__(256) void k_perm_hist(u64 n, int begin_bit, int end
 
 // Exclusive scan of each pass's histogram (bins per pass) into bucket offsets at
 // hist + RADIX_HIST_WORDS.  Thread t takes bins [t * per, (t + 1) * per).
-__global__ __launch_bounds__(256) void k_radix_offsets(u64 *hist, int npass, int bins)
+// The counts go to `host` (pinned) when given, and are cleared for the next sort, as are
+// the tile tickets: two fills and a copy less per sort.
+__global__ __launch_bounds__(256) void k_radix_offsets(u64 *hist, int npass, int bins, u32 *tile_ctr, u64 *host)
 {
+    if (threadIdx.x < RADIX_MAX_PASSES) tile_ctr[threadIdx.x] = 0;
     __shared__ u64 s_w[RS_WAVES];
     const int per = bins > 256 ? bins / 256 : 1;   // at most 8 (2048 bins)
     for (int p = 0; p < npass; p++) {
@@ -192,6 +198,8 @@ __global__ __launch_bounds__(256) void k_radix_offsets(u64 *hist, int npass, int
         for (int q = 0; q < 8; q++)
             if (q < per && d0 + q < bins) {
                 hist[RADIX_HIST_WORDS + p * bins + d0 + q] = run;
+                hist[p * bins + d0 + q] = 0;
+                if (host) host[p * bins + d0 + q] = loc[q];
                 run += loc[q];
             }
         __syncthreads();
@@ -579,11 +587,17 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
     const int npass = (end_bit - begin_bit + DB - 1) / DB;
     // 4- and 11-bit digits: onesweep only, 256-thread tiles
     const int variant = DB == 8 ? rs.variant : RADIX_ONESWEEP;
-    // short inputs (one string of a batch, a served job) take 2048-key tiles: more
-    // workgroups at once instead of a few long ones (a 16384-key tile takes about
-    // 25 us, so a 20 K-key sort would run its passes on two workgroups)
+    // Short inputs choose their tile by size: few keys spread over many workgroups, but
+    // every tile pays its start, its ticket and its look-back.  u32 pairs, us per pass with
+    // 2048- / 8192- / 16384-key tiles: 2^16 keys 22.6 / 24.5 / 27.0, 2^17 24.8 / 25.2 / 27.8,
+    // 2^19 33.4 / 29.0 / 30.8, 2^20 42.5 / 31.2 / 32.6, 2^21 59.0 / 35.6 / 36.0, 2^22 85.5 /
+    // 47.2 / 40.8 (histograms included).
     const bool small = n < rs.small_n;
-    const int items = small ? 8 : rs.items == 32 ? 32 : rs.items == 8 ? 8 : 16;
+    // Histograms decide which passes can be skipped (all keys share the digit).  Up to
+    // four times that size every pass is run instead: a pass (25 to 45 us) rarely turns
+    // out to be one of those, and the wait for the histograms on the host takes about 20 us.
+    const bool nowait = n < 4 * rs.small_n;
+    const int items = small ? (n < RS_TINY_N ? 8 : 32) : rs.items == 32 ? 32 : rs.items == 8 ? 8 : 16;
     const u64 tile_keys = (u64)RS_THREADS * items;
     const u64 tiles = (n + tile_keys - 1) / tile_keys;
     if (tiles * BINS > rs.lb_words || npass > RADIX_MAX_PASSES || (u64)npass * BINS > RADIX_HIST_WORDS ||
@@ -605,7 +619,6 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
     }
     // keys known to be a permutation of [0, n): closed-form histograms (u32 keys)
     const bool perm = rs.perm_keys && sizeof(K) == 4 && !gen && n < (1ull << 32);
-    if (!perm) SAGPU_TRY(launch_fill_u64(rs.hist, (u64)npass * BINS, 0, s));
     {
         // 64 keys per thread; 8 for short inputs, which would otherwise leave all
         // but a few workgroups idle
@@ -626,12 +639,10 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
         else
             hipLaunchKernelGGL((k_radix_hist<K, false, DB>), dim3(blocks), dim3(256), 0, s, k0, g0, n, begin_bit,
                                end_bit, npass, rs.hist);
-        hipLaunchKernelGGL(k_radix_offsets, dim3(1), dim3(256), 0, s, rs.hist, npass, BINS);
+        hipLaunchKernelGGL(k_radix_offsets, dim3(1), dim3(256), 0, s, rs.hist, npass, BINS, rs.tile_ctr,
+                           perm || nowait ? (u64 *)nullptr : rs.hist_host);
         SAGPU_CHECK(hipGetLastError());
     }
-    // Histograms decide which passes can be skipped (all keys share the digit).  A
-    // short input runs every pass instead: a pass over it costs less than the wait
-    // for the histograms on the host.
     if (perm) {
         for (int p = 0; p < npass; p++) {
             const int shift = begin_bit + DB * p;
@@ -639,18 +650,16 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
             for (u32 d = 0; d < (u32)BINS; d++)
                 rs.hist_host[p * BINS + d] = d <= dmask ? perm_digit_count(n, shift, dmask, d) : 0ull;
         }
-    } else if (!small) {
-        SAGPU_CHECK(hipMemcpyAsync(rs.hist_host, rs.hist, (u64)npass * BINS * sizeof(u64), hipMemcpyDeviceToHost, s));
+    } else if (!nowait) {
         SAGPU_CHECK(hipStreamSynchronize(s));
     }
 
-    SAGPU_TRY(launch_fill_u32(rs.tile_ctr, RADIX_MAX_PASSES, 0, s));
     K *ki = k0, *ko = k1;
     u32 *vi = v0, *vo = v1;
     int alt = 0, ran = 0;
     for (int p = 0; p < npass; p++) {
         bool trivial = false;
-        for (int d = 0; d < BINS && !small; d++)
+        for (int d = 0; d < BINS && (perm || !nowait); d++)
             if (rs.hist_host[p * BINS + d] == n) trivial = true;
         if (trivial) continue;
         rs.epoch = (rs.epoch + 1) & ((1u << 22) - 1);
@@ -684,7 +693,7 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
         const u32 *cnts = lb ? nullptr : rs.counts;
         // onesweep passes may use 512-thread workgroups (16384-key tiles with 32
         // items: twice as long digit runs per tile, same waves per CU); 8-bit digits
-        const int nt = (!small && DB == 8 && sizeof(K) == 4 && lb && rs.threads == 512 && items == 32) ? 512
+        const int nt = (!small && n >= RS_WIDE_N && DB == 8 && sizeof(K) == 4 && lb && rs.threads == 512 && items == 32) ? 512
                                                                                                           : RS_THREADS;
         const u64 ptiles = (n + (u64)nt * items - 1) / ((u64)nt * items);
 #define RS_LAUNCH(HV, LB, IT)                                                                                     \
