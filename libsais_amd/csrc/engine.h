@@ -183,7 +183,7 @@ int group_init64(WsScratch &ws, const u64 *keys, const u32 *vals, u64 n, int bit
 struct RawKey1 {
     const u32 *pw;    // null: rank form everywhere
     int bits, kbits, nspecial;
-    u32 special[32];
+    const u32 *special;   // device
 };
 // Round 1 on raw keys: key2 is the packed `kbits`-bit code of the ksym symbols at
 // i + h, so where the round splits a group, the lcp of the two adjacent subgroups
@@ -193,7 +193,7 @@ struct RawKey1 {
 struct ExactLcp {
     int on = 0;
     int bits = 0, kbits = 0, nskip = 0;
-    u32 skip[64] = {};
+    const u32 *skip = nullptr;   // device
     // PLCP hints (PlcpHint) for the suffixes the first round places with an exact
     // mark: the hint bits of the rank written to ISA
     int hint = 0, hint_off = 0;
@@ -228,6 +228,8 @@ extern int g_tile_range;
 // rows of 64 positions per wave span in the initial grouping of texts of at least
 // INIT_SMALL_N suffixes (8 or 16: tiles of 2048 or 4096 positions; the "init_rows" option)
 extern int g_init_rows;   // list entries per workgroup of the tile kernel (the "tile_range" option)
+// Groups of the last cnt suffixes (their ISA words' ranks), for RawKey1 and ExactLcp.
+int launch_tail_groups(const u32 *ISA, u64 n, u32 cnt, u32 *out, hipStream_t s);
 // Sets rp for a round whose gather takes it as it stands (a captured one).
 int launch_round_start(u64 *rp, u64 a, u64 h, hipStream_t s);
 // cnt: 8 u64 (0 list length out, 4 big groups | err << 32, 5 big-group members); the
@@ -337,7 +339,11 @@ struct SmallJob {
 int launch_small_build(const SmallJob &j, hipStream_t s);
 
 // ------------------------------------------------------------ SA kernels
-int launch_histogram(const uint8_t *T, u64 n, int gsa, u64 *hist256, u32 *gsa_bad, hipStream_t s);
+// hist: 257 u64, zero before and after; pad (may be null): 64 bytes cleared; lut, inv: 256
+// bytes each, codes of the present bytes and back; host (pinned): 256 counts, then the
+// number of positions that make a GSA text invalid.
+int launch_histogram(const uint8_t *T, u64 n, int gsa, u64 *hist, uint8_t *pad, uint8_t *lut, uint8_t *inv, u64 *host,
+                     hipStream_t s);
 // vals[p] = p, or (p << cb) | code of T[p-1] with cb > 0 (n - 1 < 2^(32 - cb)).
 int launch_pack_keys32(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, int gsa, int cb, u32 *keys,
                        u32 *vals, hipStream_t s);

@@ -377,6 +377,8 @@ constexpr int F_KERNEL0 = 64;   // + KernelId: one kernel's launches
 
 // Rounds with shorter lists are queued two at a time (sa_build).
 constexpr u64 ROUND_AHEAD = 1ull << 20;
+// Shorter texts do not wait for the length of their first list (sa_build).
+constexpr u64 LAZY_N = 1ull << 22;
 constexpr int ROUND_SIG = 32;   // words of a round's launch signature (Ctx::round_sig)
 
 struct Ctx {
@@ -402,6 +404,7 @@ struct Ctx {
     Timer timer;
     sagpu_stats stats{};
     bool sort_u32 = false;  // the radix passes being timed are u32-key passes
+    u64 *alpha = nullptr;   // device: byte counts (zero between calls), then the code tables
     uint8_t *small_io = nullptr;   // pinned: result block and host arrays of small builds
     // Executable graphs of a doubling round, one per buffer parity (rounds 2, 4, ...
     // and 3, 5, ...), kept across builds: reused as they are while every argument and
@@ -522,6 +525,7 @@ void ctx_destroy(Ctx *c)
 {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    if (c->alpha) c->pool.put(c->alpha);
     if (c->rs.hist) c->pool.put(c->rs.hist);
     if (c->rs.tile_ctr) c->pool.put(c->rs.tile_ctr);
     if (c->rs.lookback) c->pool.put(c->rs.lookback);
@@ -960,47 +964,38 @@ int read_u32(Ctx &c, const u32 *d, u32 *out)
     return SAGPU_OK;
 }
 
+// The context's byte counts (kept zero) and code tables.
+int ensure_alpha(Ctx &c)
+{
+    if (c.alpha) return SAGPU_OK;
+    c.alpha = (u64 *)c.pool.get(264 * sizeof(u64) + 512);
+    if (!c.alpha) return SAGPU_ENOMEM;
+    return launch_fill_u64(c.alpha, 264, 0, c.stream);
+}
+
 // Byte alphabet of a text: freq (optional, host), the GSA validity test, and the
 // dense symbol codes (device LUT) with their width and the symbols per 32-bit key.
-int byte_alphabet(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u64 *freq_out, int *bits_out, int *ksym_out,
+// pad: the text has 64 bytes after it, to be cleared.
+int byte_alphabet(Ctx &c, const uint8_t *dT, u64 n, int gsa, bool pad, u64 *freq_out, int *bits_out, int *ksym_out,
                   uint8_t **lut_out, uint8_t **inv_out = nullptr)
 {
     hipStream_t s = c.stream;
-    GET(d_hist, u64, 256 + 8);
-    u32 *d_bad = (u32 *)(d_hist + 256);
-    u64 freq[256];
+    SAGPU_TRY(ensure_alpha(c));
+    uint8_t *d_lut = (uint8_t *)(c.alpha + 264), *d_inv = d_lut + 256;
     {
         Span sp(c, F_INITIAL);
-        SAGPU_TRY(launch_fill_u64(d_hist, 256 + 8, 0, s));
-        SAGPU_TRY(launch_histogram(dT, n, gsa, d_hist, d_bad, s));
+        SAGPU_TRY(launch_histogram(dT, n, gsa, c.alpha, pad ? (uint8_t *)dT + n : nullptr, d_lut, d_inv, c.pinned, s));
     }
-    SAGPU_CHECK(hipMemcpyAsync(c.pinned, d_hist, (256 + 1) * sizeof(u64), hipMemcpyDeviceToHost, s));
     SAGPU_CHECK(hipStreamSynchronize(s));
-    memcpy(freq, c.pinned, sizeof freq);
-    u32 bad = *(u32 *)(c.pinned + 256);
-    if (freq_out) memcpy(freq_out, freq, sizeof freq);
-    if (gsa && bad) return SAGPU_EINVAL;
-
-    uint8_t *lut_h = (uint8_t *)(c.pinned + 4096);
+    const u64 *freq = c.pinned;
+    if (freq_out) memcpy(freq_out, freq, 256 * sizeof(u64));
+    if (gsa && freq[256]) return SAGPU_EINVAL;
     int sigma = 0;
-    for (int ch = 0; ch < 256; ch++) {
-        lut_h[ch] = (uint8_t)sigma;
-        if (freq[ch]) sigma++;
-    }
+    for (int ch = 0; ch < 256; ch++) sigma += freq[ch] != 0;
     *bits_out = sigma <= 2 ? 1 : bits_for((u64)sigma - 1);
     *ksym_out = 32 / *bits_out;
-    GET(d_lut, uint8_t, 256);
-    SAGPU_CHECK(hipMemcpyAsync(d_lut, lut_h, 256, hipMemcpyHostToDevice, s));
     *lut_out = d_lut;
-    if (inv_out) {  // code -> byte
-        uint8_t *inv_h = lut_h + 256;
-        memset(inv_h, 0, 256);
-        for (int ch = 0; ch < 256; ch++)
-            if (freq[ch]) inv_h[lut_h[ch]] = (uint8_t)ch;
-        GET(d_inv, uint8_t, 256);
-        SAGPU_CHECK(hipMemcpyAsync(d_inv, inv_h, 256, hipMemcpyHostToDevice, s));
-        *inv_out = d_inv;
-    }
+    if (inv_out) *inv_out = d_inv;
     return SAGPU_OK;
 }
 
@@ -1028,7 +1023,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         bits = sym_bits < 1 ? 1 : sym_bits;
         ksym = 32 / bits;
     } else {
-        SAGPU_TRY(byte_alphabet(c, sc, dT, n, gsa, freq_out, &bits, &ksym, &d_lut, want_seed ? &d_inv : nullptr));
+        SAGPU_TRY(byte_alphabet(c, dT, n, gsa, !sid, freq_out, &bits, &ksym, &d_lut, want_seed ? &d_inv : nullptr));
     }
     if (want_seed && ((n - 1) >> (32 - bits)) == 0) {
         GET(codes, uint8_t, n);
@@ -1083,7 +1078,6 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     }
 
     int alt = 0;
-    bool a_known = false;   // the first list's length is on the host already
     RawKey1 rk1{};   // first round from the code stream (when there is one)
     ExactLcp ex1{};  // and its exact lcps across the splits
     if (!sid) {
@@ -1128,23 +1122,19 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             // than ksym) keep ranks in round 1; none of them gets exact round-1 lcps
             const u64 cnt2 = n < 2 * (u64)ksym ? n : 2 * (u64)ksym;
             const u64 cnt = n < (u64)ksym ? n : (u64)ksym;
-            u32 *hs = (u32 *)(c.pinned + 6144);   // past the histogram and LUT staging
-            SAGPU_CHECK(hipMemcpyAsync(hs, dISA + (n - cnt2), cnt2 * sizeof(u32), hipMemcpyDeviceToHost, s));
-            SAGPU_CHECK(hipMemcpyAsync(c.pinned, ws.total, sizeof(u64), hipMemcpyDeviceToHost, s));   // the list length
-            SAGPU_CHECK(hipStreamSynchronize(s));
-            a_known = true;
+            GET(tails, u32, 64);
+            SAGPU_TRY(launch_tail_groups(dISA, n, (u32)cnt2, tails, s));
             rk1.pw = gen.pw;
             rk1.bits = bits;
             rk1.kbits = ksym * bits;
             rk1.nspecial = (int)cnt;
-            for (u64 t = 0; t < cnt2; t++) hs[t] = isa_rank(hs[t], n);
-            for (u64 t = 0; t < cnt; t++) rk1.special[t] = hs[cnt2 - cnt + t];
+            rk1.special = tails + (cnt2 - cnt);
             if (g_exact_round1) {
                 ex1.on = 1;
                 ex1.bits = bits;
                 ex1.kbits = ksym * bits;
                 ex1.nskip = (int)cnt2;
-                for (u64 t = 0; t < cnt2; t++) ex1.skip[t] = hs[t];
+                ex1.skip = tails;
                 // suffixes placed by the first round with an exact mark carry it as a
                 // PLCP hint too (their ISA words are written anyway)
                 ex1.hint = hint && hint->on ? 1 : 0;
@@ -1167,18 +1157,15 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
                                  (u32 *)(alt ? k1 : k0), (u32 *)(alt ? k1 : k0) + n));
     }
     u64 a = 0;
-    // Short texts without a code-stream round skip the wait for the first list's
-    // length: the first round is launched for n entries and reads the length from
-    // the device (its kernels stop at the list's end); the host learns it with the
-    // round's counters.
-    const bool lazy_a = !a_known && n < INIT_SMALL_N && !rk1.pw;
+    // Texts below LAZY_N skip the wait for the first list's length: the first round is
+    // launched for n entries and reads the length from the device (its kernels stop at
+    // the list's end); the host learns it with the round's report.
+    const bool lazy_a = n < LAZY_N;
     if (lazy_a) {
         a = n;
     } else {
-        if (!a_known) {
-            SAGPU_CHECK(hipMemcpyAsync(c.pinned, ws.total, sizeof(u64), hipMemcpyDeviceToHost, s));
-            SAGPU_CHECK(hipStreamSynchronize(s));
-        }
+        SAGPU_CHECK(hipMemcpyAsync(c.pinned, ws.total, sizeof(u64), hipMemcpyDeviceToHost, s));
+        SAGPU_CHECK(hipStreamSynchronize(s));
         a = c.pinned[0];
     }
 
@@ -1295,7 +1282,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             // Short rounds cost their launches and the host's wait: queue the next one
             // behind (its three kernels cost about 12 us when they find nothing to do,
             // a wait and a late launch about 20)
-            ahead = a < ROUND_AHEAD && !c.timer.on;
+            ahead = (a < ROUND_AHEAD || lazy_first) && !c.timer.on;
             if (ahead) {
                 st.rounds++;   // (a queued second round is one that replays a graph)
                 const int rc = launch(cur ^ 1, a, 0, false, false, nullptr);
@@ -1765,11 +1752,12 @@ int d2h(Ctx &c, void *dst, const void *src, u64 bytes)
 // of the library (copied directly).
 enum { SRC_DEVICE = 0, SRC_HOST = 1, SRC_PINNED = 2 };
 
-// Copies a text into a pool buffer with 64 zero bytes of padding.
-int padded_text(Ctx &c, Scope &sc, const uint8_t *src, u64 n, int src_kind, uint8_t **out)
+// Copies a text into a pool buffer with 64 zero bytes of padding (clear: cleared here;
+// a build's byte histogram clears them itself).
+int padded_text(Ctx &c, Scope &sc, const uint8_t *src, u64 n, int src_kind, uint8_t **out, bool clear = true)
 {
     GET(dT, uint8_t, n + 64);
-    SAGPU_TRY(launch_fill_u8(dT + n, 64, 0, c.stream));
+    if (clear) SAGPU_TRY(launch_fill_u8(dT + n, 64, 0, c.stream));
     if (src_kind == SRC_HOST) {
         SAGPU_TRY(h2d(c, dT, src, n));
     } else if (n) {
@@ -1879,8 +1867,10 @@ int small_host(Ctx &c, const uint8_t *T, u64 n, int gsa, int width, const void *
 }
 
 // Fused device pipeline.  Returns 0 or the primary index when U is requested.
+// later (with dU, may be null): the primary index is not waited for; *later is where it
+// will be, as a 0-based rank word, once the stream is synchronised.
 int64_t build_dev(Ctx &c, Scope &sc, const uint8_t *dTpad, u64 n, int gsa, u32 *dSA, uint8_t *dU, u32 *dPLCP,
-                  u32 *dLCP, u64 *freq, u32 *dISA = nullptr)
+                  u32 *dLCP, u64 *freq, u32 *dISA = nullptr, const u32 **later = nullptr)
 {
     if (!dSA) {
         dSA = sc.get<u32>(n);
@@ -1939,6 +1929,11 @@ int64_t build_dev(Ctx &c, Scope &sc, const uint8_t *dTpad, u64 n, int gsa, u32 *
         }
     }
     int64_t ret = 0;
+    if (later && !c.timer.on) {
+        *later = (const u32 *)(c.pinned + 64);
+        SAGPU_CHECK(hipMemcpyAsync(c.pinned + 64, dISA, sizeof(u32), hipMemcpyDeviceToHost, c.stream));
+        return 0;
+    }
     if (dU) {
         u32 j0 = 0;
         SAGPU_TRY(read_u32(c, dISA, &j0));
@@ -2057,7 +2052,7 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_sa(const uint8_t *T, void *SA, int64_
     {
         Scope sc(*c);
         uint8_t *dT;
-        SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT));
+        SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT, false));
         u32 *dSA = sc.get<u32>((u64)n);
         if (!dSA) return SAGPU_ENOMEM;
         u64 f[256];
@@ -2087,14 +2082,16 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_bwt(const uint8_t *T, uint8_t *U, int
     }
     Scope sc(*c);
     uint8_t *dT;
-    SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT));
+    SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT, false));
     uint8_t *dU = sc.get<uint8_t>((u64)n);
     if (!dU) return SAGPU_ENOMEM;
     u64 f[256];
-    int64_t primary = build_dev(*c, sc, dT, (u64)n, 0, nullptr, dU, nullptr, nullptr, f);
+    const u32 *j0 = nullptr;
+    int64_t primary = build_dev(*c, sc, dT, (u64)n, 0, nullptr, dU, nullptr, nullptr, f, nullptr, &j0);
     if (primary < 0) return primary;
     SAGPU_TRY(d2h(*c, U, dU, (u64)n));
     SAGPU_CHECK(hipStreamSynchronize(c->stream));
+    if (j0) primary = (int64_t)isa_rank(*j0, (u64)n) + 1;
     store_freq(f, freq, width);
     return primary;
 }
@@ -2226,7 +2223,7 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_bwt_aux(const uint8_t *T, uint8_t *U,
     }
     Scope sc(*c);
     uint8_t *dT;
-    SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT));
+    SAGPU_TRY(padded_text(*c, sc, T, (u64)n, SRC_HOST, &dT, false));
     uint8_t *dU = sc.get<uint8_t>((u64)n);
     u32 *dISA = sc.get<u32>((u64)n);
     const u64 count = ((u64)n - 1) / (u64)r + 1;
@@ -2936,7 +2933,7 @@ int64_t build32_on(Ctx &c, const uint8_t *d_T, u64 n, int32_t flags, int32_t *d_
     }
     Scope sc(c);
     uint8_t *dT;
-    SAGPU_TRY(padded_text(c, sc, d_T, n, SRC_DEVICE, &dT));
+    SAGPU_TRY(padded_text(c, sc, d_T, n, SRC_DEVICE, &dT, false));
     u64 f[256];
     int64_t rc = build_dev(c, sc, dT, n, (flags & SAGPU_FLAG_GSA) ? 1 : 0, (u32 *)d_SA, d_U, (u32 *)d_PLCP,
                            (u32 *)d_LCP, f);
@@ -2995,6 +2992,7 @@ int noalloc_setup(int dev)
     c->pool.arena_cap = SAGPU_NOALLOC_SCRATCH_BYTES - (64u << 10);
     Scope keep(*c);   // nothing is put back: the radix scratch stays at the bottom
     int rc = ensure_radix_scratch(*c, keep, SAGPU_NOALLOC_MAX_N);
+    if (rc == SAGPU_OK) rc = ensure_alpha(*c);
     keep.held.clear();
     if (rc == SAGPU_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = SAGPU_EDEVICE;
     if (rc != SAGPU_OK) {
@@ -3184,7 +3182,7 @@ int run_single(Ctx &c, sagpu_job *j)
     }
     Scope sc(c);
     uint8_t *dT;
-    SAGPU_TRY(padded_text(c, sc, j->T, n, SRC_HOST, &dT));
+    SAGPU_TRY(padded_text(c, sc, j->T, n, SRC_HOST, &dT, false));
     GET(dSA, u32, n);
     uint8_t *dU = nullptr;
     u32 *dL = nullptr;

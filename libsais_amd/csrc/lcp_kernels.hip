@@ -947,9 +947,10 @@ int launch_plcp_t(LcpScratch &ls, const uint8_t *T, u64 n, int gsa, const u32 *P
                            SA, V, ls.queue, ls.queue_l, ls.queue_n, ls.queue_cap, marks);
     }
     const VLongQueue vq{ls.vq_pos ? ls.queue_n + 1 : nullptr, ls.vq_pos, ls.vq_off, ls.vq_res};
-    hipLaunchKernelGGL((k_plcp_long<VT, W>), dim3(4096), dim3(256), 0, s, T, n, gsa, PHI, ISA, SA, V, ls.queue, ls.queue_l,
+    hipLaunchKernelGGL((k_plcp_long<VT, W>), dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, T, n, gsa, PHI, ISA, SA, V, ls.queue, ls.queue_l,
                        ls.queue_n, ls.queue_cap, fused_max ? tmax : (VT *)nullptr, vq);
-    if (vq.n) {
+    // (a match goes on past the first pass's steps only in a text longer than they are)
+    if (vq.n && W * n > LONG_STEPS * LONG_STEP) {
         hipLaunchKernelGGL((k_plcp_vlong<W>), dim3(2048), dim3(256), 0, s, T, n, gsa, PHI, ISA, SA, vq);
         hipLaunchKernelGGL((k_plcp_vlong_fin<VT, W>), dim3(VQ_CAP / 256), dim3(256), 0, s, V,
                            fused_max ? tmax : (VT *)nullptr, vq);

@@ -741,6 +741,11 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
     }
 }
 
+__global__ void k_tail_groups(const u32 *__restrict__ ISA, u64 n, u32 cnt, u32 *__restrict__ out)
+{
+    if (threadIdx.x < cnt) out[threadIdx.x] = isa_rank(ISA[n - cnt + threadIdx.x], n);
+}
+
 __global__ void k_round_start(u64 *rp, u64 a, u64 h)
 {
     rp[0] = a;
@@ -1572,6 +1577,13 @@ int round_gather(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const Round
     const RawKey1 r = rk ? *rk : RawKey1{};
     return wide ? round_gather_t<u64>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u64 *)key2, s, r, cb)
                 : round_gather_t<u32>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u32 *)key2, s, r, cb);
+}
+
+int launch_tail_groups(const u32 *ISA, u64 n, u32 cnt, u32 *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_tail_groups, dim3(1), dim3(64), 0, s, ISA, n, cnt, out);
+    SAGPU_CHECK(hipGetLastError());
+    return SAGPU_OK;
 }
 
 int launch_round_start(u64 *rp, u64 a, u64 h, hipStream_t s)

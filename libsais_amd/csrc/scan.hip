@@ -101,6 +101,11 @@ __global__ __launch_bounds__(SC_THREADS) void k_scan_apply(u32 *__restrict__ dat
 int scan_exclusive_u32(ScanScratch &sc, u32 *data, u64 count, hipStream_t s)
 {
     if (count == 0) return SAGPU_OK;
+    if (count <= 8192) {   // up to 8 steps of one workgroup: less than the two launches it saves
+        hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(1024), 0, s, data, count);
+        SAGPU_CHECK(hipGetLastError());
+        return SAGPU_OK;
+    }
     const u64 tiles = (count + SC_TILE - 1) / SC_TILE;
     if (tiles > sc.cap) {
         sagpu_set_error("scan scratch too small", __FILE__, __LINE__);
