@@ -104,6 +104,14 @@ __device__ __forceinline__ u64 wave_incl_max64(u64 v)
     return v;
 }
 
+// p[i] of memory that nothing writes while the kernel runs, at an index that is the same
+// in all lanes: a scalar load.
+__device__ __forceinline__ u32 const_word(const u32 *p, int i)
+{
+    typedef const __attribute__((address_space(4))) u32 *cptr;
+    return ((cptr)(uintptr_t)p)[i];
+}
+
 // Device-scope relaxed atomics on 64-bit look-back words.
 __device__ __forceinline__ u64 ld_acquire_u64(const u64 *p)
 {

@@ -183,7 +183,7 @@ int group_init64(WsScratch &ws, const u64 *keys, const u32 *vals, u64 n, int bit
 struct RawKey1 {
     const u32 *pw;    // null: rank form everywhere
     int bits, kbits, nspecial;
-    const u32 *special;   // device
+    const u32 *special;   // device (read as constant memory)
 };
 // Round 1 on raw keys: key2 is the packed `kbits`-bit code of the ksym symbols at
 // i + h, so where the round splits a group, the lcp of the two adjacent subgroups
@@ -193,7 +193,7 @@ struct RawKey1 {
 struct ExactLcp {
     int on = 0;
     int bits = 0, kbits = 0, nskip = 0;
-    const u32 *skip = nullptr;   // device
+    const u32 *skip = nullptr;   // device (read as constant memory)
     // PLCP hints (PlcpHint) for the suffixes the first round places with an exact
     // mark: the hint bits of the rank written to ISA
     int hint = 0, hint_off = 0;
@@ -204,7 +204,7 @@ struct ExactLcp {
     __device__ bool skipped(u32 g) const
     {
         for (int t = 0; t < nskip; t++)
-            if (skip[t] == g) return true;
+            if (const_word(skip, t) == g) return true;
         return false;
     }
     // symbols two different raw keys share from the top

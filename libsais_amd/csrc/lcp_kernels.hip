@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
 }
 
 constexpr int PP = 8;   // slots per thread and step
-__global__ __launch_bounds__(256) void k_plcp_pairs(const u32 *__restrict__ SA, const u32 *__restrict__ marks,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_plcp_pairs(const u32 *__restrict__ SA, const u32 *__restrict__ marks,
                                                     const uint8_t *__restrict__ U, const uint8_t *__restrict__ T,
                                                     const u32 *__restrict__ ISA, u64 n, u64 *__restrict__ pairs)
 {

@@ -715,7 +715,7 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
             if (rk.pw && k < a) {
                 const u32 g = act_g[k];
                 raw[q] = true;
-                for (int t = 0; t < rk.nspecial; t++) raw[q] = raw[q] && g != rk.special[t];
+                for (int t = 0; t < rk.nspecial; t++) raw[q] = raw[q] && g != const_word(rk.special, t);
             }
         }
 #pragma unroll
@@ -785,7 +785,7 @@ __device__ __forceinline__ void rt_big_head(u64 head, u32 g, u64 *__restrict__ s
 }
 
 template <typename KT, int RANGE>
-__global__ __launch_bounds__(RT_THREADS) void k_round_tile(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g,
+__global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) void k_round_tile(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g,
                                                            const KT *__restrict__ key2, const u64 *__restrict__ rp,
                                                            u32 *__restrict__ SA, u32 *__restrict__ ISA,
                                                            u32 *__restrict__ seg_i, u32 *__restrict__ seg_g,

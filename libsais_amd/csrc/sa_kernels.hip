@@ -7,15 +7,11 @@ namespace {
 // sub-histogram per wave so that the few hot bins of DNA text do not serialise
 // the whole workgroup.  In GSA mode it also counts the positions that make the
 // input invalid (a 0 at position 0 or a 0 directly after another 0).
-// The workgroup that finishes last turns the counts into the dense codes of the present
-// bytes (lut) and back (inv), hands counts and validity to the host (pinned) and clears
-// them for the next text: it replaces a fill, a copy back and two uploads of tables
-// made on the host.  Workgroup 0 also clears the 64 bytes of padding after the text.
-__global__ __launch_bounds__(256) void k_histogram(const uint8_t *T, u64 n, int gsa, u64 *hist, uint8_t *pad,
-                                                   uint8_t *__restrict__ lut, uint8_t *__restrict__ inv,
-                                                   u64 *__restrict__ host)
+// Workgroup 0 also clears the 64 bytes of padding after the text.
+__global__ __launch_bounds__(256) void k_histogram(const uint8_t *__restrict__ T, u64 n, int gsa,
+                                                   u64 *__restrict__ hist, uint8_t *__restrict__ pad)
 {
-    u32 *bad = (u32 *)(hist + 256), *done = bad + 1;
+    u32 *bad = (u32 *)(hist + 256);
     if (pad && blockIdx.x == 0 && threadIdx.x < 64) pad[threadIdx.x] = 0;
     // 16 sub-histograms: lanes of a wave spread over 4 copies (lane % 4), so a text of
     // few distinct bytes (DNA) has a quarter of the same-word atomics per step.  Rows
@@ -55,17 +51,20 @@ __global__ __launch_bounds__(256) void k_histogram(const uint8_t *T, u64 n, int 
         if (t) atomicAdd(&hist[c], (u64)t);
     }
     if (gsa && nbad) atomicAdd(bad, nbad);
-    __shared__ bool s_last;
+}
+
+// The counts as dense codes of the present bytes (lut) and back (inv); counts and validity
+// to the host (pinned), and cleared for the next text.  It replaces a fill, a copy back
+// and two uploads of tables made on the host.  (A kernel of its own: left to the last
+// workgroup of k_histogram, the fence that each of up to 2048 workgroups needs took 0.1
+// ms on a 48 MiB text.)
+__global__ __launch_bounds__(256) void k_alphabet(u64 *__restrict__ hist, uint8_t *__restrict__ lut,
+                                                  uint8_t *__restrict__ inv, u64 *__restrict__ host)
+{
     __shared__ u64 s_b[4];
     __shared__ uint8_t s_inv[256];
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) s_last = atomicAdd(done, 1u) == gridDim.x - 1;
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
     const u32 c = threadIdx.x, wv = c / SAGPU_WAVE;
-    const u64 cnt = ld_acquire_u64(hist + c);
+    const u64 cnt = hist[c];
     const u64 b = __ballot(cnt != 0);
     if (lane_id() == 0) s_b[wv] = b;
     s_inv[c] = 0;
@@ -77,8 +76,8 @@ __global__ __launch_bounds__(256) void k_histogram(const uint8_t *T, u64 n, int 
     host[c] = cnt;
     hist[c] = 0;
     if (c == 0) {
-        host[256] = ld_acquire_u64((u64 *)bad) & 0xFFFFFFFFull;
-        hist[256] = 0;   // bad and done
+        host[256] = hist[256] & 0xFFFFFFFFull;
+        hist[256] = 0;
     }
     __syncthreads();
     inv[c] = s_inv[c];
@@ -419,8 +418,8 @@ unsigned grid_for(u64 work, unsigned per_block, unsigned cap)
 int launch_histogram(const uint8_t *T, u64 n, int gsa, u64 *hist, uint8_t *pad, uint8_t *lut, uint8_t *inv, u64 *host,
                      hipStream_t s)
 {
-    hipLaunchKernelGGL(k_histogram, dim3(grid_for(n, 256 * 16 * 8, 2048)), dim3(256), 0, s, T, n, gsa, hist, pad, lut,
-                       inv, host);
+    hipLaunchKernelGGL(k_histogram, dim3(grid_for(n, 256 * 16 * 8, 2048)), dim3(256), 0, s, T, n, gsa, hist, pad);
+    hipLaunchKernelGGL(k_alphabet, dim3(1), dim3(256), 0, s, hist, lut, inv, host);
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
