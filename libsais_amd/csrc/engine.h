@@ -224,18 +224,34 @@ struct RoundStart {
     u64 a;              // the length, or where to read it
     const u64 *a_src;
 };
+// Chains of groups (chain_marks): bit p is set where the group of suffix p, at most
+// CHAIN_GROUP members, continues in one group: the members' next suffixes share their
+// rank too.  Such a group's order is that of its next one's, so its members compare at
+// the offset of the first position past p without a bit, plus h.  next[w]: the first
+// position without a bit from position 64 w on, when it lies in w's CHAIN_TILE words,
+// else none (~0); tile[t]: the same from tile t's first position on, over all tiles.
+constexpr int CHAIN_GROUP = 8, CHAIN_TILE = 1024;
+struct Chains {
+    const u64 *bits;   // nullptr: off
+    const u32 *next, *tile;
+    const u32 *on;   // 0: few of the list's groups can continue; nothing was marked
+};
+// words of scratch chain_marks takes for a text of n symbols (u32, 8-byte aligned)
+u64 chain_words(u64 n);
+// The chains of a list of a entries, into scratch (chain_words(n) u32).
+int chain_marks(const u32 *act_i, const u32 *act_g, u64 a, const u32 *ISA, u64 n, int cb, u32 *scratch, Chains *ch,
+                hipStream_t s);
 extern int g_tile_range;
 // rows of 64 positions per wave span in the initial grouping of texts of at least
 // INIT_SMALL_N suffixes (8 or 16: tiles of 2048 or 4096 positions; the "init_rows" option)
 extern int g_init_rows;   // list entries per workgroup of the tile kernel (the "tile_range" option)
 // Groups of the last cnt suffixes (their ISA words' ranks), for RawKey1 and ExactLcp.
 int launch_tail_groups(const u32 *ISA, u64 n, u32 cnt, u32 *out, hipStream_t s);
-// Sets rp for a round whose gather takes it as it stands (a captured one).
-int launch_round_start(u64 *rp, u64 a, u64 h, hipStream_t s);
 // cnt: 8 u64 (0 list length out, 4 big groups | err << 32, 5 big-group members); the
 // gather clears them and seg_ctr (128 u64).
 int round_gather(const u32 *act_i, const u32 *act_g, u64 a_grid, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
-                 const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk = nullptr, int cb = 0);
+                 const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk = nullptr, int cb = 0,
+                 const Chains *ch = nullptr);
 // The tile kernel's survivors go to 8 per-XCD segments of seg_i / seg_g (capacity
 // 8 * round_seg_cap(a_grid) each) and are concatenated into out_i / out_g, whose
 // length goes to cnt[0].  Big-group heads go the same way to 8 segments of bseg_h /

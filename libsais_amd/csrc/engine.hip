@@ -472,6 +472,10 @@ int g_radix_small_n = 1 << 20;
 // 1: texts of at most SMALL_MAX bytes are built by one workgroup in one kernel
 // (small.hip); 0: by the general engine
 int g_small_build = 1;
+// Rounds whose list the round before left at over seven eighths of its length compare
+// groups of up to CHAIN_GROUP members at the end of their chains, from this many list
+// entries on (0: never)
+int g_chain_min = 4096;
 u32 g_knobs_off = 0;   // bit k: general-engine knob g_knobs[k] is off its default
 
 // A context is one stream with its own pooled buffers and scratch; calls on one
@@ -1179,8 +1183,8 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     // offset live in device memory, where the round's start puts them or the round
     // before leaves them, so a round can be queued before the host knows the outcome
     // of the one before: with big groups left, it finds a length of 0 and does nothing.
-    // Rounds from the second on replay one captured graph per buffer parity, whose
-    // launch geometry is sized for a list at least as long as the round's.
+    // From the second round on tile and end replay one captured graph per buffer parity,
+    // whose launch geometry is sized for a list at least as long as the round's.
     GET(d_rp, u64, 4);   // by parity
     u64 *const rec[2] = {c.pinned, c.pinned + 32};   // a round's report, by parity
     // per-XCD survivor segments of the tile kernel, sized for the first (longest) list
@@ -1195,7 +1199,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
 
     // Queues the round of parity p: a list of at most a_most entries, of exactly that many
     // and offset h when `given`, else as the round before leaves it.
-    auto launch = [&](int p, u64 a_most, u64 h, bool given, bool raw, const u64 *a_src) -> int {
+    auto launch = [&](int p, u64 a_most, u64 h, bool given, bool raw, const u64 *a_src, bool chains = false) -> int {
         Span sp(c, F_ROUNDS);
         // the geometry of lists below 2^20 entries is sized by powers of two, so that the
         // graphs of one build serve the next one of the same size
@@ -1206,21 +1210,26 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             if (a_grid > a_first) a_grid = a_first;
         }
         rec[p][6] = NOT_RUN;
-        auto enqueue = [&](const RoundStart &st, bool timed) -> int {
-            if (timed) ktime_begin(KI_ROUND_GATHER);
-            SAGPU_TRY(round_gather(act_i[p], act_g[p], a_grid, d_rp + 2 * p, st, d_cnt, seg_ctr, dISA, n, key2, wide,
-                                   s, raw ? &rk1 : nullptr, ac.cb));
+        {
+            // (the next list's room is free until the round's end)
+            Chains ch{};
+            if (chains) SAGPU_TRY(chain_marks(act_i[p], act_g[p], a_most, dISA, n, ac.cb, act_i[p ^ 1], &ch, s));
+            ktime_begin(KI_ROUND_GATHER);
+            SAGPU_TRY(round_gather(act_i[p], act_g[p], a_grid, d_rp + 2 * p,
+                                   given ? RoundStart{h, a_most, a_src} : RoundStart{}, d_cnt, seg_ctr, dISA, n, key2,
+                                   wide, s, raw ? &rk1 : nullptr, ac.cb, chains ? &ch : nullptr));
             // suffix read, one random 4-byte read (rank, or code-stream window), key
             // written (+ the group read for the first round's form)
-            if (timed) ktime_end(KI_ROUND_GATHER, a_most * ((wide ? 16 : 12) + (raw ? 4 : 0)));
-            // (the tile kernel is timed inside round_tile; the timer is off while a
-            // round is captured)
+            ktime_end(KI_ROUND_GATHER, a_most * ((wide ? 16 : 12) + (raw ? 4 : 0)));
+        }
+        // (the tile kernel is timed inside round_tile; the timer is off while a round is
+        // captured)
+        auto tile_end = [&]() -> int {
             return round_tile(act_i[p], act_g[p], key2, wide, a_grid, d_rp + 2 * p, d_rp + 2 * (p ^ 1), rec[p], dSA,
                               dISA, act_i[p ^ 1], act_g[p ^ 1], d_cnt, big_head, big_g, big_size, big_cap, dLCP, s, ac,
                               raw ? &ex1 : nullptr, seg_i, seg_g, seg_ctr, bseg_h, bseg_g, bseg_cap, d_boff);
         };
-        if (!graphs || st.rounds < 1) return enqueue(given ? RoundStart{h, a_most, a_src} : RoundStart{}, true);
-        if (given) SAGPU_TRY(launch_round_start(d_rp + 2 * p, a_most, h, s));
+        if (!graphs || st.rounds < 1) return tile_end();
         hipGraphExec_t &exec = c.round_exec[p];
         // every argument and launch size the round's operations take
         const u64 sig[ROUND_SIG] = {(u64)act_i[p], (u64)act_g[p], (u64)act_i[p ^ 1], (u64)act_g[p ^ 1],
@@ -1234,7 +1243,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             // capture this parity's round once per build; the executable graph of
             // the previous build is updated when its topology still matches
             SAGPU_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            const int rc = enqueue(RoundStart{}, false);
+            const int rc = tile_end();
             hipGraph_t graph = nullptr;
             const hipError_t ec = hipStreamEndCapture(s, &graph);
             if (rc != SAGPU_OK || ec != hipSuccess) {
@@ -1273,12 +1282,26 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     };
 
     bool queued = false, left = false;   // this round is on the stream already; its length is in rp
+    u64 a_before = 0;                    // the length of the round before
+    int chain_rounds = 0;
     while (a > 0) {
         const bool raw = st.rounds == 0 && rk1.pw;
         const bool lazy_first = lazy_a && st.rounds == 0;
         bool ahead = false;   // the next round was queued behind this one
+        bool chains = false;
         if (!queued) {
-            SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr));
+            // A list that a round hardly shortened is one of long repeats, whose groups split
+            // only once h reaches their ends: chains take them there in one round.  Marks
+            // and the longer gather cost about 2 rounds' gathers (0.25 ms for 4.8 M
+            // entries), so the list must promise more than two such rounds: 7/8 of the
+            // length before.  48 MiB of words with repeats (lists of 4778 and 4771 K, then
+            // 145 K instead of 9 rounds): 13.80 -> 12.69 ms.  At 3/4, 256 MiB of DNA with
+            // diverged repeats (23.1 and 18.1 M, then 5.1 instead of 11.8 M) went from
+            // 21.6 to 22.3 ms.  A second time takes what groups above CHAIN_GROUP left.
+            chains = g_chain_min && left && st.rounds >= 2 && chain_rounds < 2 && a >= (u64)g_chain_min &&
+                     a > a_before / 8 * 7 && chain_words(n) <= n && n < 0xFFFFFF00ull;
+            chain_rounds += chains;
+            SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr, chains));
             // Short rounds cost their launches and the host's wait: queue the next one
             // behind (its three kernels cost about 12 us when they find nothing to do,
             // a wait and a late launch about 20)
@@ -1437,6 +1460,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             st.big_rounds++;
             st.big_elems += (int64_t)total;
         }
+        a_before = a;
         a = out_n;
         cur = nxt;
         h *= 2;
@@ -2628,7 +2652,7 @@ namespace {
 const struct { const char *name; int64_t value; } g_knobs[] = {
     {"radix_items", 32}, {"radix_threads", 512}, {"radix_variant", RADIX_ONESWEEP}, {"radix_bits", 8},
     {"radix_small_n", 1 << 20}, {"bucketed_phi", 1}, {"plcp_hint", 1}, {"exact_round1", 1}, {"stream_compare", 1},
-    {"raw_round1", 1}, {"key_stream", 1}, {"round_graphs", 1}, {"big_pivot_min", 1 << 20}, {"perm_hist", 1},
+    {"raw_round1", 1}, {"key_stream", 1}, {"round_graphs", 1}, {"big_pivot_min", 1 << 20}, {"chain_min", 4096}, {"perm_hist", 1},
     {"group_flags", 1}, {"windowed_scatter", 1}, {"plcp_pairs", 1}, {"bwt_variant", 0}, {"hist_windows", 1},
     {"init_rows", 8}, {"tile_range", 512}, {"isa_window_log2", 25}, {"wide_from", 0x7FFFFFFF}};
 
@@ -2780,6 +2804,11 @@ int set_option(const char *name, int64_t value)
     if (!strcmp(name, "wide_from")) {
         if (value < 0 || value > 0x7FFFFFFF) return SAGPU_EINVAL;
         g_wide_from = (u64)value;
+        return 0;
+    }
+    if (!strcmp(name, "chain_min")) {
+        if (value < 0 || value > 0x7FFFFFFF) return SAGPU_EINVAL;
+        g_chain_min = (int)value;
         return 0;
     }
     if (!strcmp(name, "small_build")) {

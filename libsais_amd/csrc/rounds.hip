@@ -680,10 +680,11 @@ int ws_run(WsScratch &ws, const F &f, u64 n, u64 *out_counter, hipStream_t s)
 // IG list entries per thread and step, all loads (the random ISA reads included)
 // in flight before the stores.
 constexpr int IG = 4;
-template <typename KT>
+template <typename KT, bool CHAIN>
 __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g,
-                                                      u64 *rp, RoundStart st, u64 *__restrict__ cnt, u64 *__restrict__ seg_ctr, const u32 *__restrict__ ISA, u64 n,
-                                                      KT *__restrict__ key2, RawKey1 rk, int cb)
+                                                      u64 *rp, RoundStart st, u64 *__restrict__ cnt,
+                                                      u64 *__restrict__ seg_ctr, const u32 *__restrict__ ISA, u64 n,
+                                                      KT *__restrict__ key2, RawKey1 rk, int cb, Chains ch)
 {
     // The round's list length and offset: from the host (its block 0 puts them where the
     // round's other kernels read them), or left there by the round before (a length of
@@ -712,16 +713,37 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
             // stream instead of the 4-byte ISA; groups holding a suffix shorter than
             // h keep the rank form
             raw[q] = false;
-            if (rk.pw && k < a) {
+            if (!CHAIN && rk.pw && k < a) {
                 const u32 g = act_g[k];
                 raw[q] = true;
                 for (int t = 0; t < rk.nspecial; t++) raw[q] = raw[q] && g != const_word(rk.special, t);
             }
         }
+        // where the suffix's chain ends, past i
+        u32 t[IG];
+#pragma unroll
+        for (int q = 0; q < IG; q++) t[q] = 0;
+        if (CHAIN && *ch.on) {
+            u64 w[IG];
+#pragma unroll
+            for (int q = 0; q < IG; q++) w[q] = ch.bits[i[q] >> 6] >> (i[q] & 63u);
+#pragma unroll
+            for (int q = 0; q < IG; q++) {
+                const u32 left = 64u - (i[q] & 63u);   // bits of the word from i on
+                t[q] = w[q] == ~0ull ? 64u : (u32)__ffsll((long long)~w[q]) - 1u;
+                if (t[q] < left) continue;
+                // (a word holding a position without a bit follows: the text's last one
+                // has none)
+                const u32 w1 = (i[q] >> 6) + 1u;
+                u32 e = ch.next[w1];
+                if (e == ~0u) e = ch.tile[w1 / CHAIN_TILE + 1u];
+                t[q] = e - i[q];
+            }
+        }
 #pragma unroll
         for (int q = 0; q < IG; q++) {
             const u64 k = base + (u64)q * 256 + threadIdx.x;
-            const u64 ih = (u64)i[q] + h;
+            const u64 ih = (u64)i[q] + h + t[q];
             if (k < a && raw[q]) {
                 const u64 bitpos = ih * (u64)rk.bits;
                 const u64 w = bitpos >> 5;
@@ -735,21 +757,145 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
         for (int q = 0; q < IG; q++) {
             const u64 k = base + (u64)q * 256 + threadIdx.x;
             if (k >= a) continue;
-            const u64 ih = (u64)i[q] + h;
-            key2[k] = raw[q] ? (KT)r[q] : ih < n ? (KT)(h + r[q]) : (KT)(n - 1 - i[q]);
+            const u64 ih = (u64)i[q] + h + t[q];
+            // (a group whose members compare past h has one suffix at most that ends there)
+            key2[k] = raw[q] ? (KT)r[q] : ih < n ? (KT)(h + r[q]) : CHAIN && t[q] ? (KT)0 : (KT)(n - 1 - i[q]);
         }
+    }
+}
+
+// Whether chains are worth their marks: at least half of CS_SAMPLES entries spread over
+// the list are in groups that can continue.  On texts of long periods (lists of groups of
+// ever the same size above CHAIN_GROUP) the marks would cost two gathers and give nothing.
+constexpr u32 CS_SAMPLES = 4096;
+__global__ __launch_bounds__(1024) void k_chain_sample(const u32 *__restrict__ act_g, u64 a, u32 *__restrict__ on)
+{
+    __shared__ u32 s_small[1024 / SAGPU_WAVE];
+    u32 small = 0;
+    for (u32 q = threadIdx.x; q < CS_SAMPLES; q += 1024) {
+        const u64 k = a * q / CS_SAMPLES;
+        const u32 g = act_g[k];
+        int size = 1;
+        for (int d = 1; d <= CHAIN_GROUP && k >= (u64)d && act_g[k - d] == g; d++) size++;
+        for (int d = 1; d <= CHAIN_GROUP && k + d < a && act_g[k + d] == g; d++) size++;
+        small += size <= CHAIN_GROUP;
+    }
+    small = wave_incl_sum(small);
+    if (lane_id() == SAGPU_WAVE - 1) s_small[threadIdx.x / SAGPU_WAVE] = small;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    u32 sum = 0;
+    for (u32 w = 0; w < 1024 / SAGPU_WAVE; w++) sum += s_small[w];
+    *on = sum >= CS_SAMPLES / 2;
+}
+
+// Marks of chains.  Each list entry reads the rank of its next suffix (one random 4-byte
+// read) and sets its bit when its group is small and all of the group's next suffixes
+// hold one rank; the bits of a group are alike, and since the next suffixes are of one
+// group, whose bits are alike too, all members reach a position without a bit after the
+// same number of steps.  Bound by the random read and the random atomic (about 95 us
+// each for 4.8 M entries of a 48 MiB text).  A group's members lie side by side in
+// the list, so the entries within CHAIN_GROUP of the workgroup's range are loaded too
+// (one more than a group that counts can reach: a larger one is seen from its ends).
+constexpr int CM_RANGE = 1024, CM_HALO = CHAIN_GROUP, CM_WIN = CM_RANGE + 2 * CM_HALO;
+__global__ __launch_bounds__(256) void k_chain_marks(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g, u64 a,
+                                                     const u32 *__restrict__ ISA, u64 n, int cb, u32 *__restrict__ bits,
+                                                     const u32 *__restrict__ on)
+{
+    if (!*on) return;
+    constexpr int PER = (CM_WIN + 255) / 256;
+    __shared__ u32 s_g[CM_WIN], s_r[CM_WIN];
+    const u64 lo = (u64)blockIdx.x * CM_RANGE;
+    u32 i[PER], r[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int x = j * 256 + (int)threadIdx.x;
+        const u64 k = lo + (u64)x - CM_HALO;   // wraps below 0: past a
+        i[j] = ~0u;
+        if (x < CM_WIN) {
+            s_g[x] = k < a ? act_g[k] : ~0u;   // no group word is ~0: a head is below n - 1
+            if (k < a) i[j] = act_i[k] >> cb;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) r[j] = (u64)i[j] + 1 < n ? isa_rank(ISA[i[j] + 1u], n) : ~0u;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int x = j * 256 + (int)threadIdx.x;
+        if (x < CM_WIN) s_r[x] = r[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int x = j * 256 + (int)threadIdx.x;
+        if (x < CM_HALO || x >= CM_HALO + CM_RANGE || lo + (u64)(x - CM_HALO) >= a) continue;
+        const u32 g = s_g[x];
+        int size = 1;
+        bool same = r[j] != ~0u;
+        for (int y = x - 1; y >= x - CM_HALO && s_g[y] == g; y--, size++) same = same && s_r[y] == r[j];
+        for (int y = x + 1; y <= x + CM_HALO && s_g[y] == g; y++, size++) same = same && s_r[y] == r[j];
+        if (same && size <= CHAIN_GROUP) atomicOr(&bits[i[j] >> 5], 1u << (i[j] & 31u));
+    }
+}
+
+// next[] of the words (each thread takes 4, a workgroup a tile), and the tile's own first
+// position without a bit.
+__global__ __launch_bounds__(256) void k_chain_next(const u64 *__restrict__ bits, u64 words, u32 *__restrict__ next,
+                                                    u32 *__restrict__ tile)
+{
+    static_assert(CHAIN_TILE == 256 * 4, "four words a thread");
+    __shared__ u32 s_w[256 / SAGPU_WAVE];
+    const u64 w0 = (u64)blockIdx.x * CHAIN_TILE + threadIdx.x * 4u;
+    u32 f[4];
+    u32 m = ~0u;
+#pragma unroll
+    for (int q = 3; q >= 0; q--) {
+        const u64 v = w0 + q < words ? ~bits[w0 + q] : 0ull;
+        if (v) m = (u32)((w0 + q) * 64 + (u64)__ffsll((long long)v) - 1);
+        f[q] = m;   // positions grow with the words: the nearest word's is the least
+    }
+    u32 after = ~0u, inc = m;   // least over the lanes after this one
+    for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
+        const u32 o = __shfl_down(inc, d, SAGPU_WAVE);
+        if ((int)lane_id() + d < SAGPU_WAVE) inc = o < inc ? o : inc;
+    }
+    after = __shfl_down(inc, 1, SAGPU_WAVE);
+    if (lane_id() == SAGPU_WAVE - 1) after = ~0u;
+    if (lane_id() == 0) s_w[threadIdx.x / SAGPU_WAVE] = inc;
+    __syncthreads();
+    for (u32 q = threadIdx.x / SAGPU_WAVE + 1; q < 256 / SAGPU_WAVE; q++) after = s_w[q] < after ? s_w[q] : after;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (w0 + q < words) next[w0 + q] = f[q] != ~0u ? f[q] : after;
+    if (threadIdx.x == 0) tile[blockIdx.x] = f[0] != ~0u ? f[0] : after;
+}
+
+// tile[t] = least of tile[t ..]: one workgroup, from the last tiles on.
+__global__ __launch_bounds__(1024) void k_chain_tiles(u32 *__restrict__ tile, u32 tiles)
+{
+    __shared__ u32 s_w[1024 / SAGPU_WAVE];
+    u32 carry = ~0u;
+    for (u32 t0 = (tiles - 1) / 1024u * 1024u;; t0 -= 1024u) {
+        const u32 t = t0 + threadIdx.x;
+        u32 m = t < tiles ? tile[t] : ~0u;
+        for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
+            const u32 o = __shfl_down(m, d, SAGPU_WAVE);
+            if ((int)lane_id() + d < SAGPU_WAVE) m = o < m ? o : m;
+        }
+        if (lane_id() == 0) s_w[threadIdx.x / SAGPU_WAVE] = m;
+        __syncthreads();
+        for (u32 q = threadIdx.x / SAGPU_WAVE + 1; q < 1024 / SAGPU_WAVE; q++) m = s_w[q] < m ? s_w[q] : m;
+        m = carry < m ? carry : m;
+        if (t < tiles) tile[t] = m;
+        for (u32 q = 0; q < 1024 / SAGPU_WAVE; q++) carry = s_w[q] < carry ? s_w[q] : carry;
+        if (t0 == 0) return;
+        __syncthreads();
     }
 }
 
 __global__ void k_tail_groups(const u32 *__restrict__ ISA, u64 n, u32 cnt, u32 *__restrict__ out)
 {
     if (threadIdx.x < cnt) out[threadIdx.x] = isa_rank(ISA[n - cnt + threadIdx.x], n);
-}
-
-__global__ void k_round_start(u64 *rp, u64 a, u64 h)
-{
-    rp[0] = a;
-    rp[1] = h;
 }
 
 constexpr int RT_THREADS = 256;
@@ -1506,10 +1652,15 @@ int group_init64(WsScratch &ws, const u64 *keys, const u32 *vals, u64 n, int bit
 
 template <typename KT>
 int round_gather_t(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
-                   const u32 *ISA, u64 n, KT *key2, hipStream_t s, const RawKey1 &rk, int cb)
+                   const u32 *ISA, u64 n, KT *key2, hipStream_t s, const RawKey1 &rk, int cb, const Chains *ch)
 {
-    hipLaunchKernelGGL(k_round_gather<KT>, dim3(grid_for(a, 256 * IG, 65535)), dim3(256), 0, s, act_i, act_g, rp, st,
-                       cnt, seg_ctr, ISA, n, key2, rk, cb);
+    const dim3 grid(grid_for(a, 256 * IG, 65535));
+    if (ch)
+        hipLaunchKernelGGL((k_round_gather<KT, true>), grid, dim3(256), 0, s, act_i, act_g, rp, st, cnt, seg_ctr, ISA,
+                           n, key2, rk, cb, *ch);
+    else
+        hipLaunchKernelGGL((k_round_gather<KT, false>), grid, dim3(256), 0, s, act_i, act_g, rp, st, cnt, seg_ctr, ISA,
+                           n, key2, rk, cb, Chains{});
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
@@ -1572,23 +1723,35 @@ int big_extract_t(const u32 *act_i, const KT *key2, const u32 *bhead, const u64 
 }
 
 int round_gather(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
-                 const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk, int cb)
+                 const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk, int cb, const Chains *ch)
 {
     const RawKey1 r = rk ? *rk : RawKey1{};
-    return wide ? round_gather_t<u64>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u64 *)key2, s, r, cb)
-                : round_gather_t<u32>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u32 *)key2, s, r, cb);
+    return wide ? round_gather_t<u64>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u64 *)key2, s, r, cb, ch)
+                : round_gather_t<u32>(act_i, act_g, a, rp, st, cnt, seg_ctr, ISA, n, (u32 *)key2, s, r, cb, ch);
+}
+
+static u64 chain_bit_words(u64 n) { return n / 64 + 1; }
+u64 chain_words(u64 n) { return 3 * chain_bit_words(n) + ceil_div_u(chain_bit_words(n), (u64)CHAIN_TILE) + 1; }
+int chain_marks(const u32 *act_i, const u32 *act_g, u64 a, const u32 *ISA, u64 n, int cb, u32 *scratch, Chains *ch,
+                hipStream_t s)
+{
+    const u64 words = chain_bit_words(n);
+    const u32 tiles = (u32)ceil_div_u(words, (u64)CHAIN_TILE);
+    u32 *next = scratch + 2 * words, *tile = next + words, *on = tile + tiles;
+    hipLaunchKernelGGL(k_chain_sample, dim3(1), dim3(1024), 0, s, act_g, a, on);
+    SAGPU_TRY(launch_fill_u32(scratch, 2 * words, 0, s));
+    hipLaunchKernelGGL(k_chain_marks, dim3((unsigned)ceil_div_u(a, (u64)CM_RANGE)), dim3(256), 0, s, act_i, act_g, a, ISA,
+                       n, cb, scratch, (const u32 *)on);
+    hipLaunchKernelGGL(k_chain_next, dim3(tiles), dim3(256), 0, s, (const u64 *)scratch, words, next, tile);
+    if (tiles > 1) hipLaunchKernelGGL(k_chain_tiles, dim3(1), dim3(1024), 0, s, tile, tiles);
+    SAGPU_CHECK(hipGetLastError());
+    *ch = Chains{(const u64 *)scratch, next, tile, on};
+    return SAGPU_OK;
 }
 
 int launch_tail_groups(const u32 *ISA, u64 n, u32 cnt, u32 *out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_tail_groups, dim3(1), dim3(64), 0, s, ISA, n, cnt, out);
-    SAGPU_CHECK(hipGetLastError());
-    return SAGPU_OK;
-}
-
-int launch_round_start(u64 *rp, u64 a, u64 h, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_round_start, dim3(1), dim3(1), 0, s, rp, a, h);
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }

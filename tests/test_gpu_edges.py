@@ -219,3 +219,64 @@ def test_small_gsa(n):
             bad = T.copy()
             bad[30:32] = 0
             assert la.libsais_gsa(bad, out, n, 0, None) == -1
+
+
+def _chain_texts(n, rng):
+    """Repeats whose groups continue into one another: two and nine copies (the most a
+    chain takes is eight), copies up to the text's last symbol, and copies that change
+    how many they are along the way."""
+    base = rng.integers(97, 101, n).astype(np.uint8)
+    two = base.copy()
+    two[n // 2 + 7:] = two[:n - n // 2 - 7]
+    yield "two, to the end", two
+    mixed = base.copy()
+    k = n // 16
+    for c, size in ((3, k), (6, k - 1), (9, k // 2), (12, k // 3), (14, 2 * k)):
+        mixed[c * k:c * k + size] = mixed[:size]
+    yield "two to six", mixed
+    yield "eight", np.tile(base[:n // 8], 9)[:n].copy()
+    nine = np.tile(base[:n // 10], 10)[:n].copy()
+    nine[n // 10 * 9:] = base[n // 10 * 9:][:len(nine) - n // 10 * 9]
+    yield "nine", nine
+
+
+@pytest.mark.parametrize("n", [40, 1000, 4097, 65535 * 2 + 3, 300007])
+def test_round_chains(n):
+    """Groups compared at the end of their chains (from lists of 2 entries on, and never),
+    over words, tiles and the text's last positions: plain texts and string sets, with
+    codes and marks, against the oracle."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    rng = np.random.default_rng(n)
+    for name, T in _chain_texts(n, rng):
+        for gsa in (False, True):
+            if gsa:
+                T = T.copy()
+                T[n // 5::n // 3 + 1] = 0
+                T[-2:] = (98, 0)
+            rc, SA = ol.sa(T, gsa=gsa)
+            assert rc == 0
+            P = ol.plcp(T, SA, gsa=gsa)
+            L = ol.lcp(P, SA)
+            for least in (2, 0):
+                assert lib.sagpu_set_option(b"chain_min", least) == 0
+                try:
+                    gSA, gU, gp, gP, gL, _ = fused(T, gsa=gsa)
+                    print(f"[chains] n={n} {name} gsa={gsa} from {least}: {la.stats().rounds} rounds", flush=True)
+                finally:
+                    assert lib.sagpu_set_option(b"chain_min", 4096) == 0
+                assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, L), (name, least)
+                if not gsa:
+                    U, p = ol.bwt(T, SA)
+                    assert gp == p and np.array_equal(gU, U), (name, least)
+    S = rng.integers(0, 40000, n).astype(np.uint16)
+    S[n // 2:] = S[:n - n // 2]
+    rc, SA = ol.sa16(S)
+    assert rc == 0
+    for least in (2, 0):
+        assert lib.sagpu_set_option(b"chain_min", least) == 0
+        try:
+            out = np.zeros(n, np.int32)
+            assert la.libsais16(S, out, n, 0, None) == 0 and np.array_equal(out, SA), least
+        finally:
+            assert lib.sagpu_set_option(b"chain_min", 4096) == 0
