@@ -172,6 +172,8 @@ int group_init(WsScratch &ws, const u32 *keys, const u32 *vals, u64 n, int bits,
 void set_isa_window_log2(int v);
 // log2 of the bucket size used for an n-entry permutation scatter (at most 64 buckets).
 int isa_bucket_log2(u64 n);
+// The same for the (suffix, rank) pairs of the initial grouping.
+int isa_pair_bucket_log2(u64 n);
 // List entries per workgroup of the tile round kernel: 256, 512 (default) or 1024.
 void set_tile_range(int v);
 // Batched GSA: keys = (string id << 32) | packed symbols.

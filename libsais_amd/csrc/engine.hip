@@ -931,13 +931,13 @@ int sort_u32(Ctx &c, u32 *k0, u32 *v0, u32 *k1, u32 *v1, u64 n, int begin_bit, i
 }
 
 // ISA from the (suffix, rank) pairs of the initial grouping, bucketed by suffix >> cw
-// (bucket-major).  Texts over 2^22 with at most 8 buckets: one radix pass on bits
+// (bucket-major).  Texts of 2^22 to 2^31 suffixes (at most 8 buckets): one radix pass on bits
 // [cw - 8, cw) groups the pairs into windows of 2^(cw - 8) suffixes, and each XCD
 // writes only its own windows (launch_scatter_windows); otherwise one pass over the
 // pairs in bucket order.  K1 / V1: free buffers of n words for the radix pass.
 int isa_from_pairs(Ctx &c, Scope &sc, const u32 *PV, const u32 *PG, u64 n, u32 *ISA, u32 *K1, u32 *V1)
 {
-    const int cw = isa_bucket_log2(n);
+    const int cw = isa_pair_bucket_log2(n);
     const u64 nc = ((n - 1) >> cw) + 1;
     if (g_windowed_scatter && n > (1ull << 22) && nc <= 8 && cw >= 16) {
         int alt = 0;

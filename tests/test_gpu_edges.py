@@ -280,3 +280,27 @@ def test_round_chains(n):
             assert la.libsais16(S, out, n, 0, None) == 0 and np.array_equal(out, SA), least
         finally:
             assert lib.sagpu_set_option(b"chain_min", 4096) == 0
+
+
+@pytest.mark.parametrize("n", [(1 << 28) - 1, (1 << 28) + 1, (1 << 28) + 12345])
+def test_isa_windows(n):
+    """Texts on both sides of 2^28 suffixes, above which the ISA's buckets grow: windowed
+    and direct scatter give one suffix array, and the BWT of both is the text's."""
+    lib = la.load()
+    T = workloads.iid(n, seed=n & 255, alphabet=b"ACGT")
+    from tests.test_gpu_parity import fused
+    out = []
+    for on in (1, 0):
+        print(f"[isa windows] n={n} windowed_scatter={on}", flush=True)
+        assert lib.sagpu_set_option(b"windowed_scatter", on) == 0
+        try:
+            out.append(fused(T)[:3])
+        finally:
+            assert lib.sagpu_set_option(b"windowed_scatter", 1) == 0
+    (SA, U, p), (SA0, U0, p0) = out
+    assert np.array_equal(SA, SA0) and p == p0 and np.array_equal(U, U0)
+    rng = np.random.default_rng(n)
+    j = rng.integers(1, n, 20000)
+    a, b = SA[j - 1].astype(np.int64), SA[j].astype(np.int64)
+    keys = [[T[q:q + 64].tobytes() for q in (x, y)] for x, y in zip(a, b)]
+    assert all(x <= y for x, y in keys)
