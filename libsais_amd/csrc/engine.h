@@ -92,6 +92,18 @@ enum { RADIX_ONESWEEP = 0, RADIX_REDUCE_THEN_SCAN = 1 };
 
 enum { RS_THREADS = 256, RS_ITEMS = 8, RS_TILE = RS_THREADS * RS_ITEMS };  // smallest tile: sizes the scratch
 
+// Keys [start, end) of one workgroup's tile of a segmented sort, all of segment seg,
+// whose first tile is number `first`; at most SEG_TILE_KEYS keys.
+struct SegTile {
+    u32 start, end, seg, first;
+};
+constexpr u32 SEG_TILE_KEYS = 16384;
+// Sorts every segment (a contiguous range of the keys) by itself, stably, by key bits
+// [0, end_bit), end_bit <= 32; the result is in (k1, v1) when *alt is set.  seg: the
+// segments' tiles in order (each but a segment's last one full); seg_start: their first
+// keys; hist: (passes * nseg * 256) u32 of scratch.
+int radix_sort_seg(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, const SegTile *seg, u32 ntiles,
+                   const u32 *seg_start, u32 nseg, u32 *hist, int end_bit, hipStream_t s, int *alt);
 int radix_sort_u64(RadixScratch &rs, u64 *k0, u32 *v0, u64 *k1, u32 *v1, u64 n, int begin_bit,
                    int end_bit, hipStream_t s, int *result_in_alt, int *passes_run);
 int radix_sort_u32(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, u64 n, int begin_bit,
@@ -368,6 +380,9 @@ int launch_pack_keys32(const uint8_t *T, u64 n, const uint8_t *lut, int bits, in
 // Batched GSA: sid[p] = number of 0 bytes before p (string id); keys get sid in
 // their high half.  launch_string_ids needs a ScanScratch for n entries.
 int launch_string_ids(const uint8_t *T, u64 n, u32 *sid, ScanScratch &sc, hipStream_t s);
+// The same in 32 bits: (local[string id] << (bits * k)) | symbols.
+int launch_pack_keys32_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid,
+                           const uint8_t *local, u32 *keys, u32 *vals, hipStream_t s);
 int launch_pack_keys64_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid, u64 *keys,
                            u32 *vals, hipStream_t s);
 // Checks that string k starts at offsets[k] (sid[offsets[k]] == k and the byte

@@ -930,6 +930,23 @@ int sort_u32(Ctx &c, u32 *k0, u32 *v0, u32 *k1, u32 *v1, u64 n, int begin_bit, i
     return rc;
 }
 
+int sort_seg(Ctx &c, u32 *k0, u32 *v0, u32 *k1, u32 *v1, u64 n, const SegTile *seg, u32 ntiles, const u32 *start,
+             u32 nseg, u32 *hist, int end_bit, int *alt)
+{
+    const int64_t passes = (end_bit + 7) / 8;
+    c.rs.hook = c.timer.on ? onesweep_hook : nullptr;
+    c.rs.hook_user = &c;
+    c.sort_u32 = true;
+    c.timer.hook_n = n;
+    const int rc = radix_sort_seg(c.rs, k0, v0, k1, v1, seg, ntiles, start, nseg, hist, end_bit, c.stream, alt);
+    c.sort_u32 = false;
+    c.stats.sort_passes += passes;
+    c.stats.sorted_elems += passes * (int64_t)n;
+    c.stats.sorted_bytes += passes * (int64_t)n * 16;
+    c.stats.sorted_bytes_u32 += passes * (int64_t)n * 16;
+    return rc;
+}
+
 // ISA from the (suffix, rank) pairs of the initial grouping, bucketed by suffix >> cw
 // (bucket-major).  Texts of 2^22 to 2^31 suffixes (at most 8 buckets): one radix pass on bits
 // [cw - 8, cw) groups the pairs into windows of 2^(cw - 8) suffixes, and each XCD
@@ -966,6 +983,46 @@ int read_u32(Ctx &c, const u32 *d, u32 *out)
     SAGPU_CHECK(hipStreamSynchronize(c.stream));
     *out = *(u32 *)c.pinned;
     return SAGPU_OK;
+}
+
+// Plan of a string set's segmented sort: consecutive strings, as many as the key bits
+// that the symbols leave can tell apart, make a segment.  Positions come string by string,
+// so a segment's keys stay in its own range: 32-bit keys, 16 B per key and pass, instead
+// of (string id, symbols) keys of 64 bits with 24 B and the id's passes on top.
+struct SegPlan {
+    std::vector<SegTile> tiles;
+    std::vector<u32> start;       // first key of each segment
+    std::vector<uint8_t> local;   // a string's number in its segment
+    int end_bit = 0;
+};
+// False when the 64-bit sort moves no more: every segment's last tile is only half full
+// on average, which short strings pay for.  Below 2^22 keys the tables and the extra
+// launches cost what the bytes save.
+bool plan_segments(const Ctx &c, const int64_t *off, u32 count, u64 n, int kbits, SegPlan &sp)
+try {
+    const RadixScratch &rs = c.rs;
+    if (!off || n < (1ull << 22) || n > (u64)INT32_MAX || rs.variant != RADIX_ONESWEEP || rs.bits != 8 || rs.items != 32 ||
+        rs.threads != 512)
+        return false;
+    const int spare = 32 - kbits < 8 ? 32 - kbits : 8;
+    const u32 most = 1u << spare;
+    sp.end_bit = kbits + (count < most ? bits_for(count - 1) : spare);
+    const u64 pass32 = (u64)(sp.end_bit + 7) / 8 * SEG_TILE_KEYS * 16, all64 = (u64)(32 + bits_for(count - 1) + 7) / 8 * n * 24;
+    const u64 max_tiles = all64 / pass32;
+    if ((u64)(count + most - 1) / most > max_tiles) return false;
+    sp.local.resize(count);
+    for (u32 q0 = 0; q0 < count; q0 += most) {
+        const u32 q1 = count - q0 < most ? count : q0 + most;
+        for (u32 q = q0; q < q1; q++) sp.local[q] = (uint8_t)(q - q0);
+        const u32 first = (u32)sp.tiles.size(), lo = (u32)off[q0], hi = (u32)off[q1];
+        for (u32 t = lo; t < hi; t += hi - t < SEG_TILE_KEYS ? hi - t : SEG_TILE_KEYS)
+            sp.tiles.push_back({t, hi - t < SEG_TILE_KEYS ? hi : t + SEG_TILE_KEYS, (u32)sp.start.size(), first});
+        sp.start.push_back(lo);
+        if (sp.tiles.size() > max_tiles) return false;
+    }
+    return sp.tiles.size() * 256 <= rs.lb_words;
+} catch (const std::bad_alloc &) {
+    return false;
 }
 
 // The context's byte counts (kept zero) and code tables.
@@ -1014,7 +1071,8 @@ int byte_alphabet(Ctx &c, const uint8_t *dT, u64 n, int gsa, bool pad, u64 *freq
 // launch_bwt_seeded (seed->cb > 0 on return); otherwise seed->cb stays 0.
 int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32 *dISA, u64 *freq_out, u32 *dLCP,
              const u32 *sid = nullptr, u32 nstrings = 0, const u32 *dSym = nullptr, int sym_bits = 0,
-             BwtSeed *seed = nullptr, CodeStream *cs = nullptr, PlcpHint *hint = nullptr)
+             BwtSeed *seed = nullptr, CodeStream *cs = nullptr, PlcpHint *hint = nullptr,
+             const int64_t *h_off = nullptr)
 {
     hipStream_t s = c.stream;
     sagpu_stats &st = c.stats;
@@ -1045,7 +1103,10 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     //   aA  [2n u32]: first active list (suffix, group head)
     // Groups too big for one workgroup get their own sort buffers per round.
     const bool wide = n > g_wide_from;
-    GET(kA, u32, sid ? 4 * n : 2 * n);
+    SAGPU_TRY(ensure_radix_scratch(c, sc, n));
+    SegPlan sp_plan;
+    const bool by_segment = sid && plan_segments(c, h_off, nstrings, n, ksym * bits, sp_plan);
+    GET(kA, u32, sid && !by_segment ? 4 * n : 2 * n);
     GET(vA, u32, 2 * n);
     GET(aA, u32, 2 * n);
     const u64 big_cap = n / (RT_SMALL + 1) + 16;
@@ -1072,7 +1133,6 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         ws.total = d_cnt + 2;
         ws.base = d_cnt + 3;
     }
-    SAGPU_TRY(ensure_radix_scratch(c, sc, n));
     {
         // bucket counts of the initial grouping: at most 64 buckets per tile
         ws.bcnt_cap = 64 * ws.tiles_cap;
@@ -1145,6 +1205,30 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
                 ex1.hint_off = hint ? hint->off : 0;
             }
         }
+    } else if (by_segment) {
+        // batched GSA: (string of the segment, symbols) keys sorted inside the segment.
+        // Keys of two segments may agree, but a string's first suffix in order is its
+        // separator, alone in its group, so every group stays inside one string.
+        u32 *k0 = kA, *k1 = kA + n, *v0 = vA, *v1 = vA + n;
+        const u32 ntiles = (u32)sp_plan.tiles.size(), nseg = (u32)sp_plan.start.size();
+        const int npass = (sp_plan.end_bit + 7) / 8;
+        Scope srt(c);
+        SegTile *d_seg = srt.get<SegTile>(ntiles);
+        u32 *d_start = srt.get<u32>(nseg), *d_hist = srt.get<u32>((u64)npass * nseg * 256);
+        uint8_t *d_local = srt.get<uint8_t>(nstrings);
+        if (!d_seg || !d_start || !d_hist || !d_local) return SAGPU_ENOMEM;
+        SAGPU_CHECK(hipMemcpyAsync(d_seg, sp_plan.tiles.data(), ntiles * sizeof(SegTile), hipMemcpyHostToDevice, s));
+        SAGPU_CHECK(hipMemcpyAsync(d_start, sp_plan.start.data(), nseg * sizeof(u32), hipMemcpyHostToDevice, s));
+        SAGPU_CHECK(hipMemcpyAsync(d_local, sp_plan.local.data(), nstrings, hipMemcpyHostToDevice, s));
+        {
+            Span sp(c, F_INITIAL);
+            SAGPU_TRY(launch_pack_keys32_sid(dT, n, d_lut, bits, ksym, sid, d_local, k0, v0, s));
+        }
+        SAGPU_TRY(sort_seg(c, k0, v0, k1, v1, n, d_seg, ntiles, d_start, nseg, d_hist, sp_plan.end_bit, &alt));
+        Span sp(c, F_INITIAL);
+        SAGPU_TRY(group_init(ws, alt ? k1 : k0, alt ? v1 : v0, n, bits, ksym, 1, dSA, dISA, act_i[0], act_g[0], dLCP,
+                             alt ? k0 : k1, alt ? v0 : v1, s));
+        SAGPU_TRY(isa_from_pairs(c, sc, alt ? k0 : k1, alt ? v0 : v1, n, dISA, alt ? k1 : k0, alt ? v1 : v0));
     } else {
         // batched GSA: (string id, symbols) keys, so every group stays inside one string
         u64 *k0 = (u64 *)kA, *k1 = (u64 *)kA + n;
@@ -3144,7 +3228,8 @@ extern "C" int32_t sagpu_gsa_batch32(const uint8_t *d_T, int64_t n, const int64_
     }
     {
         Span total(*c, F_TOTAL);
-        int rc = sa_build(*c, sc, dT, (u64)n, 1, gSA, ISA, nullptr, marks, sid, (u32)count);
+        int rc = sa_build(*c, sc, dT, (u64)n, 1, gSA, ISA, nullptr, marks, sid, (u32)count, nullptr, 0, nullptr, nullptr,
+                          nullptr, h_offsets);
         if (rc != SAGPU_OK) return rc;
         if (d_LCP) {
             {
@@ -3297,7 +3382,8 @@ int run_batch(Ctx &c, sagpu_job **jobs, int count)
         gL = marks;
         if (!marks || !P) return SAGPU_ENOMEM;
     }
-    SAGPU_TRY(sa_build(c, sc, dT, N, 1, gSA, ISA, nullptr, marks, sid, (u32)count));
+    SAGPU_TRY(sa_build(c, sc, dT, N, 1, gSA, ISA, nullptr, marks, sid, (u32)count, nullptr, 0, nullptr, nullptr, nullptr,
+                       off.data()));
     if (any_l) {
         SAGPU_TRY(plcp_run(c, sc, dT, N, 1, nullptr, ISA, gSA, P, marks));
         SAGPU_TRY(launch_lcp_fix(P, gSA, N, gL, s));

@@ -215,13 +215,14 @@ __global__ __launch_bounds__(256) void k_radix_offsets(u64 *hist, int npass, int
 // ranking took fewer vector instructions (wave_peers), digit starts were folded into
 // one LDS read per element and values were loaded under the key writes.  u64 keys:
 // 3.37 ms for 2^29 pairs (3.72 before).
-template <typename K, bool HAS_VALS, bool LOOKBACK, int ITEMS, bool GEN = false, int NT = RS_THREADS, int DB = 8>
+template <typename K, bool HAS_VALS, bool LOOKBACK, int ITEMS, bool GEN = false, int NT = RS_THREADS, int DB = 8,
+          bool SEG = false>
 __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, const u32 *__restrict__ vin,
                                                            K *__restrict__ kout, u32 *__restrict__ vout, u64 n,
                                                            int shift, u32 dmask, const u64 *__restrict__ offsets,
                                                            u64 *__restrict__ lookback, u32 *__restrict__ tile_ctr,
                                                            u32 epoch, const u32 *__restrict__ scanned, u64 tiles,
-                                                           KeyGen gen)
+                                                           KeyGen gen, const SegTile *__restrict__ seg)
 {
     // NT threads (256 or 512) per workgroup; BINS digits, DPT per thread in the digit
     // phase (thread t takes digits [t * DPT, (t + 1) * DPT)).
@@ -245,8 +246,16 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     for (u32 i = tid; i < (u32)NW * BINS; i += NT) (&s_wcnt[0][0])[i] = 0;
     __syncthreads();
 
-    const u64 tile = LOOKBACK ? (u64)s_tile : (u64)blockIdx.x;
-    const u64 wbase = tile * TILE_ + (u64)w * WAVE_ITEMS_;
+    // SEG: the tile's own range of the keys, inside one segment; its look-back ends at
+    // the segment's first tile and its offsets are the segment's.
+    static_assert(!SEG || (LOOKBACK && !GEN && DB == 8), "segments: onesweep passes over arrays");
+    const u64 tile = SEG ? (u64)(u32)__builtin_amdgcn_readfirstlane((int)s_tile) : LOOKBACK ? (u64)s_tile : (u64)blockIdx.x;
+    SegTile sg{};
+    if (SEG) sg = seg[tile];
+    const u64 first = SEG ? (u64)sg.first : 0ull;
+    const u64 tbase = SEG ? (u64)sg.start : tile * TILE_;
+    if (SEG) n = sg.end;
+    const u64 wbase = tbase + (u64)w * WAVE_ITEMS_;
 
     // Values are loaded after the keys have left the registers: fewer live registers
     // per wave, more waves per SIMD.
@@ -259,7 +268,7 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     K key[ITEMS];
     u32 rank[ITEMS];
     u32 prevc[GEN ? ITEMS / 4 : 1];   // GEN: code of T[pos-1] per item, 8 bits each
-    const bool full = (tile + 1) * (u64)TILE_ <= n;
+    const bool full = tbase + (u64)TILE_ <= n;
     if constexpr (GEN) {
         // The tile's stretch of the code stream (from one symbol before the tile)
         // goes to LDS with coalesced loads; keys and preceding codes are cut from
@@ -350,7 +359,7 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
 #pragma unroll
             for (int qd = 0; qd < DPT; qd++)
                 st_release_u64(lookback + tile * BINS + tid * DPT + qd,
-                               lb_pack(epoch, tile == 0 ? LB_PRE : LB_AGG, run[qd]));
+                               lb_pack(epoch, tile == first ? LB_PRE : LB_AGG, run[qd]));
         }
 #pragma unroll
         for (int qd = 0; qd < DPT; qd++) {
@@ -358,14 +367,15 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
             if (LOOKBACK) {
                 u64 *my = lookback + tile * BINS + d;
                 u64 excl = 0;
-                if (tile > 0) {
+                if (tile > first) {
                     // Windowed look-back: the loads for up to LB_WIN predecessors are
                     // issued together so their latencies overlap; entries are consumed
                     // from the nearest one until an inclusive prefix is found.
                     long long t = (long long)tile - 1;
                     bool found = false;
                     while (!found) {
-                        const int cnt = t + 1 < LB_WIN ? (int)(t + 1) : LB_WIN;
+                        const long long left = t + 1 - (long long)first;
+                        const int cnt = left < LB_WIN ? (int)left : LB_WIN;
                         u64 v[LB_WIN];
 #pragma unroll
                         for (int q = 0; q < LB_WIN; q++)
@@ -384,7 +394,8 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
                     }
                     st_release_u64(my, lb_pack(epoch, LB_PRE, excl + run[qd]));
                 }
-                gbase[qd] = (u32)(offsets[d] + excl);
+                gbase[qd] = SEG ? reinterpret_cast<const u32 *>(offsets)[(u64)sg.seg * BINS + d] + (u32)excl
+                                : (u32)(offsets[d] + excl);
             } else {
                 gbase[qd] = scanned[(u64)d * tiles + tile];
             }
@@ -433,7 +444,6 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
         }
     }
     __syncthreads();
-    const u64 tbase = tile * TILE_;
     const u32 tile_n = (u32)((n - tbase) < (u64)TILE_ ? (n - tbase) : (u64)TILE_);
     // Digits of the staged keys are recomputed and kept packed in registers for the
     // value phase, so no LDS digit array is needed (one more workgroup per CU fits).
@@ -497,6 +507,49 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
                 if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
             }
         }
+    }
+}
+
+// Segmented sorts (radix_sort_seg): digit counts of every pass per segment, a tile per
+// workgroup (hist[(p * nseg + seg) * 256 + d], cleared by the caller), then each segment's
+// counts to offsets in place.
+__global__ __launch_bounds__(512) void k_seg_hist(const u32 *__restrict__ keys, const SegTile *__restrict__ seg,
+                                                  u32 nseg, int npass, u32 *__restrict__ hist)
+{
+    constexpr int C = 4;   // copies, as in k_radix_hist
+    __shared__ u32 s_hc[4 * C][256];
+    for (int i = threadIdx.x; i < npass * C * 256; i += 512) (&s_hc[0][0])[i] = 0;
+    __syncthreads();
+    const SegTile sg = seg[blockIdx.x];
+    const u32 copy = threadIdx.x & (C - 1);
+#pragma unroll 8
+    for (u32 i = sg.start + threadIdx.x; i < sg.end; i += 512) {
+        const u32 k = keys[i];
+        for (int p = 0; p < npass; p++) atomicAdd(&s_hc[p * C + copy][((k >> (8 * p)) + copy) & 255u], 1u);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < npass * 256; i += 512) {
+        const int p = i >> 8, d = i & 255;
+        u32 v = 0;
+        for (int c = 0; c < C; c++) v += s_hc[p * C + c][(d + c) & 255];
+        if (v) atomicAdd(&hist[((u64)p * nseg + sg.seg) * 256 + d], v);
+    }
+}
+__global__ __launch_bounds__(256) void k_seg_offsets(u32 *__restrict__ hist, const u32 *__restrict__ seg_start, u32 nseg,
+                                                     int npass, u32 *__restrict__ tile_ctr)
+{
+    __shared__ u32 s_w[256 / SAGPU_WAVE];
+    if (blockIdx.x == 0 && threadIdx.x < RADIX_MAX_PASSES) tile_ctr[threadIdx.x] = 0;
+    const u32 start = seg_start[blockIdx.x];
+    for (int p = 0; p < npass; p++) {
+        u32 *h = hist + ((u64)p * nseg + blockIdx.x) * 256;
+        const u32 v = h[threadIdx.x], inc = wave_incl_sum(v);
+        if (lane_id() == SAGPU_WAVE - 1) s_w[threadIdx.x / SAGPU_WAVE] = inc;
+        __syncthreads();
+        u32 o = start + inc - v;
+        for (u32 w = 0; w < threadIdx.x / SAGPU_WAVE; w++) o += s_w[w];
+        h[threadIdx.x] = o;
+        __syncthreads();
     }
 }
 
@@ -698,14 +751,14 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
         const u64 ptiles = (n + (u64)nt * items - 1) / ((u64)nt * items);
 #define RS_LAUNCH(HV, LB, IT)                                                                                     \
     hipLaunchKernelGGL((k_radix_pass<K, HV, LB, IT, false, RS_THREADS, DB>), dim3((unsigned)tiles), dim3(RS_THREADS), \
-                       0, s, ki, vi, ko, vo, n, shift, dmask, offs, lbk, tctr, rs.epoch, cnts, tiles, g0)
+                       0, s, ki, vi, ko, vo, n, shift, dmask, offs, lbk, tctr, rs.epoch, cnts, tiles, g0, (const SegTile *)nullptr)
 #define RS_LAUNCH512(HV, GN)                                                                                      \
     hipLaunchKernelGGL((k_radix_pass<K, HV, true, 32, GN, 512>), dim3((unsigned)ptiles), dim3(512), 0, s, ki, vi, ko, \
-                       vo, n, shift, dmask, offs, lbk, tctr, rs.epoch, cnts, ptiles, g0)
+                       vo, n, shift, dmask, offs, lbk, tctr, rs.epoch, cnts, ptiles, g0, (const SegTile *)nullptr)
 #define RS_LAUNCH_GEN(IT)                                                                                          \
     hipLaunchKernelGGL((k_radix_pass<K, true, true, IT, true, RS_THREADS, DB>), dim3((unsigned)gtiles),              \
                        dim3(RS_THREADS), 0, s, ki, vi, ko, vo, n, shift, dmask, offs, lbk, tctr, rs.epoch, cnts, gtiles, \
-                       g0)
+                       g0, (const SegTile *)nullptr)
         if (nt == 512) {
             if constexpr (sizeof(K) == 4 && DB == 8) {   // 16384 u32 keys: 64 KB of LDS staging
                 if (gen_now) RS_LAUNCH512(true, true);
@@ -750,6 +803,37 @@ int radix_sort_db(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int b
     return SAGPU_OK;
 }
 
+// ---- host: segmented sort
+int radix_sort_seg_impl(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, const SegTile *seg, u32 ntiles,
+                        const u32 *seg_start, u32 nseg, u32 *hist, int end_bit, hipStream_t s, int *alt)
+{
+    const int npass = (end_bit + 7) / 8;
+    if ((u64)ntiles * 256 > rs.lb_words || npass > 4) {
+        sagpu_set_error("radix scratch too small", __FILE__, __LINE__);
+        return SAGPU_EDEVICE;
+    }
+    SAGPU_TRY(launch_fill_u32(hist, (u64)npass * nseg * 256, 0, s));
+    hipLaunchKernelGGL(k_seg_hist, dim3(ntiles), dim3(512), 0, s, (const u32 *)k0, seg, nseg, npass, hist);
+    hipLaunchKernelGGL(k_seg_offsets, dim3(nseg), dim3(256), 0, s, hist, seg_start, nseg, npass, rs.tile_ctr);
+    for (int p = 0; p < npass; p++) {
+        rs.epoch = (rs.epoch + 1) & ((1u << 22) - 1);
+        if (rs.epoch == 0) {
+            SAGPU_TRY(launch_fill_u64(rs.lookback, rs.lb_words, 0, s));
+            rs.epoch = 1;
+        }
+        if (rs.hook) rs.hook(rs.hook_user, 0);
+        hipLaunchKernelGGL((k_radix_pass<u32, true, true, 32, false, 512, 8, true>), dim3(ntiles), dim3(512), 0, s, k0, v0, k1,
+                           v1, 0ull, 8 * p, 255u, (const u64 *)(hist + (u64)p * nseg * 256), rs.lookback, rs.tile_ctr + p,
+                           rs.epoch, (const u32 *)nullptr, 0ull, KeyGen{}, seg);
+        SAGPU_CHECK(hipGetLastError());
+        if (rs.hook) rs.hook(rs.hook_user, 1);
+        u32 *t = k0; k0 = k1; k1 = t;
+        t = v0; v0 = v1; v1 = t;
+    }
+    *alt = npass & 1;
+    return SAGPU_OK;
+}
+
 template <typename K>
 int radix_sort_impl(RadixScratch &rs, K *k0, u32 *v0, K *k1, u32 *v1, u64 n, int begin_bit, int end_bit,
                     hipStream_t s, int *result_in_alt, int *passes_run)
@@ -776,6 +860,12 @@ int launch_pack_stream(const uint8_t *T, u64 n, const uint8_t *lut, int bits, u3
     hipLaunchKernelGGL(k_pack_stream, dim3((unsigned)blocks), dim3(256), 0, s, T, n, lut, bits, pw, words);
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
+}
+
+int radix_sort_seg(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, const SegTile *seg, u32 ntiles,
+                   const u32 *seg_start, u32 nseg, u32 *hist, int end_bit, hipStream_t s, int *alt)
+{
+    return radix_sort_seg_impl(rs, k0, v0, k1, v1, seg, ntiles, seg_start, nseg, hist, end_bit, s, alt);
 }
 
 int radix_sort_u64(RadixScratch &rs, u64 *k0, u32 *v0, u64 *k1, u32 *v1, u64 n, int begin_bit, int end_bit,

@@ -138,6 +138,54 @@ __global__ __launch_bounds__(256) void k_zero_flags(const uint8_t *__restrict__ 
     for (u64 p = (u64)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += stride) f[p] = T[p] == 0;
 }
 
+// Keys of string sets sorted string by string (local: a string's number among those
+// sorted together).  Each thread takes PK_ITEMS consecutive positions from right to left,
+// key(i) = code(i) in front of key(i + 1) without its last symbol, and zero at a separator;
+// the keys are written out through LDS.  Bound by its 4 + 4 bytes written and 5 read per
+// position.
+__global__ __launch_bounds__(PK_THREADS) void k_pack_keys32_sid(const uint8_t *__restrict__ T, u64 n,
+                                                                const uint8_t *__restrict__ lut, int bits, int k,
+                                                                const u32 *__restrict__ sid,
+                                                                const uint8_t *__restrict__ local,
+                                                                u32 *__restrict__ keys, u32 *__restrict__ vals)
+{
+    constexpr int ROW = PK_ITEMS + 1;   // (rows a bank apart)
+    __shared__ uint8_t s_lut[256];
+    __shared__ uint8_t s_c[PK_TILE + PK_HALO];
+    __shared__ u32 s_k[PK_THREADS * ROW];
+    s_lut[threadIdx.x] = lut[threadIdx.x];
+    __syncthreads();
+    const u64 base = (u64)blockIdx.x * PK_TILE;
+    for (int i = threadIdx.x; i < PK_TILE + PK_HALO; i += PK_THREADS) {
+        const u64 p = base + i;
+        s_c[i] = p < n ? s_lut[T[p]] : 0;
+    }
+    __syncthreads();
+    const int lo = (int)threadIdx.x * PK_ITEMS, top = bits * (k - 1);
+    u32 key = 0;
+    for (int t = k - 1; t >= 0; t--) {   // key(lo + PK_ITEMS)
+        const u32 c = s_c[lo + PK_ITEMS + t];
+        key = c ? (c << top) | (key >> bits) : 0u;
+    }
+#pragma unroll
+    for (int j = PK_ITEMS - 1; j >= 0; j--) {
+        const u32 c = s_c[lo + j];
+        key = c ? (c << top) | (key >> bits) : 0u;
+        s_k[threadIdx.x * ROW + j] = key;
+    }
+    __syncthreads();
+    const int kb = bits * k;
+#pragma unroll 4
+    for (int j = 0; j < PK_ITEMS; j++) {
+        const int li = j * PK_THREADS + (int)threadIdx.x;
+        const u64 p = base + li;
+        if (p >= n) break;
+        const u32 l = local[sid[p]];
+        keys[p] = s_k[li / PK_ITEMS * ROW + li % PK_ITEMS] | (l ? l << kb : 0u);
+        vals[p] = (u32)p;
+    }
+}
+
 __global__ __launch_bounds__(PK_THREADS) void k_pack_keys64_sid(const uint8_t *__restrict__ T, u64 n,
                                                                 const uint8_t *__restrict__ lut, int bits, int k,
                                                                 const u32 *__restrict__ sid, u64 *__restrict__ keys,
@@ -542,6 +590,19 @@ int launch_string_ids(const uint8_t *T, u64 n, u32 *sid, ScanScratch &sc, hipStr
     hipLaunchKernelGGL(k_zero_flags, dim3(grid_for(n, 256 * 8, 65535)), dim3(256), 0, s, T, n, sid);
     SAGPU_CHECK(hipGetLastError());
     return scan_exclusive_u32(sc, sid, n, s);
+}
+
+int launch_pack_keys32_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid,
+                           const uint8_t *local, u32 *keys, u32 *vals, hipStream_t s)
+{
+    if (k > PK_HALO || k < 1 || k * bits > 32) {
+        sagpu_set_error("pack_keys: bad symbol count", __FILE__, __LINE__);
+        return SAGPU_EDEVICE;
+    }
+    hipLaunchKernelGGL(k_pack_keys32_sid, dim3(ceil_div_u(n, PK_TILE)), dim3(PK_THREADS), 0, s, T, n, lut, bits, k, sid,
+                       local, keys, vals);
+    SAGPU_CHECK(hipGetLastError());
+    return SAGPU_OK;
 }
 
 int launch_pack_keys64_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid, u64 *keys,

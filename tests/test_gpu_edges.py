@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import libsais_amd as la
-from libsais_amd import workloads
+from libsais_amd import batch, workloads
 from tests import oracle_lib as ol
 
 pytestmark = pytest.mark.gpu
@@ -304,3 +304,57 @@ def test_isa_windows(n):
     a, b = SA[j - 1].astype(np.int64), SA[j].astype(np.int64)
     keys = [[T[q:q + 64].tobytes() for q in (x, y)] for x, y in zip(a, b)]
     assert all(x <= y for x, y in keys)
+
+
+SEG_KEYS = 16384   # keys of a tile of a segmented sort
+
+
+def _string_sets():
+    """(name, string lengths, symbols): sets of at least 2^22 symbols, whose strings are
+    sorted four to a segment (5 codes: 30-bit keys), one (16 and 256 codes: no bits left)
+    and sixteen (100 codes); lengths around whole tiles, one string, a few long ones."""
+    rng = np.random.default_rng(7)
+    n = 1 << 22
+    edges = [SEG_KEYS - 1, SEG_KEYS, SEG_KEYS + 1, 4 * SEG_KEYS, 2, 3, 65]
+    around = [edges[i % 7] for i in range(7 * (n // sum(edges) + 1))]
+    mixed = rng.integers(2, 60000, 160)
+    yield "around tiles", around, 4
+    yield "one string", [n], 4
+    yield "two strings", [n // 2, n // 2 + 5], 15
+    yield "long and short", [n - 100, 2, 2, 50, 70001], 255
+    yield "mixed, 4 bits", list(mixed) + [3], 15
+    yield "mixed, 7 bits", list(mixed) + [5, 2], 99
+    yield "alike", [40000] * 106, 4
+    yield "short", [90] * (n // 90 + 1), 4   # too short: the 64-bit sort
+
+
+@pytest.mark.parametrize("name,lengths,sigma", list(_string_sets()), ids=lambda v: v if isinstance(v, str) else "")
+def test_segmented_sort(name, lengths, sigma):
+    """Sets sorted string by string against the sort by (string, symbols) of the same set
+    (the form that other tiles take), and sampled strings against the oracle."""
+    lib = la.load()
+    rng = np.random.default_rng(len(lengths))
+    n = int(np.sum(lengths))
+    offs = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    T = rng.integers(1, sigma + 1, n).astype(np.uint8)
+    if name == "alike":
+        T[:] = np.tile(T[:40000], len(lengths))
+    T[offs[1:] - 1] = 0
+    out = []
+    for items in (32, 16):
+        print(f"[segments] {name}: n={n} strings={len(lengths)} radix_items={items}", flush=True)
+        assert lib.sagpu_set_option(b"radix_items", items) == 0
+        try:
+            out.append(batch.batched(T, offs))
+            print(f"[segments] bytes sorted per symbol: {la.stats().sorted_bytes / n:.0f}", flush=True)
+        finally:
+            assert lib.sagpu_set_option(b"radix_items", 32) == 0
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    SA, L = out[0]
+    for k in sorted({0, len(lengths) // 2, len(lengths) - 1}):
+        o, e = int(offs[k]), int(offs[k + 1])
+        if e - o > 100000:
+            continue
+        rc, ref = ol.sa(T[o:e].copy(), gsa=True)
+        assert rc == 0 and np.array_equal(SA[o:e], ref), k
+        assert np.array_equal(L[o:e], ol.lcp(ol.plcp(T[o:e].copy(), ref, gsa=True), ref)), k
