@@ -63,45 +63,59 @@ __device__ __forceinline__ u32 mask_below(u64 m)
     return __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
 }
 
-// Inclusive wave-level scan (sum) over 64 lanes.
+// Lane moves inside the wave by DPP, which costs a vector instruction where a shuffle
+// takes a trip through LDS.  Lanes without a source get `old`.
+template <int CTRL, int ROWS> __device__ __forceinline__ u32 dpp(u32 old, u32 v)
+{
+    return (u32)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ u64 dpp(u64 old, u64 v)
+{
+    return (u64)dpp<CTRL, ROWS>((u32)(old >> 32), (u32)(v >> 32)) << 32 | dpp<CTRL, ROWS>((u32)old, (u32)v);
+}
+// The value of the lane below (lane 0: old) and above (lane 63: old).
+template <typename V> __device__ __forceinline__ V lane_up(V old, V v) { return dpp<0x138, 0xf>(old, v); }
+template <typename V> __device__ __forceinline__ V lane_down(V old, V v) { return dpp<0x130, 0xf>(old, v); }
+// The value of one lane, in a scalar register.
+__device__ __forceinline__ u32 lane_value(u32 v, int l) { return (u32)__builtin_amdgcn_readlane((int)v, l); }
+__device__ __forceinline__ u64 lane_value(u64 v, int l)
+{
+    return (u64)lane_value((u32)(v >> 32), l) << 32 | lane_value((u32)v, l);
+}
+
+// Inclusive wave-level scans over 64 lanes: within rows of 16 lanes, then the last lane of
+// each row (and of the lower half) to the rows after it.
+template <typename V, class OP> __device__ __forceinline__ V wave_scan(V v, OP op)
+{
+    v = op(v, dpp<0x111, 0xf>((V)0, v));
+    v = op(v, dpp<0x112, 0xf>((V)0, v));
+    v = op(v, dpp<0x114, 0xf>((V)0, v));
+    v = op(v, dpp<0x118, 0xf>((V)0, v));
+    v = op(v, dpp<0x142, 0xa>((V)0, v));
+    v = op(v, dpp<0x143, 0xc>((V)0, v));
+    return v;
+}
 __device__ __forceinline__ u32 wave_incl_sum(u32 v)
 {
-#pragma unroll
-    for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
-        u32 o = __shfl_up(v, d, SAGPU_WAVE);
-        if ((int)lane_id() >= d) v += o;
-    }
-    return v;
+    return wave_scan(v, [](u32 a, u32 b) { return a + b; });
 }
-
 __device__ __forceinline__ u32 wave_incl_max(u32 v)
 {
-#pragma unroll
-    for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
-        u32 o = __shfl_up(v, d, SAGPU_WAVE);
-        if ((int)lane_id() >= d) v = v > o ? v : o;
-    }
-    return v;
+    return wave_scan(v, [](u32 a, u32 b) { return a > b ? a : b; });
 }
-
 __device__ __forceinline__ u64 wave_incl_sum64(u64 v)
 {
-#pragma unroll
-    for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
-        u64 o = __shfl_up(v, d, SAGPU_WAVE);
-        if ((int)lane_id() >= d) v += o;
-    }
-    return v;
+    return wave_scan(v, [](u64 a, u64 b) { return a + b; });
 }
-
 __device__ __forceinline__ u64 wave_incl_max64(u64 v)
 {
-#pragma unroll
-    for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
-        u64 o = __shfl_up(v, d, SAGPU_WAVE);
-        if ((int)lane_id() >= d) v = v > o ? v : o;
-    }
-    return v;
+    return wave_scan(v, [](u64 a, u64 b) { return a > b ? a : b; });
+}
+
+// row + the highest set bit of m, or `none`.
+__device__ __forceinline__ u32 last_set(u64 m, u32 row, u32 none)
+{
+    return m ? row + 63u - (u32)__clzll((long long)m) : none;
 }
 
 // p[i] of memory that nothing writes while the kernel runs, at an index that is the same

@@ -300,6 +300,8 @@ constexpr int MS_THREADS = 256, MS_ITEMS = 16, MS_TILE = MS_THREADS * MS_ITEMS;
 
 template <typename VT>
 __device__ __forceinline__ VT vmax(VT a, VT b) { return a > b ? a : b; }
+__device__ __forceinline__ u32 wave_incl_max_t(u32 v) { return wave_incl_max(v); }
+__device__ __forceinline__ u64 wave_incl_max_t(u64 v) { return wave_incl_max64(v); }
 
 // 64 stream bits from bit `bitpos` (the stream has a zero word past every window).
 __device__ __forceinline__ u64 stream_window(const u32 *__restrict__ pw, u64 bitpos)
@@ -411,8 +413,8 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
                 mx = vmax(mx, v);
             }
         }
-        for (int d = 32; d >= 1; d >>= 1) mx = vmax(mx, (VT)__shfl_xor(mx, d, SAGPU_WAVE));
-        if (lane_id() == 0) s_m[threadIdx.x / SAGPU_WAVE] = mx;
+        mx = wave_incl_max_t(mx);
+        if (lane_id() == SAGPU_WAVE - 1) s_m[threadIdx.x / SAGPU_WAVE] = mx;
         __syncthreads();
         if (threadIdx.x == 0) {
             const VT m = vmax(vmax(s_m[0], s_m[1]), vmax(s_m[2], s_m[3]));
@@ -639,17 +641,6 @@ __global__ __launch_bounds__(256) void k_plcp_vlong_fin(VT *__restrict__ V, VT *
 
 
 template <typename VT>
-__device__ __forceinline__ VT wave_incl_max_t(VT v)
-{
-#pragma unroll
-    for (int d = 1; d < SAGPU_WAVE; d <<= 1) {
-        VT o = __shfl_up(v, d, SAGPU_WAVE);
-        if ((int)lane_id() >= d) v = vmax(v, o);
-    }
-    return v;
-}
-
-template <typename VT>
 __global__ __launch_bounds__(MS_THREADS) void k_max_reduce(const VT *__restrict__ V, u64 n, VT *__restrict__ tmax)
 {
     __shared__ VT s_w[4];
@@ -695,8 +686,7 @@ __device__ VT max_step(VT *tmax, u64 tiles, u64 base, VT carry, VT *s_w, VT *s_e
     __syncthreads();
     VT c = carry;
     for (u32 q = 0; q < threadIdx.x / SAGPU_WAVE; q++) c = vmax(c, s_w[q]);
-    const VT prev = __shfl_up(inc, 1, SAGPU_WAVE);
-    if (lane_id() > 0) c = vmax(c, prev);
+    c = vmax(c, lane_up((VT)0, inc));
 #pragma unroll
     for (int q = 0; q < MX_K; q++) {   // exclusive max of the tiles before i0 + q
         if (i0 + q < tiles) tmax[i0 + q] = c;
@@ -786,7 +776,7 @@ __global__ __launch_bounds__(MS_THREADS) void k_max_apply(const VT *V, u64 n, co
         load4(V, wbase + (u64)r * 256 + 4 * lane, n, full, v[r]);
         VT m = vmax(vmax(v[r][0], v[r][1]), vmax(v[r][2], v[r][3]));
         inc[r] = wave_incl_max_t(m);
-        tot = vmax(tot, (VT)__shfl(inc[r], SAGPU_WAVE - 1, SAGPU_WAVE));
+        tot = vmax(tot, lane_value(inc[r], SAGPU_WAVE - 1));
     }
     if (lane == 0) s_w[w] = tot;
     __syncthreads();
@@ -795,8 +785,7 @@ __global__ __launch_bounds__(MS_THREADS) void k_max_apply(const VT *V, u64 n, co
 #pragma unroll
     for (int r = 0; r < ROWS; r++) {
         const u64 e0 = wbase + (u64)r * 256 + 4 * lane;
-        VT prev = __shfl_up(inc[r], 1, SAGPU_WAVE);
-        VT cl = lane > 0 ? vmax(c, prev) : c;
+        VT cl = vmax(c, lane_up((VT)0, inc[r]));
         u32 o[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -810,7 +799,7 @@ __global__ __launch_bounds__(MS_THREADS) void k_max_apply(const VT *V, u64 n, co
             for (int k = 0; k < 4; k++)
                 if (e0 + k < n) PLCP[e0 + k] = o[k];
         }
-        c = vmax(c, (VT)__shfl(inc[r], SAGPU_WAVE - 1, SAGPU_WAVE));
+        c = vmax(c, lane_value(inc[r], SAGPU_WAVE - 1));
     }
 }
 

@@ -416,9 +416,8 @@ __global__ __launch_bounds__(256) void k_piv_emit(const u32 *__restrict__ pq, Pi
         const u64 m = c0 + (u64)row * SAGPU_WAVE + lane;
         const bool in = m < npv;
         const u32 q = in ? pq[m] : NOQ;
-        const u32 left = __shfl_up(q, 1, SAGPU_WAVE);
-        const u32 qm1 = lane == 0 ? above : left;
-        above = __shfl(q, SAGPU_WAVE - 1, SAGPU_WAVE);
+        const u32 qm1 = lane_up(above, q);
+        above = lane_value(q, SAGPU_WAVE - 1);
         if (!in) continue;
         u32 b = 0;
 #pragma unroll

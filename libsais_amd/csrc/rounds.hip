@@ -49,18 +49,12 @@ __global__ __launch_bounds__(WS_THREADS) void k_ws_reduce(F f, Agg *__restrict__
     u64 s = 0;
     u32 m1 = 0, m2 = 0;
     for (int r = 0; r < R; r++) {
-        u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
-        bool act;
-        u32 v1, v2;
-        f.scan_inputs(e, act, v1, v2);   // every lane calls (rows may shuffle); e >= n yields nothing
-        s += act;
-        m1 = umax(m1, v1);
-        m2 = umax(m2, v2);
-    }
-    for (int d = 32; d >= 1; d >>= 1) {
-        s += __shfl_xor(s, d, SAGPU_WAVE);
-        m1 = umax(m1, __shfl_xor(m1, d, SAGPU_WAVE));
-        m2 = umax(m2, __shfl_xor(m2, d, SAGPU_WAVE));
+        const u64 row = wbase + (u64)r * SAGPU_WAVE;
+        bool act, b1, b2;
+        f.scan_inputs(row + lane, act, b1, b2);   // (nothing from n on)
+        s += (u32)__popcll(__ballot(act));
+        m1 = last_set(__ballot(b1), (u32)row, m1);
+        m2 = last_set(__ballot(b2), (u32)row, m2);
     }
     if (lane == 0) s_w[w] = Agg{s, m1, m2};
     __syncthreads();
@@ -115,11 +109,8 @@ __device__ Agg scan_step(Agg *tagg, u64 tiles, u64 b0, Agg carry, Agg *s_t, Agg 
         c.m1 = umax(c.m1, s_w[q].m1);
         c.m2 = umax(c.m2, s_w[q].m2);
     }
-    const u32 p1 = __shfl_up(i1, 1, SAGPU_WAVE), p2 = __shfl_up(i2, 1, SAGPU_WAVE);
-    if (lane_id() > 0) {
-        c.m1 = umax(c.m1, p1);
-        c.m2 = umax(c.m2, p2);
-    }
+    c.m1 = umax(c.m1, lane_up(0u, i1));
+    c.m2 = umax(c.m2, lane_up(0u, i2));
     c.s += is - t.s;
 #pragma unroll
     for (int q = 0; q < SC_K; q++) {   // exclusive prefixes into the thread's own row
@@ -217,28 +208,24 @@ int ws_scan(WsScratch &ws, u64 tiles, u64 *out_counter, hipStream_t s)
 }
 
 template <class F, int R>
-__global__ __launch_bounds__(WS_THREADS) void k_ws_emit(F f, const Agg *__restrict__ texcl, const u64 *__restrict__ base)
+__global__ __launch_bounds__(WS_THREADS, 6) void k_ws_emit(F f, const Agg *__restrict__ texcl, const u64 *__restrict__ base)
 {
     constexpr int SPAN = R * SAGPU_WAVE;
     __shared__ Agg s_w[WS_WAVES];
     const u32 w = threadIdx.x / SAGPU_WAVE, lane = lane_id();
     const u64 wbase = (u64)blockIdx.x * (WS_WAVES * SPAN) + (u64)w * SPAN;
-    bool act[R];
-    u32 v1[R], v2[R];
+    u32 fl[R];   // 1: stays active, 2 and 4: a first and a second head
     u64 s = 0;
     u32 m1 = 0, m2 = 0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
-        f.scan_inputs(e, act[r], v1[r], v2[r]);
-        s += act[r];
-        m1 = umax(m1, v1[r]);
-        m2 = umax(m2, v2[r]);
-    }
-    for (int d = 32; d >= 1; d >>= 1) {
-        s += __shfl_xor(s, d, SAGPU_WAVE);
-        m1 = umax(m1, __shfl_xor(m1, d, SAGPU_WAVE));
-        m2 = umax(m2, __shfl_xor(m2, d, SAGPU_WAVE));
+        const u64 row = wbase + (u64)r * SAGPU_WAVE;
+        bool act, b1, b2;
+        f.scan_inputs(row + lane, act, b1, b2);
+        s += (u32)__popcll(__ballot(act));
+        m1 = last_set(__ballot(b1), (u32)row, m1);
+        m2 = last_set(__ballot(b2), (u32)row, m2);
+        fl[r] = (act ? 1u : 0u) | (b1 ? 2u : 0u) | (b2 ? 4u : 0u);
     }
     if (lane == 0) s_w[w] = Agg{s, m1, m2};
     __syncthreads();
@@ -251,14 +238,14 @@ __global__ __launch_bounds__(WS_THREADS) void k_ws_emit(F f, const Agg *__restri
     const u64 ob = base ? *base : 0ull;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
-        u32 is = wave_incl_sum((u32)act[r]);
-        u32 i1 = umax(c.m1, wave_incl_max(v1[r]));
-        u32 i2 = umax(c.m2, wave_incl_max(v2[r]));
-        f.emit(e, act[r], ob + c.s + is - (u64)act[r], i1, i2);   // every lane calls; e >= n writes nothing
-        c.s += __shfl(is, SAGPU_WAVE - 1, SAGPU_WAVE);
-        c.m1 = __shfl(i1, SAGPU_WAVE - 1, SAGPU_WAVE);
-        c.m2 = __shfl(i2, SAGPU_WAVE - 1, SAGPU_WAVE);
+        const u64 row = wbase + (u64)r * SAGPU_WAVE;
+        const u64 ab = __ballot(fl[r] & 1u), h1 = __ballot(fl[r] & 2u), h2 = __ballot(fl[r] & 4u);
+        const u64 upto = ~0ull >> (63u - lane);
+        f.emit(row + lane, fl[r] & 1u, ob + c.s + mask_below(ab), last_set(h1 & upto, (u32)row, c.m1),
+               last_set(h2 & upto, (u32)row, c.m2));   // (nothing from n on)
+        c.s += (u32)__popcll(ab);
+        c.m1 = last_set(h1, (u32)row, c.m1);
+        c.m2 = last_set(h2, (u32)row, c.m2);
     }
 }
 
@@ -299,13 +286,12 @@ struct InitF {
     __device__ u32 div_bits(u32 x) const { return (x * bmul) >> 16; }
     __device__ bool sep(u32 k) const { return gsa && (k & sepmask) == 0; }
     // Group flags of element e from its key and its neighbours' keys.
-    __device__ void flags(u64 e, K k, K kp, K kn, bool &act, u32 &v1) const
+    __device__ void flags(u64 e, K k, K kp, K kn, bool &act, bool &head) const
     {
         const bool s = sep((u32)k);
-        const bool head = (e == 0) || s || kp != k;
+        head = e < n && ((e == 0) || s || kp != k);
         const bool tail = (e + 1 >= n) || s || kn != k;
         act = e < n && !(head && tail);
-        v1 = e < n && head ? (u32)e : 0u;
     }
     // Leading symbols two packed keys share, stopped at a separator in GSA mode.
     __device__ u32 key_lcp(u32 k, u32 kp) const
@@ -383,18 +369,17 @@ struct SpanKeys {
     // unrolled callers).
     __device__ void neighbours(int r, K &kp, K &kn) const
     {
-        const u32 lane = lane_id();
-        const K up = __shfl_up(k[r], 1, SAGPU_WAVE);
-        const K last = r > 0 ? __shfl(k[r - 1], SAGPU_WAVE - 1, SAGPU_WAVE) : before;
-        kp = lane ? up : last;
-        const K down = __shfl_down(k[r], 1, SAGPU_WAVE);
-        const K first = r + 1 < R ? __shfl(k[r + 1 < R ? r + 1 : r], 0, SAGPU_WAVE) : after;
-        kn = lane + 1 < SAGPU_WAVE ? down : first;
+        kp = lane_up(r > 0 ? lane_value(k[r > 0 ? r - 1 : 0], SAGPU_WAVE - 1) : before, k[r]);
+        kn = lane_down(r + 1 < R ? lane_value(k[r + 1 < R ? r + 1 : r], 0) : after, k[r]);
     }
 };
 
 // Initial grouping, pass 1: per tile (4 spans of R rows), the number of grouped
-// elements and the position of the last group start.
+// elements, the position of the last group start, and the elements of each ISA bucket.
+// Bound by the 8 B read per element: neighbours come by DPP, counts and positions from
+// ballots.  With shuffles, and an LDS atomic per element on the bucket counters (all on
+// one counter where a tile's elements share their bucket, as in a string set): 547 us for
+// 2^28 DNA suffixes, 2386 us for 2^29 of a string set; now 420 and 777 us.
 template <typename K, int R>
 __global__ __launch_bounds__(WS_THREADS) void k_init_reduce(InitF<K> f, Agg *__restrict__ tagg)
 {
@@ -420,17 +405,33 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_reduce(InitF<K> f, Agg *__r
         const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
         K kp, kn;
         sk.neighbours(r, kp, kn);
-        bool act;
-        u32 v1;
-        f.flags(e, sk.k[r], kp, kn, act, v1);
-        s += act;
-        m1 = umax(m1, v1);
-        // u64 shifts: wlog may be 32 (one bucket)
-        if (e < f.n) atomicAdd(&s_cnt[(u32)((u64)(vv[r] >> f.cb) >> f.wlog)], 1u);
+        bool act, head;
+        f.flags(e, sk.k[r], kp, kn, act, head);
+        s += (u32)__popcll(__ballot(act));
+        const u64 hb = __ballot(head);
+        m1 = last_set(hb, (u32)(wbase + (u64)r * SAGPU_WAVE), m1);
     }
-    for (int d = 32; d >= 1; d >>= 1) {
-        s += __shfl_xor(s, d, SAGPU_WAVE);
-        m1 = umax(m1, __shfl_xor(m1, d, SAGPU_WAVE));
+    // the wave's elements of each ISA bucket (u64 shifts: wlog may be 32, one bucket)
+    const u32 nb = (u32)(((f.n - 1) >> f.wlog) + 1);
+    if (nb <= 8) {
+        // eight counts of a lane in one word, added up over the lanes as 16-bit fields
+        static_assert(R < 256, "8 bits a count");
+        u64 c = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
+            if (e < f.n) c += 1ull << (8u * (u32)((u64)(vv[r] >> f.cb) >> f.wlog));
+        }
+        constexpr u64 EVEN = 0x00FF00FF00FF00FFull;
+        const u64 even = lane_value(wave_incl_sum64(c & EVEN), SAGPU_WAVE - 1);
+        const u64 odd = lane_value(wave_incl_sum64((c >> 8) & EVEN), SAGPU_WAVE - 1);
+        if (lane < 8) atomicAdd(&s_cnt[lane], (u32)((lane & 1 ? odd : even) >> (16 * (lane >> 1))) & 0xFFFFu);
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
+            if (e < f.n) atomicAdd(&s_cnt[(u32)((u64)(vv[r] >> f.cb) >> f.wlog)], 1u);
+        }
     }
     if (lane == 0) s_w[w] = Agg{s, m1, 0};
     __syncthreads();
@@ -442,25 +443,28 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_reduce(InitF<K> f, Agg *__r
         }
         tagg[blockIdx.x] = t;
     }
-    const u32 nb = (u32)(((f.n - 1) >> f.wlog) + 1);
     if (threadIdx.x < nb) f.bcnt[(u64)threadIdx.x * gridDim.x + blockIdx.x] = s_cnt[threadIdx.x];
 }
 
 // Initial grouping, pass 2 (after k_ws_scan_tiles): singletons into SA, grouped
 // elements into the active list, LCP marks, BWT seeds, and the (suffix, group head)
-// pairs into their ISA buckets.
+// pairs into their ISA buckets.  Bound by memory, 26 B per element and the lists; the
+// ranks inside the buckets came from returning LDS atomics: 4.1 ms for a string set of
+// 2^29 suffixes whose tiles have one bucket each, now 2.5 ms (2^28 DNA suffixes over 8
+// buckets: 2.05 ms both ways).
 template <typename K, int R>
 __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg *__restrict__ texcl)
 {
     constexpr int SPAN = R * SAGPU_WAVE;
     __shared__ Agg s_w[WS_WAVES];
-    __shared__ u32 s_cnt[IB_MAX];
+    __shared__ u32 s_cnt[WS_WAVES][IB_MAX];   // elements per wave and bucket, then the waves' offsets
     __shared__ u64 s_base[IB_MAX];
     const u32 w = threadIdx.x / SAGPU_WAVE, lane = lane_id();
     const u64 wbase = (u64)blockIdx.x * (WS_WAVES * SPAN) + (u64)w * SPAN;
     const u64 n = f.n;
     const u32 nb = (u32)(((n - 1) >> f.wlog) + 1);
-    if (threadIdx.x < IB_MAX) s_cnt[threadIdx.x] = 0;
+    s_cnt[w][lane] = 0;
+    static_assert(IB_MAX == SAGPU_WAVE, "a lane per bucket");
     SpanKeys<K, R> sk;
     sk.load(f.keys, n, wbase);
     u32 vv[R];
@@ -470,8 +474,9 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
         vv[r] = e < n ? f.vals[e] : 0u;
     }
     __syncthreads();
-    // st[r]: bit 31 grouped, bit 30 group start, low bits the rank inside the
-    // workgroup's share of the element's ISA bucket
+    // st[r]: bit 31 grouped, bit 30 group start, low bits the rank inside the wave's
+    // share of the element's ISA bucket: the lanes of one bucket find each other by
+    // ballots (3 bits for up to 8 buckets), so no two write one counter
     u32 st[R];
     u64 s = 0;
     u32 m1 = 0;
@@ -480,23 +485,34 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
         const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
         K kp, kn;
         sk.neighbours(r, kp, kn);
-        bool act;
-        u32 v1;
-        f.flags(e, sk.k[r], kp, kn, act, v1);
-        s += act;
-        m1 = umax(m1, v1);
-        u32 rank = 0;
+        bool act, head;
+        f.flags(e, sk.k[r], kp, kn, act, head);
+        s += (u32)__popcll(__ballot(act));
+        const u64 hb = __ballot(head);
+        m1 = last_set(hb, (u32)(wbase + (u64)r * SAGPU_WAVE), m1);
         // u64 shifts: wlog may be 32 (one bucket), which a 32-bit shift cannot express
-        if (e < n) rank = atomicAdd(&s_cnt[(u32)((u64)(vv[r] >> f.cb) >> f.wlog)], 1u);
-        st[r] = rank | (act ? 1u << 31 : 0u) | (e < n && v1 == (u32)e && (e == 0 || v1 != 0) ? 1u << 30 : 0u);
-    }
-    for (int d = 32; d >= 1; d >>= 1) {
-        s += __shfl_xor(s, d, SAGPU_WAVE);
-        m1 = umax(m1, __shfl_xor(m1, d, SAGPU_WAVE));
+        const u32 b = (u32)((u64)(vv[r] >> f.cb) >> f.wlog);
+        const u64 in = __ballot(e < n);
+        const u64 m = nb <= 8 ? wave_peers<3>(b, in) : wave_peers<6>(b, in);
+        u32 rank = 0;
+        if (e < n) {
+            const u32 old = s_cnt[w][b];
+            s_cnt[w][b] = old + (u32)__popcll(m);   // the same value from every peer
+            rank = old + mask_below(m);
+        }
+        st[r] = rank | (act ? 1u << 31 : 0u) | (head ? 1u << 30 : 0u);
     }
     if (lane == 0) s_w[w] = Agg{s, m1, 0};
     __syncthreads();
-    if (threadIdx.x < nb && s_cnt[threadIdx.x]) s_base[threadIdx.x] = f.bcnt[(u64)threadIdx.x * gridDim.x + blockIdx.x];
+    if (threadIdx.x < nb) {
+        u32 o = 0;
+        for (int q = 0; q < WS_WAVES; q++) {
+            const u32 c = s_cnt[q][threadIdx.x];
+            s_cnt[q][threadIdx.x] = o;
+            o += c;
+        }
+        if (o) s_base[threadIdx.x] = f.bcnt[(u64)threadIdx.x * gridDim.x + blockIdx.x];
+    }
     Agg c = texcl[blockIdx.x];
     for (u32 q = 0; q < w; q++) {
         c.s += s_w[q].s;
@@ -508,19 +524,18 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
     for (int r = 0; r < R; r++) {
         const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
         const bool act = st[r] >> 31;
-        const u32 is = wave_incl_sum((u32)act);
-        const u32 g = umax(c.m1, wave_incl_max((st[r] >> 30) & 1u ? (u32)e : 0u));
-        const u64 o = c.s + is - (u64)act;
+        const u64 ab = __ballot(act), hb = __ballot((st[r] >> 30) & 1u);
+        const u64 o = c.s + mask_below(ab);
+        // the group's first slot: the nearest head at or below this lane, else the last
+        // one before the row
+        const u32 row = (u32)(wbase + (u64)r * SAGPU_WAVE);
+        const u32 g = last_set(hb & (~0ull >> (63u - lane)), row, c.m1);
         K kp = 0, kn;
         if (f.LCP) sk.neighbours(r, kp, kn);
         // the slot before: its value (suffix) and whether it is alone in its group
         // (unknown for the first slot of the span: taken as grouped)
-        const u32 vup = __shfl_up(vv[r], 1, SAGPU_WAVE);
-        const u32 vlast = r > 0 ? __shfl(vv[r > 0 ? r - 1 : 0], SAGPU_WAVE - 1, SAGPU_WAVE) : 0u;
-        const u32 vp = lane ? vup : vlast;
-        const u32 gup = __shfl_up(st[r] >> 31, 1, SAGPU_WAVE);
-        const u32 glast = r > 0 ? __shfl(st[r > 0 ? r - 1 : 0] >> 31, SAGPU_WAVE - 1, SAGPU_WAVE) : 1u;
-        const bool onep = !(lane ? gup : glast);
+        const u32 vp = lane_up(r > 0 ? lane_value(vv[r > 0 ? r - 1 : 0], SAGPU_WAVE - 1) : 0u, vv[r]);
+        const bool onep = !(lane_up(r > 0 ? lane_value(st[r > 0 ? r - 1 : 0], SAGPU_WAVE - 1) : ~0u, st[r]) >> 31);
         if (e < n) {
             const u32 v = vv[r] >> f.cb;
             if (f.codes) f.codes[e] = (uint8_t)(vv[r] & cmask);
@@ -531,7 +546,8 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
             const u32 hint = (f.hint && f.LCP && !act && mark >= (u32)f.hint_off && mark - (u32)f.hint_off < 15u)
                                  ? (mark - (u32)f.hint_off + 1u) << 28
                                  : 0u;
-            const u64 slot = s_base[(u32)((u64)v >> f.wlog)] + (st[r] & 0x3fffffffu);
+            const u32 b = (u32)((u64)v >> f.wlog);
+            const u64 slot = s_base[b] + s_cnt[w][b] + (st[r] & 0x3fffffffu);
             f.PV[slot] = v;
             f.PG[slot] = g | hint;
             // every slot is written (full lines); slots of grouped elements are
@@ -543,8 +559,8 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
             }
             if (f.LCP) f.LCP[e] = mark;
         }
-        c.s += __shfl(is, SAGPU_WAVE - 1, SAGPU_WAVE);
-        c.m1 = __shfl(g, SAGPU_WAVE - 1, SAGPU_WAVE);
+        c.s += (u32)__popcll(ab);
+        c.m1 = last_set(hb, row, c.m1);
     }
 }
 
@@ -592,22 +608,21 @@ struct BigF {
     const u32 *grank;
     const u64 *keepkey;
 
-    __device__ void scan_inputs(u64 e, bool &act, u32 &v1, u32 &v2) const
+    // act: more than one member in its subgroup; first: a group's first element; head: a
+    // subgroup's
+    __device__ void scan_inputs(u64 e, bool &act, bool &first, bool &head) const
     {
         if (e >= n) {
-            act = false;
-            v1 = v2 = 0;
+            act = first = head = false;
             return;
         }
         const u64 c = comp[e];
         const u64 cp = e > 0 ? (u64)comp[e - 1] : ~0ull;
         const u64 cn = e + 1 < n ? (u64)comp[e + 1] : ~0ull;
-        bool head = (e == 0) || c != cp;
-        bool tail = (e + 1 == n) || c != cn;
-        bool gch = (e == 0) || (c >> kb) != (cp >> kb);
+        head = (e == 0) || c != cp;
+        const bool tail = (e + 1 == n) || c != cn;
+        first = (e == 0) || (c >> kb) != (cp >> kb);
         act = !(head && tail);
-        v1 = gch ? (u32)e : 0u;
-        v2 = head ? (u32)e : 0u;
     }
     __device__ void emit(u64 e, bool act, u64 o, u32 gstart, u32 hstart) const
     {
@@ -1015,8 +1030,7 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
         __syncthreads();
         u32 c = 0;
         for (u32 q = 0; q < tid / SAGPU_WAVE; q++) c = umax(c, s_wsum[q]);
-        const u32 prev = __shfl_up(inc, 1, SAGPU_WAVE);
-        if (lane_id() > 0) c = umax(c, prev);
+        c = umax(c, lane_up(0u, inc));
 #pragma unroll
         for (int j = 0; j < W_PER; j++) {
             const u32 x = tid * W_PER + j;
@@ -1059,14 +1073,10 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
                 rt_big_head<RANGE>(lo + x, s_w[x], seg_ctr, bseg_h, bseg_g, bseg_cap, err);
             }
         }
-        for (int d = 32; d >= 1; d >>= 1) {
-            const u32 of = __shfl_xor(f, d, SAGPU_WAVE), oe = __shfl_xor(e, d, SAGPU_WAVE);
-            const u32 om = __shfl_xor(gm, d, SAGPU_WAVE);
-            f = of < f ? of : f;
-            e = oe > e ? oe : e;
-            gm = om > gm ? om : gm;
-        }
-        if (lane_id() == 0 && f != NONE) {
+        f = ~wave_incl_max(~f);   // (in the last lane: of the whole wave)
+        e = wave_incl_max(e);
+        gm = wave_incl_max(gm);
+        if (lane_id() == SAGPU_WAVE - 1 && f != NONE) {
             atomicMin(&s_first, f);
             atomicMax(&s_end, e);
             atomicMax(&s_gmax, gm);
