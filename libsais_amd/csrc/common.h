@@ -112,6 +112,29 @@ __device__ __forceinline__ u64 wave_incl_max64(u64 v)
     return wave_scan(v, [](u64 a, u64 b) { return a > b ? a : b; });
 }
 
+// An order of `count` work items that gives each XCD (workgroups go to the XCDs
+// round-robin) runs of neighbouring items, which share its L2: up to 256 items (what an XCD
+// has in flight), at least 8 runs an XCD, so that uneven work evens out.  b < xcd_runs(count);
+// an item of count or more is none.
+__host__ __device__ __forceinline__ int xcd_run_log2(u64 count)
+{
+    const int l = count ? 63 - __builtin_clzll(count) : 0;
+    return l < 6 ? 0 : l > 14 ? 8 : l - 6;
+}
+__host__ __device__ __forceinline__ u64 xcd_runs(u64 count)
+{
+    const int s = xcd_run_log2(count) + 3;
+    return (count + (1ull << s) - 1) >> s << s;
+}
+__device__ __forceinline__ u64 xcd_run(u64 b, u64 count)
+{
+    const int s = xcd_run_log2(count);
+    const u64 j = b >> 3;   // the XCD's j-th
+    return (((j >> s) << 3 | (b & 7)) << s) | (j & ((1ull << s) - 1));
+}
+// Workgroups for b of them: whole rounds of the XCDs.
+inline unsigned xcd_grid(u64 b) { return (unsigned)(b < 8 ? 8 : b < 65528 ? b : 65528); }
+
 // row + the highest set bit of m, or `none`.
 __device__ __forceinline__ u32 last_set(u64 m, u32 row, u32 none)
 {

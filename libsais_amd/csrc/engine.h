@@ -262,18 +262,19 @@ extern int g_init_rows;   // list entries per workgroup of the tile kernel (the 
 // Groups of the last cnt suffixes (their ISA words' ranks), for RawKey1 and ExactLcp.
 int launch_tail_groups(const u32 *ISA, u64 n, u32 cnt, u32 *out, hipStream_t s);
 // cnt: 8 u64 (0 list length out, 4 big groups | err << 32, 5 big-group members); the
-// gather clears them and seg_ctr (128 u64).
+// gather clears them and seg_ctr (SEG_CTR_WORDS u64).
 int round_gather(const u32 *act_i, const u32 *act_g, u64 a_grid, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
                  const u32 *ISA, u64 n, void *key2, int wide, hipStream_t s, const RawKey1 *rk = nullptr, int cb = 0,
                  const Chains *ch = nullptr);
-// The tile kernel's survivors go to 8 per-XCD segments of seg_i / seg_g (capacity
-// 8 * round_seg_cap(a_grid) each) and are concatenated into out_i / out_g, whose
+// The list's tiles make ROUND_RUNS runs.  The tile kernel's survivors go to a segment of
+// seg_i / seg_g per run (ROUND_RUNS * round_seg_cap(a_grid) entries) and are concatenated into out_i / out_g, whose
 // length goes to cnt[0].  Big-group heads go the same way to 8 segments of bseg_h /
 // bseg_g (round_bigseg_cap(n) entries each, n >= every list length) and are
 // concatenated into big_head / big_g / big_size; boff (big_cap + 1 entries) gets their
 // offsets in the concatenation of their members.  rec (pinned, 7 u64) receives cnt's
 // words at their indexes and in rec[6], last, the length the round started with;
 // rp_next the next round's length (0 when there are big groups) and offset.
+constexpr int ROUND_RUNS = 64, SEG_CTR_WORDS = ROUND_RUNS * 16;
 u64 round_seg_cap(u64 a);
 u64 round_bigseg_cap(u64 n);
 int round_tile(const u32 *act_i, const u32 *act_g, const void *key2, int wide, u64 a_grid, const u64 *rp, u64 *rp_next,

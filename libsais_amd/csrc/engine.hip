@@ -1271,11 +1271,11 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     // whose launch geometry is sized for a list at least as long as the round's.
     GET(d_rp, u64, 4);   // by parity
     u64 *const rec[2] = {c.pinned, c.pinned + 32};   // a round's report, by parity
-    // per-XCD survivor segments of the tile kernel, sized for the first (longest) list
-    const u64 a_first = a, seg_words = 8 * round_seg_cap(a_first);
+    // survivor segments of the tile kernel, sized for the first (longest) list
+    const u64 a_first = a, seg_words = ROUND_RUNS * round_seg_cap(a_first);
     GET(seg_i, u32, seg_words);
     GET(seg_g, u32, seg_words);
-    GET(seg_ctr, u64, 128);
+    GET(seg_ctr, u64, SEG_CTR_WORDS);
     // (not in the allocation-free build: instantiating a graph allocates)
     const bool graphs = g_round_graphs && !c.timer.on && !c.pool.arena;
     bool captured[2] = {false, false};

@@ -179,13 +179,9 @@ __global__ __launch_bounds__(256) void k_phi_scatter(const u32 *__restrict__ PV,
 // zero padding so both aligned words are in bounds.
 __device__ __forceinline__ u64 load8u(const uint8_t *p)
 {
-    uintptr_t a = (uintptr_t)p;
-    const u64 *q = reinterpret_cast<const u64 *>(a & ~(uintptr_t)7);
-    u32 sh = (u32)(a & 7) * 8;
-    u64 lo = q[0];
-    if (sh == 0) return lo;
-    u64 hi = q[1];
-    return (lo >> sh) | (hi << (64 - sh));
+    u64 x;
+    __builtin_memcpy(&x, p, 8);   // (one load: the target takes any alignment)
+    return x;
 }
 
 // Lanes of x that hold a zero symbol (W-byte symbols, W = 1 or 2; for W = 4 GSA is not
@@ -309,7 +305,7 @@ __device__ __forceinline__ u64 stream_window(const u32 *__restrict__ pw, u64 bit
     const u64 w = bitpos >> 5;
     const u32 off = (u32)(bitpos & 31);
     const u64 hi = ((u64)pw[w] << 32) | (u64)pw[w + 1];
-    return off ? (hi << off) | ((u64)pw[w + 2] >> (32 - off)) : hi;
+    return (hi << off) | ((u64)pw[w + 2] << off >> 32);
 }
 
 // lcp of suffixes i and k on the packed code stream, from l (a known lower bound)
@@ -337,7 +333,10 @@ __device__ __forceinline__ u64 match_stream(const u32 *__restrict__ pw, int bits
 // Byte texts, pair-word form (k_plcp_pairs): per position one ISA read, one 8-byte
 // pair read and the symbol before it; known lcps and reducible positions finish
 // there, irreducible ones compare as k_plcp_irr.  PI positions per thread and step
-// with their loads issued together.
+// with their loads issued together, those of the comparisons' first steps too (2^28 DNA
+// suffixes: 1.75 ms with a comparison at a time, 1.55 ms now).  Bound by the random pair
+// reads; the XCDs take runs of the text, so the pairs of a string set's strings are read
+// from one L2 (2^29 suffixes of 20000 strings: 9.4 ms round-robin, 6.4 ms by runs).
 constexpr int PI = 4;
 // Each workgroup takes whole MS_TILE tiles (PI rows of 256 per step) and writes the
 // tile's max of v to tmax, so the prefix max needs no separate reduce pass
@@ -357,7 +356,12 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
     __shared__ VT s_m[4];
     const u64 tiles = (n + MS_TILE - 1) / MS_TILE;
     const u64 part_len = MS_TILE / (u64)split;
-    for (u64 wi = blockIdx.x; wi < tiles * (u64)split; wi += gridDim.x) {
+    const u32 per = pw ? 64u / (u32)bits : 8u;   // symbols a step compares
+    const u64 keep = pw ? ~0ull << (64 - per * (u32)bits) : 0ull;
+    const u64 items = tiles * (u64)split;
+    for (u64 b = blockIdx.x; b < xcd_runs(items); b += gridDim.x) {
+        const u64 wi = xcd_run(b, items);
+        if (wi >= items) continue;
         const u64 tile = wi / (u64)split, p0 = tile * MS_TILE + (wi % (u64)split) * part_len;
         VT mx = 0;
         for (u64 base = p0; base < p0 + part_len && base < n; base += STEP) {
@@ -374,6 +378,37 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
             }
 #pragma unroll
             for (int q = 0; q < PI; q++) w[q] = (r[q] && !hint[q]) ? pairs[r[q]] : 0ull;
+            // the first step of every comparison: all loads in flight together (lanes
+            // without one read the text's first symbols)
+            u64 d[PI];
+            u32 l0[PI];
+            bool cmp[PI], any = false;
+#pragma unroll
+            for (int q = 0; q < PI; q++) {
+                const u64 i = base + (u64)q * 256 + threadIdx.x;
+                const u32 k = (u32)w[q];
+                // unknown and not reducible (PLCP[i] = PLCP[i-1] - 1)
+                cmp[q] = (w[q] >> 63) && !(i > 0 && k > 0 && a[q] == (uint8_t)(w[q] >> 32) && !(gsa && a[q] == 0));
+                const u32 lg = (u32)(w[q] >> 58) & 31u;
+                l0[q] = lg ? 1u << (lg - 1) : 0u;
+                const u64 m = n - (i > k ? i : k);
+                if ((u64)l0[q] > m) l0[q] = (u32)m;
+                any |= cmp[q];
+                d[q] = 0;
+            }
+#pragma unroll
+            for (int q = 0; q < PI; q++) {
+                if (!__ballot(any)) break;
+                const u64 i = base + (u64)q * 256 + threadIdx.x;
+                const u32 k = (u32)w[q];
+                const u64 pi = cmp[q] ? i + l0[q] : 0, pk = cmp[q] ? (u64)k + l0[q] : 0;
+                if (pw) {
+                    d[q] = (stream_window(pw, pi * (u64)bits) ^ stream_window(pw, pk * (u64)bits)) & keep;
+                } else {
+                    const u64 x = load8u(T + pi);
+                    d[q] = (x ^ load8u(T + pk)) | (gsa ? zero_lanes<1>(x) : 0ull);
+                }
+            }
 #pragma unroll
             for (int q = 0; q < PI; q++) {
                 const u64 i = base + (u64)q * 256 + threadIdx.x;
@@ -385,29 +420,34 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
                     v = (VT)i;
                 } else if (!(w[q] >> 63)) {
                     v = (VT)((u64)(u32)w[q] + i);
+                } else if (!cmp[q]) {
+                    v = 0;   // reducible: PLCP[i] = PLCP[i-1] - 1
                 } else {
                     const u64 k = (u32)w[q];
-                    const u32 lg = (u32)(w[q] >> 58) & 31u;
-                    const u64 lb = lg ? (1ull << (lg - 1)) : 0;
-                    if (i > 0 && k > 0 && a[q] == (uint8_t)(w[q] >> 32) && !(gsa && a[q] == 0)) {
-                        v = 0;   // reducible: PLCP[i] = PLCP[i-1] - 1
-                    } else {
-                        const u64 m = n - (i > k ? i : k);
-                        bool done = false;
+                    const u64 m = n - (i > k ? i : k);
+                    u64 l = l0[q];
+                    bool done = true;
+                    if (l >= m) {
+                        l = m;
+                    } else if (d[q]) {
+                        l += pw ? (u64)((u32)__clzll((long long)d[q]) / (u32)bits) : (u64)(__builtin_ctzll(d[q]) >> 3);
+                        l = l < m ? l : m;
+                    } else {   // longer than the first step
+                        l += per;
                         // with the code stream (no GSA), 64 / bits symbols per step
-                        u64 l = pw ? match_stream(pw, bits, i, k, lb < m ? lb : m, m, PL_THREAD_LIMIT, &done)
-                                   : match_bytes<1>(T, i, k, lb < m ? lb : m, m, gsa, PL_THREAD_LIMIT, &done);
-                        if (!done) {
-                            u32 slot = atomicAdd(queue_n, 1u);
-                            if (slot < queue_cap) {
-                                queue[slot] = (u32)i;   // provisional value; k_plcp_long finishes it
-                                queue_l[slot] = (u32)l;
-                            } else {
-                                l = match_bytes<1>(T, i, k, l, m, gsa, ~0ull >> 1, &done);
-                            }
-                        }
-                        v = (VT)(l + i);
+                        l = pw ? match_stream(pw, bits, i, k, l < m ? l : m, m, PL_THREAD_LIMIT, &done)
+                               : match_bytes<1>(T, i, k, l < m ? l : m, m, gsa, PL_THREAD_LIMIT, &done);
                     }
+                    if (!done) {
+                        u32 slot = atomicAdd(queue_n, 1u);
+                        if (slot < queue_cap) {
+                            queue[slot] = (u32)i;   // provisional value; k_plcp_long finishes it
+                            queue_l[slot] = (u32)l;
+                        } else {
+                            l = match_bytes<1>(T, i, k, l, m, gsa, ~0ull >> 1, &done);
+                        }
+                    }
+                    v = (VT)(l + i);
                 }
                 V[i] = v;
                 mx = vmax(mx, v);
@@ -925,8 +965,7 @@ int launch_plcp_t(LcpScratch &ls, const uint8_t *T, u64 n, int gsa, const u32 *P
             const int split = n < (1ull << 20) ? (int)(MS_TILE / (256 * PI)) : 1;
             if (split > 1) SAGPU_TRY(launch_fill_u32((u32 *)tmax, tiles * sizeof(VT) / 4, 0, s));
             if (ls.hook) ls.hook(ls.hook_user, 0);
-            const u64 wg = tiles * (u64)split;
-            hipLaunchKernelGGL((k_plcp_irr_pairs<VT>), dim3((unsigned)(wg < 65535 ? wg : 65535)), dim3(256), 0, s, T, n,
+            hipLaunchKernelGGL((k_plcp_irr_pairs<VT>), dim3(xcd_grid(xcd_runs(tiles * (u64)split))), dim3(256), 0, s, T, n,
                                gsa, ISA, pairs, V, ls.queue, ls.queue_l, ls.queue_n, ls.queue_cap,
                                gsa ? nullptr : pw, bits, tmax, hint_off, split);
             if (ls.hook) ls.hook(ls.hook_user, 1);

@@ -693,7 +693,9 @@ int ws_run(WsScratch &ws, const F &f, u64 n, u64 *out_counter, hipStream_t s)
 
 // ------------------------------------------------------------- round kernels
 // IG list entries per thread and step, all loads (the random ISA reads included)
-// in flight before the stores.
+// in flight before the stores.  Bound by those reads (53 G/s over a large ISA); the XCDs
+// take runs of the list, whose entries read near each other where the list keeps to its
+// strings (512 MiB of ACGT strings: 2.09 ms round-robin, 1.63 ms by runs).
 constexpr int IG = 4;
 template <typename KT, bool CHAIN>
 __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g,
@@ -708,15 +710,17 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
     const u64 a = st.h ? (st.a_src ? *st.a_src : st.a) : rp[0], h = st.h ? st.h : rp[1];
     if (!st.h && a == 0) return;
     if (blockIdx.x == 0) {
-        if (threadIdx.x < 128) seg_ctr[threadIdx.x] = 0;
+        for (u32 x = threadIdx.x; x < SEG_CTR_WORDS; x += 256) seg_ctr[x] = 0;
         if (threadIdx.x == 128) cnt[0] = cnt[4] = cnt[5] = 0;
         if (threadIdx.x == 129 && st.h) {
             rp[0] = a;
             rp[1] = h;
         }
     }
-    const u64 chunk = 256ull * IG;
-    for (u64 base = (u64)blockIdx.x * chunk; base < a; base += (u64)gridDim.x * chunk) {
+    const u64 chunk = 256ull * IG, items = (a + chunk - 1) / chunk;
+    for (u64 b = blockIdx.x; b < xcd_runs(items); b += gridDim.x) {
+        const u64 base = xcd_run(b, items) * chunk;
+        if (base >= a) continue;
         u32 i[IG], r[IG];
         bool raw[IG];
 #pragma unroll
@@ -987,8 +991,19 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
     const u64 a = rp[0];
     const u32 h = rp[1] < LCP_BOUND_CAP ? (u32)rp[1] : LCP_BOUND_CAP;   // marks carry h capped
     const u32 tid = threadIdx.x;
-    const u64 lo = (u64)blockIdx.x * RANGE;
-    if (lo >= a) return;
+    if (a == 0) return;
+    // The tile: the list's tiles make ROUND_RUNS runs, and each XCD takes every eighth run.
+    // The next list is the runs' survivors in run order, so it stays sorted as the groups
+    // and, in groups that run over the whole text, as their suffixes are: later rounds'
+    // random reads and writes stay close together.  Gathers and tiles of a 64 MiB
+    // Fibonacci string's 21 rounds, us, with tiles round-robin over the XCDs and one
+    // segment each: 23370 and 14740; 256 runs 21020 and 15040; 64 runs 15670 and 14310; 8
+    // runs 13830 and 14000, but those leave the XCDs uneven loads (48 MiB of words, tiles:
+    // 2030, 2080, 2090 and 2260).
+    const u32 per_run = (u32)((a + (u64)RANGE * ROUND_RUNS - 1) / ((u64)RANGE * ROUND_RUNS));
+    const u32 nth = blockIdx.x >> 3, run = nth / per_run * 8 + (blockIdx.x & 7u);
+    const u64 lo = ((u64)run * per_run + nth % per_run) * RANGE;
+    if (lo >= a || run >= (u32)ROUND_RUNS) return;
     const u64 hi = lo + RANGE < a ? lo + RANGE : a;
     const u32 wlen = (u32)((a - lo) < (u64)WIN ? (a - lo) : (u64)WIN);
     const u32 rlen = (u32)(hi - lo);
@@ -1288,11 +1303,10 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
     }
     __syncthreads();
 
-    // 6. survivors: output ranks by position, their range reserved in this XCD's
-    //    segment (one atomic on the XCD's counter).  A counter shared by all
+    // 6. survivors: output ranks by position, their range reserved in this run's
+    //    segment (one atomic on the run's counter).  A counter shared by all
     //    workgroups serialises them: 300 K returning atomics on one address take
-    //    3.6 ms, on 8 addresses 0.57 ms; workgroups go to the XCDs round-robin
-    //    (blockIdx % 8).
+    //    3.6 ms, on 8 addresses 0.57 ms; the XCDs work on a run each.
     u32 cnt_s[RT_PER];
     u32 tot = 0;
 #pragma unroll
@@ -1306,8 +1320,7 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
     __syncthreads();
     if (tid == 0) {
         const u32 all = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
-        const u32 xcd = blockIdx.x & 7u;
-        s_base = (u64)xcd * seg_cap + (all ? atomicAdd(&seg_ctr[xcd * 16], (u64)all) : 0ull);
+        s_base = (u64)run * seg_cap + (all ? atomicAdd(&seg_ctr[run * 16], (u64)all) : 0ull);
     }
     {
         u32 o = inc - tot;
@@ -1420,9 +1433,9 @@ __global__ __launch_bounds__(1024) void k_big_offsets(const u32 *__restrict__ bi
     if (bad) atomicOr(err, 2u);
 }
 
-// Ends a round: the next active list from the 8 XCD segments of the tile kernel's output
-// (segment x: [x * seg_cap, x * seg_cap + seg_ctr[16 x])), concatenated in segment
-// order; *out_counter = its length (the big-group emission appends behind it).  Block 0
+// Ends a round: the next active list from the runs' segments of the tile kernel's output
+// (segment x: [x * seg_cap, x * seg_cap + seg_ctr[16 x])), concatenated in run order, so
+// that the list keeps its order but for tiles in flight together; *out_counter = its length (the big-group emission appends behind it).  Block 0
 // then reports to the host (rec, pinned: list length, big groups | err << 32, their
 // members, the length the round started with) and leaves the next round's length and
 // offset in rp_next; with big groups, whose members the host adds first, a length of
@@ -1445,17 +1458,21 @@ __global__ __launch_bounds__(256) void k_round_end(const u32 *__restrict__ seg_i
         if (blockIdx.x == 0 && threadIdx.x == 0) rp_next[0] = 0;
         return;
     }
-    u64 pre[9];
-    pre[0] = 0;
-#pragma unroll
-    for (int x = 0; x < 8; x++) pre[x + 1] = pre[x] + seg_ctr[x * 16];
-    const u64 total = pre[8];
+    static_assert(ROUND_RUNS == SAGPU_WAVE, "a lane per run");
+    __shared__ u64 s_pre[ROUND_RUNS + 1];   // the runs' first entries of the next list
+    if (threadIdx.x < (u32)ROUND_RUNS) {
+        const u64 c = seg_ctr[threadIdx.x * 16], inc = wave_incl_sum64(c);
+        s_pre[threadIdx.x] = inc - c;
+        if (threadIdx.x == ROUND_RUNS - 1) s_pre[ROUND_RUNS] = inc;
+    }
+    __syncthreads();
+    const u64 total = s_pre[ROUND_RUNS];
     const u64 stride = (u64)gridDim.x * blockDim.x;
     for (u64 k = (u64)blockIdx.x * blockDim.x + threadIdx.x; k < total; k += stride) {
-        int x = 0;
+        u32 x = 0;   // the last run that starts at or before k
 #pragma unroll
-        for (int q = 1; q < 8; q++) x += k >= pre[q];
-        const u64 src = (u64)x * seg_cap + (k - pre[x]);
+        for (u32 q = ROUND_RUNS / 2; q > 0; q >>= 1) x += k >= s_pre[x + q] ? q : 0u;
+        const u64 src = (u64)x * seg_cap + (k - s_pre[x]);
         out_i[k] = seg_i[src];
         out_g[k] = seg_g[src];
     }
@@ -1678,7 +1695,7 @@ template <typename KT>
 int round_gather_t(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const RoundStart &st, u64 *cnt, u64 *seg_ctr,
                    const u32 *ISA, u64 n, KT *key2, hipStream_t s, const RawKey1 &rk, int cb, const Chains *ch)
 {
-    const dim3 grid(grid_for(a, 256 * IG, 65535));
+    const dim3 grid(xcd_grid(xcd_runs((a + 256 * IG - 1) / (256 * IG))));
     if (ch)
         hipLaunchKernelGGL((k_round_gather<KT, true>), grid, dim3(256), 0, s, act_i, act_g, rp, st, cnt, seg_ctr, ISA,
                            n, key2, rk, cb, *ch);
@@ -1689,15 +1706,21 @@ int round_gather_t(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const Rou
     return SAGPU_OK;
 }
 
-// Segment capacity of each XCD for a list of a entries: the workgroups of XCD x are
-// the tiles x, x + 8, ..., each emitting at most RANGE + RT_SMALL survivors.
-u64 round_seg_cap(u64 a) { return (ceil_div_u(a, (u64)g_tile_range) / 8 + 1) * (u64)(g_tile_range + RT_SMALL); }
+// Segment capacity of each run for a list of a entries: its workgroups emit at most
+// RANGE + RT_SMALL survivors each.
+u64 round_seg_cap(u64 a)
+{
+    return (u64)ceil_div_u(a, (u64)g_tile_range * ROUND_RUNS) * (u64)(g_tile_range + RT_SMALL);
+}
 
 // Big-head segment capacity of each XCD for lists of at most n entries: heads of
 // groups of more than RT_SMALL = 256 members lie at least 257 entries apart, so a
-// workgroup of RANGE entries holds at most RANGE / 256 of them, and an XCD's
-// ceil(ceil(n / RANGE) / 8) workgroups at most n / 2048 + RANGE / 128.
-u64 round_bigseg_cap(u64 n) { return n / 2048 + 16; }
+// workgroup of RANGE entries holds at most RANGE / 256 + 1 of them, and an XCD has
+// ROUND_RUNS / 8 runs of workgroups.
+u64 round_bigseg_cap(u64 n)
+{
+    return (u64)ceil_div_u(n, (u64)g_tile_range * ROUND_RUNS) * (ROUND_RUNS / 8) * (u64)(g_tile_range / 256 + 1);
+}
 
 template <typename KT>
 int round_tile_t(const u32 *act_i, const u32 *act_g, const KT *key2, u64 a, const u64 *rp, u64 *rp_next, u64 *rec,
@@ -1708,7 +1731,7 @@ int round_tile_t(const u32 *act_i, const u32 *act_g, const KT *key2, u64 a, cons
     const u64 seg_cap = round_seg_cap(a);
     u32 *big_counter = (u32 *)(cnt + 4), *err = big_counter + 1;
 #define RT_LAUNCH(R)                                                                                              \
-    hipLaunchKernelGGL((k_round_tile<KT, R>), dim3(ceil_div_u(a, R)), dim3(RT_THREADS), 0, s, act_i, act_g, key2, rp, \
+    hipLaunchKernelGGL((k_round_tile<KT, R>), dim3(ceil_div_u(a, (u64)R * ROUND_RUNS) * ROUND_RUNS), dim3(RT_THREADS), 0, s, act_i, act_g, key2, rp, \
                        SA, ISA, seg_i, seg_g, seg_ctr, seg_cap, err, bseg_h, bseg_g, bseg_cap, LCP, ac, ex)
     // the kernel alone is timed: list entry and key read (8 + sizeof(KT) B), about
     // 16 B written per entry (ranks, placed suffixes, marks and survivors)
