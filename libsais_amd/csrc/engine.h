@@ -99,7 +99,8 @@ struct SegTile {
 };
 constexpr u32 SEG_TILE_KEYS = 16384;
 // Sorts every segment (a contiguous range of the keys) by itself, stably, by key bits
-// [0, end_bit), end_bit <= 32; the result is in (k1, v1) when *alt is set.  seg: the
+// [0, end_bit), 0 < end_bit <= 32, with the keys' positions as values (v0 is not read);
+// the result is in (k1, v1) when *alt is set.  seg: the
 // segments' tiles in order (each but a segment's last one full); seg_start: their first
 // keys; hist: (passes * nseg * 256) u32 of scratch.
 int radix_sort_seg(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, const SegTile *seg, u32 ntiles,
@@ -379,11 +380,13 @@ int launch_histogram(const uint8_t *T, u64 n, int gsa, u64 *hist, uint8_t *pad, 
 int launch_pack_keys32(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, int gsa, int cb, u32 *keys,
                        u32 *vals, hipStream_t s);
 // Batched GSA: sid[p] = number of 0 bytes before p (string id); keys get sid in
-// their high half.  launch_string_ids needs a ScanScratch for n entries.
-int launch_string_ids(const uint8_t *T, u64 n, u32 *sid, ScanScratch &sc, hipStream_t s);
+// their high half.  launch_string_ids: sid[p] = separators before p; the text has 64 bytes
+// after it; part: string_ids_words(n) u32 of scratch.
+u64 string_ids_words(u64 n);
+int launch_string_ids(const uint8_t *T, u64 n, u32 *sid, u32 *part, hipStream_t s);
 // The same in 32 bits: (local[string id] << (bits * k)) | symbols.
 int launch_pack_keys32_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid,
-                           const uint8_t *local, u32 *keys, u32 *vals, hipStream_t s);
+                           const uint8_t *local, u32 *keys, hipStream_t s);
 int launch_pack_keys64_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid, u64 *keys,
                            u32 *vals, hipStream_t s);
 // Checks that string k starts at offsets[k] (sid[offsets[k]] == k and the byte

@@ -1222,7 +1222,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         SAGPU_CHECK(hipMemcpyAsync(d_local, sp_plan.local.data(), nstrings, hipMemcpyHostToDevice, s));
         {
             Span sp(c, F_INITIAL);
-            SAGPU_TRY(launch_pack_keys32_sid(dT, n, d_lut, bits, ksym, sid, d_local, k0, v0, s));
+            SAGPU_TRY(launch_pack_keys32_sid(dT, n, d_lut, bits, ksym, sid, d_local, k0, s));
         }
         SAGPU_TRY(sort_seg(c, k0, v0, k1, v1, n, d_seg, ntiles, d_start, nseg, d_hist, sp_plan.end_bit, &alt));
         Span sp(c, F_INITIAL);
@@ -3207,10 +3207,9 @@ extern "C" int32_t sagpu_gsa_batch32(const uint8_t *d_T, int64_t n, const int64_
     u32 *sid = sc.get<u32>((u64)n);
     int64_t *d_off = sc.get<int64_t>((u64)count + 1);
     u32 *d_bad = sc.get<u32>(64);
-    u32 *part = sc.get<u32>((u64)n / 4096 + 2);
+    u32 *part = sc.get<u32>(string_ids_words((u64)n));
     if (!sid || !d_off || !d_bad || !part) return SAGPU_ENOMEM;
-    ScanScratch ssc{part, (u64)n / 4096 + 2};
-    SAGPU_TRY(launch_string_ids(dT, (u64)n, sid, ssc, s));
+    SAGPU_TRY(launch_string_ids(dT, (u64)n, sid, part, s));
     SAGPU_CHECK(hipMemcpyAsync(d_off, h_offsets, ((size_t)count + 1) * sizeof(int64_t), hipMemcpyHostToDevice, s));
     SAGPU_TRY(launch_fill_u32(d_bad, 1, 0, s));
     SAGPU_TRY(launch_check_offsets(dT, sid, d_off, (u32)count, d_bad, s));
@@ -3363,9 +3362,8 @@ int run_batch(Ctx &c, sagpu_job **jobs, int count)
     GET(sid, u32, N);
     GET(d_off, int64_t, (u64)count + 1);
     GET(d_bad, u32, 64);
-    GET(part, u32, N / 4096 + 2);
-    ScanScratch ssc{part, N / 4096 + 2};
-    SAGPU_TRY(launch_string_ids(dT, N, sid, ssc, s));
+    GET(part, u32, string_ids_words(N));
+    SAGPU_TRY(launch_string_ids(dT, N, sid, part, s));
     SAGPU_CHECK(hipMemcpyAsync(d_off, off.data(), ((size_t)count + 1) * sizeof(int64_t), hipMemcpyHostToDevice, s));
     SAGPU_TRY(launch_fill_u32(d_bad, 1, 0, s));
     SAGPU_TRY(launch_check_offsets(dT, sid, d_off, (u32)count, d_bad, s));

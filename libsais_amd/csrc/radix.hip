@@ -432,7 +432,10 @@ __global__ __launch_bounds__(NT) void k_radix_pass(const K *__restrict__ kin, co
     constexpr bool LOAD_VALS = HAS_VALS && !GEN;
     u32 val[LOAD_VALS ? ITEMS : 1];
     if constexpr (LOAD_VALS) {
-        if (full) {
+        if (SEG && !vin) {   // the values are the positions
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) val[j] = (u32)wbase + (u32)j * SAGPU_WAVE + lane;
+        } else if (full) {
 #pragma unroll
             for (int j = 0; j < ITEMS; j++) val[j] = vin[wbase + (u64)j * SAGPU_WAVE + lane];
         } else {
@@ -815,6 +818,7 @@ int radix_sort_seg_impl(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, co
     SAGPU_TRY(launch_fill_u32(hist, (u64)npass * nseg * 256, 0, s));
     hipLaunchKernelGGL(k_seg_hist, dim3(ntiles), dim3(512), 0, s, (const u32 *)k0, seg, nseg, npass, hist);
     hipLaunchKernelGGL(k_seg_offsets, dim3(nseg), dim3(256), 0, s, hist, seg_start, nseg, npass, rs.tile_ctr);
+    u32 *vi = nullptr;   // (the first pass takes the positions)
     for (int p = 0; p < npass; p++) {
         rs.epoch = (rs.epoch + 1) & ((1u << 22) - 1);
         if (rs.epoch == 0) {
@@ -822,13 +826,14 @@ int radix_sort_seg_impl(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, co
             rs.epoch = 1;
         }
         if (rs.hook) rs.hook(rs.hook_user, 0);
-        hipLaunchKernelGGL((k_radix_pass<u32, true, true, 32, false, 512, 8, true>), dim3(ntiles), dim3(512), 0, s, k0, v0, k1,
+        hipLaunchKernelGGL((k_radix_pass<u32, true, true, 32, false, 512, 8, true>), dim3(ntiles), dim3(512), 0, s, k0, vi, k1,
                            v1, 0ull, 8 * p, 255u, (const u64 *)(hist + (u64)p * nseg * 256), rs.lookback, rs.tile_ctr + p,
                            rs.epoch, (const u32 *)nullptr, 0ull, KeyGen{}, seg);
         SAGPU_CHECK(hipGetLastError());
         if (rs.hook) rs.hook(rs.hook_user, 1);
         u32 *t = k0; k0 = k1; k1 = t;
         t = v0; v0 = v1; v1 = t;
+        vi = v0;
     }
     *alt = npass & 1;
     return SAGPU_OK;

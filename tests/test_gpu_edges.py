@@ -358,3 +358,23 @@ def test_segmented_sort(name, lengths, sigma):
         rc, ref = ol.sa(T[o:e].copy(), gsa=True)
         assert rc == 0 and np.array_equal(SA[o:e], ref), k
         assert np.array_equal(L[o:e], ol.lcp(ol.plcp(T[o:e].copy(), ref, gsa=True), ref)), k
+
+
+@pytest.mark.parametrize("n", [2, 5, 1023, 1025, 4095, 4096, 4097, 8193, 12290])
+def test_string_ids(n):
+    """Sets whose separators fall on every position of a tile's words and steps."""
+    rng = np.random.default_rng(n)
+    T = rng.integers(1, 4, n).astype(np.uint8)
+    at = np.flatnonzero(rng.random(n) < 0.3)
+    T[at[at > 0]] = 0
+    T[1:][(T[1:] == 0) & (T[:-1] == 0)] = 3   # no empty strings
+    T[-2:] = (1, 0)
+    ends = np.flatnonzero(T == 0) + 1
+    offs = np.concatenate([[0], ends]).astype(np.int64)
+    print(f"[string ids] n={n} strings={len(offs) - 1}", flush=True)
+    SA, L = batch.batched(T, offs)
+    for k in range(len(offs) - 1):
+        S = T[offs[k]:offs[k + 1]].copy()
+        rc, ref = ol.sa(S, gsa=True)
+        assert rc == 0 and np.array_equal(SA[offs[k]:offs[k + 1]], ref), k
+        assert np.array_equal(L[offs[k]:offs[k + 1]], ol.lcp(ol.plcp(S, ref, gsa=True), ref)), k
