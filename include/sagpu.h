@@ -227,7 +227,7 @@ SAGPU_API int32_t sagpu_sort_pairs_u64(uint64_t *d_keys, uint32_t *d_vals, int64
  *                    packed key that follows (same order as its rank; default); 0 = by rank
  *   "exact_round1"   1 = with raw_round1, the first round records the exact lcp across each
  *                    split, from the two raw keys (default); 0 = a lower bound, left to the PLCP pass
- *   "plcp_hint"      1 = the fused build with LCP (texts up to 2^28) packs the exact lcp of each
+ *   "plcp_hint"      1 = the fused build with LCP (texts and large string sets up to 2^30) packs the exact lcp of each
  *                    suffix alone in its initial group into bits 28-31 of its ISA word (15 values
  *                    on the largest marks the initial key allows), and the PLCP pass takes it
  *                    instead of reading a pair word (default); 0 = no hints

@@ -111,16 +111,27 @@ int radix_sort_u32(RadixScratch &rs, u32 *k0, u32 *v0, u32 *k1, u32 *v1, u64 n, 
                    int end_bit, hipStream_t s, int *result_in_alt, int *passes_run);
 
 // ------------------------------------------------------- rounds (rounds.hip)
-// ISA words of texts of at most 2^28 suffixes may carry a PLCP hint in bits 28-31
-// (the fused build with LCP: the lcp of a suffix alone in its initial group, coded
-// as in PlcpHint; 0 = none).  Every ISA reader takes the rank through isa_rank; for
-// longer texts nothing is packed and the word is the rank.
-__host__ __device__ __forceinline__ u32 isa_rank(u32 x, u64 n) { return n <= (1ull << 28) ? (x & 0x0FFFFFFFu) : x; }
-__host__ __device__ __forceinline__ u32 isa_hint(u32 x, u64 n) { return n <= (1ull << 28) ? (x >> 28) : 0u; }
-// A hint h (1..15) stands for the lcp off + h - 1: off = max(0, ksym - 10) puts the
-// 15 values on the largest marks an initial key allows and the exact marks of the
-// first doubling round (ksym plus the few symbols two raw keys share; DNA with
-// 16-symbol keys: 6..20).  on (in) asks for the hints; on (out) tells whether they
+// ISA words of texts of at most 2^30 suffixes may carry a PLCP hint in the bits above the
+// rank's (builds with LCP: the lcp of a suffix alone in its initial group, coded as in
+// PlcpHint; 0 = none): from bit 28 on up to 2^28 suffixes (15 values), 29 up to 2^29 (7),
+// 30 up to 2^30 (3).  Every ISA reader takes the rank through isa_rank; for longer texts
+// nothing is packed and the word is the rank.
+__host__ __device__ __forceinline__ int isa_shift(u64 n)
+{
+    return n <= (1ull << 28) ? 28 : n <= (1ull << 29) ? 29 : n <= (1ull << 30) ? 30 : 32;
+}
+__host__ __device__ __forceinline__ u32 isa_rank(u32 x, u64 n) { return x & (u32)((1ull << isa_shift(n)) - 1); }
+__host__ __device__ __forceinline__ u32 isa_hint(u32 x, u64 n) { return (u32)((u64)x >> isa_shift(n)); }
+// The hint bits of an lcp mark: shift = isa_shift(n), off = the first value's lcp.
+__device__ __forceinline__ u32 isa_hint_bits(u32 mark, int shift, u32 off)
+{
+    return mark >= off && mark - off < (1u << (32 - shift)) - 1u ? (mark - off + 1u) << shift : 0u;
+}
+// A hint h >= 1 stands for the lcp off + h - 1: off = max(0, ksym - 10) puts 15 values
+// on the largest marks an initial key allows and the exact marks of the first doubling
+// round (ksym plus the few symbols two raw keys share; DNA with 16-symbol keys: 6..20);
+// 7 values start at ksym - 5, 3 at ksym - 2.  In string sets, whose first round gives no
+// exact marks, the values end at ksym - 1.  on (in) asks for the hints; on (out) tells whether they
 // were packed.
 struct PlcpHint {
     int on = 0;
@@ -211,11 +222,8 @@ struct ExactLcp {
     const u32 *skip = nullptr;   // device (read as constant memory)
     // PLCP hints (PlcpHint) for the suffixes the first round places with an exact
     // mark: the hint bits of the rank written to ISA
-    int hint = 0, hint_off = 0;
-    __device__ u32 hint_bits(u32 mark) const
-    {
-        return hint && mark >= (u32)hint_off && mark - (u32)hint_off < 15u ? (mark - (u32)hint_off + 1u) << 28 : 0u;
-    }
+    int hint = 0, hint_off = 0;   // hint: isa_shift, or 0 for none
+    __device__ u32 hint_bits(u32 mark) const { return hint ? isa_hint_bits(mark, hint, (u32)hint_off) : 0u; }
     __device__ bool skipped(u32 g) const
     {
         for (int t = 0; t < nskip; t++)
@@ -414,6 +422,7 @@ struct LcpScratch {
     u64 *vq_res;      // [256] and first mismatch
     void *tile_max;   // [tiles_cap] per-tile max for the prefix-max scan (u32 or u64), then chunk maxima
     u64 tiles_cap;
+    bool direct;      // byte texts with marks: ranks lie near positions, no pair words
     // optional: called with 0 / 1 around the launch of the pair-word text-order pass
     void (*hook)(void *user, int phase);
     void *hook_user;

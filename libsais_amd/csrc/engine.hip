@@ -1169,12 +1169,13 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         c.rs.gen = nullptr;
         SAGPU_TRY(src);
         Span sp(c, F_INITIAL);
-        if (hint) {   // byte texts without separators, up to 2^28 suffixes
-            hint->on = hint->on && !gsa && !dSym && n <= (1ull << 28);
-            // the 15 hint values cover marks [off, off + 14]: the largest marks of the
+        if (hint) {   // byte texts without separators
+            hint->on = hint->on && !gsa && !dSym && n <= (1ull << 30);
+            // the 15 (7, 3) hint values cover marks from off on: the largest marks of the
             // initial grouping (below ksym) and the first round's exact marks (ksym
             // and a few above)
-            hint->off = ksym > 10 ? ksym - 10 : 0;
+            const int below = isa_shift(n) == 28 ? 10 : isa_shift(n) == 29 ? 5 : 2;
+            hint->off = ksym > below ? ksym - below : 0;
         }
         // the unsorted key buffer is free now: it holds the per-slot group heads
         SAGPU_TRY(group_init(ws, alt ? k1 : k0, alt ? v1 : v0, n, bits, ksym, gsa, dSA, dISA, act_i[0], act_g[0], dLCP,
@@ -1201,7 +1202,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
                 ex1.skip = tails;
                 // suffixes placed by the first round with an exact mark carry it as a
                 // PLCP hint too (their ISA words are written anyway)
-                ex1.hint = hint && hint->on ? 1 : 0;
+                ex1.hint = hint && hint->on ? isa_shift(n) : 0;
                 ex1.hint_off = hint ? hint->off : 0;
             }
         }
@@ -1226,13 +1227,19 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         }
         SAGPU_TRY(sort_seg(c, k0, v0, k1, v1, n, d_seg, ntiles, d_start, nseg, d_hist, sp_plan.end_bit, &alt));
         Span sp(c, F_INITIAL);
+        if (hint) {   // all marks of the initial grouping are below ksym
+            hint->on = hint->on && n <= (1ull << 30);
+            const int values = (1 << (32 - isa_shift(n))) - 1;
+            hint->off = ksym > values ? ksym - values : 0;
+        }
         SAGPU_TRY(group_init(ws, alt ? k1 : k0, alt ? v1 : v0, n, bits, ksym, 1, dSA, dISA, act_i[0], act_g[0], dLCP,
-                             alt ? k0 : k1, alt ? v0 : v1, s));
+                             alt ? k0 : k1, alt ? v0 : v1, s, nullptr, hint));
         SAGPU_TRY(isa_from_pairs(c, sc, alt ? k0 : k1, alt ? v0 : v1, n, dISA, alt ? k1 : k0, alt ? v1 : v0));
     } else {
         // batched GSA: (string id, symbols) keys, so every group stays inside one string
         u64 *k0 = (u64 *)kA, *k1 = (u64 *)kA + n;
         u32 *v0 = vA, *v1 = vA + n;
+        if (hint) hint->on = 0;
         {
             Span sp(c, F_INITIAL);
             SAGPU_TRY(launch_pack_keys64_sid(dT, n, d_lut, bits, ksym, sid, k0, v0, s));
@@ -1568,11 +1575,14 @@ int phi_run(Ctx &c, Scope &sc, const u32 *dSA, u64 n, u32 *dPHI)
     return launch_phi_bucketed(dSA, n, dPHI, pv, pg, bcur, isa_bucket_log2(n), c.stream);
 }
 
+constexpr u64 DIRECT_MEAN = 1u << 17;   // mean string length up to which PLCP takes the direct form
 int plcp_run(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, const u32 *PHI, const u32 *ISA, const u32 *SA,
              u32 *PLCP, const u32 *marks, int sym_bytes = 1, const uint8_t *dU = nullptr,
-             const CodeStream *cs = nullptr, int hint_off = 0)
+             const CodeStream *cs = nullptr, int hint_off = 0, u64 strings = 1)
 {
     LcpScratch ls{};
+    // String sets of short strings keep a string's marks and suffixes within an XCD's L2
+    ls.direct = g_plcp_pairs && strings > 1 && n / strings <= DIRECT_MEAN;
     ls.queue_cap = n / 16 + 4096;
     ls.tiles_cap = n / 4096 + 2;
     GET(q, u32, ls.queue_cap);
@@ -1598,7 +1608,7 @@ int plcp_run(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, const u32 *PH
         if (!V64) return SAGPU_ENOMEM;
     }
     u64 *pairs = nullptr;
-    if (marks && sym_bytes == 1 && g_plcp_pairs) {
+    if (marks && sym_bytes == 1 && g_plcp_pairs && !ls.direct) {
         pairs = sc.get<u64>(n);
         if (!pairs) return SAGPU_ENOMEM;
     }
@@ -3227,13 +3237,16 @@ extern "C" int32_t sagpu_gsa_batch32(const uint8_t *d_T, int64_t n, const int64_
     }
     {
         Span total(*c, F_TOTAL);
+        PlcpHint hint;
+        hint.on = marks && g_plcp_hint;
         int rc = sa_build(*c, sc, dT, (u64)n, 1, gSA, ISA, nullptr, marks, sid, (u32)count, nullptr, 0, nullptr, nullptr,
-                          nullptr, h_offsets);
+                          &hint, h_offsets);
         if (rc != SAGPU_OK) return rc;
         if (d_LCP) {
             {
                 Span sp(*c, F_PLCP);
-                SAGPU_TRY(plcp_run(*c, sc, dT, (u64)n, 1, nullptr, ISA, gSA, P, marks));
+                SAGPU_TRY(plcp_run(*c, sc, dT, (u64)n, 1, nullptr, ISA, gSA, P, marks, 1, nullptr, nullptr,
+                                   hint.on ? hint.off : 0, (u64)count));
             }
             Span sp(*c, F_LCP);
             SAGPU_TRY(launch_lcp_fix(P, gSA, (u64)n, (u32 *)d_LCP, s));
@@ -3383,7 +3396,7 @@ int run_batch(Ctx &c, sagpu_job **jobs, int count)
     SAGPU_TRY(sa_build(c, sc, dT, N, 1, gSA, ISA, nullptr, marks, sid, (u32)count, nullptr, 0, nullptr, nullptr, nullptr,
                        off.data()));
     if (any_l) {
-        SAGPU_TRY(plcp_run(c, sc, dT, N, 1, nullptr, ISA, gSA, P, marks));
+        SAGPU_TRY(plcp_run(c, sc, dT, N, 1, nullptr, ISA, gSA, P, marks, 1, nullptr, nullptr, 0, (u64)count));
         SAGPU_TRY(launch_lcp_fix(P, gSA, N, gL, s));
     }
     GET(oSA, u32, M);

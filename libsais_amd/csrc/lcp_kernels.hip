@@ -333,21 +333,27 @@ __device__ __forceinline__ u64 match_stream(const u32 *__restrict__ pw, int bits
 // Byte texts, pair-word form (k_plcp_pairs): per position one ISA read, one 8-byte
 // pair read and the symbol before it; known lcps and reducible positions finish
 // there, irreducible ones compare as k_plcp_irr.  PI positions per thread and step
-// with their loads issued together, those of the comparisons' first steps too (2^28 DNA
-// suffixes: 1.75 ms with a comparison at a time, 1.55 ms now).  Bound by the random pair
-// reads; the XCDs take runs of the text, so the pairs of a string set's strings are read
-// from one L2 (2^29 suffixes of 20000 strings: 9.4 ms round-robin, 6.4 ms by runs).
+// with their loads issued together, those of the comparisons' first steps too, and
+// without branches around them; ISA and values stream past the L2 (2^28 DNA suffixes:
+// 1.75 ms with a comparison at a time, 1.35 ms now).  Bound by the random reads that miss
+// the L2 (about 60 G/s); the XCDs take runs of the text, so that a string set's strings
+// are read from one L2 each.
 constexpr int PI = 4;
 // Each workgroup takes whole MS_TILE tiles (PI rows of 256 per step) and writes the
 // tile's max of v to tmax, so the prefix max needs no separate reduce pass
 // (k_plcp_long raises the entries of the positions it finishes).
-template <typename VT>
+// DIRECT: the mark, SA[r-1] and T[k-1] instead of the pair words, for texts whose ranks
+// lie near their positions (string sets), where those reads hit the L2 more often and
+// k_plcp_pairs costs more than it saves: 2^29 suffixes of 20000 strings 4.8 ms, against
+// 3.5 ms and 2.0 ms for k_plcp_pairs (without hints 6.4 and 2.0, round-robin 9.4 and 2.0).
+template <typename VT, bool DIRECT, bool STREAM>
 __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restrict__ T, u64 n, int gsa,
                                                         const u32 *__restrict__ ISA, const u64 *__restrict__ pairs,
                                                         VT *__restrict__ V, u32 *__restrict__ queue,
                                                         u32 *__restrict__ queue_l, u32 *__restrict__ queue_n,
                                                         u64 queue_cap, const u32 *__restrict__ pw, int bits,
-                                                        VT *__restrict__ tmax, int hint_off, int split)
+                                                        VT *__restrict__ tmax, int hint_off, int split,
+                                                        const u32 *__restrict__ marks, const u32 *__restrict__ SA)
 {
     // split > 1 (short texts): a tile's steps go to `split` workgroups, which raise
     // the tile's maximum (zeroed first) with atomics instead of storing it
@@ -356,8 +362,8 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
     __shared__ VT s_m[4];
     const u64 tiles = (n + MS_TILE - 1) / MS_TILE;
     const u64 part_len = MS_TILE / (u64)split;
-    const u32 per = pw ? 64u / (u32)bits : 8u;   // symbols a step compares
-    const u64 keep = pw ? ~0ull << (64 - per * (u32)bits) : 0ull;
+    const u32 per = STREAM ? 64u / (u32)bits : 8u;   // symbols a step compares
+    const u64 keep = STREAM ? ~0ull << (64 - per * (u32)bits) : 0ull;
     const u64 items = tiles * (u64)split;
     for (u64 b = blockIdx.x; b < xcd_runs(items); b += gridDim.x) {
         const u64 wi = xcd_run(b, items);
@@ -365,92 +371,114 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
         const u64 tile = wi / (u64)split, p0 = tile * MS_TILE + (wi % (u64)split) * part_len;
         VT mx = 0;
         for (u64 base = p0; base < p0 + part_len && base < n; base += STEP) {
-            u32 r[PI], hint[PI];
-            u64 w[PI];
-            uint8_t a[PI];
-#pragma unroll
-            for (int q = 0; q < PI; q++) {
-                const u64 i = base + (u64)q * 256 + threadIdx.x;
-                const u32 x = i < n ? ISA[i] : 0u;
-                r[q] = isa_rank(x, n);
-                hint[q] = isa_hint(x, n);   // 1 + PLCP[i] known from the initial grouping
-                a[q] = (i > 0 && i < n) ? T[i - 1] : 0;
-            }
-#pragma unroll
-            for (int q = 0; q < PI; q++) w[q] = (r[q] && !hint[q]) ? pairs[r[q]] : 0ull;
-            // the first step of every comparison: all loads in flight together (lanes
-            // without one read the text's first symbols)
-            u64 d[PI];
-            u32 l0[PI];
+            // Positions, lengths and values in VT (32 bits up to 2^31 - 1 positions).
+            // Lanes without a load read entry 0 instead of branching around it.
+            const VT nn = (VT)n, i0 = (VT)base + threadIdx.x;
+            u32 x[PI], k[PI], known[PI];   // the ISA word; T[i..]'s neighbour, or the lcp
+            uint8_t a[PI], before[PI];     // the symbols before i and k
+            VT l0[PI];
             bool cmp[PI], any = false;
 #pragma unroll
             for (int q = 0; q < PI; q++) {
-                const u64 i = base + (u64)q * 256 + threadIdx.x;
-                const u32 k = (u32)w[q];
-                // unknown and not reducible (PLCP[i] = PLCP[i-1] - 1)
-                cmp[q] = (w[q] >> 63) && !(i > 0 && k > 0 && a[q] == (uint8_t)(w[q] >> 32) && !(gsa && a[q] == 0));
-                const u32 lg = (u32)(w[q] >> 58) & 31u;
-                l0[q] = lg ? 1u << (lg - 1) : 0u;
-                const u64 m = n - (i > k ? i : k);
-                if ((u64)l0[q] > m) l0[q] = (u32)m;
+                const VT i = i0 + (VT)(q * 256);
+                x[q] = __builtin_nontemporal_load(ISA + (i < nn ? i : (VT)0));
+                a[q] = T[i > 0 && i < nn ? i - 1 : (VT)0];
+            }
+            bool look[PI];
+#pragma unroll
+            for (int q = 0; q < PI; q++) {
+                const VT i = i0 + (VT)(q * 256);
+                // (a hint: the lcp known from the initial grouping, plus 1)
+                look[q] = i < nn && isa_rank(x[q], n) && !isa_hint(x[q], n);
+            }
+            if constexpr (DIRECT) {
+                u32 m[PI];
+#pragma unroll
+                for (int q = 0; q < PI; q++) m[q] = marks[look[q] ? isa_rank(x[q], n) : 0u];
+#pragma unroll
+                for (int q = 0; q < PI; q++) {
+                    cmp[q] = look[q] && (m[q] & LCP_UNKNOWN);
+                    k[q] = SA[cmp[q] ? isa_rank(x[q], n) - 1u : 0u];
+                }
+#pragma unroll
+                for (int q = 0; q < PI; q++) {
+                    before[q] = T[cmp[q] && k[q] ? k[q] - 1u : 0u];
+                    known[q] = m[q];
+                    l0[q] = (VT)(m[q] & ~LCP_UNKNOWN);
+                }
+            } else {
+                u64 w[PI];
+#pragma unroll
+                for (int q = 0; q < PI; q++) w[q] = pairs[look[q] ? isa_rank(x[q], n) : 0u];
+#pragma unroll
+                for (int q = 0; q < PI; q++) {
+                    k[q] = known[q] = (u32)w[q];
+                    before[q] = (uint8_t)(w[q] >> 32);
+                    const u32 lg = (u32)(w[q] >> 58) & 31u;
+                    l0[q] = lg ? (VT)1 << (lg - 1) : (VT)0;
+                    cmp[q] = look[q] && w[q] >> 63;
+                }
+            }
+            // unknown, and reducible when the symbols before agree (PLCP[i] = PLCP[i-1] - 1);
+            // DIRECT: the first step's loads don't wait for T[k-1]
+            bool red[PI];
+            u64 d[PI];
+#pragma unroll
+            for (int q = 0; q < PI; q++) {
+                const VT i = i0 + (VT)(q * 256);
+                const VT m = nn - vmax(i, (VT)k[q]);
+                l0[q] = cmp[q] && l0[q] > m ? m : l0[q];
+                red[q] = cmp[q] && i > 0 && k[q] > 0 && a[q] == before[q] && !(gsa && a[q] == 0);
+                if (!DIRECT) cmp[q] = cmp[q] && !red[q];
                 any |= cmp[q];
                 d[q] = 0;
             }
+            // the first step of every comparison: all loads in flight together
+            if (__ballot(any)) {
 #pragma unroll
-            for (int q = 0; q < PI; q++) {
-                if (!__ballot(any)) break;
-                const u64 i = base + (u64)q * 256 + threadIdx.x;
-                const u32 k = (u32)w[q];
-                const u64 pi = cmp[q] ? i + l0[q] : 0, pk = cmp[q] ? (u64)k + l0[q] : 0;
-                if (pw) {
-                    d[q] = (stream_window(pw, pi * (u64)bits) ^ stream_window(pw, pk * (u64)bits)) & keep;
-                } else {
-                    const u64 x = load8u(T + pi);
-                    d[q] = (x ^ load8u(T + pk)) | (gsa ? zero_lanes<1>(x) : 0ull);
+                for (int q = 0; q < PI; q++) {
+                    const VT pi = cmp[q] ? i0 + (VT)(q * 256) + l0[q] : (VT)0, pk = cmp[q] ? (VT)k[q] + l0[q] : (VT)0;
+                    if (STREAM) {
+                        d[q] = (stream_window(pw, (u64)pi * (u32)bits) ^ stream_window(pw, (u64)pk * (u32)bits)) & keep;
+                    } else {
+                        const u64 s = load8u(T + pi);
+                        d[q] = (s ^ load8u(T + pk)) | (gsa ? zero_lanes<1>(s) : 0ull);
+                    }
                 }
             }
 #pragma unroll
             for (int q = 0; q < PI; q++) {
-                const u64 i = base + (u64)q * 256 + threadIdx.x;
-                if (i >= n) continue;
-                VT v;
-                if (hint[q]) {
-                    v = (VT)((u64)hint_off + hint[q] - 1 + i);
-                } else if (r[q] == 0) {   // first suffix in SA order: lcp 0
-                    v = (VT)i;
-                } else if (!(w[q] >> 63)) {
-                    v = (VT)((u64)(u32)w[q] + i);
-                } else if (!cmp[q]) {
-                    v = 0;   // reducible: PLCP[i] = PLCP[i-1] - 1
-                } else {
-                    const u64 k = (u32)w[q];
-                    const u64 m = n - (i > k ? i : k);
-                    u64 l = l0[q];
-                    bool done = true;
-                    if (l >= m) {
-                        l = m;
-                    } else if (d[q]) {
-                        l += pw ? (u64)((u32)__clzll((long long)d[q]) / (u32)bits) : (u64)(__builtin_ctzll(d[q]) >> 3);
+                const VT i = i0 + (VT)(q * 256);
+                VT v = (VT)known[q];
+                if (!look[q]) v = isa_hint(x[q], n) ? (VT)hint_off + (VT)isa_hint(x[q], n) - 1 : (VT)0;   // (first suffix: 0)
+                if (cmp[q] && !red[q]) {
+                    const VT m = nn - vmax(i, (VT)k[q]);
+                    const u32 s = STREAM ? (u32)__clzll((long long)d[q]) / (u32)bits : (u32)__builtin_ctzll(d[q]) >> 3;
+                    v = l0[q] + (VT)s;
+                    v = v < m ? v : m;
+                    if (!d[q] && l0[q] < m) {   // longer than the first step
+                        bool done;
+                        u64 l = (u64)l0[q] + per;
                         l = l < m ? l : m;
-                    } else {   // longer than the first step
-                        l += per;
-                        // with the code stream (no GSA), 64 / bits symbols per step
-                        l = pw ? match_stream(pw, bits, i, k, l < m ? l : m, m, PL_THREAD_LIMIT, &done)
-                               : match_bytes<1>(T, i, k, l < m ? l : m, m, gsa, PL_THREAD_LIMIT, &done);
-                    }
-                    if (!done) {
-                        u32 slot = atomicAdd(queue_n, 1u);
-                        if (slot < queue_cap) {
-                            queue[slot] = (u32)i;   // provisional value; k_plcp_long finishes it
-                            queue_l[slot] = (u32)l;
-                        } else {
-                            l = match_bytes<1>(T, i, k, l, m, gsa, ~0ull >> 1, &done);
+                        l = STREAM ? match_stream(pw, bits, i, k[q], l, m, PL_THREAD_LIMIT, &done)
+                                   : match_bytes<1>(T, i, k[q], l, m, gsa, PL_THREAD_LIMIT, &done);
+                        if (!done) {
+                            u32 slot = atomicAdd(queue_n, 1u);
+                            if (slot < queue_cap) {
+                                queue[slot] = (u32)i;   // provisional value; k_plcp_long finishes it
+                                queue_l[slot] = (u32)l;
+                            } else {
+                                l = match_bytes<1>(T, i, k[q], l, m, gsa, ~0ull >> 1, &done);
+                            }
                         }
+                        v = (VT)l;
                     }
-                    v = (VT)(l + i);
                 }
-                V[i] = v;
-                mx = vmax(mx, v);
+                v = red[q] ? (VT)0 : v + i;
+                if (i < nn) {
+                    __builtin_nontemporal_store(v, V + i);
+                    mx = vmax(mx, v);
+                }
             }
         }
         mx = wave_incl_max_t(mx);
@@ -478,7 +506,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_pl
 #pragma unroll
         for (int q = 0; q < PP; q++) {
             const u64 j = base + (u64)q * 256 + threadIdx.x;
-            m[q] = (j > 0 && j < n) ? marks[j] : 0u;
+            m[q] = (j > 0 && j < n) ? __builtin_nontemporal_load(marks + j) : 0u;
         }
 #pragma unroll
         for (int q = 0; q < PP; q++) {
@@ -504,7 +532,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_pl
                 const u32 lg = lb ? 32u - (u32)__clz(lb) : 0u;
                 w = (1ull << 63) | ((u64)lg << 58) | ((u64)b[q] << 32) | (u64)k[q];
             }
-            pairs[j] = w;
+            __builtin_nontemporal_store(w, pairs + j);
         }
     }
 }
@@ -958,16 +986,23 @@ int launch_plcp_t(LcpScratch &ls, const uint8_t *T, u64 n, int gsa, const u32 *P
     }
     VT *tmax = (VT *)ls.tile_max;
     SAGPU_TRY(launch_fill_u32(ls.queue_n, 2, 0, s));
-    const bool fused_max = pairs && W == 1;   // the pair-word pass writes the tile maxima itself
+    const bool direct = ls.direct && marks && W == 1;
+    const bool fused_max = (pairs || direct) && W == 1;   // the pass writes the tile maxima itself
     if (fused_max) {
         if constexpr (W == 1) {
             // short texts: one 1024-position step per workgroup
             const int split = n < (1ull << 20) ? (int)(MS_TILE / (256 * PI)) : 1;
             if (split > 1) SAGPU_TRY(launch_fill_u32((u32 *)tmax, tiles * sizeof(VT) / 4, 0, s));
             if (ls.hook) ls.hook(ls.hook_user, 0);
-            hipLaunchKernelGGL((k_plcp_irr_pairs<VT>), dim3(xcd_grid(xcd_runs(tiles * (u64)split))), dim3(256), 0, s, T, n,
-                               gsa, ISA, pairs, V, ls.queue, ls.queue_l, ls.queue_n, ls.queue_cap,
-                               gsa ? nullptr : pw, bits, tmax, hint_off, split);
+            const dim3 grid(xcd_grid(xcd_runs(tiles * (u64)split)));
+            const bool stream = !gsa && pw;
+#define IRR(D, ST)                                                                                                 \
+    hipLaunchKernelGGL((k_plcp_irr_pairs<VT, D, ST>), grid, dim3(256), 0, s, T, n, gsa, ISA, pairs, V, ls.queue,     \
+                       ls.queue_l, ls.queue_n, ls.queue_cap, pw, bits, tmax, hint_off, split, marks, SA)
+            if (direct) IRR(true, false);
+            else if (stream) IRR(false, true);
+            else IRR(false, false);
+#undef IRR
             if (ls.hook) ls.hook(ls.hook_user, 1);
         }
     } else {

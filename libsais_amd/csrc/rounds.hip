@@ -269,9 +269,8 @@ struct InitF {
     // tile t's first slot in bucket b directly, with no atomics.
     u32 *PV, *PG, *bcnt;
     int wlog;
-    // 1: the head of a slot alone in its group carries its exact lcp mark as a PLCP
-    // hint in bits 28-31 (mark - hint_off + 1, for marks in [hint_off, hint_off + 14];
-    // texts of at most 2^28 suffixes)
+    // hint = isa_shift (0: none): the head of a slot alone in its group carries its exact
+    // lcp mark as a PLCP hint above the rank (isa_hint_bits; texts of at most 2^30 suffixes)
     int hint, hint_off;
     u32 lowbits;   // the lowest bit of each of the ksym symbol slots of a key
     // BWT seeding (cb > 0): vals carry (suffix << cb) | code of the symbol before
@@ -543,9 +542,7 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
             if (f.LCP && e > 0)
                 mark = f.lcp_mark((u32)sk.k[r], (u32)kp, !act, n - (u64)(vv[r] >> f.cb), onep, n - (u64)(vp >> f.cb));
             // (an unknown mark is >= 2^31 and gets none)
-            const u32 hint = (f.hint && f.LCP && !act && mark >= (u32)f.hint_off && mark - (u32)f.hint_off < 15u)
-                                 ? (mark - (u32)f.hint_off + 1u) << 28
-                                 : 0u;
+            const u32 hint = f.hint && f.LCP && !act ? isa_hint_bits(mark, f.hint, (u32)f.hint_off) : 0u;
             const u32 b = (u32)((u64)v >> f.wlog);
             const u64 slot = s_base[b] + s_cnt[w][b] + (st[r] & 0x3fffffffu);
             f.PV[slot] = v;
@@ -645,7 +642,7 @@ struct BigF {
         // rank then stored at its first slot + 1); new ranks here are first slots
         const bool flagged = (gw & ac.gf) != 0;
         const bool kept = flagged ? key == keepkey[q] : r == g;
-        u32 hint = 0;   // PLCP hint of a suffix placed with an exact mark (ISA bits 28-31)
+        u32 hint = 0;   // PLCP hint of a suffix placed with an exact mark (above its rank)
         if (LCP && hstart == (u32)e && r != g) {
             // a subgroup after the group's first: e - 1 is the last entry of the
             // previous subgroup (exact marks come only without pivot classes)
@@ -726,7 +723,7 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
 #pragma unroll
         for (int q = 0; q < IG; q++) {
             const u64 k = base + (u64)q * 256 + threadIdx.x;
-            i[q] = k < a ? act_i[k] >> cb : 0u;
+            i[q] = k < a ? __builtin_nontemporal_load(act_i + k) >> cb : 0u;
             // round 1 with a code stream: the packed key of i + h orders the group as
             // its rank does (equal keys, equal ranks), read from the 2-bits-per-symbol
             // stream instead of the 4-byte ISA; groups holding a suffix shorter than
@@ -1136,7 +1133,7 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
         // unflagged
         const u32 gv = (gw & ac.gf) ? SA[g + 1] : g;
         const bool kept = gv - g >= lt && gv - g < lt + eq;
-        u32 hint = 0;   // PLCP hint of a suffix placed with an exact mark (ISA bits 28-31)
+        u32 hint = 0;   // PLCP hint of a suffix placed with an exact mark (above its rank)
         if (kept && (gw & ac.gf) && lt > 0 && eq > 1 && eqb == 0) SA[r + 1] = gv;
         if (LCP && lt > 0 && eqb == 0) {
             u32 mark = LCP_UNKNOWN | (h < LCP_BOUND_CAP ? h : LCP_BOUND_CAP);
@@ -1611,7 +1608,7 @@ int group_init_t(WsScratch &ws, const K *keys, const u32 *vals, u64 n, int bits,
     const int cb = seed ? seed->cb : 0;
     const int wlog = isa_pair_bucket_log2(n);
     InitF<K> f{keys, vals, n, (1u << bits) - 1u, bits, ksym, gsa, SA, act_i, act_g, LCP, PV, PG, ws.bcnt, wlog,
-               hint && hint->on && n <= (1ull << 28) ? 1 : 0, hint ? hint->off : 0, 0u, cb,
+               hint && hint->on ? isa_shift(n) : 0, hint ? hint->off : 0, 0u, cb,
                seed ? seed->codes : nullptr, 65536u / (u32)bits + 1u};
     for (int i = 0; i < ksym; i++) f.lowbits |= 1u << (bits * i);
     // short texts: 512-position tiles (2 rows per wave), so more workgroups share them

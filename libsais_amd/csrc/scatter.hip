@@ -88,8 +88,9 @@ __global__ __launch_bounds__(XW_THREADS) void k_scatter_windows(const u32 *__res
 #pragma unroll
         for (int k = 0; k < XW_ITEMS; k++) {
             const u64 e = base + (u64)k * XW_THREADS + tid;
-            v[k] = e < lim ? PV[e] : 0u;
-            g[k] = e < lim ? PG[e] : 0u;
+            // (past the L2, which holds the windows: 2 to 5 % of the kernel)
+            v[k] = e < lim ? __builtin_nontemporal_load(PV + e) : 0u;
+            g[k] = e < lim ? __builtin_nontemporal_load(PG + e) : 0u;
         }
 #pragma unroll
         for (int k = 0; k < XW_ITEMS; k++)

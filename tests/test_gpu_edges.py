@@ -378,3 +378,58 @@ def test_string_ids(n):
         rc, ref = ol.sa(S, gsa=True)
         assert rc == 0 and np.array_equal(SA[offs[k]:offs[k + 1]], ref), k
         assert np.array_equal(L[offs[k]:offs[k + 1]], ol.lcp(ol.plcp(S, ref, gsa=True), ref)), k
+
+
+def _check_lcp(T, SA, L, n, rng):
+    j = rng.integers(1, n, 5000)
+    for a, b, l in zip(SA[j - 1], SA[j], L[j]):
+        assert np.array_equal(T[a:a + l], T[b:b + l])
+        assert max(a, b) + l == n or T[a + l] != T[b + l]
+
+
+@pytest.mark.parametrize("n", [1 << 28, (1 << 28) + 1, (1 << 29) + 1])
+def test_plcp_hint_ranges(n):
+    """PLCP hints on both sides of the sizes where the bits for them get fewer: the same
+    LCP and PLCP with hints and without, and sampled lcps of the text."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    T = workloads.iid(n, seed=n & 255, alphabet=b"ACGT")
+    T[n // 2: n // 2 + 3000] = T[:3000]
+    out = []
+    for on in (1, 0):
+        print(f"[hints] n={n} plcp_hint={on}", flush=True)
+        assert lib.sagpu_set_option(b"plcp_hint", on) == 0
+        try:
+            SA, _, _, P, L, _ = fused(T)
+        finally:
+            assert lib.sagpu_set_option(b"plcp_hint", 1) == 0
+        out.append((SA, P, L))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    _check_lcp(T, out[0][0], out[0][2], n, np.random.default_rng(n))
+
+
+@pytest.mark.parametrize("n", [1 << 23, (1 << 28) + 5])
+def test_plcp_hint_sets(n):
+    """The same for string sets sorted string by string."""
+    lib = la.load()
+    rng = np.random.default_rng(n)
+    T = workloads.iid(n, seed=n & 255, alphabet=b"ACGT")
+    T[np.cumsum(rng.integers(3, 90000, n // 45000 - 100))] = 0
+    T[-1] = 0
+    T[(n - 50):(n - 1)] = 67
+    ends = np.flatnonzero(T == 0) + 1
+    offs = np.concatenate([[0], ends]).astype(np.int64)
+    out = []
+    for on in (1, 0):
+        print(f"[hint sets] n={n} strings={len(offs) - 1} plcp_hint={on}", flush=True)
+        assert lib.sagpu_set_option(b"plcp_hint", on) == 0
+        try:
+            out.append(batch.batched(T, offs))
+        finally:
+            assert lib.sagpu_set_option(b"plcp_hint", 1) == 0
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    for k in (0, len(offs) // 2, len(offs) - 2):
+        S = T[offs[k]:offs[k + 1]].copy()
+        rc, ref = ol.sa(S, gsa=True)
+        assert rc == 0 and np.array_equal(out[0][0][offs[k]:offs[k + 1]], ref), k
+        assert np.array_equal(out[0][1][offs[k]:offs[k + 1]], ol.lcp(ol.plcp(S, ref, gsa=True), ref)), k
