@@ -187,10 +187,10 @@ struct ActCode {
     u32 gf = 0;
 };
 // PV, PG: scratch of n entries each ((suffix, group head) pairs bucketed for the
-// ISA scatter).
+// ISA scatter).  direct: no pairs, the ranks are written to ISA.
 int group_init(WsScratch &ws, const u32 *keys, const u32 *vals, u64 n, int bits, int ksym, int gsa, u32 *SA, u32 *ISA,
                u32 *act_i, u32 *act_g, u32 *LCP, u32 *PV, u32 *PG, hipStream_t s, const BwtSeed *seed = nullptr,
-               const PlcpHint *hint = nullptr);
+               const PlcpHint *hint = nullptr, bool direct = false);
 // ISA scatter after the initial sort: buckets of 2^v suffixes (v in [10, 32]; at most
 // 64 buckets, larger ones for longer texts).
 void set_isa_window_log2(int v);

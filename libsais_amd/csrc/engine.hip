@@ -1025,6 +1025,10 @@ try {
     return false;
 }
 
+// Whether a set's strings are short enough that reads and writes all over one string (4
+// to 9 bytes per symbol) mostly stay in an XCD's 4 MB of L2.
+bool short_strings(u64 n, u64 strings) { return strings > 1 && n / strings <= (1u << 17); }
+
 // The context's byte counts (kept zero) and code tables.
 int ensure_alpha(Ctx &c)
 {
@@ -1233,8 +1237,9 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             hint->off = ksym > values ? ksym - values : 0;
         }
         SAGPU_TRY(group_init(ws, alt ? k1 : k0, alt ? v1 : v0, n, bits, ksym, 1, dSA, dISA, act_i[0], act_g[0], dLCP,
-                             alt ? k0 : k1, alt ? v0 : v1, s, nullptr, hint));
-        SAGPU_TRY(isa_from_pairs(c, sc, alt ? k0 : k1, alt ? v0 : v1, n, dISA, alt ? k1 : k0, alt ? v1 : v0));
+                             alt ? k0 : k1, alt ? v0 : v1, s, nullptr, hint, short_strings(n, nstrings)));
+        if (!short_strings(n, nstrings))
+            SAGPU_TRY(isa_from_pairs(c, sc, alt ? k0 : k1, alt ? v0 : v1, n, dISA, alt ? k1 : k0, alt ? v1 : v0));
     } else {
         // batched GSA: (string id, symbols) keys, so every group stays inside one string
         u64 *k0 = (u64 *)kA, *k1 = (u64 *)kA + n;
@@ -1575,14 +1580,12 @@ int phi_run(Ctx &c, Scope &sc, const u32 *dSA, u64 n, u32 *dPHI)
     return launch_phi_bucketed(dSA, n, dPHI, pv, pg, bcur, isa_bucket_log2(n), c.stream);
 }
 
-constexpr u64 DIRECT_MEAN = 1u << 17;   // mean string length up to which PLCP takes the direct form
 int plcp_run(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, const u32 *PHI, const u32 *ISA, const u32 *SA,
              u32 *PLCP, const u32 *marks, int sym_bytes = 1, const uint8_t *dU = nullptr,
              const CodeStream *cs = nullptr, int hint_off = 0, u64 strings = 1)
 {
     LcpScratch ls{};
-    // String sets of short strings keep a string's marks and suffixes within an XCD's L2
-    ls.direct = g_plcp_pairs && strings > 1 && n / strings <= DIRECT_MEAN;
+    ls.direct = g_plcp_pairs && short_strings(n, strings);
     ls.queue_cap = n / 16 + 4096;
     ls.tiles_cap = n / 4096 + 2;
     GET(q, u32, ls.queue_cap);

@@ -269,6 +269,9 @@ struct InitF {
     // tile t's first slot in bucket b directly, with no atomics.
     u32 *PV, *PG, *bcnt;
     int wlog;
+    // instead of the pairs (ISA given): the ranks go straight to the ISA, for string sets
+    // sorted string by string, whose tiles write near their own positions
+    u32 *ISA;
     // hint = isa_shift (0: none): the head of a slot alone in its group carries its exact
     // lcp mark as a PLCP hint above the rank (isa_hint_bits; texts of at most 2^30 suffixes)
     int hint, hint_off;
@@ -390,11 +393,12 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_reduce(InitF<K> f, Agg *__r
     if (threadIdx.x < IB_MAX) s_cnt[threadIdx.x] = 0;
     SpanKeys<K, R> sk;
     sk.load(f.keys, f.n, wbase);
+    const bool buckets = !f.ISA;
     u32 vv[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
-        vv[r] = e < f.n ? f.vals[e] : 0u;
+        vv[r] = buckets && e < f.n ? f.vals[e] : 0u;
     }
     __syncthreads();
     u64 s = 0;
@@ -411,8 +415,9 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_reduce(InitF<K> f, Agg *__r
         m1 = last_set(hb, (u32)(wbase + (u64)r * SAGPU_WAVE), m1);
     }
     // the wave's elements of each ISA bucket (u64 shifts: wlog may be 32, one bucket)
-    const u32 nb = (u32)(((f.n - 1) >> f.wlog) + 1);
-    if (nb <= 8) {
+    const u32 nb = buckets ? (u32)(((f.n - 1) >> f.wlog) + 1) : 0u;
+    if (nb == 0) {
+    } else if (nb <= 8) {
         // eight counts of a lane in one word, added up over the lanes as 16-bit fields
         static_assert(R < 256, "8 bits a count");
         u64 c = 0;
@@ -449,9 +454,11 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_reduce(InitF<K> f, Agg *__r
 // elements into the active list, LCP marks, BWT seeds, and the (suffix, group head)
 // pairs into their ISA buckets.  Bound by memory, 26 B per element and the lists; the
 // ranks inside the buckets came from returning LDS atomics: 4.1 ms for a string set of
-// 2^29 suffixes whose tiles have one bucket each, now 2.5 ms (2^28 DNA suffixes over 8
-// buckets: 2.05 ms both ways).
-template <typename K, int R>
+// 2^29 suffixes whose tiles have one bucket each, then 2.5 ms (2^28 DNA suffixes over 8
+// buckets: 2.05 ms both ways).  In sets of short strings a tile writes its ranks near its
+// own positions: straight to the ISA 5.8 ms, against 2.6 ms for this kernel with pairs and
+// 5.0 ms for their pass into windows and the scatter.
+template <typename K, int R, bool LOCAL = false>
 __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg *__restrict__ texcl)
 {
     constexpr int SPAN = R * SAGPU_WAVE;
@@ -459,9 +466,12 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
     __shared__ u32 s_cnt[WS_WAVES][IB_MAX];   // elements per wave and bucket, then the waves' offsets
     __shared__ u64 s_base[IB_MAX];
     const u32 w = threadIdx.x / SAGPU_WAVE, lane = lane_id();
-    const u64 wbase = (u64)blockIdx.x * (WS_WAVES * SPAN) + (u64)w * SPAN;
     const u64 n = f.n;
-    const u32 nb = (u32)(((n - 1) >> f.wlog) + 1);
+    const u64 tiles = (n + WS_WAVES * SPAN - 1) / (WS_WAVES * SPAN);
+    const u64 tile = LOCAL ? xcd_run(blockIdx.x, tiles) : (u64)blockIdx.x;
+    if (tile >= tiles) return;
+    const u64 wbase = tile * (WS_WAVES * SPAN) + (u64)w * SPAN;
+    const u32 nb = LOCAL ? 0u : (u32)(((n - 1) >> f.wlog) + 1);
     s_cnt[w][lane] = 0;
     static_assert(IB_MAX == SAGPU_WAVE, "a lane per bucket");
     SpanKeys<K, R> sk;
@@ -470,7 +480,7 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
-        vv[r] = e < n ? f.vals[e] : 0u;
+        vv[r] = e >= n ? 0u : LOCAL ? __builtin_nontemporal_load(f.vals + e) : f.vals[e];
     }
     __syncthreads();
     // st[r]: bit 31 grouped, bit 30 group start, low bits the rank inside the wave's
@@ -489,15 +499,17 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
         s += (u32)__popcll(__ballot(act));
         const u64 hb = __ballot(head);
         m1 = last_set(hb, (u32)(wbase + (u64)r * SAGPU_WAVE), m1);
-        // u64 shifts: wlog may be 32 (one bucket), which a 32-bit shift cannot express
-        const u32 b = (u32)((u64)(vv[r] >> f.cb) >> f.wlog);
-        const u64 in = __ballot(e < n);
-        const u64 m = nb <= 8 ? wave_peers<3>(b, in) : wave_peers<6>(b, in);
         u32 rank = 0;
-        if (e < n) {
-            const u32 old = s_cnt[w][b];
-            s_cnt[w][b] = old + (u32)__popcll(m);   // the same value from every peer
-            rank = old + mask_below(m);
+        if (!LOCAL) {
+            // u64 shifts: wlog may be 32 (one bucket), which a 32-bit shift cannot express
+            const u32 b = (u32)((u64)(vv[r] >> f.cb) >> f.wlog);
+            const u64 in = __ballot(e < n);
+            const u64 m = nb <= 8 ? wave_peers<3>(b, in) : wave_peers<6>(b, in);
+            if (e < n) {
+                const u32 old = s_cnt[w][b];
+                s_cnt[w][b] = old + (u32)__popcll(m);   // the same value from every peer
+                rank = old + mask_below(m);
+            }
         }
         st[r] = rank | (act ? 1u << 31 : 0u) | (head ? 1u << 30 : 0u);
     }
@@ -510,15 +522,21 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
             s_cnt[q][threadIdx.x] = o;
             o += c;
         }
-        if (o) s_base[threadIdx.x] = f.bcnt[(u64)threadIdx.x * gridDim.x + blockIdx.x];
+        if (o) s_base[threadIdx.x] = f.bcnt[(u64)threadIdx.x * tiles + tile];
     }
-    Agg c = texcl[blockIdx.x];
+    Agg c = texcl[tile];
     for (u32 q = 0; q < w; q++) {
         c.s += s_w[q].s;
         c.m1 = umax(c.m1, s_w[q].m1);
     }
     __syncthreads();
     const u32 cmask = (1u << f.cb) - 1u;
+    // written in order; past the L2 where the ISA's lines fill up in it (string sets: 6.2 ->
+    // 5.8 ms for 2^29 suffixes; shorter texts find what is written in the caches later)
+    auto put = [&](u32 *p, u32 x) {
+        if (LOCAL) __builtin_nontemporal_store(x, p);
+        else *p = x;
+    };
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const u64 e = wbase + (u64)r * SAGPU_WAVE + lane;
@@ -543,18 +561,22 @@ __global__ __launch_bounds__(WS_THREADS) void k_init_emit(InitF<K> f, const Agg 
                 mark = f.lcp_mark((u32)sk.k[r], (u32)kp, !act, n - (u64)(vv[r] >> f.cb), onep, n - (u64)(vp >> f.cb));
             // (an unknown mark is >= 2^31 and gets none)
             const u32 hint = f.hint && f.LCP && !act ? isa_hint_bits(mark, f.hint, (u32)f.hint_off) : 0u;
-            const u32 b = (u32)((u64)v >> f.wlog);
-            const u64 slot = s_base[b] + s_cnt[w][b] + (st[r] & 0x3fffffffu);
-            f.PV[slot] = v;
-            f.PG[slot] = g | hint;
+            if (LOCAL) {
+                f.ISA[v] = g | hint;
+            } else {
+                const u32 b = (u32)((u64)v >> f.wlog);
+                const u64 slot = s_base[b] + s_cnt[w][b] + (st[r] & 0x3fffffffu);
+                f.PV[slot] = v;
+                f.PG[slot] = g | hint;
+            }
             // every slot is written (full lines); slots of grouped elements are
             // overwritten when their suffixes are placed
-            f.SA[e] = v;
+            put(f.SA + e, v);
             if (act) {
-                f.act_i[o] = vv[r];   // with the BWT seed the code travels in the list entry
-                f.act_g[o] = g;
+                put(f.act_i + o, vv[r]);   // with the BWT seed the code travels in the list entry
+                put(f.act_g + o, g);
             }
-            if (f.LCP) f.LCP[e] = mark;
+            if (f.LCP) put(f.LCP + e, mark);
         }
         c.s += (u32)__popcll(ab);
         c.m1 = last_set(hb, row, c.m1);
@@ -1603,17 +1625,17 @@ int g_init_rows = 8;
 template <typename K>
 int group_init_t(WsScratch &ws, const K *keys, const u32 *vals, u64 n, int bits, int ksym, int gsa, u32 *SA, u32 *ISA,
                  u32 *act_i, u32 *act_g, u32 *LCP, u32 *PV, u32 *PG, hipStream_t s, const BwtSeed *seed = nullptr,
-                 const PlcpHint *hint = nullptr)
+                 const PlcpHint *hint = nullptr, bool direct = false)
 {
     const int cb = seed ? seed->cb : 0;
     const int wlog = isa_pair_bucket_log2(n);
-    InitF<K> f{keys, vals, n, (1u << bits) - 1u, bits, ksym, gsa, SA, act_i, act_g, LCP, PV, PG, ws.bcnt, wlog,
+    InitF<K> f{keys, vals, n, (1u << bits) - 1u, bits, ksym, gsa, SA, act_i, act_g, LCP, PV, PG, ws.bcnt, wlog, direct ? ISA : nullptr,
                hint && hint->on ? isa_shift(n) : 0, hint ? hint->off : 0, 0u, cb,
                seed ? seed->codes : nullptr, 65536u / (u32)bits + 1u};
     for (int i = 0; i < ksym; i++) f.lowbits |= 1u << (bits * i);
     // short texts: 512-position tiles (2 rows per wave), so more workgroups share them
     const bool small = n < INIT_SMALL_N;
-    const int rows = small ? 2 : g_init_rows;
+    const int rows = small ? 2 : direct ? 8 : g_init_rows;
     const u64 tile = (u64)WS_WAVES * rows * SAGPU_WAVE;
     const u64 tiles = (n + tile - 1) / tile;
     if (tiles > ws.tiles_cap) {
@@ -1630,19 +1652,23 @@ int group_init_t(WsScratch &ws, const K *keys, const u32 *vals, u64 n, int bits,
     else if (rows == 8) hipLaunchKernelGGL((k_init_reduce<K, 8>), dim3((unsigned)tiles), dim3(WS_THREADS), 0, s, f, tagg);
     else hipLaunchKernelGGL((k_init_reduce<K, WS_ROWS>), dim3((unsigned)tiles), dim3(WS_THREADS), 0, s, f, tagg);
     SAGPU_TRY(ws_scan(ws, tiles, (u64 *)nullptr, s));
-    SAGPU_TRY(scan_exclusive_u32(ws.scan, ws.bcnt, nb * tiles, s));
+    if (!direct) SAGPU_TRY(scan_exclusive_u32(ws.scan, ws.bcnt, nb * tiles, s));
+    const dim3 ge((unsigned)(direct ? xcd_runs(tiles) : tiles));
     ktime_begin(KI_INIT_EMIT);
-    if (rows == 2)
-        hipLaunchKernelGGL((k_init_emit<K, 2>), dim3((unsigned)tiles), dim3(WS_THREADS), 0, s, f, (const Agg *)tagg);
+    if (direct) {
+        if constexpr (sizeof(K) == 4)
+            hipLaunchKernelGGL((k_init_emit<K, 8, true>), ge, dim3(WS_THREADS), 0, s, f, (const Agg *)tagg);
+    } else if (rows == 2)
+        hipLaunchKernelGGL((k_init_emit<K, 2>), ge, dim3(WS_THREADS), 0, s, f, (const Agg *)tagg);
     else if (rows == 8)
-        hipLaunchKernelGGL((k_init_emit<K, 8>), dim3((unsigned)tiles), dim3(WS_THREADS), 0, s, f, (const Agg *)tagg);
+        hipLaunchKernelGGL((k_init_emit<K, 8>), ge, dim3(WS_THREADS), 0, s, f, (const Agg *)tagg);
     else
-        hipLaunchKernelGGL((k_init_emit<K, WS_ROWS>), dim3((unsigned)tiles), dim3(WS_THREADS), 0, s, f,
+        hipLaunchKernelGGL((k_init_emit<K, WS_ROWS>), ge, dim3(WS_THREADS), 0, s, f,
                            (const Agg *)tagg);
     // key and value read; SA, the (suffix, rank) pair, LCP mark and BWT code written
     // per position (the active-list entries are not counted)
     ktime_end(KI_INIT_EMIT, n * (sizeof(K) + 4 + 4 + 8 + (LCP ? 4 : 0) + (f.codes ? 1 : 0)));
-    (void)ISA;   // the caller scatters the pairs (launch_isa_scatter or the windowed form)
+    // (without direct the caller scatters the pairs: launch_isa_scatter or the windowed form)
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
@@ -1676,10 +1702,10 @@ void set_tile_range(int v) { g_tile_range = v; }
 
 int group_init(WsScratch &ws, const u32 *keys, const u32 *vals, u64 n, int bits, int ksym, int gsa, u32 *SA, u32 *ISA,
                u32 *act_i, u32 *act_g, u32 *LCP, u32 *PV, u32 *PG, hipStream_t s, const BwtSeed *seed,
-               const PlcpHint *hint)
+               const PlcpHint *hint, bool direct)
 {
-    return group_init_t<u32>(ws, keys, vals, n, bits, ksym, gsa, SA, ISA, act_i, act_g, LCP, PV, PG, s, seed,
-                             hint);
+    return group_init_t<u32>(ws, keys, vals, n, bits, ksym, gsa, SA, ISA, act_i, act_g, LCP, PV, PG, s, seed, hint,
+                             direct);
 }
 
 int group_init64(WsScratch &ws, const u64 *keys, const u32 *vals, u64 n, int bits, int ksym, u32 *SA, u32 *ISA,

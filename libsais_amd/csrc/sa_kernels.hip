@@ -308,12 +308,19 @@ __global__ void k_check_offsets(const uint8_t *__restrict__ T, const u32 *__rest
     }
 }
 
+// out[j] = SA[j] less its string's first position.  The slots of a string are its own
+// positions; most tiles of 4096 lie inside one string and take its offset once.
+constexpr u64 LZ_TILE = 4096;
 __global__ __launch_bounds__(256) void k_localize(const u32 *__restrict__ SA, const u32 *__restrict__ sid,
                                                   const int64_t *__restrict__ off, u64 n, u32 *__restrict__ out)
 {
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    for (u64 j = (u64)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride)
-        out[j] = SA[j] - (u32)off[sid[j]];
+    const u64 base = (u64)blockIdx.x * LZ_TILE;
+    const u64 last = n - base < LZ_TILE ? n - 1 : base + LZ_TILE - 1;
+    const u32 q0 = sid[base], q1 = sid[last];
+    const u32 o0 = (u32)off[q0];
+#pragma unroll
+    for (u64 j = base + threadIdx.x; j < base + LZ_TILE; j += 256)
+        if (j <= last) out[j] = SA[j] - (q0 == q1 ? o0 : (u32)off[sid[j]]);
 }
 
 __global__ __launch_bounds__(256) void k_batch_extract(const u32 *__restrict__ gSA, const u32 *__restrict__ gLCP,
@@ -713,7 +720,7 @@ int launch_check_offsets(const uint8_t *T, const u32 *sid, const int64_t *offset
 
 int launch_localize(const u32 *SA, const u32 *sid, const int64_t *offsets, u64 n, u32 *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_localize, dim3(grid_for(n, 256 * 8, 65535)), dim3(256), 0, s, SA, sid, offsets, n, out);
+    hipLaunchKernelGGL(k_localize, dim3((unsigned)((n + LZ_TILE - 1) / LZ_TILE)), dim3(256), 0, s, SA, sid, offsets, n, out);
     SAGPU_CHECK(hipGetLastError());
     return SAGPU_OK;
 }
