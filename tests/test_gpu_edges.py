@@ -433,3 +433,95 @@ def test_plcp_hint_sets(n):
         rc, ref = ol.sa(S, gsa=True)
         assert rc == 0 and np.array_equal(out[0][0][offs[k]:offs[k + 1]], ref), k
         assert np.array_equal(out[0][1][offs[k]:offs[k + 1]], ol.lcp(ol.plcp(S, ref, gsa=True), ref)), k
+
+
+RADIX_SIZES = [1, 2, 255, 2047, 2049, 8191, 8193, (1 << 18) - 1, (1 << 18) + 1, (1 << 20) - 1, (1 << 20) + 1,
+               (3 << 19) - 1, (3 << 19) + 1, (1 << 22) - 1, (1 << 22) + 1]
+
+
+@pytest.mark.parametrize("n", RADIX_SIZES)
+def test_radix_tile_rules(n):
+    """Sorted pairs at the sizes where tiles, the skipped wait for the histograms and
+    generated keys change; digits all alike, and key bits that end inside a digit."""
+    from tests.test_gpu_parity import fused
+    T = workloads.iid(max(n, 2), seed=n & 255, alphabet=b"ACGT")
+    print(f"[radix] n={n}", flush=True)
+    SA, U, p, P, L, f = fused(T)
+    rc, ref = ol.sa(T)
+    assert rc == 0 and np.array_equal(SA, ref)
+    rU, rp = ol.bwt(T, ref)
+    assert p == rp and np.array_equal(U, rU)
+    S = np.full(max(n, 2), 7, np.int32)   # 3-bit symbols, most digits alike
+    S[::97] = 1
+    out = np.zeros(len(S), np.int32)
+    assert la.libsais_int(S.copy(), out, len(S), 8, 0) == 0
+    assert np.array_equal(out, ol.sa_int(S))
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 1, (1 << 20) + 1, (1 << 22) - 1, (1 << 22) + 1])
+def test_round_rules(n):
+    """Rounds at the sizes where the first list's length is left on the device, the next
+    round is queued ahead and the round's end takes the big groups along: lists of small
+    groups, of big ones (pivots and not), both, and empty ones; plain and string sets."""
+    from tests.test_gpu_parity import fused
+    rng = np.random.default_rng(n)
+    words = workloads.iid(n, seed=3, alphabet=b"ab")
+    words[n // 3:n // 3 + n // 4] = words[:n // 4]
+    big = np.tile(rng.integers(97, 123, 601).astype(np.uint8), n // 601 + 1)[:n].copy()
+    runs = np.full(n, 97, np.uint8)
+    runs[::1000] = 98
+    for name, T in (("unique", rng.integers(0, 256, n).astype(np.uint8)), ("small", words), ("big", big), ("runs", runs)):
+        for gsa in (False, True):
+            if gsa:
+                T = np.where(T == 0, 1, T).astype(np.uint8)
+                T[5000::70001] = 0
+                T[-2:] = (98, 0)
+            rc, SA = ol.sa(T, gsa=gsa)
+            assert rc == 0
+            P = ol.plcp(T, SA, gsa=gsa)
+            gSA, gU, gp, gP, gL, _ = fused(T, gsa=gsa)
+            print(f"[rounds] n={n} {name} gsa={gsa}: {la.stats().rounds} rounds", flush=True)
+            assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA)), (name, gsa)
+            if not gsa:
+                U, p = ol.bwt(T, SA)
+                assert gp == p and np.array_equal(gU, U), name
+
+
+@pytest.mark.parametrize("n", [131071, 131073, 1048575, 1048577, 4194303, 4194305, 8388609, 12582913])
+def test_staged_copies(n):
+    """Host arrays of both index widths around the sizes where their copies are staged, the
+    chunk and ring sizes, in calls that carry several arrays up and down."""
+    T = workloads.iid(n, seed=n & 255, alphabet=b"ACGT")
+    rc, SA = ol.sa(T)
+    assert rc == 0
+    U, p = ol.bwt(T, SA)
+    P = ol.plcp(T, SA)
+    L = ol.lcp(P, SA)
+    for dt, sa, bwt, unbwt, plcp, lcp in (
+            (np.int32, la.libsais, la.libsais_bwt, la.libsais_unbwt, la.libsais_plcp, la.libsais_lcp),
+            (np.int64, la.libsais64, la.libsais64_bwt, la.libsais64_unbwt, la.libsais64_plcp, la.libsais64_lcp)):
+        print(f"[staged] n={n} {dt.__name__}", flush=True)
+        out, hU, A = np.zeros(n, dt), np.zeros(n, np.uint8), np.zeros(n + 1, dt)
+        assert sa(T, out, n, 0, None) == 0 and np.array_equal(out, SA)
+        assert bwt(T, hU, A, n, 0, None) == p and np.array_equal(hU, U)
+        back = np.zeros(n, np.uint8)
+        assert unbwt(hU, back, A, n, None, p) == 0 and np.array_equal(back, T)
+        S, PL = SA.astype(dt), np.zeros(n, dt)
+        assert plcp(T, S, PL, n) == 0 and np.array_equal(PL, P)
+        out[:] = 0
+        assert lcp(PL, S, out, n) == 0 and np.array_equal(out, L)
+
+
+@pytest.mark.parametrize("n", [24577, 65536, 65537, (1 << 20) + 3])
+def test_alphabet_kernel(n):
+    """Symbol counts and codes: one, two and 256 symbols, and symbols that occur once, at
+    the text's ends and around its words."""
+    from tests.test_gpu_parity import fused
+    rng = np.random.default_rng(n)
+    for name, T in (("one", np.full(n, 255, np.uint8)), ("all", rng.integers(0, 256, n).astype(np.uint8)),
+                    ("two", rng.integers(0, 2, n).astype(np.uint8) * 255)):
+        T[0], T[-1], T[n // 2] = 3, 9, 250
+        print(f"[alphabet] n={n} {name}", flush=True)
+        SA, _, _, _, _, f = fused(T)
+        rc, ref = ol.sa(T)
+        assert rc == 0 and np.array_equal(SA, ref) and np.array_equal(f, np.bincount(T, minlength=256)), name
