@@ -1026,8 +1026,17 @@ try {
 }
 
 // Whether a set's strings are short enough that reads and writes all over one string (4
-// to 9 bytes per symbol) mostly stay in an XCD's 4 MB of L2.
-bool short_strings(u64 n, u64 strings) { return strings > 1 && n / strings <= (1u << 17); }
+// to 9 bytes per symbol) often stay in an XCD's 4 MB of L2: the length of the string that
+// an average symbol lies in.  Sets of 2^29 symbols in strings of one length, SA + LCP, ms
+// with the forms for long / short strings: 4096 22.5 / 18.2, 2^15 25.4 / 21.0, 2^18 30.8 /
+// 26.6, 2^19 34.5 / 31.4, 2^20 43.7 / 44.2, 2^21 57.6 / 60.4, 2^22 69.9 / 73.8.
+constexpr double SHORT_STRING = 3 << 18;
+bool short_strings(const int64_t *off, u64 count)
+{
+    double sq = 0;
+    for (u64 q = 0; q < count; q++) sq += (double)(off[q + 1] - off[q]) * (double)(off[q + 1] - off[q]);
+    return count > 1 && sq <= SHORT_STRING * (double)off[count];
+}
 
 // The context's byte counts (kept zero) and code tables.
 int ensure_alpha(Ctx &c)
@@ -1076,7 +1085,7 @@ int byte_alphabet(Ctx &c, const uint8_t *dT, u64 n, int gsa, bool pad, u64 *freq
 int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32 *dISA, u64 *freq_out, u32 *dLCP,
              const u32 *sid = nullptr, u32 nstrings = 0, const u32 *dSym = nullptr, int sym_bits = 0,
              BwtSeed *seed = nullptr, CodeStream *cs = nullptr, PlcpHint *hint = nullptr,
-             const int64_t *h_off = nullptr)
+             const int64_t *h_off = nullptr, bool near = false)
 {
     hipStream_t s = c.stream;
     sagpu_stats &st = c.stats;
@@ -1237,8 +1246,8 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             hint->off = ksym > values ? ksym - values : 0;
         }
         SAGPU_TRY(group_init(ws, alt ? k1 : k0, alt ? v1 : v0, n, bits, ksym, 1, dSA, dISA, act_i[0], act_g[0], dLCP,
-                             alt ? k0 : k1, alt ? v0 : v1, s, nullptr, hint, short_strings(n, nstrings)));
-        if (!short_strings(n, nstrings))
+                             alt ? k0 : k1, alt ? v0 : v1, s, nullptr, hint, near));
+        if (!near)
             SAGPU_TRY(isa_from_pairs(c, sc, alt ? k0 : k1, alt ? v0 : v1, n, dISA, alt ? k1 : k0, alt ? v1 : v0));
     } else {
         // batched GSA: (string id, symbols) keys, so every group stays inside one string
@@ -1582,10 +1591,10 @@ int phi_run(Ctx &c, Scope &sc, const u32 *dSA, u64 n, u32 *dPHI)
 
 int plcp_run(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, const u32 *PHI, const u32 *ISA, const u32 *SA,
              u32 *PLCP, const u32 *marks, int sym_bytes = 1, const uint8_t *dU = nullptr,
-             const CodeStream *cs = nullptr, int hint_off = 0, u64 strings = 1)
+             const CodeStream *cs = nullptr, int hint_off = 0, bool near = false)
 {
     LcpScratch ls{};
-    ls.direct = g_plcp_pairs && short_strings(n, strings);
+    ls.direct = g_plcp_pairs && near;
     ls.queue_cap = n / 16 + 4096;
     ls.tiles_cap = n / 4096 + 2;
     GET(q, u32, ls.queue_cap);
@@ -3242,14 +3251,15 @@ extern "C" int32_t sagpu_gsa_batch32(const uint8_t *d_T, int64_t n, const int64_
         Span total(*c, F_TOTAL);
         PlcpHint hint;
         hint.on = marks && g_plcp_hint;
+        const bool near = short_strings(h_offsets, (u64)count);
         int rc = sa_build(*c, sc, dT, (u64)n, 1, gSA, ISA, nullptr, marks, sid, (u32)count, nullptr, 0, nullptr, nullptr,
-                          &hint, h_offsets);
+                          &hint, h_offsets, near);
         if (rc != SAGPU_OK) return rc;
         if (d_LCP) {
             {
                 Span sp(*c, F_PLCP);
                 SAGPU_TRY(plcp_run(*c, sc, dT, (u64)n, 1, nullptr, ISA, gSA, P, marks, 1, nullptr, nullptr,
-                                   hint.on ? hint.off : 0, (u64)count));
+                                   hint.on ? hint.off : 0, near));
             }
             Span sp(*c, F_LCP);
             SAGPU_TRY(launch_lcp_fix(P, gSA, (u64)n, (u32 *)d_LCP, s));
@@ -3396,10 +3406,11 @@ int run_batch(Ctx &c, sagpu_job **jobs, int count)
         gL = marks;
         if (!marks || !P) return SAGPU_ENOMEM;
     }
+    const bool near = short_strings(off.data(), (u64)count);
     SAGPU_TRY(sa_build(c, sc, dT, N, 1, gSA, ISA, nullptr, marks, sid, (u32)count, nullptr, 0, nullptr, nullptr, nullptr,
-                       off.data()));
+                       off.data(), near));
     if (any_l) {
-        SAGPU_TRY(plcp_run(c, sc, dT, N, 1, nullptr, ISA, gSA, P, marks, 1, nullptr, nullptr, 0, (u64)count));
+        SAGPU_TRY(plcp_run(c, sc, dT, N, 1, nullptr, ISA, gSA, P, marks, 1, nullptr, nullptr, 0, near));
         SAGPU_TRY(launch_lcp_fix(P, gSA, N, gL, s));
     }
     GET(oSA, u32, M);
