@@ -998,7 +998,8 @@ struct SegPlan {
 // False when the 64-bit sort moves no more: every segment's last tile is only half full
 // on average, which short strings pay for.  Below 2^22 keys the tables and the extra
 // launches cost what the bytes save.
-bool plan_segments(const Ctx &c, const int64_t *off, u32 count, u64 n, int kbits, SegPlan &sp)
+// tight: nor when more than 3/2 of the keys' tiles are needed.
+bool plan_segments(const Ctx &c, const int64_t *off, u32 count, u64 n, int kbits, bool tight, SegPlan &sp)
 try {
     const RadixScratch &rs = c.rs;
     if (!off || n < (1ull << 22) || n > (u64)INT32_MAX || rs.variant != RADIX_ONESWEEP || rs.bits != 8 || rs.items != 32 ||
@@ -1006,9 +1007,12 @@ try {
         return false;
     const int spare = 32 - kbits < 8 ? 32 - kbits : 8;
     const u32 most = 1u << spare;
+    sp.tiles.clear();
+    sp.start.clear();
     sp.end_bit = kbits + (count < most ? bits_for(count - 1) : spare);
     const u64 pass32 = (u64)(sp.end_bit + 7) / 8 * SEG_TILE_KEYS * 16, all64 = (u64)(32 + bits_for(count - 1) + 7) / 8 * n * 24;
-    const u64 max_tiles = all64 / pass32;
+    u64 max_tiles = all64 / pass32;
+    if (tight && n / 2 * 3 / SEG_TILE_KEYS < max_tiles) max_tiles = n / 2 * 3 / SEG_TILE_KEYS;
     if ((u64)(count + most - 1) / most > max_tiles) return false;
     sp.local.resize(count);
     for (u32 q0 = 0; q0 < count; q0 += most) {
@@ -1118,7 +1122,18 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     const bool wide = n > g_wide_from;
     SAGPU_TRY(ensure_radix_scratch(c, sc, n));
     SegPlan sp_plan;
-    const bool by_segment = sid && plan_segments(c, h_off, nstrings, n, ksym * bits, sp_plan);
+    bool by_segment = false;
+    // Short strings need fewer symbols, whose bits tell more strings of a segment apart:
+    // the most symbols that need at most 3/2 of the keys' tiles, else the most that pay.
+    // 2^28 symbols, SA + LCP, ms with all symbols (or by (string, symbols) where those do
+    // not pay) / by this rule: strings of 128 23.4 / 11.6, 1000 21.8 / 10.4, 1700 12.3 /
+    // 10.7, 2100 11.5 / 10.8, 5000 11.4 / 11.2, 9000 the same (at 9/8 10.7 / 11.4).
+    for (int tight = 1; sid && !by_segment && tight >= 0; tight--)
+        for (int k = ksym; !by_segment && 2 * k > ksym; k--)
+            if (plan_segments(c, h_off, nstrings, n, k * bits, tight, sp_plan)) {
+                by_segment = true;
+                ksym = k;
+            }
     GET(kA, u32, sid && !by_segment ? 4 * n : 2 * n);
     GET(vA, u32, 2 * n);
     GET(aA, u32, 2 * n);

@@ -311,8 +311,9 @@ SEG_KEYS = 16384   # keys of a tile of a segmented sort
 
 def _string_sets():
     """(name, string lengths, symbols): sets of at least 2^22 symbols, whose strings are
-    sorted four to a segment (5 codes: 30-bit keys), one (16 and 256 codes: no bits left)
-    and sixteen (100 codes); lengths around whole tiles, one string, a few long ones."""
+    sorted four to a segment (5 codes: 30-bit keys), one (16 and 256 codes: no bits left),
+    sixteen (100 codes) and more with fewer symbols; lengths around whole tiles, one string,
+    a few long ones."""
     rng = np.random.default_rng(7)
     n = 1 << 22
     edges = [SEG_KEYS - 1, SEG_KEYS, SEG_KEYS + 1, 4 * SEG_KEYS, 2, 3, 65]
@@ -325,7 +326,9 @@ def _string_sets():
     yield "mixed, 4 bits", list(mixed) + [3], 15
     yield "mixed, 7 bits", list(mixed) + [5, 2], 99
     yield "alike", [40000] * 106, 4
-    yield "short", [90] * (n // 90 + 1), 4   # too short: the 64-bit sort
+    yield "short", [90] * (n // 90 + 1), 4   # fewer symbols, 256 strings to a segment
+    yield "reads", list(rng.integers(30, 400, n // 200)), 4
+    yield "tiny", [4] * (n // 4 + 1), 4      # too short: the 64-bit sort
 
 
 @pytest.mark.parametrize("name,lengths,sigma", list(_string_sets()), ids=lambda v: v if isinstance(v, str) else "")
