@@ -528,3 +528,25 @@ def test_alphabet_kernel(n):
         SA, _, _, _, _, f = fused(T)
         rc, ref = ol.sa(T)
         assert rc == 0 and np.array_equal(SA, ref) and np.array_equal(f, np.bincount(T, minlength=256)), name
+
+
+@pytest.mark.parametrize("n", [1048577, 6000001, 8388608])
+def test_concurrent_staged_copies(n):
+    """Downloads of several calls at once, which take turns on the bus a half ring at a
+    time: both index widths, lengths around the half."""
+    from concurrent.futures import ThreadPoolExecutor
+    T = [workloads.iid(n, seed=k, alphabet=b"ACGT") for k in range(2)]
+    ref = [ol.sa(t)[1] for t in T]
+
+    def one(k):
+        dt, sa = (np.int32, la.libsais) if k % 2 else (np.int64, la.libsais64)
+        out = np.zeros(n, dt)
+        for _ in range(3):
+            out[:] = 0
+            if sa(T[k // 2 % 2], out, n, 0, None) != 0 or not np.array_equal(out, ref[k // 2 % 2]):
+                return False
+        return True
+
+    print(f"[concurrent copies] n={n}", flush=True)
+    with ThreadPoolExecutor(6) as ex:
+        assert all(ex.map(one, range(6)))
