@@ -289,16 +289,20 @@ class CopyPool {
     }
 
   public:
-    // Opens a job (no parts yet) for up to `threads` threads.
+    // Opens a job (no parts yet) for up to `threads` threads; fewer where the system gives
+    // no more (the owner takes parts, too).
     void begin(Job &j, int threads)
     {
         std::lock_guard<std::mutex> lk(m);
-        while (workers < threads - 1) {
-            std::thread([this] { loop(); }).detach();
-            workers++;
-        }
         open.push_back(&j);
         opens++;
+        try {
+            while (workers < threads - 1) {
+                std::thread([this] { loop(); }).detach();
+                workers++;
+            }
+        } catch (const std::exception &) {
+        }
     }
     int jobs() const { return opens.load(); }
     void end(Job &j)   // waits for every part granted, and for the workers to leave the job
@@ -836,11 +840,19 @@ int ensure_radix_scratch(Ctx &c, Scope &sc, u64 n)
 {
     u64 tiles = (n + RS_TILE - 1) / RS_TILE + 1;
     if (!c.rs.hist) {
-        c.rs.hist = (u64 *)c.pool.get(2 * RADIX_HIST_WORDS * sizeof(u64));
-        c.rs.tile_ctr = (u32 *)c.pool.get(64 * sizeof(u32));
-        if (!c.rs.hist || !c.rs.tile_ctr) return SAGPU_ENOMEM;
+        if (!c.rs.tile_ctr) c.rs.tile_ctr = (u32 *)c.pool.get(64 * sizeof(u32));
+        u64 *hist = (u64 *)c.pool.get(2 * RADIX_HIST_WORDS * sizeof(u64));
+        if (!hist || !c.rs.tile_ctr) {
+            if (hist) c.pool.put(hist);
+            return SAGPU_ENOMEM;
+        }
         // (every sort leaves its counts cleared)
-        SAGPU_TRY(launch_fill_u64(c.rs.hist, RADIX_HIST_WORDS, 0, c.stream));
+        const int rc = launch_fill_u64(hist, RADIX_HIST_WORDS, 0, c.stream);
+        if (rc != SAGPU_OK) {
+            c.pool.put(hist);
+            return rc;
+        }
+        c.rs.hist = hist;
     }
     if (c.rs.counts_cap < tiles * 256) {
         if (c.rs.counts) c.pool.put(c.rs.counts);
@@ -1054,9 +1066,15 @@ bool short_strings(const int64_t *off, u64 count)
 int ensure_alpha(Ctx &c)
 {
     if (c.alpha) return SAGPU_OK;
-    c.alpha = (u64 *)c.pool.get(264 * sizeof(u64) + 512);
-    if (!c.alpha) return SAGPU_ENOMEM;
-    return launch_fill_u64(c.alpha, 264, 0, c.stream);
+    u64 *alpha = (u64 *)c.pool.get(264 * sizeof(u64) + 512);
+    if (!alpha) return SAGPU_ENOMEM;
+    const int rc = launch_fill_u64(alpha, 264, 0, c.stream);
+    if (rc != SAGPU_OK) {
+        c.pool.put(alpha);
+        return rc;
+    }
+    c.alpha = alpha;
+    return SAGPU_OK;
 }
 
 // Byte alphabet of a text: freq (optional, host), the GSA validity test, and the
@@ -1678,9 +1696,13 @@ bool xs_ready(Ctx &c, u64 bytes, u64 least = XS_MIN)
             return false;
         }
     if (!c.xs_ctr) {
-        c.xs_ctr = (u32 *)c.pool.get(XP_CHUNKS * sizeof(u32));
-        if (!c.xs_ctr) return false;
-        if (launch_fill_u32(c.xs_ctr, XP_CHUNKS, 0, c.stream) != SAGPU_OK) return false;
+        u32 *ctr = (u32 *)c.pool.get(XP_CHUNKS * sizeof(u32));
+        if (!ctr) return false;
+        if (launch_fill_u32(ctr, XP_CHUNKS, 0, c.stream) != SAGPU_OK) {
+            c.pool.put(ctr);
+            return false;
+        }
+        c.xs_ctr = ctr;
     }
     // the ring, then the flags of a download's chunks
     g_device_allocs++;
@@ -1766,7 +1788,7 @@ struct XsGuard {
 // caller may then overwrite it (outputs that alias inputs); the DMA of the last
 // chunks may still be running.
 int h2d_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool narrow)
-{
+try {
     CopyPool::Job j(bytes / xs_part() + bytes / xs_chunk(0) + 2);   // (every chunk may end in a short part)
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
@@ -1801,6 +1823,8 @@ int h2d_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool narrow)
     SAGPU_TRY(xs_mark(c));
     guard.fine = true;
     return SAGPU_OK;
+} catch (const std::bad_alloc &) {
+    return SAGPU_ENOMEM;
 }
 
 // Copies device memory into the pinned ring, chunk after chunk, each divided over all
@@ -1864,7 +1888,7 @@ int d2h_shared(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, 
 // bytes (src aligned to 16); widen: u32 entries become int64.  Returns with every byte
 // in dst.
 int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool widen)
-{
+try {
     CopyPool::Job j(bytes / xs_part() + bytes / xs_chunk(0) + 2);
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
@@ -1923,6 +1947,8 @@ int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool widen)
     copies().wait(j, j.granted.load());
     guard.fine = true;
     return SAGPU_OK;
+} catch (const std::bad_alloc &) {
+    return SAGPU_ENOMEM;
 }
 
 int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
