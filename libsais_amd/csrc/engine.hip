@@ -1309,8 +1309,10 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     u64 a = 0;
     // Texts below LAZY_N skip the wait for the first list's length: the first round is
     // launched for n entries and reads the length from the device (its kernels stop at
-    // the list's end); the host learns it with the round's report.
-    const bool lazy_a = n < LAZY_N;
+    // the list's end); the host learns it with the round's report.  The survivor segments
+    // are then sized for n entries (12 B each; 1 MiB of ACGT: 65 MB in all instead of 49),
+    // so a call under a memory limit, which may just hold the list, waits.
+    const bool lazy_a = n < LAZY_N && !g_mem_limit.load();
     if (lazy_a) {
         a = n;
     } else {

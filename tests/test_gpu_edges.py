@@ -550,3 +550,26 @@ def test_concurrent_staged_copies(n):
     print(f"[concurrent copies] n={n}", flush=True)
     with ThreadPoolExecutor(6) as ex:
         assert all(ex.map(one, range(6)))
+
+
+@pytest.mark.parametrize("n", [30000, 1 << 20, (1 << 22) - 1])
+def test_build_under_a_memory_limit(n):
+    """Under a limit, texts below 2^22 wait for the first list's length: the same results."""
+    print(f"[limit] n={n}", flush=True)
+    T = workloads.iid_acgt(n, seed=n)
+    lib = la.load()
+    SA0 = np.zeros(n, np.int32)
+    assert la.libsais(T, SA0, n, 0, None) == 0, la.last_error()
+    rc, ref = ol.sa(T)
+    assert rc == 0 and np.array_equal(SA0, ref)
+    try:
+        lib.sagpu_set_memory_limit(1 << 36)   # (the context keeps scratch of earlier calls)
+        SA = np.zeros(n, np.int32)
+        assert la.libsais(T, SA, n, 0, None) == 0, la.last_error()
+        U = np.zeros(n, np.uint8)
+        p = la.libsais_bwt(T, U, np.zeros(n, np.int32), n, 0, None)
+    finally:
+        lib.sagpu_set_memory_limit(0)
+    U_r, p_r = ol.bwt(T, ref)
+    assert np.array_equal(SA, ref)
+    assert p == p_r and np.array_equal(U, U_r)
