@@ -1,0 +1,228 @@
+// copy_pool.h -- host copies split over worker threads, and the shape of the staged copies
+// that use them (engine.hip).  Plain C++ without GPU code, so host programs can include it
+// by itself.
+#pragma once
+
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <cstdint>
+#include <cstring>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+typedef unsigned long long u64;
+typedef uint32_t u32;
+
+namespace {
+
+// Copies split over worker threads.  Workers are detached and live until the process
+// ends; a forked child starts a new pool.  Parts are small (128 KiB take a thread about
+// 40 us while 16 of them share the memory), so that the first ones are soon ready for
+// the DMA; they are taken and reported without a lock, and a thread looks for the next
+// one for some time before it sleeps (waking one takes longer than a part).
+class CopyPool {
+  public:
+    struct Part {
+        uint8_t *d;
+        const uint8_t *s;
+        u64 len;     // bytes written
+        int conv;    // 0: bytes; 1: int64 narrowed to u32; 2: u32 widened to int64
+    };
+    // At most `most` parts, granted by the owner in order as they become ready, taken in
+    // that order, and done in any.
+    struct Job {
+        explicit Job(u64 most) : part(most), done(new std::atomic<char>[most])
+        {
+            for (u64 k = 0; k < most; k++) done[k].store(0, std::memory_order_relaxed);
+        }
+        std::vector<Part> part;
+        std::unique_ptr<std::atomic<char>[]> done;
+        std::atomic<int> granted{0}, next{0}, users{0};
+        std::atomic<bool> closing{false};
+        int prefix = 0;   // the owner's: parts [0, prefix) are done
+    };
+
+  private:
+    std::mutex m;   // open, workers, sleeping
+    std::condition_variable work_cv;
+    std::vector<Job *> open;
+    std::atomic<int> sleeping{0};
+    std::atomic<u32> epoch{0};   // grants so far, of all jobs
+    std::atomic<int> opens{0};   // jobs in `open`
+    int workers = 0;
+
+    static void run(const Part &p)
+    {
+        if (p.conv == 1) {
+            const int64_t *s = (const int64_t *)p.s;
+            u32 *d = (u32 *)p.d;
+            for (u64 i = 0; i < p.len / 4; i++) d[i] = (u32)s[i];
+        } else if (p.conv == 2) {
+            const u32 *s = (const u32 *)p.s;
+            int64_t *d = (int64_t *)p.d;
+            for (u64 i = 0; i < p.len / 8; i++) d[i] = (int64_t)s[i];
+        } else {
+            memcpy(p.d, p.s, p.len);
+        }
+    }
+    // Takes and runs one part, if there is one.
+    static bool take(Job &j)
+    {
+        int k = j.next.load();
+        while (k < j.granted.load())
+            if (j.next.compare_exchange_weak(k, k + 1)) {
+                run(j.part[k]);
+                j.done[k].store(1, std::memory_order_release);
+                return true;
+            }
+        return false;
+    }
+    Job *find()   // m is held: of the jobs with parts to take, one with the fewest threads
+    {
+        Job *best = nullptr;
+        for (Job *j : open)
+            if (j->next.load() < j->granted.load() && (!best || j->users.load() < best->users.load())) best = j;
+        return best;
+    }
+    void loop()
+    {
+        std::unique_lock<std::mutex> lk(m);
+        for (;;) {
+            Job *j = find();
+            if (!j) {   // look out for a grant for some 50 us, then sleep
+                const u32 seen = epoch.load();
+                lk.unlock();
+                for (int k = 0; k < 2000 && epoch.load() == seen; k++) __builtin_ia32_pause();
+                lk.lock();
+                if (epoch.load() != seen) continue;
+                sleeping++;
+                work_cv.wait(lk, [&] { return (j = find()) != nullptr; });
+                sleeping--;
+            }
+            j->users++;
+            lk.unlock();
+            // (with other jobs open, back to look there at once)
+            for (int idle = 0; idle < (opens.load() > 1 ? 20 : 2000) && !j->closing.load(); idle++) {
+                if (take(*j)) idle = 0;
+                else __builtin_ia32_pause();
+            }
+            j->users--;
+            lk.lock();
+        }
+    }
+
+  public:
+    // Opens a job (no parts yet) for up to `threads` threads; fewer where the system gives
+    // no more (the owner takes parts, too).
+    void begin(Job &j, int threads)
+    {
+        std::lock_guard<std::mutex> lk(m);
+        open.push_back(&j);
+        opens++;
+        try {
+            while (workers < threads - 1) {
+                std::thread([this] { loop(); }).detach();
+                workers++;
+            }
+        } catch (const std::exception &) {
+        }
+    }
+    int jobs() const { return opens.load(); }
+    void end(Job &j)   // waits for every part granted, and for the workers to leave the job
+    {
+        wait(j, j.granted.load());
+        j.closing.store(true);
+        {
+            std::lock_guard<std::mutex> lk(m);
+            open.erase(std::find(open.begin(), open.end(), &j));
+            opens--;
+        }
+        while (j.users.load() > 0) __builtin_ia32_pause();
+    }
+    // Grants a stretch in parts of `per` written bytes.  False, and nothing granted, when
+    // the job has no room for them.
+    bool grant(Job &j, Part all, u64 per)
+    {
+        const u64 sper = all.conv == 1 ? 2 * per : all.conv == 2 ? per / 2 : per;
+        int g = j.granted.load();
+        if (parts_of(all.len, per) > j.part.size() - (u64)g) return false;
+        for (; all.len; all.d += per, all.s += sper) {
+            Part p = all;
+            p.len = all.len < per ? all.len : per;
+            all.len -= p.len;
+            j.part[g++] = p;
+        }
+        j.granted.store(g);
+        epoch++;
+        if (sleeping.load() > 0) {
+            { std::lock_guard<std::mutex> lk(m); }
+            work_cv.notify_all();
+        }
+        return true;
+    }
+    // Waits until parts [0, upto) are done; takes parts itself when that is not soon.
+    void wait(Job &j, int upto)
+    {
+        for (int idle = 0; j.prefix < upto; idle++) {
+            if (j.done[j.prefix].load(std::memory_order_acquire)) {
+                j.prefix++;
+                idle = 0;
+            } else if (idle < 2000 && workers > 0) {
+                __builtin_ia32_pause();
+            } else if (!take(j)) {
+                std::this_thread::yield();
+            }
+        }
+    }
+    static u64 parts_of(u64 len, u64 per) { return (len + per - 1) / per; }
+    void copy(void *d, const void *s, u64 len, int threads)
+    {
+        if (threads <= 1 || len < (1u << 20)) {
+            memcpy(d, s, len);
+            return;
+        }
+        // parts of whole pages, at least 1 MiB
+        u64 per = (len + threads - 1) / threads;
+        per = per < (1u << 20) ? (1u << 20) : (per + 4095) & ~(u64)4095;
+        Job j(parts_of(len, per));
+        begin(j, threads);
+        if (!grant(j, Part{(uint8_t *)d, (const uint8_t *)s, len, 0}, per)) memcpy(d, s, len);
+        end(j);
+    }
+    void lock() { m.lock(); }
+    void unlock() { m.unlock(); }
+};
+
+// The shape of one staged copy: settled when it starts, since the options may change while
+// it runs.  Sizes are device bytes where nothing else is said; conv is Part::conv.
+struct CopyForm {
+    bool tiny;   // 64 KiB chunks of 16 KiB parts, whatever the size (host_staging 2)
+    int conv;
+
+    u64 written(u64 bytes) const { return conv == 2 ? 2 * bytes : bytes; }   // by the host copies
+    u64 taken(u64 bytes) const { return conv == 1 ? 2 * bytes : bytes; }     // from the caller's array
+    // Upload chunk k.  The first ones are small, so that DMA and host copies overlap from
+    // early on; later ones keep the DMA's start-up small beside it (a 4 MiB chunk takes 73 us).
+    u64 up_chunk(int k) const
+    {
+        return tiny ? 64u << 10 : k < 4 ? (512ull << 10) << k : k < 8 ? 4ull << 20 : 8ull << 20;
+    }
+    // Chunk of a download of `bytes`.
+    u64 down_chunk(u64 bytes) const { return tiny ? 64u << 10 : bytes < (32u << 20) ? 1u << 20 : 4u << 20; }
+    // Written bytes of a part; of a download that shares the bus, parts of a huge page.
+    u64 part(bool shared = false) const
+    {
+        return shared && !tiny ? 2u << 20 : written(tiny ? 16u << 10 : 128u << 10);
+    }
+    // Parts that a copy of `bytes` may be granted: a short one at the end of every stretch,
+    // and none of the stretches but the last is shorter than the first upload chunk.
+    u64 room(u64 bytes) const
+    {
+        return CopyPool::parts_of(written(bytes), part()) + CopyPool::parts_of(bytes, up_chunk(0));
+    }
+};
+
+} // namespace

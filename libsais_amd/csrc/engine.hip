@@ -7,6 +7,7 @@
 //       -> regroup, retire singletons, compact the active list   until none left
 //   ->  optional BWT gather, PLCP (irreducible + prefix max), LCP gather.
 #include "engine.h"
+#include "copy_pool.h"
 #include "../../include/sagpu.h"
 
 #include <algorithm>
@@ -182,7 +183,7 @@ constexpr int XS_EVENTS = 8, XS_AHEAD = 24;   // upload chunks whose host copies
 enum { XS_TODO = -1, XS_QUEUED = -2 };        // a region's DMA is not queued / queued, no event after it yet
 // 1: copies of at least XS_MIN bytes staged (default); 0: every copy direct; 2: every
 // copy staged in 64 KiB chunks (exercises the chunk logic on small inputs)
-int g_host_staging = 1;
+std::atomic<int> g_host_staging{1};
 int g_copy_threads = 0;   // 0: min(16, hardware threads)
 
 int copy_threads()
@@ -191,181 +192,6 @@ int copy_threads()
     const unsigned hw = std::thread::hardware_concurrency();
     return hw == 0 ? 4 : (int)(hw < 16 ? hw : 16);
 }
-
-// Copies split over worker threads.  Workers are detached and live until the process
-// ends; a forked child starts a new pool.  Parts are small (128 KiB take a thread about
-// 40 us while 16 of them share the memory), so that the first ones are soon ready for
-// the DMA; they are taken and reported without a lock, and a thread looks for the next
-// one for some time before it sleeps (waking one takes longer than a part).
-class CopyPool {
-  public:
-    struct Part {
-        uint8_t *d;
-        const uint8_t *s;
-        u64 len;     // bytes written
-        int conv;    // 0: bytes; 1: int64 narrowed to u32; 2: u32 widened to int64
-    };
-    // At most `most` parts, granted by the owner in order as they become ready, taken in
-    // that order, and done in any.
-    struct Job {
-        explicit Job(u64 most) : part(most), done(new std::atomic<char>[most])
-        {
-            for (u64 k = 0; k < most; k++) done[k].store(0, std::memory_order_relaxed);
-        }
-        std::vector<Part> part;
-        std::unique_ptr<std::atomic<char>[]> done;
-        std::atomic<int> granted{0}, next{0}, users{0};
-        std::atomic<bool> closing{false};
-        int prefix = 0;   // the owner's: parts [0, prefix) are done
-    };
-
-  private:
-    std::mutex m;   // open, workers, sleeping
-    std::condition_variable work_cv;
-    std::vector<Job *> open;
-    std::atomic<int> sleeping{0};
-    std::atomic<u32> epoch{0};   // grants so far, of all jobs
-    std::atomic<int> opens{0};   // jobs in `open`
-    int workers = 0;
-
-    static void run(const Part &p)
-    {
-        if (p.conv == 1) {
-            const int64_t *s = (const int64_t *)p.s;
-            u32 *d = (u32 *)p.d;
-            for (u64 i = 0; i < p.len / 4; i++) d[i] = (u32)s[i];
-        } else if (p.conv == 2) {
-            const u32 *s = (const u32 *)p.s;
-            int64_t *d = (int64_t *)p.d;
-            for (u64 i = 0; i < p.len / 8; i++) d[i] = (int64_t)s[i];
-        } else {
-            memcpy(p.d, p.s, p.len);
-        }
-    }
-    // Takes and runs one part, if there is one.
-    static bool take(Job &j)
-    {
-        int k = j.next.load();
-        while (k < j.granted.load())
-            if (j.next.compare_exchange_weak(k, k + 1)) {
-                run(j.part[k]);
-                j.done[k].store(1, std::memory_order_release);
-                return true;
-            }
-        return false;
-    }
-    Job *find()   // m is held: of the jobs with parts to take, one with the fewest threads
-    {
-        Job *best = nullptr;
-        for (Job *j : open)
-            if (j->next.load() < j->granted.load() && (!best || j->users.load() < best->users.load())) best = j;
-        return best;
-    }
-    void loop()
-    {
-        std::unique_lock<std::mutex> lk(m);
-        for (;;) {
-            Job *j = find();
-            if (!j) {   // look out for a grant for some 50 us, then sleep
-                const u32 seen = epoch.load();
-                lk.unlock();
-                for (int k = 0; k < 2000 && epoch.load() == seen; k++) __builtin_ia32_pause();
-                lk.lock();
-                if (epoch.load() != seen) continue;
-                sleeping++;
-                work_cv.wait(lk, [&] { return (j = find()) != nullptr; });
-                sleeping--;
-            }
-            j->users++;
-            lk.unlock();
-            // (with other jobs open, back to look there at once)
-            for (int idle = 0; idle < (opens.load() > 1 ? 20 : 2000) && !j->closing.load(); idle++) {
-                if (take(*j)) idle = 0;
-                else __builtin_ia32_pause();
-            }
-            j->users--;
-            lk.lock();
-        }
-    }
-
-  public:
-    // Opens a job (no parts yet) for up to `threads` threads; fewer where the system gives
-    // no more (the owner takes parts, too).
-    void begin(Job &j, int threads)
-    {
-        std::lock_guard<std::mutex> lk(m);
-        open.push_back(&j);
-        opens++;
-        try {
-            while (workers < threads - 1) {
-                std::thread([this] { loop(); }).detach();
-                workers++;
-            }
-        } catch (const std::exception &) {
-        }
-    }
-    int jobs() const { return opens.load(); }
-    void end(Job &j)   // waits for every part granted, and for the workers to leave the job
-    {
-        wait(j, j.granted.load());
-        j.closing.store(true);
-        {
-            std::lock_guard<std::mutex> lk(m);
-            open.erase(std::find(open.begin(), open.end(), &j));
-            opens--;
-        }
-        while (j.users.load() > 0) __builtin_ia32_pause();
-    }
-    // Grants a stretch in parts of `per` written bytes.
-    void grant(Job &j, Part all, u64 per)
-    {
-        const u64 sper = all.conv == 1 ? 2 * per : all.conv == 2 ? per / 2 : per;
-        int g = j.granted.load();
-        for (; all.len; all.d += per, all.s += sper) {
-            Part p = all;
-            p.len = all.len < per ? all.len : per;
-            all.len -= p.len;
-            j.part[g++] = p;
-        }
-        j.granted.store(g);
-        epoch++;
-        if (sleeping.load() > 0) {
-            { std::lock_guard<std::mutex> lk(m); }
-            work_cv.notify_all();
-        }
-    }
-    // Waits until parts [0, upto) are done; takes parts itself when that is not soon.
-    void wait(Job &j, int upto)
-    {
-        for (int idle = 0; j.prefix < upto; idle++) {
-            if (j.done[j.prefix].load(std::memory_order_acquire)) {
-                j.prefix++;
-                idle = 0;
-            } else if (idle < 2000 && workers > 0) {
-                __builtin_ia32_pause();
-            } else if (!take(j)) {
-                std::this_thread::yield();
-            }
-        }
-    }
-    static u64 parts_of(u64 len, u64 per) { return (len + per - 1) / per; }
-    void copy(void *d, const void *s, u64 len, int threads)
-    {
-        if (threads <= 1 || len < (1u << 20)) {
-            memcpy(d, s, len);
-            return;
-        }
-        // parts of whole pages, at least 1 MiB
-        u64 per = (len + threads - 1) / threads;
-        per = per < (1u << 20) ? (1u << 20) : (per + 4095) & ~(u64)4095;
-        Job j(parts_of(len, per));
-        begin(j, threads);
-        grant(j, Part{(uint8_t *)d, (const uint8_t *)s, len, 0}, per);
-        end(j);
-    }
-    void lock() { m.lock(); }
-    void unlock() { m.unlock(); }
-};
 
 CopyPool *g_copies = nullptr;
 std::once_flag g_copies_once;
@@ -1682,10 +1508,12 @@ constexpr u64 XS_MIN = 4u << 20, XS_MIN_INDEX64 = 1u << 20;
 // 128 49 GB/s; a plain copy 56.
 constexpr u32 XP_CHUNKS = 64, XP_WGS = 64;
 
-// Whether a copy of this size is staged (and pinned memory is available).
-bool xs_ready(Ctx &c, u64 bytes, u64 least = XS_MIN)
+// Whether a copy of this size is staged (and pinned memory is available), and its form.
+bool xs_ready(Ctx &c, u64 bytes, CopyForm *f, u64 least = XS_MIN)
 {
-    if (g_host_staging == 0 || (g_host_staging == 1 && bytes < least)) return false;
+    const int mode = g_host_staging.load();
+    if (mode == 0 || (mode == 1 && bytes < least)) return false;
+    f->tiny = mode == 2;
     if (c.xs) return true;
     for (auto &e : c.xs_ev)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
@@ -1716,12 +1544,6 @@ bool xs_ready(Ctx &c, u64 bytes, u64 least = XS_MIN)
     memset(c.xs + XS_RING, 0, XP_CHUNKS * sizeof(u32));
     return true;
 }
-
-// Bytes of upload chunk k, and of the parts its host copy is split into.  The first
-// chunks are small, so that DMA and host copies overlap from early on; later ones keep
-// the DMA's start-up small beside it (a 4 MiB chunk takes 73 us).
-u64 xs_chunk(int k) { return g_host_staging == 2 ? 64u << 10 : k < 4 ? (512ull << 10) << k : k < 8 ? 4ull << 20 : 8ull << 20; }
-u64 xs_part() { return g_host_staging == 2 ? 16u << 10 : 128u << 10; }
 
 // An event after everything queued so far: it frees every region queued before it.
 int xs_mark(Ctx &c)
@@ -1785,13 +1607,22 @@ struct XsGuard {
     }
 };
 
-// Host to device on the context's stream: `bytes` device bytes; narrow: src holds int64
+// A stretch of a copy's host side for the pool: `bytes` device bytes, from the s-th byte of
+// the source and to the d-th of the destination on.
+int xs_grant(CopyPool::Job &j, const CopyForm &f, uint8_t *d, const uint8_t *s, u64 bytes, bool shared = false)
+{
+    if (copies().grant(j, {d, s, f.written(bytes), f.conv}, f.part(shared))) return SAGPU_OK;
+    sagpu_set_error("host copy in more parts than planned", __FILE__, __LINE__);
+    return SAGPU_EDEVICE;
+}
+
+// Host to device on the context's stream: `bytes` device bytes; f.conv 1: src holds int64
 // entries that become u32.  Returns once every byte of src has been read, so the
 // caller may then overwrite it (outputs that alias inputs); the DMA of the last
 // chunks may still be running.
-int h2d_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool narrow)
+int h2d_staged(Ctx &c, void *dst, const void *src, u64 bytes, const CopyForm &f)
 try {
-    CopyPool::Job j(bytes / xs_part() + bytes / xs_chunk(0) + 2);   // (every chunk may end in a short part)
+    CopyPool::Job j(f.room(bytes));
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
     // an idle ring starts over: its first pages are the ones the CPU has mapped and cached
@@ -1804,13 +1635,12 @@ try {
     for (int k = 0; given < bytes || !ahead.empty();) {
         // regions and host copies of the chunks ahead of the DMA
         while (given < bytes && (int)ahead.size() < XS_AHEAD) {
-            const u64 len = bytes - given < xs_chunk(k) ? bytes - given : xs_chunk(k);
+            const u64 len = bytes - given < f.up_chunk(k) ? bytes - given : f.up_chunk(k);
             u64 at = 0;
             bool ok;
             SAGPU_TRY(xs_take(c, len, ahead.empty(), &at, &ok));
             if (!ok) break;
-            copies().grant(j, {c.xs + at, (const uint8_t *)src + (narrow ? 2 : 1) * given, len, narrow ? 1 : 0},
-                           xs_part());
+            SAGPU_TRY(xs_grant(j, f, c.xs + at, (const uint8_t *)src + f.taken(given), len));
             ahead.push_back({given, j.granted.load()});
             given += len;
             k++;
@@ -1860,7 +1690,7 @@ __global__ __launch_bounds__(256) void k_push(const uint8_t *__restrict__ src, u
 // once the bus is busy anyway, and kernels that push chunks compete with the others'
 // kernels for the CUs: 300 served jobs (2.1 GB of text) at once took 280 ms, 241 this
 // way; into pages not touched before 470 and 336.
-int d2h_shared(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, bool widen)
+int d2h_shared(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, const CopyForm &f)
 {
     const u64 half = XS_RING / 2, nb = (bytes + half - 1) / half;
     std::vector<int> upto(nb + 1, 0);   // parts through the end of every half
@@ -1874,8 +1704,7 @@ int d2h_shared(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, 
     for (u64 b = 0; b < nb; b++) {
         const u64 off = b * half, len = bytes - off < half ? bytes - off : half;
         SAGPU_CHECK(hipEventSynchronize(c.xs_down[b & 1]));
-        copies().grant(j, {(uint8_t *)dst + (widen ? 2 : 1) * off, c.xs + (b & 1) * half, widen ? 2 * len : len,
-                           widen ? 2 : 0}, g_host_staging == 2 ? xs_part() : 2u << 20);
+        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + (b & 1) * half, len, true));
         upto[b + 1] = j.granted.load();
         if (b + 2 < nb) {
             copies().wait(j, upto[b + 1]);
@@ -1887,24 +1716,23 @@ int d2h_shared(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, 
 }
 
 // Device to host after the work already queued on the context's stream: `bytes` device
-// bytes (src aligned to 16); widen: u32 entries become int64.  Returns with every byte
+// bytes (src aligned to 16); f.conv 2: u32 entries become int64.  Returns with every byte
 // in dst.
-int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, bool widen)
+int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, const CopyForm &f)
 try {
-    CopyPool::Job j(bytes / xs_part() + bytes / xs_chunk(0) + 2);
+    CopyPool::Job j(f.room(bytes));
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
     if (copies().jobs() > 1) {
-        SAGPU_TRY(d2h_shared(c, j, dst, src, bytes, widen));
+        SAGPU_TRY(d2h_shared(c, j, dst, src, bytes, f));
         guard.fine = true;
         return SAGPU_OK;
     }
     volatile u32 *flags = (volatile u32 *)(c.xs + XS_RING);
     // two halves of the ring, a kernel each; a half is filled again once it is drained
-    const u64 half = XS_RING / 2, chunk = g_host_staging == 2 ? 64u << 10 : bytes < (32u << 20) ? 1u << 20 : 4u << 20;
+    const u64 half = XS_RING / 2, chunk = f.down_chunk(bytes);
     const u64 batch = chunk * (XP_CHUNKS / 2) < half ? chunk * (XP_CHUNKS / 2) : half;
     const u64 nb = (bytes + batch - 1) / batch;
-    const u64 per = widen ? 2 * xs_part() : xs_part();
     std::vector<int> upto(nb + 1, 0);   // parts through the end of every batch
     u32 ticks[2] = {0, 0};
     auto launch = [&](u64 b) -> int {
@@ -1936,8 +1764,7 @@ try {
             }
             std::atomic_thread_fence(std::memory_order_acquire);
             const u64 l = len - o < chunk ? len - o : chunk;
-            copies().grant(j, {(uint8_t *)dst + (widen ? 2 : 1) * (off + o), c.xs + side * half + o, widen ? 2 * l : l,
-                               widen ? 2 : 0}, per);
+            SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off + o), c.xs + side * half + o, l));
         }
         upto[b + 1] = j.granted.load();
         // the half of batch b + 1 is being filled or drained; batch b + 2 needs this one
@@ -1956,7 +1783,8 @@ try {
 int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    if (xs_ready(c, bytes)) return h2d_staged(c, dst, src, bytes, false);
+    CopyForm f{false, 0};
+    if (xs_ready(c, bytes, &f)) return h2d_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
     return SAGPU_OK;
 }
@@ -1965,7 +1793,8 @@ int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 int d2h(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    if ((uintptr_t)src % 16 == 0 && xs_ready(c, bytes)) return d2h_staged(c, dst, src, bytes, false);
+    CopyForm f{false, 0};
+    if ((uintptr_t)src % 16 == 0 && xs_ready(c, bytes, &f)) return d2h_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
     return SAGPU_OK;
 }
@@ -2187,10 +2016,11 @@ unsigned grid_n(u64 n)
 // Download u32 device array into an int32 or int64 host array.
 int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 {
+    CopyForm f{false, 2};
     if (width == 4) {
         SAGPU_TRY(d2h(c, h, d, n * 4));
-    } else if (n && xs_ready(c, n * 4, XS_MIN_INDEX64)) {
-        SAGPU_TRY(d2h_staged(c, h, d, n * 4, true));
+    } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {
+        SAGPU_TRY(d2h_staged(c, h, d, n * 4, f));
     } else {
         GET(w, int64_t, n);
         hipLaunchKernelGGL(k_widen, dim3(grid_n(n)), dim3(256), 0, c.stream, d, w, n);
@@ -2202,10 +2032,11 @@ int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 int upload_idx(Ctx &c, Scope &sc, const void *h, u64 n, int width, u32 **out)
 {
     GET(d, u32, n);
+    CopyForm f{false, 1};
     if (width == 4) {
         SAGPU_TRY(h2d(c, d, h, n * 4));
-    } else if (n && xs_ready(c, n * 4, XS_MIN_INDEX64)) {
-        SAGPU_TRY(h2d_staged(c, d, h, n * 4, true));
+    } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {
+        SAGPU_TRY(h2d_staged(c, d, h, n * 4, f));
     } else {
         GET(w, int64_t, n);
         SAGPU_TRY(h2d(c, w, h, n * 8));

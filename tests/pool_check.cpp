@@ -1,0 +1,104 @@
+// Checks of libsais_amd/csrc/copy_pool.h that need its parts: test_copy_pool_parts.py builds
+// this with a sanitizer and runs one check by name.  Prints "ok" and returns 0, or says
+// what is wrong.
+#include "../libsais_amd/csrc/copy_pool.h"
+
+#include <stdio.h>
+
+namespace {
+
+#define EXPECT(c)                                                                                  \
+    do {                                                                                           \
+        if (!(c)) {                                                                                \
+            printf("line %d: %s\n", __LINE__, #c);                                                 \
+            return 1;                                                                              \
+        }                                                                                          \
+    } while (0)
+
+CopyPool &pool = *new CopyPool;   // (its workers live as long as the process)
+constexpr u64 HALF = 16ull << 20;   // of the staged copies' ring: the stretch of a shared download
+
+// Every form of a staged copy, in the stretches that the engine grants: its parts fit the
+// room that the job was given, and every entry arrives.
+int copy_form(bool tiny, int conv, u64 entries, bool up, bool shared)
+{
+    const CopyForm f{tiny, conv};
+    const u64 bytes = 4 * entries;
+    std::vector<u32> dev(entries);
+    std::vector<int64_t> wide(entries);
+    for (u64 i = 0; i < entries; i++) {
+        dev[i] = up ? 0u : (u32)(i * 2654435761ull);
+        wide[i] = up ? (int64_t)(u32)(i * 2654435761ull) : -1;
+    }
+    std::vector<u32> plain(entries);
+    uint8_t *host = conv ? (uint8_t *)wide.data() : (uint8_t *)plain.data();
+    if (up && !conv)
+        for (u64 i = 0; i < entries; i++) plain[i] = (u32)wide[i];
+    CopyPool::Job j(f.room(bytes));
+    pool.begin(j, 4);
+    u64 off = 0;
+    for (int k = 0; off < bytes; k++) {
+        u64 len = up ? f.up_chunk(k) : shared ? HALF : f.down_chunk(bytes);
+        len = bytes - off < len ? bytes - off : len;
+        const bool ok = up ? pool.grant(j, {(uint8_t *)dev.data() + off, host + f.taken(off), len, conv}, f.part())
+                           : pool.grant(j, {host + f.written(off), (const uint8_t *)dev.data() + off, f.written(len), conv},
+                                        f.part(shared));
+        if (!ok) break;
+        off += len;
+    }
+    pool.end(j);
+    EXPECT(off == bytes);
+    for (u64 i = 0; i < entries; i++) {
+        const u32 v = (u32)(i * 2654435761ull);
+        EXPECT(dev[i] == v);
+        EXPECT(conv ? wide[i] == (int64_t)v : plain[i] == v);
+    }
+    return 0;
+}
+
+int forms()
+{
+    const u64 sizes[] = {1, 4095, 4096, 100003, 300007, 1u << 20, (5u << 20) + 1};
+    for (u64 n : sizes)
+        for (int tiny = 0; tiny < 2; tiny++)
+            for (int conv = 0; conv < 3; conv++)
+                for (int how = 0; how < 3; how++) {   // upload, download alone, download beside others
+                    if (how == 0 ? conv == 2 : conv == 1) continue;
+                    if (copy_form(tiny != 0, conv, n, how == 0, how == 2)) {
+                        printf("entries %llu, tiny %d, conv %d, way %d\n", n, tiny, conv, how);
+                        return 1;
+                    }
+                }
+    return 0;
+}
+
+// A stretch of more parts than the job has left is refused whole.
+int refused()
+{
+    std::vector<uint8_t> a(1 << 20, 7), b(1 << 20, 0);
+    CopyPool::Job j(3);
+    pool.begin(j, 2);
+    EXPECT(pool.grant(j, {b.data(), a.data(), 100, 0}, 64));            // two parts
+    EXPECT(!pool.grant(j, {b.data() + 100, a.data(), 128, 0}, 64));     // two more
+    EXPECT(j.granted.load() == 2);
+    EXPECT(pool.grant(j, {b.data() + 100, a.data(), 64, 0}, 64));
+    EXPECT(!pool.grant(j, {b.data() + 164, a.data(), 1, 0}, 64));
+    pool.end(j);
+    for (int i = 0; i < 200; i++) EXPECT(b[i] == (i < 164 ? 7 : 0));
+    return 0;
+}
+
+} // namespace
+
+int main(int argc, char **argv)
+{
+    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}};
+    for (const auto &c : checks)
+        if (argc > 1 && !strcmp(argv[1], c.name)) {
+            const int rc = c.run();
+            if (!rc) printf("ok\n");
+            return rc;
+        }
+    printf("no such check\n");
+    return 2;
+}
