@@ -46,13 +46,13 @@ class CopyPool {
     };
 
   private:
-    std::mutex m;   // open, workers, sleeping
+    std::mutex m;   // open, sleeping; workers grow under it
     std::condition_variable work_cv;
     std::vector<Job *> open;
     std::atomic<int> sleeping{0};
     std::atomic<u32> epoch{0};   // grants so far, of all jobs
     std::atomic<int> opens{0};   // jobs in `open`
-    int workers = 0;
+    std::atomic<int> workers{0};
 
     static void run(const Part &p)
     {
@@ -123,7 +123,7 @@ class CopyPool {
         open.push_back(&j);
         opens++;
         try {
-            while (workers < threads - 1) {
+            while (workers.load() < threads - 1) {
                 std::thread([this] { loop(); }).detach();
                 workers++;
             }
@@ -170,7 +170,7 @@ class CopyPool {
             if (j.done[j.prefix].load(std::memory_order_acquire)) {
                 j.prefix++;
                 idle = 0;
-            } else if (idle < 2000 && workers > 0) {
+            } else if (idle < 2000 && workers.load() > 0) {
                 __builtin_ia32_pause();
             } else if (!take(j)) {
                 std::this_thread::yield();

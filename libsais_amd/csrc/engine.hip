@@ -184,11 +184,12 @@ enum { XS_TODO = -1, XS_QUEUED = -2 };        // a region's DMA is not queued / 
 // 1: copies of at least XS_MIN bytes staged (default); 0: every copy direct; 2: every
 // copy staged in 64 KiB chunks (exercises the chunk logic on small inputs)
 std::atomic<int> g_host_staging{1};
-int g_copy_threads = 0;   // 0: min(16, hardware threads)
+std::atomic<int> g_copy_threads{0};   // 0: min(16, hardware threads)
 
 int copy_threads()
 {
-    if (g_copy_threads > 0) return g_copy_threads;
+    const int asked = g_copy_threads.load();
+    if (asked > 0) return asked;
     const unsigned hw = std::thread::hardware_concurrency();
     return hw == 0 ? 4 : (int)(hw < 16 ? hw : 16);
 }

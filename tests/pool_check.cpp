@@ -88,11 +88,33 @@ int refused()
     return 0;
 }
 
+// Callers with different thread counts at once: one waits for its parts while another
+// starts more workers.
+int counts()
+{
+    CopyPool &p = *new CopyPool;
+    constexpr u64 LEN = 8ull << 20;
+    std::vector<std::thread> ts;
+    std::atomic<int> wrong{0};
+    for (int k = 1; k <= 6; k++)
+        ts.emplace_back([&, k] {
+            std::vector<uint8_t> a(LEN + k, (uint8_t)k), b(LEN + k, 0);
+            for (int q = 0; q < 4; q++) {
+                p.copy(b.data(), a.data(), a.size(), 2 * k);
+                if (a != b) wrong++;
+                memset(b.data(), 0, b.size());
+            }
+        });
+    for (auto &t : ts) t.join();
+    EXPECT(wrong == 0);
+    return 0;
+}
+
 } // namespace
 
 int main(int argc, char **argv)
 {
-    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}};
+    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}, {"counts", counts}};
     for (const auto &c : checks)
         if (argc > 1 && !strcmp(argv[1], c.name)) {
             const int rc = c.run();

@@ -2,7 +2,7 @@
 
 tests/pool_check.cpp includes the pool and the shapes of the staged copies, so that what no
 entry point shows can be checked: the room of a job against the parts that each form of a
-copy grants, and a grant that does not fit.
+copy grants, a grant that does not fit, and callers with different thread counts at once.
 """
 import os
 import shutil
@@ -30,6 +30,6 @@ def _run(program, check):
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout[-2000:] + r.stderr[-4000:]
 
 
-@pytest.mark.parametrize("check", ["forms", "refused"])
+@pytest.mark.parametrize("check", ["forms", "refused", "counts"])
 def test_parts(program, check):
     _run(program, check)
