@@ -42,6 +42,7 @@ class CopyPool {
         std::unique_ptr<std::atomic<char>[]> done;
         std::atomic<int> granted{0}, next{0}, users{0};
         std::atomic<bool> closing{false};
+        int limit = 0;    // workers that may be on it at once; set before it is opened
         int prefix = 0;   // the owner's: parts [0, prefix) are done
     };
 
@@ -80,11 +81,15 @@ class CopyPool {
             }
         return false;
     }
-    Job *find()   // m is held: of the jobs with parts to take, one with the fewest threads
+    // m is held (users only grow under it): of the jobs with parts to take and room for one
+    // more thread, one with the fewest threads
+    Job *find()
     {
         Job *best = nullptr;
         for (Job *j : open)
-            if (j->next.load() < j->granted.load() && (!best || j->users.load() < best->users.load())) best = j;
+            if (j->next.load() < j->granted.load() && j->users.load() < j->limit &&
+                (!best || j->users.load() < best->users.load()))
+                best = j;
         return best;
     }
     void loop()
@@ -115,10 +120,11 @@ class CopyPool {
     }
 
   public:
-    // Opens a job (no parts yet) for up to `threads` threads; fewer where the system gives
-    // no more (the owner takes parts, too).
+    // Opens a job (no parts yet) for up to `threads` threads, the owner (who takes parts, too)
+    // among them; fewer where the system gives no more.
     void begin(Job &j, int threads)
     {
+        j.limit = threads - 1;
         std::lock_guard<std::mutex> lk(m);
         open.push_back(&j);
         opens++;
@@ -156,6 +162,8 @@ class CopyPool {
             j.part[g++] = p;
         }
         j.granted.store(g);
+        // (at the limit nobody is called: a worker that leaves the job looks for parts again)
+        if (j.users.load() >= j.limit) return true;
         epoch++;
         if (sleeping.load() > 0) {
             { std::lock_guard<std::mutex> lk(m); }
@@ -170,7 +178,7 @@ class CopyPool {
             if (j.done[j.prefix].load(std::memory_order_acquire)) {
                 j.prefix++;
                 idle = 0;
-            } else if (idle < 2000 && workers.load() > 0) {
+            } else if (idle < 2000 && workers.load() > 0 && j.limit > 0) {
                 __builtin_ia32_pause();
             } else if (!take(j)) {
                 std::this_thread::yield();

@@ -3,6 +3,7 @@
 // what is wrong.
 #include "../libsais_amd/csrc/copy_pool.h"
 
+#include <chrono>
 #include <stdio.h>
 
 namespace {
@@ -110,11 +111,49 @@ int counts()
     return 0;
 }
 
+// A job's thread count caps the workers that take its parts, however many there are:
+// with one thread the caller copies alone.
+int limits()
+{
+    CopyPool &p = *new CopyPool;
+    constexpr u64 LEN = 64ull << 20, PER = 64 << 10;
+    std::vector<uint8_t> a(LEN, 5), b(LEN, 0);
+    p.copy(b.data(), a.data(), LEN, 8);   // seven workers from here on
+    for (int threads = 1; threads <= 4; threads++) {
+        memset(b.data(), 0, LEN);
+        CopyPool::Job j(CopyPool::parts_of(LEN, PER));
+        p.begin(j, threads);
+        EXPECT(p.grant(j, {b.data(), a.data(), LEN / 2, 0}, PER));
+        EXPECT(p.grant(j, {b.data() + LEN / 2, a.data() + LEN / 2, LEN / 2, 0}, PER));
+        int most = 0, done = 0;
+        for (int k = 0; k < 50; k++) {   // the workers by themselves
+            std::this_thread::sleep_for(std::chrono::milliseconds(1));
+            most = std::max(most, j.users.load());
+        }
+        for (u64 k = 0; k < LEN / PER; k++) done += j.done[k].load();
+        EXPECT(most <= threads - 1);
+        EXPECT(threads > 1 ? done > 0 : done == 0);
+        p.end(j);
+        EXPECT(a == b);
+    }
+    // a job without workers beside one that has them
+    CopyPool::Job j1(1), j2(1);
+    p.begin(j1, 1);
+    p.begin(j2, 2);
+    EXPECT(p.grant(j1, {b.data(), a.data(), 64, 0}, 64));
+    EXPECT(p.grant(j2, {b.data() + 64, a.data(), 64, 0}, 64));
+    for (int k = 0; k < 5000 && !j2.done[0].load(); k++) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+    EXPECT(j2.done[0].load() && !j1.done[0].load());
+    p.end(j1);
+    p.end(j2);
+    return 0;
+}
+
 } // namespace
 
 int main(int argc, char **argv)
 {
-    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}, {"counts", counts}};
+    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}, {"counts", counts}, {"limits", limits}};
     for (const auto &c : checks)
         if (argc > 1 && !strcmp(argv[1], c.name)) {
             const int rc = c.run();

@@ -2,7 +2,8 @@
 
 tests/pool_check.cpp includes the pool and the shapes of the staged copies, so that what no
 entry point shows can be checked: the room of a job against the parts that each form of a
-copy grants, a grant that does not fit, and callers with different thread counts at once.
+copy grants, a grant that does not fit, callers with different thread counts at once, and the threads that
+may work on a job.
 """
 import os
 import shutil
@@ -30,6 +31,6 @@ def _run(program, check):
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout[-2000:] + r.stderr[-4000:]
 
 
-@pytest.mark.parametrize("check", ["forms", "refused", "counts"])
+@pytest.mark.parametrize("check", ["forms", "refused", "counts", "limits"])
 def test_parts(program, check):
     _run(program, check)
