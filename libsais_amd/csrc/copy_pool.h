@@ -10,6 +10,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -186,8 +187,9 @@ class CopyPool {
         }
     }
     static u64 parts_of(u64 len, u64 per) { return (len + per - 1) / per; }
+    // (where there is no memory for the job, the caller copies alone)
     void copy(void *d, const void *s, u64 len, int threads)
-    {
+    try {
         if (threads <= 1 || len < (1u << 20)) {
             memcpy(d, s, len);
             return;
@@ -199,6 +201,8 @@ class CopyPool {
         begin(j, threads);
         if (!grant(j, Part{(uint8_t *)d, (const uint8_t *)s, len, 0}, per)) memcpy(d, s, len);
         end(j);
+    } catch (const std::bad_alloc &) {
+        memcpy(d, s, len);
     }
     void lock() { m.lock(); }
     void unlock() { m.unlock(); }

@@ -2646,7 +2646,12 @@ extern "C" int32_t sagpu_memcpy_d2h(void *h, const void *d, size_t bytes)
 extern "C" int32_t sagpu_host_memcpy(void *h, const void *s, size_t bytes, int32_t threads)
 {
     if (threads < 0) return SAGPU_EINVAL;
-    if (bytes) copies().copy(h, s, bytes, threads ? threads : copy_threads());
+    if (!bytes) return 0;
+    try {
+        copies().copy(h, s, bytes, threads ? threads : copy_threads());
+    } catch (const std::bad_alloc &) {   // no pool could be made
+        memcpy(h, s, bytes);
+    }
     return 0;
 }
 

@@ -4,7 +4,26 @@
 #include "../libsais_amd/csrc/copy_pool.h"
 
 #include <chrono>
+#include <new>
 #include <stdio.h>
+#include <stdlib.h>
+
+static std::atomic<int> g_fail_after{-1};   // allocations until every one fails; -1: none does
+
+void *operator new(size_t n)
+{
+    if (g_fail_after >= 0 && g_fail_after-- == 0) {
+        g_fail_after = 0;
+        throw std::bad_alloc();
+    }
+    if (void *p = malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void *operator new[](size_t n) { return operator new(n); }
+void operator delete(void *p) noexcept { free(p); }
+void operator delete[](void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+void operator delete[](void *p, size_t) noexcept { free(p); }
 
 namespace {
 
@@ -149,11 +168,33 @@ int limits()
     return 0;
 }
 
+// A copy finishes, and throws nothing, wherever the memory for its job or its threads ends.
+int no_memory()
+{
+    constexpr u64 LEN = 3ull << 20;
+    std::vector<uint8_t> a(LEN, 9), b(LEN);
+    for (int k = 0; k < 8; k++) {
+        CopyPool &p = *new CopyPool;
+        memset(b.data(), 0, LEN);
+        bool threw = false;
+        g_fail_after = k;
+        try {
+            p.copy(b.data(), a.data(), LEN, 3);
+        } catch (...) {
+            threw = true;
+        }
+        g_fail_after = -1;
+        EXPECT(!threw && a == b);
+    }
+    return 0;
+}
+
 } // namespace
 
 int main(int argc, char **argv)
 {
-    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}, {"counts", counts}, {"limits", limits}};
+    const struct { const char *name; int (*run)(); } checks[] = {{"forms", forms}, {"refused", refused}, {"counts", counts}, {"limits", limits},
+                                                         {"no_memory", no_memory}};
     for (const auto &c : checks)
         if (argc > 1 && !strcmp(argv[1], c.name)) {
             const int rc = c.run();

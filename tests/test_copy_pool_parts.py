@@ -2,8 +2,8 @@
 
 tests/pool_check.cpp includes the pool and the shapes of the staged copies, so that what no
 entry point shows can be checked: the room of a job against the parts that each form of a
-copy grants, a grant that does not fit, callers with different thread counts at once, and the threads that
-may work on a job.
+copy grants, a grant that does not fit, callers with different thread counts at once, the threads that may
+work on a job, and a copy for which there is no memory.
 """
 import os
 import shutil
@@ -31,6 +31,6 @@ def _run(program, check):
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout[-2000:] + r.stderr[-4000:]
 
 
-@pytest.mark.parametrize("check", ["forms", "refused", "counts", "limits"])
+@pytest.mark.parametrize("check", ["forms", "refused", "counts", "limits", "no_memory"])
 def test_parts(program, check):
     _run(program, check)
