@@ -398,7 +398,7 @@ int launch_pack_keys32_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits
 int launch_pack_keys64_sid(const uint8_t *T, u64 n, const uint8_t *lut, int bits, int k, const u32 *sid, u64 *keys,
                            u32 *vals, hipStream_t s);
 // Checks that string k starts at offsets[k] (sid[offsets[k]] == k and the byte
-// before it is a separator); sets *bad otherwise.
+// before it is a separator) and holds one separator, its last symbol; sets *bad otherwise.
 int launch_check_offsets(const uint8_t *T, const u32 *sid, const int64_t *offsets, u32 count, u32 *bad, hipStream_t s);
 // Batched plain-text jobs: job k's text is followed by one separator and occupies
 // [off[k], off[k+1]); slot off[k] of the batched suffix array is that separator's

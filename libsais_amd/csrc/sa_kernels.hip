@@ -304,6 +304,9 @@ __global__ void k_check_offsets(const uint8_t *__restrict__ T, const u32 *__rest
     for (u32 q = blockIdx.x * blockDim.x + threadIdx.x; q < count; q += gridDim.x * blockDim.x) {
         int64_t o = off[q];
         bool ok = sid[o] == q && off[q + 1] > o + 1 && T[off[q + 1] - 1] == 0 && (q == 0 || T[o - 1] == 0);
+        // no separator before the string's last symbol (that of the last string would make
+        // ids past every table that is read by id)
+        ok = ok && sid[off[q + 1] - 1] == q;
         if (!ok) atomicOr(bad, 1u);
     }
 }

@@ -75,3 +75,26 @@ def test_medium_batch_sampled_against_reference():
             assert np.array_equal(L[o:e], ol.ref_lcp(Pk, SAk)), k
     else:
         _check_against_oracle(T, offs, SA, L, sample)
+
+
+@pytest.mark.parametrize("lengths,at", [([7], [2]), ([9], [1, 3, 5]), ([5, 4000, 900], [4905 - 300]),
+                                        ([70000, 1 << 22], [70000 + 5, 200000])])
+def test_separators_inside_the_last_string(lengths, at):
+    """A set whose last string holds separators of its own is refused like one whose other
+    strings do: a string's id is the number of separators before it."""
+    rng = np.random.default_rng(len(lengths))
+    offs = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    T = rng.integers(1, 5, int(offs[-1])).astype(np.uint8)
+    T[offs[1:] - 1] = 0
+    print(f"[batch] inner separators, n={len(T)}", flush=True)
+    dev = batch.DeviceText(T)
+    try:
+        assert batch.batched_on_device(dev, offs) == 0
+    finally:
+        dev.free()
+    T[at] = 0
+    dev = batch.DeviceText(T)
+    try:
+        assert batch.batched_on_device(dev, offs) == -1
+    finally:
+        dev.free()
