@@ -962,9 +962,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         *seed = BwtSeed{bits, codes, d_inv};
     }
     const int cb = seed ? seed->cb : 0;
-    st.initial_symbols = ksym;
     st.bits_per_symbol = bits;
-
 
     // Buffer plan (each block is reused once its first use is over):
     //   kA  [2n u32, 4n for batched u64 keys]: initial sort keys (ping-pong), then
@@ -987,6 +985,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
                 by_segment = true;
                 ksym = k;
             }
+    st.initial_symbols = ksym;
     GET(kA, u32, sid && !by_segment ? 4 * n : 2 * n);
     GET(vA, u32, 2 * n);
     GET(aA, u32, 2 * n);

@@ -573,3 +573,31 @@ def test_build_under_a_memory_limit(n):
     U_r, p_r = ol.bwt(T, ref)
     assert np.array_equal(SA, ref)
     assert p == p_r and np.array_equal(U, U_r)
+
+
+@pytest.mark.parametrize("length,sigma,segmented,fewer", [(90, 4, True, True), (1 << 22, 4, True, False),
+                                                          (60000, 255, True, False), (4, 4, False, False)])
+def test_string_set_route(length, sigma, segmented, fewer):
+    """Which sort a set takes, and the symbols in its keys, from the statistics: 32-bit keys by
+    segment move 16 bytes a symbol and pass, the others 24; short strings' keys hold fewer
+    symbols than 32 bits do.  One more pass of 16 bytes groups the ranks into windows, unless
+    they go straight to the ISA (segmented sets of strings below 3 * 2^18 symbols)."""
+    count = (1 << 22) // length + 1
+    lengths = [length] * count
+    offs = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    n = int(offs[-1])
+    T = np.random.default_rng(length).integers(1, sigma + 1, n).astype(np.uint8)
+    T[offs[1:] - 1] = 0
+    print(f"[set route] {count} strings of {length}", flush=True)
+    batch.batched(T, offs)
+    st = la.stats()
+    most = 32 // st.bits_per_symbol
+    per_symbol = st.sorted_bytes / n
+    print(f"[set route] bytes per symbol {per_symbol:.1f}, symbols {st.initial_symbols} of {most}", flush=True)
+    if not segmented or length > 3 << 18:
+        per_symbol -= 16
+    if segmented:
+        assert per_symbol % 16 == 0 and per_symbol <= 4 * 16
+    else:
+        assert per_symbol % 24 == 0
+    assert st.initial_symbols < most if fewer else st.initial_symbols == most
