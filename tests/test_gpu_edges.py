@@ -601,3 +601,25 @@ def test_string_set_route(length, sigma, segmented, fewer):
     else:
         assert per_symbol % 24 == 0
     assert st.initial_symbols < most if fewer else st.initial_symbols == most
+
+
+@pytest.mark.parametrize("n", [1 << 16, 300007])
+def test_round_chains_save_rounds(n):
+    """Two copies of one random text: every group continues in one group up to the copies'
+    end, so with chains the build ends within a round or two of the first that uses them."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    T = np.random.default_rng(n).integers(97, 101, n).astype(np.uint8)
+    T[n // 2:] = T[:n - n // 2]
+    rounds = []
+    for least in (2, 0):
+        assert lib.sagpu_set_option(b"chain_min", least) == 0
+        try:
+            out = fused(T)
+            rounds.append(la.stats().rounds)
+        finally:
+            assert lib.sagpu_set_option(b"chain_min", 4096) == 0
+    print(f"[chains] n={n}: {rounds} rounds", flush=True)
+    rc, SA = ol.sa(T)
+    assert rc == 0 and np.array_equal(out[0], SA)
+    assert rounds[0] + 3 < rounds[1]
