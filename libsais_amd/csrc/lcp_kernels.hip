@@ -453,7 +453,8 @@ __global__ __launch_bounds__(256) void k_plcp_irr_pairs(const uint8_t *__restric
                 if (!look[q]) v = isa_hint(x[q], n) ? (VT)hint_off + (VT)isa_hint(x[q], n) - 1 : (VT)0;   // (first suffix: 0)
                 if (cmp[q] && !red[q]) {
                     const VT m = nn - vmax(i, (VT)k[q]);
-                    const u32 s = STREAM ? (u32)__clzll((long long)d[q]) / (u32)bits : (u32)__builtin_ctzll(d[q]) >> 3;
+                    const u32 s = !d[q] ? per : STREAM ? (u32)__clzll((long long)d[q]) / (u32)bits
+                                                       : (u32)__builtin_ctzll(d[q]) >> 3;
                     v = l0[q] + (VT)s;
                     v = v < m ? v : m;
                     if (!d[q] && l0[q] < m) {   // longer than the first step

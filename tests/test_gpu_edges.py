@@ -623,3 +623,37 @@ def test_round_chains_save_rounds(n):
     rc, SA = ol.sa(T)
     assert rc == 0 and np.array_equal(out[0], SA)
     assert rounds[0] + 3 < rounds[1]
+
+
+@pytest.mark.parametrize("length", [8, 16, 32, 64])
+@pytest.mark.parametrize("n", [30011, 70000])
+def test_plcp_bound_at_the_end(n, length):
+    """The text's last `length` symbols stand earlier, before zero bytes: the known bound of
+    their lcp is all that is left of the text, and the bytes past both places agree (the
+    padding is zero).  Byte comparisons (plain and with separators) and the code stream."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    rng = np.random.default_rng(n + length)
+    T = rng.integers(1, 5, n).astype(np.uint8)
+    for at in (101, n // 2):
+        T[at:at + length] = T[n - length:]
+        T[at + length:at + length + 40] = 0
+    rc, SA = ol.sa(T)
+    assert rc == 0
+    P = ol.plcp(T, SA)
+    for compare in (1, 0):
+        print(f"[plcp end] n={n} length={length} stream_compare={compare}", flush=True)
+        assert lib.sagpu_set_option(b"stream_compare", compare) == 0
+        try:
+            gSA, _, _, gP, gL, _ = fused(T)
+        finally:
+            assert lib.sagpu_set_option(b"stream_compare", 1) == 0
+        assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA))
+    for at in (101, n // 2):
+        T[at + length + 1:at + length + 40] = 1
+    T[-1] = 0
+    rc, SA = ol.sa(T, gsa=True)
+    assert rc == 0
+    P = ol.plcp(T, SA, gsa=True)
+    gSA, _, _, gP, gL, _ = fused(T, gsa=True)
+    assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA))
