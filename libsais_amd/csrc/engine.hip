@@ -1137,8 +1137,9 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     // launched for n entries and reads the length from the device (its kernels stop at
     // the list's end); the host learns it with the round's report.  The survivor segments
     // are then sized for n entries (12 B each; 1 MiB of ACGT: 65 MB in all instead of 49),
-    // so a call under a memory limit, which may just hold the list, waits.
-    const bool lazy_a = n < LAZY_N && !g_mem_limit.load();
+    // so a call under a memory limit, which may just hold the list, waits; and so does a
+    // timed one, whose kernels' bytes are counted for the list.
+    const bool lazy_a = n < LAZY_N && !g_mem_limit.load() && !c.timer.on;
     if (lazy_a) {
         a = n;
     } else {
@@ -1178,7 +1179,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
         // the geometry of lists below 2^20 entries is sized by powers of two, so that the
         // graphs of one build serve the next one of the same size
         u64 a_grid = a_most;
-        if (a_most < (1ull << 20)) {
+        if (graphs && a_most < (1ull << 20)) {
             a_grid = 4096;
             while (a_grid < a_most) a_grid *= 2;
             if (a_grid > a_first) a_grid = a_first;

@@ -657,3 +657,23 @@ def test_plcp_bound_at_the_end(n, length):
     P = ol.plcp(T, SA, gsa=True)
     gSA, _, _, gP, gL, _ = fused(T, gsa=True)
     assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA))
+
+
+@pytest.mark.parametrize("n", [30000, 1 << 18, (1 << 22) - 1, (1 << 22) + 1])
+def test_timed_bytes(n):
+    """Timing mode counts the gathers' and tile kernels' bytes for the lists that the rounds
+    had: 12 and 28 bytes an entry, and 4 more where the first round reads the groups."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    T = workloads.dna_like(n, seed=n & 255)
+    print(f"[timed bytes] n={n}", flush=True)
+    lib.sagpu_set_timing(1)
+    try:
+        fused(T)
+        st = la.stats()
+    finally:
+        lib.sagpu_set_timing(0)
+    entries = sum(st.active[:st.rounds])
+    assert st.rounds > 1 and st.active[0] < n
+    assert st.kernel_bytes[5] == 12 * entries + 4 * st.active[0]
+    assert st.kernel_bytes[6] == 28 * entries
