@@ -356,7 +356,7 @@ int big_piv_emit(const u32 *pq, const PivRegions &reg, const u32 *rk, const u32 
 // A build of at most SMALL_MAX bytes in one workgroup, all of it in LDS.  T and the
 // outputs may be device memory or pinned host memory; out is pinned host memory.
 constexpr u32 SMALL_MAX = 24 * 1024;
-enum { SMALL_NOT_TAKEN = 1 };   // status: a GSA text that does not end in a separator
+enum { SMALL_NOT_TAKEN = 1 };   // status: a GSA text that does not end in a separator (or no pinned block to be had)
 struct SmallOut {
     int32_t status;          // SAGPU_OK, SAGPU_EINVAL (GSA validity) or SMALL_NOT_TAKEN
     u32 primary, rounds, ksym, sigma;

@@ -1848,8 +1848,7 @@ int small_block(Ctx &c, SmallOut **out, uint8_t **arrays)
         if (hipHostMalloc((void **)&c.small_io, SMALL_IO, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             c.small_io = nullptr;
-            sagpu_set_error("pinned host allocation failed", __FILE__, __LINE__);
-            return SAGPU_ENOMEM;
+            return SMALL_NOT_TAKEN;   // (the general engine needs no such block)
         }
     }
     *out = (SmallOut *)c.small_io;
@@ -2129,10 +2128,10 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_bwt(const uint8_t *T, uint8_t *U, int
     stats_reset(*c);
     if (small_text(*c, (u64)n)) {
         u64 fr[256], primary = 0;
-        SAGPU_TRY(small_host(*c, T, (u64)n, 0, width, nullptr, nullptr, U, nullptr, nullptr, nullptr, 0,
-                             freq ? fr : nullptr, &primary));
-        store_freq(fr, freq, width);
-        return (int64_t)primary;
+        const int rc = small_host(*c, T, (u64)n, 0, width, nullptr, nullptr, U, nullptr, nullptr, nullptr, 0,
+                                  freq ? fr : nullptr, &primary);
+        if (rc == SAGPU_OK) store_freq(fr, freq, width);
+        if (rc != SMALL_NOT_TAKEN) return rc == SAGPU_OK ? (int64_t)primary : rc;
     }
     Scope sc(*c);
     uint8_t *dT;
@@ -2270,10 +2269,10 @@ extern "C" SAGPU_HIDDEN int64_t sagpu_host_bwt_aux(const uint8_t *T, uint8_t *U,
     stats_reset(*c);
     if (small_text(*c, (u64)n)) {
         u64 fr[256];
-        SAGPU_TRY(small_host(*c, T, (u64)n, 0, width, nullptr, nullptr, U, nullptr, nullptr, I, (u64)r,
-                             freq ? fr : nullptr, nullptr));
-        store_freq(fr, freq, width);
-        return 0;
+        const int rc = small_host(*c, T, (u64)n, 0, width, nullptr, nullptr, U, nullptr, nullptr, I, (u64)r,
+                                  freq ? fr : nullptr, nullptr);
+        if (rc == SAGPU_OK) store_freq(fr, freq, width);
+        if (rc != SMALL_NOT_TAKEN) return rc;
     }
     Scope sc(*c);
     uint8_t *dT;
@@ -2980,7 +2979,7 @@ int64_t build32_on(Ctx &c, const uint8_t *d_T, u64 n, int32_t flags, int32_t *d_
     if (small_text(c, n)) {
         SmallJob j{};
         uint8_t *arrays;
-        SAGPU_TRY(small_block(c, &j.out, &arrays));
+        int rc = small_block(c, &j.out, &arrays);
         j.T = d_T;
         j.n = (u32)n;
         j.gsa = (flags & SAGPU_FLAG_GSA) ? 1 : 0;
@@ -2989,7 +2988,7 @@ int64_t build32_on(Ctx &c, const uint8_t *d_T, u64 n, int32_t flags, int32_t *d_
         j.U = d_U;
         j.PLCP = d_PLCP;
         j.LCP = d_LCP;
-        const int rc = small_run(c, j);
+        if (rc == SAGPU_OK) rc = small_run(c, j);
         if (rc == SAGPU_OK && h_freq)
             for (int ch = 0; ch < 256; ch++) h_freq[ch] = (int64_t)j.out->freq[ch];
         if (rc == SAGPU_OK) return d_U ? (int64_t)j.out->primary : 0;
@@ -3243,10 +3242,10 @@ int run_single(Ctx &c, sagpu_job *j)
     stats_reset(c);
     if (small_text(c, n)) {
         u64 primary = 0;
-        SAGPU_TRY(small_host(c, j->T, n, 0, 4, nullptr, j->SA, j->kind == SAGPU_JOB_BWT ? j->U : nullptr, nullptr,
-                             j->kind == SAGPU_JOB_LCP ? j->LCP : nullptr, nullptr, 0, nullptr, &primary));
-        if (j->kind == SAGPU_JOB_BWT) j->primary = (int64_t)primary;
-        return 0;
+        const int rc = small_host(c, j->T, n, 0, 4, nullptr, j->SA, j->kind == SAGPU_JOB_BWT ? j->U : nullptr, nullptr,
+                                  j->kind == SAGPU_JOB_LCP ? j->LCP : nullptr, nullptr, 0, nullptr, &primary);
+        if (rc == SAGPU_OK && j->kind == SAGPU_JOB_BWT) j->primary = (int64_t)primary;
+        if (rc != SMALL_NOT_TAKEN) return rc;
     }
     Scope sc(c);
     uint8_t *dT;
