@@ -208,11 +208,14 @@ class CopyPool {
     void unlock() { m.unlock(); }
 };
 
+constexpr u64 COPY_MID = 32ull << 20, COPY_LARGE = 40ull << 20;   // device bytes
+
 // The shape of one staged copy: settled when it starts, since the options may change while
 // it runs.  Sizes are device bytes where nothing else is said; conv is Part::conv.
 struct CopyForm {
-    bool tiny;   // 64 KiB chunks of 16 KiB parts, whatever the size (host_staging 2)
+    bool tiny;    // 64 KiB chunks of 16 KiB parts, whatever the size (host_staging 2)
     int conv;
+    bool large;   // no conversion, at least COPY_LARGE, and a larger ring to pass through
 
     u64 written(u64 bytes) const { return conv == 2 ? 2 * bytes : bytes; }   // by the host copies
     u64 taken(u64 bytes) const { return conv == 1 ? 2 * bytes : bytes; }     // from the caller's array
@@ -220,20 +223,24 @@ struct CopyForm {
     // early on; later ones keep the DMA's start-up small beside it (a 4 MiB chunk takes 73 us).
     u64 up_chunk(int k) const
     {
+        if (large) return k < 3 ? (2ull << 20) << k : 16ull << 20;
         return tiny ? 64u << 10 : k < 4 ? (512ull << 10) << k : k < 8 ? 4ull << 20 : 8ull << 20;
     }
     // Chunk of a download of `bytes`.
-    u64 down_chunk(u64 bytes) const { return tiny ? 64u << 10 : bytes < (32u << 20) ? 1u << 20 : 4u << 20; }
-    // Written bytes of a part; of a download that shares the bus, parts of a huge page.
-    u64 part(bool shared = false) const
-    {
-        return shared && !tiny ? 2u << 20 : written(tiny ? 16u << 10 : 128u << 10);
-    }
+    u64 down_chunk(u64 bytes) const { return tiny ? 64u << 10 : bytes < COPY_MID ? 1u << 20 : 4u << 20; }
+    // Written bytes of a part: of an upload,
+    u64 up_part() const { return written(tiny ? 16u << 10 : 128u << 10); }
+    // of a download of `bytes` (larger parts from COPY_MID on, so that fewer threads fault in
+    // one huge page of an array not touched before: 64 MB 1.69 -> 1.45 ms, 192 MB 4.75 -> 3.96,
+    // touched arrays the same; 16 MB 0.38 -> 0.51 ms, as the threads then have too few),
+    u64 down_part(u64 bytes) const { return written(tiny ? 16u << 10 : bytes < COPY_MID ? 128u << 10 : 512u << 10); }
+    // and of one by DMA, in slots (a huge page).
+    u64 slot_part() const { return tiny ? written(16u << 10) : 2u << 20; }
     // Parts that a copy of `bytes` may be granted: a short one at the end of every stretch,
     // and none of the stretches but the last is shorter than the first upload chunk.
     u64 room(u64 bytes) const
     {
-        return CopyPool::parts_of(written(bytes), part()) + CopyPool::parts_of(bytes, up_chunk(0));
+        return CopyPool::parts_of(written(bytes), up_part()) + CopyPool::parts_of(bytes, up_chunk(0));
     }
 };
 

@@ -178,8 +178,15 @@ struct Timer {
 // to the device and 4 GB/s into pages the caller has not touched yet (first-touch faults
 // taken by one thread); pinned DMA 57 GB/s.  64-bit index arrays are narrowed and widened
 // by the copy threads, so only 4 bytes per index cross the bus.
-constexpr u64 XS_RING = 32ull << 20;
-constexpr int XS_EVENTS = 8, XS_AHEAD = 24;   // upload chunks whose host copies may run ahead of the DMA
+// Copies of COPY_LARGE and more pass through a ring of twice the size: uploads in 16 MiB
+// chunks with an event every 32 MiB (in the small ring the DMA runs dry whenever the ring is
+// full, since its first region is free only after an event behind all that is queued),
+// downloads by DMA.  libsais_lcp of 48,000,000 entries (three copies of 192 MB): 12.5 ->
+// 12.0 ms, of 128,000,000 32.4 -> 31.2 ms, of 12,000,000 3.43 -> 3.32 ms; at 38 MB the two
+// forms are equal.  (64-bit arrays wait for the threads that convert them, not for the bus.)
+constexpr u64 XS_RING = 32ull << 20, XS_RING_LARGE = 64ull << 20, XS_MARK = 32ull << 20, XS_SLOT = 16ull << 20;
+constexpr int XS_EVENTS = 8, XS_DOWN = XS_RING_LARGE / XS_SLOT;
+constexpr int XS_AHEAD = 24;                  // upload chunks whose host copies may run ahead of the DMA
 enum { XS_TODO = -1, XS_QUEUED = -2 };        // a region's DMA is not queued / queued, no event after it yet
 // 1: copies of at least XS_MIN bytes staged (default); 0: every copy direct; 2: every
 // copy staged in 64 KiB chunks (exercises the chunk logic on small inputs)
@@ -232,9 +239,10 @@ struct Ctx {
     // ring to itself (its kernel follows the uploads on the stream)
     struct XsRegion { u64 at, len; int ev; };   // ev: the event after its DMA, or XS_TODO / XS_QUEUED
     uint8_t *xs = nullptr;
+    u64 xs_cap = 0;           // the ring's bytes; the flags of a download's chunks follow
     u64 xs_head = 0;
     std::deque<XsRegion> xs_used;
-    hipEvent_t xs_ev[XS_EVENTS] = {}, xs_down[2] = {};
+    hipEvent_t xs_ev[XS_EVENTS] = {}, xs_down[XS_DOWN] = {};
     int xs_next_ev = 0;
     u32 *xs_ctr = nullptr;    // device: workgroups done with each chunk of a download
     u32 xs_tick = 0;          // value that marks the current download's chunks in the pinned flags
@@ -1515,7 +1523,9 @@ bool xs_ready(Ctx &c, u64 bytes, CopyForm *f, u64 least = XS_MIN)
     const int mode = g_host_staging.load();
     if (mode == 0 || (mode == 1 && bytes < least)) return false;
     f->tiny = mode == 2;
-    if (c.xs) return true;
+    f->large = mode == 1 && f->conv == 0 && bytes >= COPY_LARGE;
+    const u64 cap = f->large ? XS_RING_LARGE : XS_RING;
+    if (c.xs_cap >= cap) return true;
     for (auto &e : c.xs_ev)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -1535,14 +1545,22 @@ bool xs_ready(Ctx &c, u64 bytes, CopyForm *f, u64 least = XS_MIN)
         }
         c.xs_ctr = ctr;
     }
-    // the ring, then the flags of a download's chunks
     g_device_allocs++;
-    if (hipHostMalloc((void **)&c.xs, XS_RING + XP_CHUNKS * sizeof(u32), hipHostMallocDefault) != hipSuccess) {
+    uint8_t *ring = nullptr;
+    if (hipHostMalloc((void **)&ring, cap + XP_CHUNKS * sizeof(u32), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
-        c.xs = nullptr;
-        return false;
+        f->large = false;
+        return c.xs != nullptr;
     }
-    memset(c.xs + XS_RING, 0, XP_CHUNKS * sizeof(u32));
+    memset(ring + cap, 0, XP_CHUNKS * sizeof(u32));
+    if (c.xs) {   // (its last copies may be under way)
+        if (hipStreamSynchronize(c.stream) != hipSuccess) (void)hipGetLastError();
+        (void)hipHostFree(c.xs);
+        c.xs_used.clear();
+        c.xs_head = 0;
+    }
+    c.xs = ring;
+    c.xs_cap = cap;
     return true;
 }
 
@@ -1563,13 +1581,13 @@ int xs_mark(Ctx &c)
     return SAGPU_OK;
 }
 
-// Takes the ring's next `len` bytes for an upload.  Regions of finished DMAs in the way
-// are given back, after waiting for them when `block`.  *ok = false when the space is
-// not free yet.
-int xs_take(Ctx &c, u64 len, bool block, u64 *at, bool *ok)
+// Takes the next `len` bytes of the ring's first `cap` for an upload.  Regions of finished
+// DMAs in the way are given back, after waiting for them when `block`.  *ok = false when
+// the space is not free yet.
+int xs_take(Ctx &c, u64 cap, u64 len, bool block, u64 *at, bool *ok)
 {
     *ok = false;
-    const u64 head = c.xs_head + len > XS_RING ? 0 : c.xs_head;
+    const u64 head = c.xs_head + len > cap ? 0 : c.xs_head;
     for (;;) {
         bool clash = false;
         for (const auto &r : c.xs_used)
@@ -1610,9 +1628,9 @@ struct XsGuard {
 
 // A stretch of a copy's host side for the pool: `bytes` device bytes, from the s-th byte of
 // the source and to the d-th of the destination on.
-int xs_grant(CopyPool::Job &j, const CopyForm &f, uint8_t *d, const uint8_t *s, u64 bytes, bool shared = false)
+int xs_grant(CopyPool::Job &j, const CopyForm &f, uint8_t *d, const uint8_t *s, u64 bytes, u64 part)
 {
-    if (copies().grant(j, {d, s, f.written(bytes), f.conv}, f.part(shared))) return SAGPU_OK;
+    if (copies().grant(j, {d, s, f.written(bytes), f.conv}, part)) return SAGPU_OK;
     sagpu_set_error("host copy in more parts than planned", __FILE__, __LINE__);
     return SAGPU_EDEVICE;
 }
@@ -1632,16 +1650,17 @@ try {
     if (c.xs_used.empty()) c.xs_head = 0;
     struct Sent { u64 off; int upto; };   // a chunk's place in dst, and the parts through its end
     std::deque<Sent> ahead;               // chunks whose DMA is not queued yet
-    u64 given = 0;
+    const u64 cap = f.large ? XS_RING_LARGE : XS_RING;
+    u64 given = 0, unmarked = 0;
     for (int k = 0; given < bytes || !ahead.empty();) {
         // regions and host copies of the chunks ahead of the DMA
         while (given < bytes && (int)ahead.size() < XS_AHEAD) {
             const u64 len = bytes - given < f.up_chunk(k) ? bytes - given : f.up_chunk(k);
             u64 at = 0;
             bool ok;
-            SAGPU_TRY(xs_take(c, len, ahead.empty(), &at, &ok));
+            SAGPU_TRY(xs_take(c, cap, len, ahead.empty(), &at, &ok));
             if (!ok) break;
-            SAGPU_TRY(xs_grant(j, f, c.xs + at, (const uint8_t *)src + f.taken(given), len));
+            SAGPU_TRY(xs_grant(j, f, c.xs + at, (const uint8_t *)src + f.taken(given), len, f.up_part()));
             ahead.push_back({given, j.granted.load()});
             given += len;
             k++;
@@ -1652,6 +1671,11 @@ try {
                                    c.stream));
         r.ev = XS_QUEUED;
         ahead.pop_front();
+        unmarked += r.len;
+        if (f.large && unmarked >= XS_MARK) {
+            SAGPU_TRY(xs_mark(c));
+            unmarked = 0;
+        }
     }
     SAGPU_TRY(xs_mark(c));
     guard.fine = true;
@@ -1686,30 +1710,32 @@ __global__ __launch_bounds__(256) void k_push(const uint8_t *__restrict__ src, u
     }
 }
 
-// A download while other calls copy too: a DMA per half of the ring, then its host copies
-// in parts of a huge page, so that no two threads fault in one.  With several calls at
-// once the bus is busy anyway, and kernels that push chunks compete with the others'
-// kernels for the CUs: 300 served jobs (2.1 GB of text) at once took 280 ms, 241 this
-// way; into pages not touched before 470 and 336.
-int d2h_shared(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, const CopyForm &f)
+// A download by a DMA per 16 MiB slot of the ring, then the slot's host copies in parts of a
+// huge page, so that no two threads fault in one: large copies (53 GB/s for 192 MB, where the
+// kernel, started again and again, gives 50), and those while other calls copy too.  With
+// several calls at once the bus is busy anyway, and kernels that push chunks compete with
+// the others' kernels for the CUs: 300 served jobs (2.1 GB of text) at once took 280 ms,
+// 241 this way; into pages not touched before 470 and 336.
+int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, const CopyForm &f)
 {
-    const u64 half = XS_RING / 2, nb = (bytes + half - 1) / half;
-    std::vector<int> upto(nb + 1, 0);   // parts through the end of every half
+    const u64 slots = (f.large ? XS_RING_LARGE : XS_RING) / XS_SLOT, nb = (bytes + XS_SLOT - 1) / XS_SLOT;
+    std::vector<int> upto(nb + 1, 0);   // parts through the end of every slot
     auto launch = [&](u64 b) -> int {
-        const u64 off = b * half, len = bytes - off < half ? bytes - off : half;
-        SAGPU_CHECK(hipMemcpyAsync(c.xs + (b & 1) * half, (const uint8_t *)src + off, len, hipMemcpyDeviceToHost, c.stream));
-        SAGPU_CHECK(hipEventRecord(c.xs_down[b & 1], c.stream));
+        const u64 off = b * XS_SLOT, len = bytes - off < XS_SLOT ? bytes - off : XS_SLOT;
+        SAGPU_CHECK(hipMemcpyAsync(c.xs + b % slots * XS_SLOT, (const uint8_t *)src + off, len, hipMemcpyDeviceToHost,
+                                   c.stream));
+        SAGPU_CHECK(hipEventRecord(c.xs_down[b % slots], c.stream));
         return SAGPU_OK;
     };
-    for (u64 b = 0; b < nb && b < 2; b++) SAGPU_TRY(launch(b));
+    for (u64 b = 0; b < nb && b < slots; b++) SAGPU_TRY(launch(b));
     for (u64 b = 0; b < nb; b++) {
-        const u64 off = b * half, len = bytes - off < half ? bytes - off : half;
-        SAGPU_CHECK(hipEventSynchronize(c.xs_down[b & 1]));
-        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + (b & 1) * half, len, true));
+        const u64 off = b * XS_SLOT, len = bytes - off < XS_SLOT ? bytes - off : XS_SLOT;
+        SAGPU_CHECK(hipEventSynchronize(c.xs_down[b % slots]));
+        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + b % slots * XS_SLOT, len, f.slot_part()));
         upto[b + 1] = j.granted.load();
-        if (b + 2 < nb) {
+        if (b + slots < nb) {
             copies().wait(j, upto[b + 1]);
-            SAGPU_TRY(launch(b + 2));
+            SAGPU_TRY(launch(b + slots));
         }
     }
     copies().wait(j, j.granted.load());
@@ -1724,12 +1750,12 @@ try {
     CopyPool::Job j(f.room(bytes));
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
-    if (copies().jobs() > 1) {
-        SAGPU_TRY(d2h_shared(c, j, dst, src, bytes, f));
+    if (f.large || copies().jobs() > 1) {
+        SAGPU_TRY(d2h_slots(c, j, dst, src, bytes, f));
         guard.fine = true;
         return SAGPU_OK;
     }
-    volatile u32 *flags = (volatile u32 *)(c.xs + XS_RING);
+    volatile u32 *flags = (volatile u32 *)(c.xs + c.xs_cap);
     // two halves of the ring, a kernel each; a half is filled again once it is drained
     const u64 half = XS_RING / 2, chunk = f.down_chunk(bytes);
     const u64 batch = chunk * (XP_CHUNKS / 2) < half ? chunk * (XP_CHUNKS / 2) : half;
@@ -1765,7 +1791,7 @@ try {
             }
             std::atomic_thread_fence(std::memory_order_acquire);
             const u64 l = len - o < chunk ? len - o : chunk;
-            SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off + o), c.xs + side * half + o, l));
+            SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off + o), c.xs + side * half + o, l, f.down_part(bytes)));
         }
         upto[b + 1] = j.granted.load();
         // the half of batch b + 1 is being filled or drained; batch b + 2 needs this one
@@ -1784,7 +1810,7 @@ try {
 int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    CopyForm f{false, 0};
+    CopyForm f{false, 0, false};
     if (xs_ready(c, bytes, &f)) return h2d_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
     return SAGPU_OK;
@@ -1794,7 +1820,7 @@ int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 int d2h(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    CopyForm f{false, 0};
+    CopyForm f{false, 0, false};
     if ((uintptr_t)src % 16 == 0 && xs_ready(c, bytes, &f)) return d2h_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
     return SAGPU_OK;
@@ -2016,7 +2042,7 @@ unsigned grid_n(u64 n)
 // Download u32 device array into an int32 or int64 host array.
 int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 {
-    CopyForm f{false, 2};
+    CopyForm f{false, 2, false};
     if (width == 4) {
         SAGPU_TRY(d2h(c, h, d, n * 4));
     } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {
@@ -2032,7 +2058,7 @@ int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 int upload_idx(Ctx &c, Scope &sc, const void *h, u64 n, int width, u32 **out)
 {
     GET(d, u32, n);
-    CopyForm f{false, 1};
+    CopyForm f{false, 1, false};
     if (width == 4) {
         SAGPU_TRY(h2d(c, d, h, n * 4));
     } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {

@@ -20,7 +20,8 @@ pytestmark = pytest.mark.skipif(CXX is None, reason="no host C++ compiler")
 @pytest.fixture(scope="module", params=["address", "thread"])
 def program(request, tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("pool") / ("pool_" + request.param))
-    subprocess.run([CXX, "-std=c++17", "-O1", "-g", "-Wall", "-Werror", "-fsanitize=" + request.param,
+    subprocess.run([CXX, "-std=c++17", "-O2", "-g", "-Wall", "-Werror",
+                    "-Wno-mismatched-new-delete", "-fsanitize=" + request.param,
                     os.path.join(ROOT, "tests", "pool_check.cpp"), "-o", exe, "-pthread"], check=True, timeout=300)
     return exe
 

@@ -107,3 +107,28 @@ def test_form_settled_at_the_start(reset_staging):
     finally:
         stop.set()
         t.join(30)
+
+
+@pytest.mark.parametrize("n", [(10 << 20) - 1, 10 << 20, (16 << 20) + 1, (40 << 20) + 4099])
+def test_large_arrays(n, reset_staging):
+    """32-bit arrays on both sides of 40 MiB, from where copies take a larger ring: uploads
+    that wrap in it, downloads by DMA slot, and smaller and converted copies between them,
+    on one context and after another that never grew."""
+    print(f"[copies] large arrays, n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    SA = rng.integers(0, n, n, dtype=np.int32)
+    P = rng.integers(0, 1 << 30, n, dtype=np.int32)
+    ref = P[SA]
+    m = 3_000_001
+    sa64, p64 = rng.integers(0, m, m), rng.integers(0, 1 << 30, m)
+    for _ in range(2):
+        L = np.full(n, -1, np.int32)
+        assert la.libsais_lcp(P, SA, L, n) == 0 and np.array_equal(L, ref), la.last_error()
+        L64 = np.full(m, -1, np.int64)
+        assert la.libsais64_lcp(p64, sa64, L64, m) == 0 and np.array_equal(L64, p64[sa64])
+        A = SA.copy()
+        assert la.libsais_lcp(P, A, A, n) == 0 and np.array_equal(A, ref)   # over its input
+        k = m // 2
+        L = np.full(k, -1, np.int32)
+        small = SA[:k] % k
+        assert la.libsais_lcp(P[:k].copy(), small, L, k) == 0 and np.array_equal(L, P[:k][small])
