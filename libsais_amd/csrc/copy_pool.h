@@ -137,7 +137,6 @@ class CopyPool {
         } catch (const std::exception &) {
         }
     }
-    int jobs() const { return opens.load(); }
     void end(Job &j)   // waits for every part granted, and for the workers to leave the job
     {
         wait(j, j.granted.load());
@@ -155,6 +154,7 @@ class CopyPool {
     {
         const u64 sper = all.conv == 1 ? 2 * per : all.conv == 2 ? per / 2 : per;
         int g = j.granted.load();
+        const int g0 = g;
         if (parts_of(all.len, per) > j.part.size() - (u64)g) return false;
         for (; all.len; all.d += per, all.s += sper) {
             Part p = all;
@@ -163,23 +163,28 @@ class CopyPool {
             j.part[g++] = p;
         }
         j.granted.store(g);
-        // (at the limit nobody is called: a worker that leaves the job looks for parts again)
-        if (j.users.load() >= j.limit) return true;
+        // All workers that may join it are called (more parts follow soon), and beside other
+        // jobs at most one a part.  (At the limit none: a worker that leaves the job looks for
+        // parts again.)
+        int call = j.limit - j.users.load();
+        if (call <= 0) return true;
         epoch++;
         if (sleeping.load() > 0) {
             { std::lock_guard<std::mutex> lk(m); }
-            work_cv.notify_all();
+            if (opens.load() <= 1) work_cv.notify_all();
+            else for (call = std::min(call, g - g0); call > 0; call--) work_cv.notify_one();
         }
         return true;
     }
-    // Waits until parts [0, upto) are done; takes parts itself when that is not soon.
+    // Waits until parts [0, upto) are done; takes parts itself when that is not soon, or at
+    // once while other jobs want the workers, too.
     void wait(Job &j, int upto)
     {
         for (int idle = 0; j.prefix < upto; idle++) {
             if (j.done[j.prefix].load(std::memory_order_acquire)) {
                 j.prefix++;
                 idle = 0;
-            } else if (idle < 2000 && workers.load() > 0 && j.limit > 0) {
+            } else if (idle < 2000 && workers.load() > 0 && j.limit > 0 && opens.load() <= 1) {
                 __builtin_ia32_pause();
             } else if (!take(j)) {
                 std::this_thread::yield();
@@ -208,39 +213,45 @@ class CopyPool {
     void unlock() { m.unlock(); }
 };
 
-constexpr u64 COPY_MID = 32ull << 20, COPY_LARGE = 40ull << 20;   // device bytes
+constexpr u64 COPY_MID = 32ull << 20, COPY_LARGE = 40ull << 20, COPY_SHARED_LARGE = 8ull << 20;   // device bytes
 
 // The shape of one staged copy: settled when it starts, since the options may change while
 // it runs.  Sizes are device bytes where nothing else is said; conv is Part::conv.
 struct CopyForm {
     bool tiny;    // 64 KiB chunks of 16 KiB parts, whatever the size (host_staging 2)
     int conv;
-    bool large;   // no conversion, at least COPY_LARGE, and a larger ring to pass through
+    bool shared;  // other calls are under way
+    bool large;   // passes through the larger ring
 
     u64 written(u64 bytes) const { return conv == 2 ? 2 * bytes : bytes; }   // by the host copies
     u64 taken(u64 bytes) const { return conv == 1 ? 2 * bytes : bytes; }     // from the caller's array
     // Upload chunk k.  The first ones are small, so that DMA and host copies overlap from
     // early on; later ones keep the DMA's start-up small beside it (a 4 MiB chunk takes 73 us).
+    // Beside other calls, whose DMAs run meanwhile, whole stretches.
     u64 up_chunk(int k) const
     {
+        if (tiny) return 64u << 10;
+        if (shared) return 16ull << 20;
         if (large) return k < 3 ? (2ull << 20) << k : 16ull << 20;
-        return tiny ? 64u << 10 : k < 4 ? (512ull << 10) << k : k < 8 ? 4ull << 20 : 8ull << 20;
+        return k < 4 ? (512ull << 10) << k : k < 8 ? 4ull << 20 : 8ull << 20;
     }
     // Chunk of a download of `bytes`.
     u64 down_chunk(u64 bytes) const { return tiny ? 64u << 10 : bytes < COPY_MID ? 1u << 20 : 4u << 20; }
-    // Written bytes of a part: of an upload,
-    u64 up_part() const { return written(tiny ? 16u << 10 : 128u << 10); }
+    // Written bytes of a part: of an upload (beside other calls larger ones: 8 threads in
+    // libsais_lcp of 4 M entries each 42 ms with 128 KiB, 37 with 1 MiB),
+    u64 up_part() const { return written(tiny ? 16u << 10 : shared ? 1u << 20 : 128u << 10); }
     // of a download of `bytes` (larger parts from COPY_MID on, so that fewer threads fault in
     // one huge page of an array not touched before: 64 MB 1.69 -> 1.45 ms, 192 MB 4.75 -> 3.96,
     // touched arrays the same; 16 MB 0.38 -> 0.51 ms, as the threads then have too few),
     u64 down_part(u64 bytes) const { return written(tiny ? 16u << 10 : bytes < COPY_MID ? 128u << 10 : 512u << 10); }
-    // and of one by DMA, in slots (a huge page).
-    u64 slot_part() const { return tiny ? written(16u << 10) : 2u << 20; }
-    // Parts that a copy of `bytes` may be granted: a short one at the end of every stretch,
-    // and none of the stretches but the last is shorter than the first upload chunk.
+    // and of one by DMA, in slots.
+    u64 slot_part() const { return tiny ? written(16u << 10) : shared ? 1u << 20 : 2u << 20; }
+    // Room for the parts of a copy of `bytes`: every stretch that is granted may end in a
+    // short one, and no part or stretch but the last is smaller than the least of any form.
     u64 room(u64 bytes) const
     {
-        return CopyPool::parts_of(written(bytes), up_part()) + CopyPool::parts_of(bytes, up_chunk(0));
+        return CopyPool::parts_of(written(bytes), tiny ? 16u << 10 : 128u << 10) +
+               CopyPool::parts_of(bytes, tiny ? 64u << 10 : 512u << 10);
     }
 };
 

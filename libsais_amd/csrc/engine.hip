@@ -184,14 +184,15 @@ struct Timer {
 // downloads by DMA.  libsais_lcp of 48,000,000 entries (three copies of 192 MB): 12.5 ->
 // 12.0 ms, of 128,000,000 32.4 -> 31.2 ms, of 12,000,000 3.43 -> 3.32 ms; at 38 MB the two
 // forms are equal.  (64-bit arrays wait for the threads that convert them, not for the bus.)
-constexpr u64 XS_RING = 32ull << 20, XS_RING_LARGE = 64ull << 20, XS_MARK = 32ull << 20, XS_SLOT = 16ull << 20;
-constexpr int XS_EVENTS = 8, XS_DOWN = XS_RING_LARGE / XS_SLOT;
+constexpr u64 XS_RING = 32ull << 20, XS_RING_LARGE = 64ull << 20, XS_MARK = 32ull << 20;
+constexpr int XS_EVENTS = 8, XS_DOWN = 4;    // a download by DMA takes a quarter of its ring at a time
 constexpr int XS_AHEAD = 24;                  // upload chunks whose host copies may run ahead of the DMA
 enum { XS_TODO = -1, XS_QUEUED = -2 };        // a region's DMA is not queued / queued, no event after it yet
 // 1: copies of at least XS_MIN bytes staged (default); 0: every copy direct; 2: every
 // copy staged in 64 KiB chunks (exercises the chunk logic on small inputs)
 std::atomic<int> g_host_staging{1};
 std::atomic<int> g_copy_threads{0};   // 0: min(16, hardware threads)
+std::atomic<int> g_calls{0};          // calls under way: beside others, copies take other forms
 
 int copy_threads()
 {
@@ -521,12 +522,14 @@ struct Lease {
         ctx->pool.reset_peak();
         prev_ctx = t_ctx;
         t_ctx = ctx;
+        g_calls++;
         return SAGPU_OK;
     }
 
     ~Lease()
     {
         if (!ctx) return;
+        g_calls--;
         t_ctx = prev_ctx;
         if (ctx->stats_fresh) {
             ctx->stats.peak_bytes = (int64_t)ctx->pool.peak_bytes;
@@ -1523,7 +1526,8 @@ bool xs_ready(Ctx &c, u64 bytes, CopyForm *f, u64 least = XS_MIN)
     const int mode = g_host_staging.load();
     if (mode == 0 || (mode == 1 && bytes < least)) return false;
     f->tiny = mode == 2;
-    f->large = mode == 1 && f->conv == 0 && bytes >= COPY_LARGE;
+    f->shared = g_calls.load() > 1;
+    f->large = mode == 1 && (f->shared ? bytes >= COPY_SHARED_LARGE : f->conv == 0 && bytes >= COPY_LARGE);
     const u64 cap = f->large ? XS_RING_LARGE : XS_RING;
     if (c.xs_cap >= cap) return true;
     for (auto &e : c.xs_ev)
@@ -1710,32 +1714,34 @@ __global__ __launch_bounds__(256) void k_push(const uint8_t *__restrict__ src, u
     }
 }
 
-// A download by a DMA per 16 MiB slot of the ring, then the slot's host copies in parts of a
-// huge page, so that no two threads fault in one: large copies (53 GB/s for 192 MB, where the
-// kernel, started again and again, gives 50), and those while other calls copy too.  With
-// several calls at once the bus is busy anyway, and kernels that push chunks compete with
-// the others' kernels for the CUs: 300 served jobs (2.1 GB of text) at once took 280 ms,
-// 241 this way; into pages not touched before 470 and 336.
+// A download by a DMA per slot of the ring, then the slot's host copies: large copies (53
+// GB/s for 192 MB, where the kernel, started again and again, gives 50), and those while
+// other calls are under way, with whose kernels the push kernel would compete for the CUs.
+// The latter take small slots, and the work before them is waited for first: DMAs queued
+// behind it hold up the other calls' DMAs.  Calls of libsais and libsais_plcp in turn on 12
+// MB each, 8 pairs a thread, ms for 4 / 8 threads: 110 / 186 with four slots of 16 MiB, 94 /
+// 179 with the wait, 85 / 170 with slots of 8 MiB too.  300 served jobs (2.1 GB of text) at
+// once 240 -> 237 ms, into pages not touched before 262 -> 246.
 int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, const CopyForm &f)
 {
-    const u64 slots = (f.large ? XS_RING_LARGE : XS_RING) / XS_SLOT, nb = (bytes + XS_SLOT - 1) / XS_SLOT;
+    const u64 slot = (f.shared ? XS_RING : XS_RING_LARGE) / XS_DOWN, nb = (bytes + slot - 1) / slot;
     std::vector<int> upto(nb + 1, 0);   // parts through the end of every slot
     auto launch = [&](u64 b) -> int {
-        const u64 off = b * XS_SLOT, len = bytes - off < XS_SLOT ? bytes - off : XS_SLOT;
-        SAGPU_CHECK(hipMemcpyAsync(c.xs + b % slots * XS_SLOT, (const uint8_t *)src + off, len, hipMemcpyDeviceToHost,
+        const u64 off = b * slot, len = bytes - off < slot ? bytes - off : slot;
+        SAGPU_CHECK(hipMemcpyAsync(c.xs + b % XS_DOWN * slot, (const uint8_t *)src + off, len, hipMemcpyDeviceToHost,
                                    c.stream));
-        SAGPU_CHECK(hipEventRecord(c.xs_down[b % slots], c.stream));
+        SAGPU_CHECK(hipEventRecord(c.xs_down[b % XS_DOWN], c.stream));
         return SAGPU_OK;
     };
-    for (u64 b = 0; b < nb && b < slots; b++) SAGPU_TRY(launch(b));
+    for (u64 b = 0; b < nb && b < XS_DOWN; b++) SAGPU_TRY(launch(b));
     for (u64 b = 0; b < nb; b++) {
-        const u64 off = b * XS_SLOT, len = bytes - off < XS_SLOT ? bytes - off : XS_SLOT;
-        SAGPU_CHECK(hipEventSynchronize(c.xs_down[b % slots]));
-        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + b % slots * XS_SLOT, len, f.slot_part()));
+        const u64 off = b * slot, len = bytes - off < slot ? bytes - off : slot;
+        SAGPU_CHECK(hipEventSynchronize(c.xs_down[b % XS_DOWN]));
+        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + b % XS_DOWN * slot, len, f.slot_part()));
         upto[b + 1] = j.granted.load();
-        if (b + slots < nb) {
+        if (b + XS_DOWN < nb) {
             copies().wait(j, upto[b + 1]);
-            SAGPU_TRY(launch(b + slots));
+            SAGPU_TRY(launch(b + XS_DOWN));
         }
     }
     copies().wait(j, j.granted.load());
@@ -1747,10 +1753,11 @@ int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, c
 // in dst.
 int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, const CopyForm &f)
 try {
+    if (f.shared) SAGPU_CHECK(hipStreamSynchronize(c.stream));
     CopyPool::Job j(f.room(bytes));
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
-    if (f.large || copies().jobs() > 1) {
+    if (f.large || f.shared) {
         SAGPU_TRY(d2h_slots(c, j, dst, src, bytes, f));
         guard.fine = true;
         return SAGPU_OK;
@@ -1810,7 +1817,7 @@ try {
 int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    CopyForm f{false, 0, false};
+    CopyForm f{false, 0, false, false};
     if (xs_ready(c, bytes, &f)) return h2d_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
     return SAGPU_OK;
@@ -1820,7 +1827,7 @@ int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 int d2h(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    CopyForm f{false, 0, false};
+    CopyForm f{false, 0, false, false};
     if ((uintptr_t)src % 16 == 0 && xs_ready(c, bytes, &f)) return d2h_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
     return SAGPU_OK;
@@ -2042,7 +2049,7 @@ unsigned grid_n(u64 n)
 // Download u32 device array into an int32 or int64 host array.
 int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 {
-    CopyForm f{false, 2, false};
+    CopyForm f{false, 2, false, false};
     if (width == 4) {
         SAGPU_TRY(d2h(c, h, d, n * 4));
     } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {
@@ -2058,7 +2065,7 @@ int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 int upload_idx(Ctx &c, Scope &sc, const void *h, u64 n, int width, u32 **out)
 {
     GET(d, u32, n);
-    CopyForm f{false, 1, false};
+    CopyForm f{false, 1, false, false};
     if (width == 4) {
         SAGPU_TRY(h2d(c, d, h, n * 4));
     } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {
@@ -3482,6 +3489,7 @@ void worker(Server *svp, int slot)
         for (sagpu_job *j : take) j->t_start = t0;
         apply_options(c);
         int rc;
+        g_calls++;
         if (take.size() == 1) {
             rc = run_single(c, take[0]);
         } else {
@@ -3494,6 +3502,7 @@ void worker(Server *svp, int slot)
                 }
             }
         }
+        g_calls--;
         {
             std::lock_guard<std::mutex> lk(sv.mu);
             sv.reserved -= need;

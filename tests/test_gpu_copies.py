@@ -132,3 +132,34 @@ def test_large_arrays(n, reset_staging):
         L = np.full(k, -1, np.int32)
         small = SA[:k] % k
         assert la.libsais_lcp(P[:k].copy(), small, L, k) == 0 and np.array_equal(L, P[:k][small])
+
+
+@pytest.mark.parametrize("n", [(2 << 20) - 1, 2 << 20, (5 << 20) + 3, (12 << 20) + 1])
+def test_large_arrays_at_once(n, reset_staging):
+    """Four callers with 32- and 64-bit arrays on both sides of 8 MiB, from where copies beside
+    other calls take the larger ring, and of several slots and chunks."""
+    print(f"[copies] large arrays at once, n={n}", flush=True)
+    wrong = []
+
+    def work(k):
+        try:
+            rng = np.random.default_rng(n + k)
+            m = n + 7 * k
+            SA = rng.integers(0, m, m, dtype=np.int32)
+            P = rng.integers(0, 1 << 30, m, dtype=np.int32)
+            ref = P[SA]
+            for t, lcp in ((np.int32, la.libsais_lcp), (np.int64, la.libsais64_lcp)):
+                A, B = SA.astype(t), P.astype(t)
+                for _ in range(2):
+                    L = np.full(m, -1, t)
+                    if lcp(B, A, L, m) != 0 or not np.array_equal(L, ref):
+                        wrong.append((k, lcp.__name__, la.last_error()))
+        except Exception as e:  # pragma: no cover - reported below
+            wrong.append((k, repr(e)))
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(100)
+    assert not any(t.is_alive() for t in ts) and wrong == []
