@@ -254,10 +254,10 @@ struct RoundStart {
 // position without a bit from position 64 w on, when it lies in w's CHAIN_TILE words,
 // else none (~0); tile[t]: the same from tile t's first position on, over all tiles.
 constexpr int CHAIN_GROUP = 8, CHAIN_TILE = 1024;
+constexpr u32 CHAIN_GAIN = 6;   // what a round with chains gains for a member of a pair
 struct Chains {
     const u64 *bits;   // nullptr: off
     const u32 *next, *tile;
-    const u32 *on;   // 0: few of the list's groups can continue; nothing was marked
 };
 // words of scratch chain_marks takes for a text of n symbols (u32, 8-byte aligned)
 u64 chain_words(u64 n);
@@ -281,7 +281,8 @@ int round_gather(const u32 *act_i, const u32 *act_g, u64 a_grid, u64 *rp, const 
 // bseg_g (round_bigseg_cap(n) entries each, n >= every list length) and are
 // concatenated into big_head / big_g / big_size; boff (big_cap + 1 entries) gets their
 // offsets in the concatenation of their members.  rec (pinned, 7 u64) receives cnt's
-// words at their indexes and in rec[6], last, the length the round started with;
+// words at their indexes, in rec[1] what a round with chains promises for the survivors of
+// the tiles (at most CHAIN_GAIN each), and in rec[6], last, the length the round started with;
 // rp_next the next round's length (0 when there are big groups) and offset.
 constexpr int ROUND_RUNS = 64, SEG_CTR_WORDS = ROUND_RUNS * 16;
 u64 round_seg_cap(u64 a);

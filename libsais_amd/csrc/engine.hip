@@ -1268,7 +1268,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
     };
 
     bool queued = false, left = false;   // this round is on the stream already; its length is in rp
-    u64 a_before = 0;                    // the length of the round before
+    u64 a_before = 0, gain = 0;          // the length of the round before, and what chains promise now
     int chain_rounds = 0;
     while (a > 0) {
         const bool raw = st.rounds == 0 && rk1.pw;
@@ -1281,11 +1281,17 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             // and the longer gather cost about 2 rounds' gathers (0.25 ms for 4.8 M
             // entries), so the list must promise more than two such rounds: 7/8 of the
             // length before.  48 MiB of words with repeats (lists of 4778 and 4771 K, then
-            // 145 K instead of 9 rounds): 13.80 -> 12.69 ms.  At 3/4, 256 MiB of DNA with
+            // 145 K instead of 9 rounds): 13.30 -> 12.76 ms.  At 3/4, 256 MiB of DNA with
             // diverged repeats (23.1 and 18.1 M, then 5.1 instead of 11.8 M) went from
-            // 21.6 to 22.3 ms.  A second time takes what groups above CHAIN_GROUP left.
+            // 21.6 to 22.3 ms.  And it must consist of small groups: copies that end in
+            // different places cost a group one chain round for each.  308 texts of 2 and
+            // 32 Mi symbols with 2 to 20 copies of 300 to 30000 symbols, some inside one
+            // another or with mutations, against no chains: 0.93 of the time in the mean
+            // (0.44 to 1.19) from 7/16 of CHAIN_GAIN on, 0.96 from 9/16 on; with any groups up
+            // to CHAIN_GROUP 0.94 (0.44 to 1.20).  A second time takes what larger groups left.
             chains = g_chain_min && left && st.rounds >= 2 && chain_rounds < 2 && a >= (u64)g_chain_min &&
-                     a > a_before / 8 * 7 && chain_words(n) <= n && n < 0xFFFFFF00ull;
+                     a > a_before / 8 * 7 && 16 * gain >= 7 * CHAIN_GAIN * a && chain_words(n) <= n &&
+                     n < 0xFFFFFF00ull;
             chain_rounds += chains;
             SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr, chains));
             // Short rounds cost their launches and the host's wait: queue the next one
@@ -1449,6 +1455,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             st.big_elems += (int64_t)total;
         }
         a_before = a;
+        gain = rec[cur][1];
         a = out_n;
         cur = nxt;
         h *= 2;

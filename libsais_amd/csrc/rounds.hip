@@ -761,7 +761,7 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
         u32 t[IG];
 #pragma unroll
         for (int q = 0; q < IG; q++) t[q] = 0;
-        if (CHAIN && *ch.on) {
+        if (CHAIN) {
             u64 w[IG];
 #pragma unroll
             for (int q = 0; q < IG; q++) w[q] = ch.bits[i[q] >> 6] >> (i[q] & 63u);
@@ -802,31 +802,6 @@ __global__ __launch_bounds__(256) void k_round_gather(const u32 *__restrict__ ac
     }
 }
 
-// Whether chains are worth their marks: at least half of CS_SAMPLES entries spread over
-// the list are in groups that can continue.  On texts of long periods (lists of groups of
-// ever the same size above CHAIN_GROUP) the marks would cost two gathers and give nothing.
-constexpr u32 CS_SAMPLES = 4096;
-__global__ __launch_bounds__(1024) void k_chain_sample(const u32 *__restrict__ act_g, u64 a, u32 *__restrict__ on)
-{
-    __shared__ u32 s_small[1024 / SAGPU_WAVE];
-    u32 small = 0;
-    for (u32 q = threadIdx.x; q < CS_SAMPLES; q += 1024) {
-        const u64 k = a * q / CS_SAMPLES;
-        const u32 g = act_g[k];
-        int size = 1;
-        for (int d = 1; d <= CHAIN_GROUP && k >= (u64)d && act_g[k - d] == g; d++) size++;
-        for (int d = 1; d <= CHAIN_GROUP && k + d < a && act_g[k + d] == g; d++) size++;
-        small += size <= CHAIN_GROUP;
-    }
-    small = wave_incl_sum(small);
-    if (lane_id() == SAGPU_WAVE - 1) s_small[threadIdx.x / SAGPU_WAVE] = small;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    u32 sum = 0;
-    for (u32 w = 0; w < 1024 / SAGPU_WAVE; w++) sum += s_small[w];
-    *on = sum >= CS_SAMPLES / 2;
-}
-
 // Marks of chains.  Each list entry reads the rank of its next suffix (one random 4-byte
 // read) and sets its bit when its group is small and all of the group's next suffixes
 // hold one rank; the bits of a group are alike, and since the next suffixes are of one
@@ -837,10 +812,8 @@ __global__ __launch_bounds__(1024) void k_chain_sample(const u32 *__restrict__ a
 // (one more than a group that counts can reach: a larger one is seen from its ends).
 constexpr int CM_RANGE = 1024, CM_HALO = CHAIN_GROUP, CM_WIN = CM_RANGE + 2 * CM_HALO;
 __global__ __launch_bounds__(256) void k_chain_marks(const u32 *__restrict__ act_i, const u32 *__restrict__ act_g, u64 a,
-                                                     const u32 *__restrict__ ISA, u64 n, int cb, u32 *__restrict__ bits,
-                                                     const u32 *__restrict__ on)
+                                                     const u32 *__restrict__ ISA, u64 n, int cb, u32 *__restrict__ bits)
 {
-    if (!*on) return;
     constexpr int PER = (CM_WIN + 255) / 256;
     __shared__ u32 s_g[CM_WIN], s_r[CM_WIN];
     const u64 lo = (u64)blockIdx.x * CM_RANGE;
@@ -966,6 +939,13 @@ __device__ __forceinline__ void rt_big_head(u64 head, u32 g, u64 *__restrict__ s
     } else {
         atomicOr(err, 1u);
     }
+}
+
+// What a chain round promises for a member of a group of `size`, of CHAIN_GAIN: the group loses
+// at least one member to it, and a pair is done.
+__device__ __forceinline__ u32 chain_gain(u32 size)
+{
+    return size == 2 ? CHAIN_GAIN : size == 3 ? CHAIN_GAIN / 2 : size == 4 ? CHAIN_GAIN / 3 : size < 8 ? CHAIN_GAIN / 6 : 0u;
 }
 
 template <typename KT, int RANGE>
@@ -1142,7 +1122,8 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
     //    list order), pk the largest smaller key; local positions throughout.  The
     //    entry goes to position hx + lt + eqb, its subgroup's first slot is g + lt.
     //    Per entry of the thread: output position (NONE: none), group word for the
-    //    next list, the rank written to ISA, flags (1: survives, 2: ISA written).
+    //    next list, the rank written to ISA, flags (1: survives, 2: ISA written; above them
+    //    chain_gain).
     u32 e_pos[RT_PER], e_word[RT_PER], e_isa[RT_PER], e_fl[RT_PER];
     auto place = [&](int j, u32 hx, u32 lt, u32 eq, u32 eqb, KT key, KT pk) {
         const u32 gw = s_w[hx];   // first slot | flag
@@ -1168,7 +1149,7 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
         e_pos[j] = hx + lt + eqb;
         e_word[j] = r | (kept ? (gw & ac.gf) : 0u);
         e_isa[j] = r | hint;
-        e_fl[j] = (eq > 1 ? 1u : 0u) | (kept ? 0u : 2u);
+        e_fl[j] = (eq > 1 ? 1u : 0u) | (kept ? 0u : 2u) | chain_gain(eq) << 2;
     };
 #pragma unroll
     for (int j = 0; j < RT_PER; j++) e_pos[j] = NONE;
@@ -1317,13 +1298,13 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
             SA[r] = v;
             if (ac.codes) ac.codes[r] = (uint8_t)(e_ai[j] & ((1u << ac.cb) - 1u));
         } else {
-            s_os[e_pos[j]] = 1;
+            s_os[e_pos[j]] = (uint8_t)(1u | (e_fl[j] & ~3u));
         }
     }
     __syncthreads();
 
-    // 6. survivors: output ranks by position, their range reserved in this run's
-    //    segment (one atomic on the run's counter).  A counter shared by all
+    // 6. survivors (counted in the low halves, their chain_gain in the high halves): output
+    //    ranks by position, their range reserved in this run's segment (one atomic on the run's counter).  A counter shared by all
     //    workgroups serialises them: 300 K returning atomics on one address take
     //    3.6 ms, on 8 addresses 0.57 ms; the XCDs work on a run each.
     u32 cnt_s[RT_PER];
@@ -1331,7 +1312,8 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
 #pragma unroll
     for (int j = 0; j < RT_PER; j++) {
         const u32 x = first + tid * RT_PER + j;
-        cnt_s[j] = (x < end && s_os[x]) ? 1u : 0u;
+        const u32 f = x < end ? s_os[x] : 0u;
+        cnt_s[j] = (f & 1u) | (f >> 2) << 16;
         tot += cnt_s[j];
     }
     const u32 inc = wave_incl_sum(tot);
@@ -1339,7 +1321,8 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
     __syncthreads();
     if (tid == 0) {
         const u32 all = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
-        s_base = (u64)run * seg_cap + (all ? atomicAdd(&seg_ctr[run * 16], (u64)all) : 0ull);
+        const u64 add = (u64)(all >> 16) << 32 | (all & 0xFFFFu);
+        s_base = (u64)run * seg_cap + (all ? (u32)atomicAdd(&seg_ctr[run * 16], add) : 0u);
     }
     {
         u32 o = inc - tot;
@@ -1479,10 +1462,15 @@ __global__ __launch_bounds__(256) void k_round_end(const u32 *__restrict__ seg_i
     }
     static_assert(ROUND_RUNS == SAGPU_WAVE, "a lane per run");
     __shared__ u64 s_pre[ROUND_RUNS + 1];   // the runs' first entries of the next list
+    __shared__ u64 s_gain;
     if (threadIdx.x < (u32)ROUND_RUNS) {
-        const u64 c = seg_ctr[threadIdx.x * 16], inc = wave_incl_sum64(c);
+        const u64 w = seg_ctr[threadIdx.x * 16], c = (u32)w;
+        const u64 inc = wave_incl_sum64(c), gain = wave_incl_sum64(w >> 32);
         s_pre[threadIdx.x] = inc - c;
-        if (threadIdx.x == ROUND_RUNS - 1) s_pre[ROUND_RUNS] = inc;
+        if (threadIdx.x == ROUND_RUNS - 1) {
+            s_pre[ROUND_RUNS] = inc;
+            s_gain = gain;
+        }
     }
     __syncthreads();
     const u64 total = s_pre[ROUND_RUNS];
@@ -1554,6 +1542,7 @@ __global__ __launch_bounds__(256) void k_round_end(const u32 *__restrict__ seg_i
         rp_next[0] = nb ? 0 : total;
         rp_next[1] = 2 * rp[1];
         rec[0] = total;
+        rec[1] = s_gain;
         rec[4] = (nb & 0xFFFFFFFFull) | (u64)err << 32;
         rec[5] = members;
         __threadfence_system();
@@ -1801,21 +1790,20 @@ int round_gather(const u32 *act_i, const u32 *act_g, u64 a, u64 *rp, const Round
 }
 
 static u64 chain_bit_words(u64 n) { return n / 64 + 1; }
-u64 chain_words(u64 n) { return 3 * chain_bit_words(n) + ceil_div_u(chain_bit_words(n), (u64)CHAIN_TILE) + 1; }
+u64 chain_words(u64 n) { return 3 * chain_bit_words(n) + ceil_div_u(chain_bit_words(n), (u64)CHAIN_TILE); }
 int chain_marks(const u32 *act_i, const u32 *act_g, u64 a, const u32 *ISA, u64 n, int cb, u32 *scratch, Chains *ch,
                 hipStream_t s)
 {
     const u64 words = chain_bit_words(n);
     const u32 tiles = (u32)ceil_div_u(words, (u64)CHAIN_TILE);
-    u32 *next = scratch + 2 * words, *tile = next + words, *on = tile + tiles;
-    hipLaunchKernelGGL(k_chain_sample, dim3(1), dim3(1024), 0, s, act_g, a, on);
+    u32 *next = scratch + 2 * words, *tile = next + words;
     SAGPU_TRY(launch_fill_u32(scratch, 2 * words, 0, s));
     hipLaunchKernelGGL(k_chain_marks, dim3((unsigned)ceil_div_u(a, (u64)CM_RANGE)), dim3(256), 0, s, act_i, act_g, a, ISA,
-                       n, cb, scratch, (const u32 *)on);
+                       n, cb, scratch);
     hipLaunchKernelGGL(k_chain_next, dim3(tiles), dim3(256), 0, s, (const u64 *)scratch, words, next, tile);
     if (tiles > 1) hipLaunchKernelGGL(k_chain_tiles, dim3(1), dim3(1024), 0, s, tile, tiles);
     SAGPU_CHECK(hipGetLastError());
-    *ch = Chains{(const u64 *)scratch, next, tile, on};
+    *ch = Chains{(const u64 *)scratch, next, tile};
     return SAGPU_OK;
 }
 

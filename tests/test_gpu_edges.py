@@ -677,3 +677,33 @@ def test_timed_bytes(n):
     assert st.rounds > 1 and st.active[0] < n
     assert st.kernel_bytes[5] == 12 * entries + 4 * st.active[0]
     assert st.kernel_bytes[6] == 28 * entries
+
+
+@pytest.mark.parametrize("n", [70001, 300007])
+def test_round_chains_mixed_groups(n):
+    """Lists of mostly pairs, which take chains, with groups of 3 to 12 among them: some small
+    enough to be marked, some not, some ending inside another's copies."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    rng = np.random.default_rng(n)
+    T = rng.integers(97, 101, n).astype(np.uint8)
+    k = n // 40
+    T[20 * k:36 * k] = T[:16 * k]   # pairs
+    for c, (copies, size) in enumerate(((3, k), (4, k // 2), (7, k // 8), (8, k // 9), (9, k // 10), (12, k // 13))):
+        at = 36 * k + c * (k // 2) + np.arange(copies) * size // 2   # overlapping
+        for q in at:
+            T[q:q + size // 2] = T[c * k:c * k + size // 2]
+    rc, SA = ol.sa(T)
+    assert rc == 0
+    P = ol.plcp(T, SA)
+    rounds = []
+    for least in (2, 0):
+        assert lib.sagpu_set_option(b"chain_min", least) == 0
+        try:
+            gSA, gU, gp, gP, gL, _ = fused(T)
+            rounds.append(la.stats().rounds)
+        finally:
+            assert lib.sagpu_set_option(b"chain_min", 4096) == 0
+        assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA)), least
+    print(f"[chains] n={n}: {rounds} rounds", flush=True)
+    assert rounds[0] < rounds[1]
