@@ -242,8 +242,13 @@ struct CopyForm {
     u64 up_part() const { return written(tiny ? 16u << 10 : shared ? 1u << 20 : 128u << 10); }
     // of a download of `bytes` (larger parts from COPY_MID on, so that fewer threads fault in
     // one huge page of an array not touched before: 64 MB 1.69 -> 1.45 ms, 192 MB 4.75 -> 3.96,
-    // touched arrays the same; 16 MB 0.38 -> 0.51 ms, as the threads then have too few),
-    u64 down_part(u64 bytes) const { return written(tiny ? 16u << 10 : bytes < COPY_MID ? 128u << 10 : 512u << 10); }
+    // touched arrays the same; 16 MB 0.38 -> 0.51 ms, as the threads then have too few; nor for
+    // 64-bit arrays, which wait for the threads: libsais64, libsais64_plcp and libsais64_lcp of
+    // 12,000,001 symbols 10.7 -> 11.2 ms, and 12.7 -> 11.9 into arrays not touched before),
+    u64 down_part(u64 bytes) const
+    {
+        return written(tiny ? 16u << 10 : bytes < COPY_MID || conv == 2 ? 128u << 10 : 512u << 10);
+    }
     // and of one by DMA, in slots.
     u64 slot_part() const { return tiny ? written(16u << 10) : shared ? 1u << 20 : 2u << 20; }
     // Room for the parts of a copy of `bytes`: every stretch that is granted may end in a
