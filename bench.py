@@ -12,10 +12,11 @@ sagpu_stats.kernel_ms, in up to 5 extra steps after the timed ones: the timed
 steps run without events, with the doubling rounds replaying captured graphs).  achieved = its algorithmic
 bytes per launch (reads + writes at element size, counted by the engine per
 launch: e.g. k_round_tile 28 B per active list entry, k_isa_scatter 12 B per
-position) / its average launch duration.  roofline.kernels lists the five kernels
-with the largest time per build the same way.  traffic is the HBM bytes per
+position) / its average launch duration.  roofline.kernels lists the kernels by
+time per build the same way.  traffic is the HBM bytes per
 launch measured with rocprofv3 FETCH_SIZE / WRITE_SIZE (scaled by a copy kernel of
-known size), read from profiles/pmc_traffic.json.
+known size), read from profiles/pmc_traffic.json; null for kernels whose code has
+changed since.
 pipeline: B_model = 269 n + 244 sum_r a_r bytes per step (prefix-doubling yardstick
 with 8 initial symbols; a_r counts suffixes with max(LCP[j], LCP[j+1]) >= 8*2^(r-1),
 computed from the LCP this run produced), divided by the step time.
@@ -31,8 +32,10 @@ from __future__ import annotations
 
 import argparse
 import ctypes
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -47,6 +50,10 @@ KERNELS = ["k_radix_pass<u32 key, u32 value>", "k_radix_pass (generating first p
            "k_radix_pass<u64 key, u32 value>", "k_init_emit", "k_scatter_windows (initial ranks)", "k_round_gather",
            "k_round_tile",
            "k_plcp_pairs", "k_plcp_irr_pairs", "k_lcp_fix", "k_bwt_seeded"]
+# the start of a kernel's name -> its source file
+KERNEL_SOURCES = [("k_radix_pass", "radix.hip"), ("k_scatter_windows", "scatter.hip"), ("k_init_emit", "rounds.hip"),
+                  ("k_round_", "rounds.hip"), ("k_plcp_", "lcp_kernels.hip"), ("k_lcp_fix", "lcp_kernels.hip"),
+                  ("k_bwt_seeded", "lcp_kernels.hip")]
 METRIC = "SA+BWT input MB/s @256 MiB DNA; batched vs plain aggregate MB/s; p99 latency"
 
 
@@ -74,16 +81,27 @@ def copy_peak(lib, nbytes: int = 1 << 30, reps: int = 5):
     return 2 * nbytes / best / 1e9
 
 
+def kernel_code(kernel: str) -> str:
+    """Digest of the code (without // comments) of a kernel's source file and the headers it includes."""
+    src = next(f for k, f in KERNEL_SOURCES if kernel.startswith(k))
+    h = hashlib.sha256()
+    for name in (src, "engine.h", "common.h"):
+        with open(os.path.join(ROOT, "libsais_amd", "csrc", name)) as f:
+            h.update(re.sub(r"\s+", " ", re.sub(r"//[^\n]*", "", f.read())).encode())
+    return h.hexdigest()[:16]
+
+
 def measured_traffic(workload: str, kernel: str):
     """HBM bytes per launch of a kernel from the committed PMC summary (rocprofv3
-    FETCH_SIZE and WRITE_SIZE runs, scaled by the copy-kernel calibration), or None."""
+    FETCH_SIZE and WRITE_SIZE runs, scaled by the copy-kernel calibration), or None,
+    also where the kernel's code is no longer the one that was counted."""
     path = os.path.join(ROOT, "profiles", "pmc_traffic.json")
     try:
         with open(path) as f:
             d = json.load(f)
-    except (OSError, ValueError):
-        return None
-    if d.get("workload") != workload:
+        if d.get("workload") != workload or d.get("code", {}).get(kernel) != kernel_code(kernel):
+            return None
+    except (OSError, ValueError, StopIteration):
         return None
     return d.get("bytes_per_launch", {}).get(kernel)
 
