@@ -227,17 +227,21 @@ SAGPU_API int32_t sagpu_sort_pairs_u64(uint64_t *d_keys, uint32_t *d_vals, int64
  *                    packed key that follows (same order as its rank; default); 0 = by rank
  *   "exact_round1"   1 = with raw_round1, the first round records the exact lcp across each
  *                    split, from the two raw keys (default); 0 = a lower bound, left to the PLCP pass
- *   "plcp_hint"      1 = the fused build with LCP (texts and large string sets up to 2^30) packs the exact lcp of each
- *                    suffix alone in its initial group into bits 28-31 of its ISA word (15 values
- *                    on the largest marks the initial key allows), and the PLCP pass takes it
- *                    instead of reading a pair word (default); 0 = no hints
+ *   "plcp_hint"      1 = the fused build with LCP (texts and large string sets up to 2^30) packs
+ *                    the exact lcp of each suffix alone in its initial group into its ISA word,
+ *                    above the rank: into bits 28-31 for up to 2^28 suffixes (15 values, on the
+ *                    largest marks the initial key allows), 29-31 for up to 2^29 (7 values), 30
+ *                    and 31 for up to 2^30 (3 values).  The PLCP pass takes it instead of reading
+ *                    a pair word (default); 0 = no hints
  *   "stream_compare" 1 = with key_stream, the PLCP pass compares suffixes on the packed code
  *                    stream, 64 / bits symbols per step (default); 0 = on the bytes
  *   "host_staging"   copies between caller host memory and the device: 1 = copies of at least
  *                    4 MiB (64-bit index arrays: 2 MiB) through a pinned ring in chunks, host
- *                    side split over copy threads (default); 0 = direct hipMemcpy from pageable memory; 2 =
- *                    every copy staged in 64 KiB chunks
- *   "copy_threads"   host threads for staged copies, 1-64; 0 = min(16, hardware threads) (default)
+ *                    side split over copy threads (default; the ring holds 32 MiB, or 64 MiB once
+ *                    a context has copied 40 MiB at once, 8 MiB beside other calls); 0 = direct
+ *                    hipMemcpy from pageable memory; 2 = every copy staged in 64 KiB chunks
+ *   "copy_threads"   host threads that work on one staged copy at a time, the calling one among
+ *                    them, 1-64 (1: the caller alone); 0 = min(16, hardware threads) (default)
  *   "bucketed_phi"   1 = Φ of a caller's suffix array (libsais_plcp and the like) through
  *                    pairs bucketed by target, scattered bucket after bucket (default); 0 = one pass
  *   "plcp_pairs"     1 = the fused PLCP pass reads one 8-byte pair word per position, built in
@@ -248,8 +252,8 @@ SAGPU_API int32_t sagpu_sort_pairs_u64(uint64_t *d_keys, uint32_t *d_vals, int64
  *   "wide_from"      texts longer than this use 64-bit rank keys (default 2^31 - 1, the
  *                    largest the 32-bit keys hold; lower values exercise the wide mode)
  *   "round_graphs"   1 = doubling rounds from the second on replay a captured HIP graph per
- *                    buffer parity (parameter copy, gather, tile kernel, counter copy), updated
- *                    in place across builds (default; not in timing mode or the allocation-free
+ *                    buffer parity (tile kernel and end of the round), updated in place across
+ *                    builds (default; not in timing mode or the allocation-free
  *                    build); 0 = kernels launched one by one
  *   "windowed_scatter" 1 = texts over 2^22 write the initial ranks through a radix pass into
  *                    windows of the ISA and a scatter in which each XCD writes only its own windows

@@ -285,8 +285,8 @@ int g_stream_compare = 1;
 // 1: round 1 on raw keys records exact lcps across its splits; 0: lower bounds
 int g_exact_round1 = 1;
 // 1: the fused build with LCP packs the exact lcp of each suffix alone in its
-// initial group into its ISA word (texts up to 2^28), so the PLCP pass skips its
-// pair-word read; 0: every position reads its pair word
+// initial group into its ISA word (texts up to 2^30, see isa_shift), so the PLCP pass
+// skips its pair-word read; 0: every position reads its pair word
 int g_plcp_hint = 1;
 // 1: Φ of a caller's suffix array by the bucketed two-pass scatter; 0: one pass
 int g_bucketed_phi = 1;
@@ -3245,8 +3245,6 @@ extern "C" int32_t sagpu_gsa_batch32(const uint8_t *d_T, int64_t n, const int64_
 
 #include <chrono>
 #include <condition_variable>
-#include <deque>
-#include <deque>
 #include <thread>
 
 namespace {

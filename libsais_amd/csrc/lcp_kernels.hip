@@ -334,8 +334,8 @@ __device__ __forceinline__ u64 match_stream(const u32 *__restrict__ pw, int bits
 // pair read and the symbol before it; known lcps and reducible positions finish
 // there, irreducible ones compare as k_plcp_irr.  PI positions per thread and step
 // with their loads issued together, those of the comparisons' first steps too, and
-// without branches around them; ISA and values stream past the L2 (2^28 DNA suffixes:
-// 1.75 ms with a comparison at a time, 1.35 ms now).  Bound by the random reads that miss
+// without branches around them; ISA and values stream past the L2 (2^28 DNA-like suffixes:
+// 2.27 ms with a comparison at a time, 1.70 ms now).  Bound by the random reads that miss
 // the L2 (about 60 G/s); the XCDs take runs of the text, so that a string set's strings
 // are read from one L2 each.
 constexpr int PI = 4;

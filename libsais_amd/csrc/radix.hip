@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void k_radix_offsets(u64 *hist, int npass, int
 // global digit offsets were produced by an upsweep + scan (reduce-then-scan).
 // GEN: the input keys and values are generated (KeyGen) instead of read.
 // Bound by memory: 2^28 u32 pairs take 1.11 ms, 3.87 TB/s of the 16 bytes per pair that a
-// pass cannot do without (a 4 GiB copy on the same card: 4.76 TB/s); 1.21 ms before the
+// pass cannot do without (a 1 GiB copy by the engine's kernel: 4.54 TB/s); 1.21 ms before the
 // ranking took fewer vector instructions (wave_peers), digit starts were folded into
 // one LDS read per element and values were loaded under the key writes.  u64 keys:
 // 3.37 ms for 2^29 pairs (3.72 before).

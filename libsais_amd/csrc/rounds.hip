@@ -1304,9 +1304,10 @@ __global__ __launch_bounds__(RT_THREADS) __attribute__((amdgpu_num_sgpr(96))) vo
     __syncthreads();
 
     // 6. survivors (counted in the low halves, their chain_gain in the high halves): output
-    //    ranks by position, their range reserved in this run's segment (one atomic on the run's counter).  A counter shared by all
-    //    workgroups serialises them: 300 K returning atomics on one address take
-    //    3.6 ms, on 8 addresses 0.57 ms; the XCDs work on a run each.
+    //    ranks by position, their range reserved in this run's segment (one atomic on the
+    //    run's counter).  A counter shared by all workgroups serialises them: 300 K
+    //    returning atomics on one address take 3.6 ms, on 8 addresses 0.57 ms; the XCDs work
+    //    on a run each.
     u32 cnt_s[RT_PER];
     u32 tot = 0;
 #pragma unroll
