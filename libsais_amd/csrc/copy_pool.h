@@ -250,7 +250,7 @@ struct CopyForm {
         return written(tiny ? 16u << 10 : bytes < COPY_MID || conv == 2 ? 128u << 10 : 512u << 10);
     }
     // and of one by DMA, in slots.
-    u64 slot_part() const { return tiny ? written(16u << 10) : shared ? 1u << 20 : 2u << 20; }
+    u64 slot_part() const { return tiny ? written(16u << 10) : 1u << 20; }
     // Room for the parts of a copy of `bytes`: every stretch that is granted may end in a
     // short one, and no part or stretch but the last is smaller than the least of any form.
     u64 room(u64 bytes) const

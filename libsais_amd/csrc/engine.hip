@@ -181,11 +181,12 @@ struct Timer {
 // Copies of COPY_LARGE and more pass through a ring of twice the size: uploads in 16 MiB
 // chunks with an event every 32 MiB (in the small ring the DMA runs dry whenever the ring is
 // full, since its first region is free only after an event behind all that is queued),
-// downloads by DMA.  libsais_lcp of 48,000,000 entries (three copies of 192 MB): 12.5 ->
-// 12.0 ms, of 128,000,000 32.4 -> 31.2 ms, of 12,000,000 3.43 -> 3.32 ms; at 38 MB the two
-// forms are equal.  (64-bit arrays wait for the threads that convert them, not for the bus.)
+// downloads with half as many starts of the kernel.  libsais_lcp of 48,000,000 entries
+// (three copies of 192 MB): 12.6 -> 12.1 ms, of 128,000,000 33.0 -> 31.8 ms, of 12,000,000
+// 3.41 -> 3.21 ms; at 38 MB the two forms are equal.  (64-bit arrays wait for the threads
+// that convert them, not for the bus.)
 constexpr u64 XS_RING = 32ull << 20, XS_RING_LARGE = 64ull << 20, XS_MARK = 32ull << 20;
-constexpr int XS_EVENTS = 8, XS_DOWN = 4;    // a download by DMA takes a quarter of its ring at a time
+constexpr int XS_EVENTS = 8, XS_DOWN = 4;    // a download by DMA takes a quarter of the ring at a time
 constexpr int XS_AHEAD = 24;                  // upload chunks whose host copies may run ahead of the DMA
 enum { XS_TODO = -1, XS_QUEUED = -2 };        // a region's DMA is not queued / queued, no event after it yet
 // 1: copies of at least XS_MIN bytes staged (default); 0: every copy direct; 2: every
@@ -1723,17 +1724,18 @@ __global__ __launch_bounds__(256) void k_push(const uint8_t *__restrict__ src, u
     }
 }
 
-// A download by a DMA per slot of the ring, then the slot's host copies: large copies (53
-// GB/s for 192 MB, where the kernel, started again and again, gives 50), and those while
-// other calls are under way, with whose kernels the push kernel would compete for the CUs.
-// The latter take small slots, and the work before them is waited for first: DMAs queued
-// behind it hold up the other calls' DMAs.  Calls of libsais and libsais_plcp in turn on 12
-// MB each, 8 pairs a thread, ms for 4 / 8 threads: 110 / 186 with four slots of 16 MiB, 94 /
-// 179 with the wait, 85 / 170 with slots of 8 MiB too.  300 served jobs (2.1 GB of text) at
-// once 240 -> 237 ms, into pages not touched before 262 -> 246.
+// A download by a DMA per slot of the ring, then the slot's host copies, while other calls
+// are under way, with whose kernels the push kernel would compete for the CUs.  Slots are
+// small, and the work before them is waited for first: DMAs queued behind it hold up the
+// other calls' DMAs.  Calls of libsais and libsais_plcp in turn on 12 MB each, 8 pairs a
+// thread, ms for 4 / 8 threads: 110 / 186 with four slots of 16 MiB, 94 / 179 with the wait,
+// 85 / 170 with slots of 8 MiB too.  300 served jobs (2.1 GB of text) at once 240 -> 237 ms,
+// into pages not touched before 262 -> 246.  Not for single calls: behind a build, DMAs run
+// at half their rate once the process has used several streams (libsais of 16 Mi symbols
+// after a server 3.9 ms, by the kernel 2.65).
 int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, const CopyForm &f)
 {
-    const u64 slot = (f.shared ? XS_RING : XS_RING_LARGE) / XS_DOWN, nb = (bytes + slot - 1) / slot;
+    const u64 slot = XS_RING / XS_DOWN, nb = (bytes + slot - 1) / slot;
     std::vector<int> upto(nb + 1, 0);   // parts through the end of every slot
     auto launch = [&](u64 b) -> int {
         const u64 off = b * slot, len = bytes - off < slot ? bytes - off : slot;
@@ -1766,14 +1768,14 @@ try {
     CopyPool::Job j(f.room(bytes));
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
-    if (f.large || f.shared) {
+    if (f.shared) {
         SAGPU_TRY(d2h_slots(c, j, dst, src, bytes, f));
         guard.fine = true;
         return SAGPU_OK;
     }
     volatile u32 *flags = (volatile u32 *)(c.xs + c.xs_cap);
     // two halves of the ring, a kernel each; a half is filled again once it is drained
-    const u64 half = XS_RING / 2, chunk = f.down_chunk(bytes);
+    const u64 half = (f.large ? XS_RING_LARGE : XS_RING) / 2, chunk = f.down_chunk(bytes);
     const u64 batch = chunk * (XP_CHUNKS / 2) < half ? chunk * (XP_CHUNKS / 2) : half;
     const u64 nb = (bytes + batch - 1) / batch;
     std::vector<int> upto(nb + 1, 0);   // parts through the end of every batch

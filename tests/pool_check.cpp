@@ -63,7 +63,7 @@ int copy_form(bool tiny, int conv, u64 entries, bool up, bool shared)
         len = bytes - off < len ? bytes - off : len;
         const bool ok = up ? pool.grant(j, {(uint8_t *)dev.data() + off, host + f.taken(off), len, conv}, f.up_part())
                            : pool.grant(j, {host + f.written(off), (const uint8_t *)dev.data() + off, f.written(len), conv},
-                                        f.shared || f.large ? f.slot_part() : f.down_part(bytes));
+                                        f.shared ? f.slot_part() : f.down_part(bytes));
         if (!ok) break;
         off += len;
     }
