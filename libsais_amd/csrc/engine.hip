@@ -1270,7 +1270,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
 
     bool queued = false, left = false;   // this round is on the stream already; its length is in rp
     u64 a_before = 0, gain = 0;          // the length of the round before, and what chains promise now
-    int chain_rounds = 0;
+    int chain_rounds = 0, big_run = 0;   // big_run: rounds with big groups since the last without
     while (a > 0) {
         const bool raw = st.rounds == 0 && rk1.pw;
         const bool lazy_first = lazy_a && st.rounds == 0;
@@ -1297,10 +1297,11 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr, chains));
             // Short rounds cost their launches and the host's wait: queue the next one
             // behind (its three kernels cost about 12 us when they find nothing to do,
-            // a wait and a late launch about 20).  Not after a round with big groups, which
-            // mostly come round after round: libsais of 400,000 equal bytes 2.77 ms with rounds
-            // queued in vain, 2.46 without.
-            ahead = (st.rounds == 0 || left) && (a < ROUND_AHEAD || lazy_first) && !c.timer.on;
+            // a wait and a late launch about 20).  Not after two rounds with big groups in a row,
+            // which mostly go on: libsais of 400,000 equal bytes 2.73 ms with rounds queued in
+            // vain, 2.47 without.  (After one, many texts have no more: libsais_int of 200,000
+            // symbols of 4 kinds 472 us with none queued then, 438 with.)
+            ahead = big_run < 2 && (a < ROUND_AHEAD || lazy_first) && !c.timer.on;
             if (ahead) {
                 st.rounds++;   // (a queued second round is one that replays a graph)
                 const int rc = launch(cur ^ 1, a, 0, false, false, nullptr);
@@ -1334,6 +1335,7 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             return SAGPU_EDEVICE;
         }
         left = nb == 0;                  // the next round's length is in rp
+        big_run = left ? 0 : big_run + 1;
         queued = ahead && left && out_n > 0;
         if (nb > 0) {
             // Big groups in the order k_big_sizes listed them (the outputs do not

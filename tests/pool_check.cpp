@@ -59,7 +59,7 @@ int copy_form(bool tiny, int conv, u64 entries, bool up, bool shared)
     pool.begin(j, 4);
     u64 off = 0;
     for (int k = 0; off < bytes; k++) {
-        u64 len = up ? f.up_chunk(k) : f.shared || f.large ? slot(f) : f.down_chunk(bytes);
+        u64 len = up ? f.up_chunk(k) : f.shared ? slot(f) : f.down_chunk(bytes);
         len = bytes - off < len ? bytes - off : len;
         const bool ok = up ? pool.grant(j, {(uint8_t *)dev.data() + off, host + f.taken(off), len, conv}, f.up_part())
                            : pool.grant(j, {host + f.written(off), (const uint8_t *)dev.data() + off, f.written(len), conv},
