@@ -222,6 +222,7 @@ struct CopyForm {
     int conv;
     bool shared;  // other calls are under way
     bool large;   // passes through the larger ring
+    bool dma;     // a download by DMA, in slots (else by a kernel, in chunks)
 
     u64 written(u64 bytes) const { return conv == 2 ? 2 * bytes : bytes; }   // by the host copies
     u64 taken(u64 bytes) const { return conv == 1 ? 2 * bytes : bytes; }     // from the caller's array
@@ -249,8 +250,8 @@ struct CopyForm {
     {
         return written(tiny ? 16u << 10 : bytes < COPY_MID || conv == 2 ? 128u << 10 : 512u << 10);
     }
-    // and of one by DMA, in slots.
-    u64 slot_part() const { return tiny ? written(16u << 10) : 1u << 20; }
+    // and of one beside other calls.
+    u64 shared_part() const { return tiny ? written(16u << 10) : 1u << 20; }
     // Room for the parts of a copy of `bytes`: every stretch that is granted may end in a
     // short one, and no part or stretch but the last is smaller than the least of any form.
     u64 room(u64 bytes) const

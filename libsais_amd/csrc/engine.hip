@@ -1538,7 +1538,9 @@ bool xs_ready(Ctx &c, u64 bytes, CopyForm *f, u64 least = XS_MIN)
     const int mode = g_host_staging.load();
     if (mode == 0 || (mode == 1 && bytes < least)) return false;
     f->tiny = mode == 2;
-    f->shared = g_calls.load() > 1;
+    const int calls = g_calls.load();
+    f->shared = calls > 1;
+    f->dma = calls > 2 || (f->shared && bytes < COPY_MID);   // see d2h_slots
     f->large = mode == 1 && (f->shared ? bytes >= COPY_SHARED_LARGE : f->conv == 0 && bytes >= COPY_LARGE);
     const u64 cap = f->large ? XS_RING_LARGE : XS_RING;
     if (c.xs_cap >= cap) return true;
@@ -1732,9 +1734,11 @@ __global__ __launch_bounds__(256) void k_push(const uint8_t *__restrict__ src, u
 // other calls' DMAs.  Calls of libsais and libsais_plcp in turn on 12 MB each, 8 pairs a
 // thread, ms for 4 / 8 threads: 110 / 186 with four slots of 16 MiB, 94 / 179 with the wait,
 // 85 / 170 with slots of 8 MiB too.  300 served jobs (2.1 GB of text) at once 240 -> 237 ms,
-// into pages not touched before 262 -> 246.  Not for single calls: behind a build, DMAs run
-// at half their rate once the process has used several streams (libsais of 16 Mi symbols
-// after a server 3.9 ms, by the kernel 2.65).
+// into pages not touched before 262 -> 246.  Not for single calls, nor for large copies beside
+// one other call: behind a build, DMAs run at half their rate once the process has used
+// several streams (libsais of 16 Mi symbols after a server 3.9 ms, by the kernel 2.65; two
+// threads in libsais and libsais_plcp, ms by DMAs / by the kernel: 24 M symbols 47 / 40, 12 M
+// 23.2 / 20.3, 9 M 19.6 / 17.5, but 4 M 7.8 / 9.0).
 int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, const CopyForm &f)
 {
     const u64 slot = XS_RING / XS_DOWN, nb = (bytes + slot - 1) / slot;
@@ -1750,7 +1754,7 @@ int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, c
     for (u64 b = 0; b < nb; b++) {
         const u64 off = b * slot, len = bytes - off < slot ? bytes - off : slot;
         SAGPU_CHECK(hipEventSynchronize(c.xs_down[b % XS_DOWN]));
-        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + b % XS_DOWN * slot, len, f.slot_part()));
+        SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off), c.xs + b % XS_DOWN * slot, len, f.shared_part()));
         upto[b + 1] = j.granted.load();
         if (b + XS_DOWN < nb) {
             copies().wait(j, upto[b + 1]);
@@ -1766,11 +1770,11 @@ int d2h_slots(Ctx &c, CopyPool::Job &j, void *dst, const void *src, u64 bytes, c
 // in dst.
 int d2h_staged(Ctx &c, void *dst, const void *src, u64 bytes, const CopyForm &f)
 try {
-    if (f.shared) SAGPU_CHECK(hipStreamSynchronize(c.stream));
+    if (f.dma) SAGPU_CHECK(hipStreamSynchronize(c.stream));
     CopyPool::Job j(f.room(bytes));
     copies().begin(j, copy_threads());
     XsGuard guard{c, j};
-    if (f.shared) {
+    if (f.dma) {
         SAGPU_TRY(d2h_slots(c, j, dst, src, bytes, f));
         guard.fine = true;
         return SAGPU_OK;
@@ -1811,7 +1815,8 @@ try {
             }
             std::atomic_thread_fence(std::memory_order_acquire);
             const u64 l = len - o < chunk ? len - o : chunk;
-            SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off + o), c.xs + side * half + o, l, f.down_part(bytes)));
+            SAGPU_TRY(xs_grant(j, f, (uint8_t *)dst + f.written(off + o), c.xs + side * half + o, l,
+                              f.shared ? f.shared_part() : f.down_part(bytes)));
         }
         upto[b + 1] = j.granted.load();
         // the half of batch b + 1 is being filled or drained; batch b + 2 needs this one
@@ -1830,7 +1835,7 @@ try {
 int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    CopyForm f{false, 0, false, false};
+    CopyForm f{false, 0, false, false, false};
     if (xs_ready(c, bytes, &f)) return h2d_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
     return SAGPU_OK;
@@ -1840,7 +1845,7 @@ int h2d(Ctx &c, void *dst, const void *src, u64 bytes)
 int d2h(Ctx &c, void *dst, const void *src, u64 bytes)
 {
     if (!bytes) return SAGPU_OK;
-    CopyForm f{false, 0, false, false};
+    CopyForm f{false, 0, false, false, false};
     if ((uintptr_t)src % 16 == 0 && xs_ready(c, bytes, &f)) return d2h_staged(c, dst, src, bytes, f);
     SAGPU_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
     return SAGPU_OK;
@@ -2062,7 +2067,7 @@ unsigned grid_n(u64 n)
 // Download u32 device array into an int32 or int64 host array.
 int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 {
-    CopyForm f{false, 2, false, false};
+    CopyForm f{false, 2, false, false, false};
     if (width == 4) {
         SAGPU_TRY(d2h(c, h, d, n * 4));
     } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {
@@ -2078,7 +2083,7 @@ int download_idx(Ctx &c, Scope &sc, const u32 *d, void *h, u64 n, int width)
 int upload_idx(Ctx &c, Scope &sc, const void *h, u64 n, int width, u32 **out)
 {
     GET(d, u32, n);
-    CopyForm f{false, 1, false, false};
+    CopyForm f{false, 1, false, false, false};
     if (width == 4) {
         SAGPU_TRY(h2d(c, d, h, n * 4));
     } else if (n && xs_ready(c, n * 4, &f, XS_MIN_INDEX64)) {

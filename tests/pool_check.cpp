@@ -37,14 +37,14 @@ namespace {
 
 CopyPool &pool = *new CopyPool;   // (its workers live as long as the process)
 // The stretch of a download by DMA: a slot of the staged copies' ring.
-u64 slot(const CopyForm &f) { return f.shared ? 8ull << 20 : 16ull << 20; }
+constexpr u64 SLOT = 8ull << 20;
 
 // Every form of a staged copy, in the stretches that the engine grants: its parts fit the
 // room that the job was given, and every entry arrives.
-int copy_form(bool tiny, int conv, u64 entries, bool up, bool shared)
+int copy_form(bool tiny, int conv, u64 entries, bool up, bool shared, bool dma = false)
 {
     const u64 bytes = 4 * entries;
-    const CopyForm f{tiny, conv, shared, !tiny && bytes >= (shared ? COPY_SHARED_LARGE : COPY_LARGE)};
+    const CopyForm f{tiny, conv, shared, !tiny && bytes >= (shared ? COPY_SHARED_LARGE : COPY_LARGE), dma};
     std::vector<u32> dev(entries);
     std::vector<int64_t> wide(entries);
     for (u64 i = 0; i < entries; i++) {
@@ -59,11 +59,11 @@ int copy_form(bool tiny, int conv, u64 entries, bool up, bool shared)
     pool.begin(j, 4);
     u64 off = 0;
     for (int k = 0; off < bytes; k++) {
-        u64 len = up ? f.up_chunk(k) : f.shared ? slot(f) : f.down_chunk(bytes);
+        u64 len = up ? f.up_chunk(k) : dma ? SLOT : f.down_chunk(bytes);
         len = bytes - off < len ? bytes - off : len;
         const bool ok = up ? pool.grant(j, {(uint8_t *)dev.data() + off, host + f.taken(off), len, conv}, f.up_part())
                            : pool.grant(j, {host + f.written(off), (const uint8_t *)dev.data() + off, f.written(len), conv},
-                                        f.shared ? f.slot_part() : f.down_part(bytes));
+                                        f.shared ? f.shared_part() : f.down_part(bytes));
         if (!ok) break;
         off += len;
     }
@@ -83,11 +83,11 @@ int forms()
     for (u64 n : sizes)
         for (int tiny = 0; tiny < 2; tiny++)
             for (int conv = 0; conv < 3; conv++)
-                for (int how = 0; how < 4; how++) {   // upload or download, alone or beside others
+                for (int how = 0; how < 5; how++) {   // upload or download, alone or beside others (4: by DMA)
                     const bool up = how < 2;
                     if (conv == (up ? 2 : 1)) continue;
                     if (n > 1u << 20 && tiny) continue;   // (the sizes of larger chunks and parts)
-                    if (copy_form(tiny != 0, conv, n, up, how % 2 != 0)) {
+                    if (copy_form(tiny != 0, conv, n, up, how % 2 != 0 || how == 4, how == 4)) {
                         printf("entries %llu, tiny %d, conv %d, way %d\n", n, tiny, conv, how);
                         return 1;
                     }

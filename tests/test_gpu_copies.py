@@ -134,11 +134,13 @@ def test_large_arrays(n, reset_staging):
         assert la.libsais_lcp(P[:k].copy(), small, L, k) == 0 and np.array_equal(L, P[:k][small])
 
 
-@pytest.mark.parametrize("n", [(2 << 20) - 1, 2 << 20, (5 << 20) + 3, (12 << 20) + 1])
-def test_large_arrays_at_once(n, reset_staging):
-    """Four callers with 32- and 64-bit arrays on both sides of 8 MiB, from where copies beside
-    other calls take the larger ring, and of several slots and chunks."""
-    print(f"[copies] large arrays at once, n={n}", flush=True)
+@pytest.mark.parametrize("n,callers", [((2 << 20) - 1, 4), (2 << 20, 4), ((5 << 20) + 3, 4), ((12 << 20) + 1, 4),
+                                       ((8 << 20) - 9, 2), (8 << 20, 2), ((12 << 20) + 1, 2)])
+def test_large_arrays_at_once(n, callers, reset_staging):
+    """Callers with 32- and 64-bit arrays on both sides of 8 MiB, from where copies beside other
+    calls take the larger ring, and of several slots and chunks; two of them on both sides of
+    32 MiB, from where their downloads take the kernel instead of DMAs."""
+    print(f"[copies] large arrays at once, n={n}, callers={callers}", flush=True)
     wrong = []
 
     def work(k):
@@ -157,7 +159,7 @@ def test_large_arrays_at_once(n, reset_staging):
         except Exception as e:  # pragma: no cover - reported below
             wrong.append((k, repr(e)))
 
-    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(callers)]
     for t in ts:
         t.start()
     for t in ts:
