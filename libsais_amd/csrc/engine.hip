@@ -1297,11 +1297,12 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr, chains));
             // Short rounds cost their launches and the host's wait: queue the next one
             // behind (its three kernels cost about 12 us when they find nothing to do,
-            // a wait and a late launch about 20).  Not after two rounds with big groups in a row,
-            // which mostly go on: libsais of 400,000 equal bytes 2.73 ms with rounds queued in
-            // vain, 2.47 without.  (After one, many texts have no more: libsais_int of 200,000
-            // symbols of 4 kinds 472 us with none queued then, 438 with.)
-            ahead = big_run < 2 && (a < ROUND_AHEAD || lazy_first) && !c.timer.on;
+            // a wait and a late launch about 20).  Not after three rounds with big groups in a row,
+            // which mostly go on: libsais of 500,000 equal bytes 2.73 ms with rounds queued in
+            // vain, 2.46 without.  (After one or two, many texts have no more: libsais_int of
+            // 200,000 symbols of 4 kinds 472 us with none queued after one, 438 with; 100,000
+            // bytes of words 606 us with none after two, 565 with.)
+            ahead = big_run < 3 && (a < ROUND_AHEAD || lazy_first) && !c.timer.on;
             if (ahead) {
                 st.rounds++;   // (a queued second round is one that replays a graph)
                 const int rc = launch(cur ^ 1, a, 0, false, false, nullptr);
