@@ -279,7 +279,7 @@ SAGPU_API int32_t sagpu_sort_pairs_u64(uint64_t *d_keys, uint32_t *d_vals, int64
  *                    with whole symbols per 8-bit digit, are derived from one histogram of the
  *                    stream's 8-bit windows (default); 0 = counted per pass
  *   "chain_min"      doubling rounds that follow one which left more than seven eighths of its list,
- *                    mostly in groups of two to four, compare small groups at the end of their
+ *                    mostly in small groups, compare those at the end of their
  *                    chains of shared repeats when the list has at least this many entries
  *                    (default 4096; 0 = never)
  *   "small_build"    1 = texts of at most 24 KiB are built by one workgroup in one kernel, while the

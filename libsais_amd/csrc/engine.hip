@@ -1285,14 +1285,18 @@ int sa_build(Ctx &c, Scope &sc, const uint8_t *dT, u64 n, int gsa, u32 *dSA, u32
             // 145 K instead of 9 rounds): 13.30 -> 12.76 ms.  At 3/4, 256 MiB of DNA with
             // diverged repeats (23.1 and 18.1 M, then 5.1 instead of 11.8 M) went from
             // 21.6 to 22.3 ms.  And it must consist of small groups: copies that end in
-            // different places cost a group one chain round for each.  308 texts of 2 and
-            // 32 Mi symbols with 2 to 20 copies of 300 to 30000 symbols, some inside one
-            // another or with mutations, against no chains: 0.93 of the time in the mean
-            // (0.44 to 1.19) from 7/16 of CHAIN_GAIN on, 0.96 from 9/16 on; with any groups up
-            // to CHAIN_GROUP 0.94 (0.44 to 1.20).  A second time takes what larger groups left.
+            // different places cost a group one chain round for each.  Pairs are sure to be done
+            // (7/16 of CHAIN_GAIN); where 63/64 of the list are left, copies are long and exact,
+            // and groups of up to 7 mostly end in one place (1/8).  308 texts of 2 and 32 Mi
+            // symbols with 2 to 20 copies of 300 to 30000 symbols, some inside one another or
+            // with mutations, against no chains: 0.922 of the time in the mean (0.44 to 1.18);
+            // 0.935 (to 1.19) without the second rule, 0.930 with it from 15/16 on, 0.924 from
+            // 127/128 on; 0.978 (to 1.33) with any list in groups up to CHAIN_GROUP.  A second
+            // time takes what larger groups left.
+            const bool small = 16 * gain >= 7 * CHAIN_GAIN * a ||
+                               (a > a_before / 64 * 63 && 8 * gain >= CHAIN_GAIN * a);
             chains = g_chain_min && left && st.rounds >= 2 && chain_rounds < 2 && a >= (u64)g_chain_min &&
-                     a > a_before / 8 * 7 && 16 * gain >= 7 * CHAIN_GAIN * a && chain_words(n) <= n &&
-                     n < 0xFFFFFF00ull;
+                     a > a_before / 8 * 7 && small && chain_words(n) <= n && n < 0xFFFFFF00ull;
             chain_rounds += chains;
             SAGPU_TRY(launch(cur, a, h, !left, raw, lazy_first ? ws.total : nullptr, chains));
             // Short rounds cost their launches and the host's wait: queue the next one
