@@ -707,3 +707,31 @@ def test_round_chains_mixed_groups(n):
         assert np.array_equal(gSA, SA) and np.array_equal(gP, P) and np.array_equal(gL, ol.lcp(P, SA)), least
     print(f"[chains] n={n}: {rounds} rounds", flush=True)
     assert rounds[0] < rounds[1]
+
+
+@pytest.mark.parametrize("copies", [3, 5, 7])
+@pytest.mark.parametrize("length", [9001, 40000])
+def test_round_chains_exact_copies(length, copies):
+    """Exact copies of one block in a random text: their groups of up to seven all end in one
+    place, and chains take them there."""
+    from tests.test_gpu_parity import fused
+    lib = la.load()
+    T = np.random.default_rng(length + copies).integers(97, 101, (length + 300) * copies).astype(np.uint8)
+    block = T[:length].copy()
+    for k in range(copies):
+        at = k * (length + 300) + 7 * k
+        T[at:at + length] = block
+    rounds = []
+    for least in (2, 0):
+        assert lib.sagpu_set_option(b"chain_min", least) == 0
+        try:
+            out = fused(T)
+            rounds.append(la.stats().rounds)
+        finally:
+            assert lib.sagpu_set_option(b"chain_min", 4096) == 0
+    print(f"[chains] {copies} copies of {length}: {rounds} rounds", flush=True)
+    rc, SA = ol.sa(T)
+    assert rc == 0
+    P = ol.plcp(T, SA)
+    assert np.array_equal(out[0], SA) and np.array_equal(out[3], P) and np.array_equal(out[4], ol.lcp(P, SA))
+    assert rounds[0] + 3 < rounds[1]
